@@ -103,15 +103,14 @@ __device__ __forceinline__ int ftlf() { return c_cfg.fgeo0 + NGEO; }
 // split into:
 //   saha_kernel  one thread per (height, column): partition functions and the
 //                Saha factors of all 92 elements -> sbuf[k][e][4][column]
-//   rho_group_kernel  eight lanes per column, heights bottom->top: only the
+//   rho_group_kernel  16 to 64 lanes per column, heights bottom->top: only the
 //                warm-started electron-density fixed point (GET_RHO), reading
 //                the factors from sbuf -> rho, mu, Pe and (n_e, N_H) per height
 //   opac_kernel  one thread per (height, column): implicit EOS derivatives,
 //                continuum and line opacity, damping -> the per-height record
 //   tau_kernel   one thread per column: the REAL(4) log tau5 trapezoid
 // FP64 throughout; the fixed point keeps the reference's iteration path
-// (stopping rule 1e-4, warm start), so the EOS outputs are those of the
-// sequential column loop.
+// (stopping rule 1e-4, warm start).
 struct MicroTile {
   int ncol, col0, ntile, der;
   float* atm;
@@ -145,136 +144,178 @@ __global__ void __launch_bounds__(256) saha_kernel(MicroTile a) {
   }
 }
 
-// GET_RHO for one column by a group of RHO_G lanes: lane q holds the Saha
-// factors of elements q, q + RHO_G, ... of the current height in registers
-// (loaded once per height, not once per iteration), evaluates their stage
-// populations, and every lane of the group folds the 91 terms in the
-// reference's order j = 1 .. 91 through cross-lane reads, so the fixed point
-// and its iteration path are those of get_rho bit for bit.  Eight lanes per
-// column give eight times the waves of one lane per column for the same
-// cube: the height recurrence is sequential, so the column count alone
-// cannot fill the SIMDs.
-constexpr int RHO_G = 8;
-constexpr int RHO_NS = (FZ_NELEM + RHO_G - 1) / RHO_G;
-// 32 columns per workgroup: the LDS rows of the groups (48.5 KB) fit three
-// workgroups per CU
-constexpr int RHO_BLOCK = 32 * RHO_G;
-
-// sh: this group's LDS rows, nii of element j at sh[j], niii at sh[RHO_LD + j],
-// ni of element 0 at sh[FZ_NELEM].  The lanes of a group belong to one wave,
-// whose LDS operations complete in program order, so the fold reads what the
-// stage pass wrote without a workgroup barrier.
-constexpr int RHO_LD = 96;
-// Row stride of the groups: the 64 / RHO_G groups of a wave read the same
-// element index of their own rows at once (every lane of a group the same
-// address, a broadcast); a stride of 2 RHO_LD + RHO_G / 4 doubles puts those
-// rows 32 / (64 / RHO_G) banks apart, so the reads of a wave hit distinct
-// banks instead of all one.
-constexpr int RHO_ROW = 2 * RHO_LD + RHO_G / 4;
-
-__device__ inline int get_rho_group(const double (&a1)[RHO_NS], const double (&a2)[RHO_NS], int q, double* sh,
-                                    double T, double PG, double& ne, double& nh, double& pelec, double& dens,
-                                    double& mu) {
-  const double kT = KBOL * T;
-  double n = ne;
-  if (n != n) n = 0.0;
-  if (n < 1.0) n = PG / (101.0 * kT);
-  pelec = n * kT;
-  if (pelec > PG) n = (PG * 0.5) / kT;
-  double err = 1.0, nnew = n, h = 0.0;
-  int iter = 1;
-  while (err > 1.0e-4 && iter <= 100 && h >= 0.0) {
-    const double nold = nnew;
-    h = (PG - nnew * kT) / (g_c.deno_sa * kT);
-#pragma unroll
-    for (int m = 0; m < RHO_NS; ++m) {
-      const int j = q + RHO_G * m;
-      if (j < FZ_NELEM) {
-        double ni, nii, niii;
-        stages(h * g_c.abfac[j], nnew, a1[m], a2[m], ni, nii, niii);
-        sh[j] = nii;
-        sh[RHO_LD + j] = niii;
-        if (j == 0) sh[FZ_NELEM] = ni;
-      }
-    }
-    __builtin_amdgcn_wave_barrier();
-    // the reference's fold: est = (niii_0 - ni_0) + (sum_{j>=1} nii_j) + (sum_{j>=1} niii_j)
-    double s2 = 0.0, s3 = 0.0;
-#pragma unroll 13
-    for (int j = 1; j < FZ_NELEM; ++j) {
-      s2 += sh[j];
-      s3 += sh[RHO_LD + j];
-    }
-    double est = sh[RHO_LD] - sh[FZ_NELEM];
-    __builtin_amdgcn_wave_barrier();
-    est = est + s2 + s3;
-    nnew = (fmax(est, 0.0) + nold) / 2.0;
-    err = fabs((nnew - nold) / nnew);
-    ++iter;
-  }
-  if (iter >= 100 || h < 0.0) return ERR_EOS;
-  n = nnew;
-  h = (PG - n * kT) / (g_c.deno_sa * kT);
-  dens = h * g_c.deno_sam + n * MELE;
-  mu = ((dens * kT) / MAMU) * (1.0 / PG);
-  if (h != h || n != n) return ERR_NAN;
-  if (n < 0.0 || h <= 0.0) return ERR_EOS;
-  ne = n;
-  nh = h;
-  return ERR_OK;
+// GET_RHO (chemical_equilibrium.f90:165-278) for one column by a group of G
+// lanes: lane q holds the Saha factors of elements q, q + G, ... of a height
+// in registers.  Per iteration an element adds
+//   abf (1 + i) / (x + 1 + i),  x = n_e a1, i = 1 / (n_e a2)
+// (n_II + n_III over N_H; hydrogen adds n_III - n_I, abf (i - x) / (x + 1 + i)),
+// one FP64 reciprocal where the reference's quotients (:1601-1652) take four
+// divisions, and no quotient that overflows before the fractions themselves
+// underflow.  1 / a2 is formed once per height and 1 / n_e once per iteration.
+//
+// The terms are summed by one fixed tree whatever G is: elements j and j + 64,
+// then residues 32, 16 and 8 apart, then 1, 2 and 4 apart, the levels below G
+// by cross-lane moves and the others within the lane.  Every group size thus
+// gives the same bits, so a column's result does not depend on the tile it
+// is launched in.
+//
+// Bound: the chain of one iteration (the reciprocals, the tree and the
+// stopping test), and with many columns the issue of its FP64 instructions.
+// Against the sequential fold of 91 terms through LDS with eight lanes per
+// column that this replaces: hydrostatic integration of 16 columns x 64
+// heights 8.9 -> 0.55 ms, of 9216 x 96 heights 26.9 -> 2.2 ms; the forward's
+// fixed point of 82944 columns x 96 heights 24.4 -> 6.5 ms.
+__device__ __forceinline__ double rcp64(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.0), r, r);
+  return fma(fma(-x, r, 1.0), r, r);
 }
 
-// get_rho_group on the factors of one height (base: [element][4][column]),
-// out of line so that a caller with several fixed points (the RK4 steps)
-// does not carry one unrolled copy of the element loop per call
-struct RhoOut {
-  double ne, nh, pel, dens, mu;
-  int err;
+template <int CTRL>
+__device__ __forceinline__ double dpp64(double x) {
+  const int lo = __double2loint(x), hi = __double2hiint(x);
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, hi, CTRL, 0xf, 0xf, true),
+                          __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xf, 0xf, true));
+}
+
+// x of a row of 16 lanes (of 32 lanes) plus x of its neighbour
+__device__ __forceinline__ double add_swap16(double x) {
+  const unsigned lo = (unsigned)__double2loint(x), hi = (unsigned)__double2hiint(x);
+  const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+  return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+}
+__device__ __forceinline__ double add_swap32(double x) {
+  const unsigned lo = (unsigned)__double2loint(x), hi = (unsigned)__double2hiint(x);
+  const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+  const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+  return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+}
+
+// the fixed tree over the lane's terms t[m] of elements q + G m
+template <int G, int NS>
+__device__ __forceinline__ double group_sum(double (&t)[NS]) {
+  constexpr int M = 64 / G;            // residues mod 64 held by a lane
+#pragma unroll
+  for (int m = 0; m + M < NS; ++m) t[m] += t[m + M];
+#pragma unroll
+  for (int w = M / 2; w > 0; w /= 2)
+#pragma unroll
+    for (int m = 0; m < w; ++m) t[m] += t[m + w];
+  double s = t[0];
+  if constexpr (G >= 64) s = add_swap32(s);
+  if constexpr (G >= 32) s = add_swap16(s);
+  if constexpr (G >= 16) s += dpp64<0x128>(s);   // row_ror:8
+  s += dpp64<0xB1>(s);                           // lanes 1 apart
+  s += dpp64<0x4E>(s);                           // 2 apart
+  s += dpp64<0x141>(s);                          // row_half_mirror: 4 apart, quads being uniform
+  return s;
+}
+
+template <int G>
+struct RhoGroup {
+  static constexpr int NS = (FZ_NELEM + G - 1) / G;
+  int q;
+  double ab[NS];   // abundances of the lane's elements (0 past the last one)
+  __device__ __forceinline__ explicit RhoGroup(int lane) : q(lane & (G - 1)) {
+#pragma unroll
+    for (int m = 0; m < NS; ++m) ab[m] = q + G * m < FZ_NELEM ? g_c.abfac[q + G * m] : 0.0;
+  }
+  // a1, a2 of a height; base: [element][4][stride] of the column
+  __device__ __forceinline__ void load(const double* __restrict__ base, long stride, double (&a1)[NS],
+                                       double (&a2)[NS]) const {
+#pragma unroll
+    for (int m = 0; m < NS; ++m) {
+      const int j = q + G * m;
+      a1[m] = j < FZ_NELEM ? base[(long)(j * 4 + 0) * stride] : 1.0;
+      a2[m] = j < FZ_NELEM ? base[(long)(j * 4 + 1) * stride] : 1.0;
+    }
+  }
+  static __device__ __forceinline__ void invert(double (&a2)[NS]) {
+#pragma unroll
+    for (int m = 0; m < NS; ++m) a2[m] = rcp64(a2[m]);
+  }
+  // the warm-started fixed point on a1 and ia2 = 1 / a2: the reference's
+  // iteration path (damping 1/2, stop at 1e-4, at most 100).  ne: start in,
+  // result out; pelec is the start's electron pressure, as the reference returns
+  __device__ __forceinline__ int solve(const double (&a1)[NS], const double (&ia2)[NS], double T, double PG,
+                                       double& ne, double& nh, double& pelec, double& dens, double& mu) const {
+    const double kT = KBOL * T;
+    double n = ne;
+    if (n != n) n = 0.0;
+    if (n < 1.0) n = PG / (101.0 * kT);
+    pelec = n * kT;
+    if (pelec > PG) n = (PG * 0.5) / kT;
+    const double isa = 1.0 / (g_c.deno_sa * kT);
+    double nnew = n, h = 0.0;
+    int iter = 1;
+    bool more = true;
+    while (more && iter <= 100 && h >= 0.0) {
+      const double nold = nnew, ine = rcp64(nold);
+      h = fma(-nold, kT, PG) * isa;
+      double t[NS];
+#pragma unroll
+      for (int m = 0; m < NS; ++m) {
+        const double x = nold * a1[m], i = ia2[m] * ine;
+        const double s = (m == 0 && q == 0) ? -x : 1.0;
+        t[m] = fma(ab[m], i, ab[m] * s) * rcp64((x + 1.0) + i);
+      }
+      const double est = h * group_sum<G, NS>(t);
+      nnew = (fmax(est, 0.0) + nold) * 0.5;
+      more = fabs(nnew - nold) > 1.0e-4 * fabs(nnew);
+      ++iter;
+    }
+    if (iter >= 100 || h < 0.0) return ERR_EOS;
+    n = nnew;
+    h = (PG - n * kT) / (g_c.deno_sa * kT);
+    dens = h * g_c.deno_sam + n * MELE;
+    mu = ((dens * kT) / MAMU) * (1.0 / PG);
+    if (h != h || n != n) return ERR_NAN;
+    if (n < 0.0 || h <= 0.0) return ERR_EOS;
+    ne = n;
+    nh = h;
+    return ERR_OK;
+  }
 };
 
-__device__ __noinline__ RhoOut rho_group_at(const double* __restrict__ base, long stride, int q, double* sh, double T,
-                                            double PG, double ne) {
-  double a1[RHO_NS], a2[RHO_NS];
-#pragma unroll
-  for (int m = 0; m < RHO_NS; ++m) {
-    const int j = q + RHO_G * m;
-    a1[m] = j < FZ_NELEM ? base[(long)(j * 4 + 0) * stride] : 1.0;
-    a2[m] = j < FZ_NELEM ? base[(long)(j * 4 + 1) * stride] : 1.0;
-  }
-  RhoOut o;
-  o.ne = ne;
-  o.err = get_rho_group(a1, a2, q, sh, T, PG, o.ne, o.nh, o.pel, o.dens, o.mu);
-  return o;
-}
+constexpr int RHO_BLOCK = 256;
 
-__global__ void __launch_bounds__(RHO_BLOCK) rho_group_kernel(MicroTile a) {
-  __shared__ double shall[RHO_BLOCK / RHO_G][RHO_ROW];
-  const int lane = threadIdx.x & 63;
-  const int q = lane & (RHO_G - 1);
-  double* sh = shall[threadIdx.x / RHO_G];
-  const int ct = (int)(((long)blockIdx.x * blockDim.x + threadIdx.x) / RHO_G);
+template <int G>
+__global__ void __launch_bounds__(RHO_BLOCK, G == 16 ? 3 : 4) rho_group_kernel(MicroTile a) {
+  using R = RhoGroup<G>;
+  const R g(threadIdx.x & 63);
+  const int ct = (int)(((long)blockIdx.x * blockDim.x + threadIdx.x) / G);
   const bool active = ct < a.ntile;
   // a group past the tile repeats the last column without writing, so that
   // every group of a wave runs the same code
   const int cc = active ? ct : a.ntile - 1;
+  const bool wr = active && g.q == 0;
   const int nz = c_cfg.nz, col = a.col0 + cc;
-  const long cs = a.ncol, ps = (long)nz * a.ncol;
+  const long cs = a.ncol, ps = (long)nz * a.ncol, hs = (long)FZ_NELEM * 4 * a.ntile;
+  const double* sb = a.sbuf + cc;
   double ne = 0.0;
   int err = ERR_OK;
+  // the next height's factors are loaded while this one iterates
+  double n1[R::NS], n2[R::NS];
+  g.load(sb, a.ntile, n1, n2);
+  float Tn = a.atm[A_T * ps + col], Pn = a.atm[A_PG * ps + col];
   for (int k = 0; k < nz; ++k) {
-    const double T = (double)a.atm[A_T * ps + k * cs + col], P = (double)a.atm[A_PG * ps + k * cs + col];
-    const double* sb = a.sbuf + (long)k * FZ_NELEM * 4 * a.ntile + cc;
-    double a1[RHO_NS], a2[RHO_NS];
+    const double T = (double)Tn, P = (double)Pn;
+    double a1[R::NS], ia2[R::NS];
 #pragma unroll
-    for (int m = 0; m < RHO_NS; ++m) {
-      const int j = q + RHO_G * m;
-      a1[m] = j < FZ_NELEM ? sb[(long)(j * 4 + 0) * a.ntile] : 1.0;
-      a2[m] = j < FZ_NELEM ? sb[(long)(j * 4 + 1) * a.ntile] : 1.0;
+    for (int m = 0; m < R::NS; ++m) {
+      a1[m] = n1[m];
+      ia2[m] = n2[m];
     }
+    const int kn = min(k + 1, nz - 1);
+    g.load(sb + kn * hs, a.ntile, n1, n2);
+    Tn = a.atm[A_T * ps + kn * cs + col];
+    Pn = a.atm[A_PG * ps + kn * cs + col];
+    R::invert(ia2);
     double nh, pel, dens, mu;
-    err = get_rho_group(a1, a2, q, sh, T, P, ne, nh, pel, dens, mu);
+    err = g.solve(a1, ia2, T, P, ne, nh, pel, dens, mu);
     if (err) break;
-    if (active && q == 0) {
+    if (wr) {
       a.atm[A_RHO * ps + k * cs + col] = (float)dens;
       a.atm[A_MU * ps + k * cs + col] = (float)mu;
       a.atm[A_PEL * ps + k * cs + col] = (float)pel;
@@ -282,7 +323,7 @@ __global__ void __launch_bounds__(RHO_BLOCK) rho_group_kernel(MicroTile a) {
       a.eos[((long)nz + k) * a.ntile + cc] = nh;
     }
   }
-  if (active && q == 0) a.status[col] = err;
+  if (wr) a.status[col] = err;
 }
 
 // The implicit EOS derivatives (GET_DNHYDDTEMP and its four solves,
@@ -413,7 +454,7 @@ __global__ void __launch_bounds__(64) tau_kernel(MicroTile a) {
 // RK4_INTEGRATION_LOG (hydrostatic_tools.f90:150-222, RK4_LOG :350-396) over
 // a tile: the Saha factors at the heights come from saha_kernel, those at the
 // RK4 mid-step temperatures from saha_mid_kernel, and he_rk4_group_kernel
-// (eight lanes per column, top -> bottom) runs only the fixed points.
+// (16 to 64 lanes per column, top -> bottom) runs only the fixed points.
 __device__ __forceinline__ double he_tmid(int k, double tm0, double tm1) {
   const double dz = c_cfg.he_dz[k];
   return tm0 / dz * c_cfg.he_a[k] + tm1 / dz * c_cfg.he_b[k];
@@ -439,28 +480,20 @@ __global__ void __launch_bounds__(256) saha_mid_kernel(MicroTile a, double* __re
   }
 }
 
-__device__ __forceinline__ double he_step_rhs_group(const double* base, long stride, int q, double* sh, double lnp,
-                                                    double tem, double& nel, int& err) {
-  const RhoOut o = rho_group_at(base, stride, q, sh, tem, exp(lnp), nel);
-  nel = o.ne;
-  if (o.err) err = o.err;
-  return -o.mu * MAMU * GRAV / (KBOL * tem);        // RK4_SOLVE_LOG (hydrostatic_tools.f90:53-71)
-}
-
-// RK4_INTEGRATION_LOG by groups of RHO_G lanes per column, each fixed point as
-// get_rho_group (the values of the one-thread get_rho, bit for bit); the
-// integration scalars are identical in the lanes of a group.  Writes Pg, rho,
-// Pe, mu of every height and, for the forward, (n_e, N_H) with n_e = Pe/(k T)
-// from the REAL(4) Pe and T (forward.f90:904).
-__global__ void __launch_bounds__(RHO_BLOCK) he_rk4_group_kernel(MicroTile a, const double* __restrict__ smid) {
-  __shared__ double shall[RHO_BLOCK / RHO_G][RHO_ROW];
-  const int lane = threadIdx.x & 63;
-  const int q = lane & (RHO_G - 1);
-  double* sh = shall[threadIdx.x / RHO_G];
-  const int ct = (int)(((long)blockIdx.x * blockDim.x + threadIdx.x) / RHO_G);
+// RK4_INTEGRATION_LOG by groups of G lanes per column, each fixed point as in
+// rho_group_kernel; the integration scalars are identical in the lanes of a
+// group.  The factors of height k + 1 (first step) are those of the previous
+// height's last two; the mid-step and the new height's are loaded a height
+// ahead.  Writes Pg, rho, Pe, mu of every height and, for the forward, (n_e, N_H) with
+// n_e = Pe/(k T) from the REAL(4) Pe and T (forward.f90:904).
+template <int G>
+__global__ void __launch_bounds__(RHO_BLOCK, 2) he_rk4_group_kernel(MicroTile a, const double* __restrict__ smid) {
+  using R = RhoGroup<G>;
+  const R g(threadIdx.x & 63);
+  const int ct = (int)(((long)blockIdx.x * blockDim.x + threadIdx.x) / G);
   const bool active = ct < a.ntile;
   const int cc = active ? ct : a.ntile - 1;
-  const bool wr = active && q == 0;
+  const bool wr = active && g.q == 0;
   const int nz = c_cfg.nz, col = a.col0 + cc;
   const long cs = a.ncol, ps = (long)nz * a.ncol;
   const long hs = (long)FZ_NELEM * 4 * a.ntile;
@@ -471,11 +504,19 @@ __global__ void __launch_bounds__(RHO_BLOCK) he_rk4_group_kernel(MicroTile a, co
   const int top = nz - 1;
   double u0 = log((double)A(A_PG, top));
   double nel = (double)A(A_PEL, top) / KBOL / (double)A(A_T, top);
-  double nh, pel, dens, mw;
+  double nh = 0.0, pel = 0.0, dens = 0.0, mw = 0.0;
+  // factors (a1, 1/a2) of the height above, of the mid step and of the new height
+  double h1[R::NS], h2[R::NS], m1[R::NS], m2[R::NS], k1a[R::NS], k2a[R::NS];
+  double pm1[R::NS], pm2[R::NS], pk1[R::NS], pk2[R::NS];
+  g.load(SH + top * hs, a.ntile, h1, h2);
   {
-    const RhoOut o = rho_group_at(SH + top * hs, a.ntile, q, sh, (double)A(A_T, top), exp(u0), nel);
-    nel = o.ne, nh = o.nh, pel = o.pel, dens = o.dens, mw = o.mu, err = o.err;
+    const int kn = max(top - 1, 0);
+    g.load(SM + kn * hs, a.ntile, pm1, pm2);
+    g.load(SH + kn * hs, a.ntile, pk1, pk2);
   }
+  R::invert(h2);
+  double tm0 = (double)A(A_T, top);
+  err = g.solve(h1, h2, tm0, exp(u0), nel, nh, pel, dens, mw);
   if (wr) {
     A(A_PG, top) = (float)exp(u0);
     A(A_RHO, top) = (float)dens;
@@ -483,25 +524,49 @@ __global__ void __launch_bounds__(RHO_BLOCK) he_rk4_group_kernel(MicroTile a, co
     A(A_MU, top) = (float)mw;
     if (a.eos) a.eos[((long)nz + top) * a.ntile + cc] = nh;
   }
+  // RK4_SOLVE_LOG (hydrostatic_tools.f90:53-71)
+  auto rhs = [&](const double (&f1)[R::NS], const double (&f2)[R::NS], double lnp, double tem) -> double {
+    double mu = 0.0;
+    const int e = g.solve(f1, f2, tem, exp(lnp), nel, nh, pel, dens, mu);
+    if (e) err = e;
+    return -mu * MAMU * GRAV / (KBOL * tem);
+  };
   for (int k = nz - 2; k >= 0 && !err; --k) {
     const double dz = c_cfg.he_dz[k];
-    const double tm0 = (double)A(A_T, k + 1), tm1 = (double)A(A_T, k);
-    const double k1 = he_step_rhs_group(SH + (k + 1) * hs, a.ntile, q, sh, u0, tm0, nel, err) * dz;
-    const double tmid = he_tmid(k, tm0, tm1);
-    const double k2 = he_step_rhs_group(SM + k * hs, a.ntile, q, sh, u0 + k1 / 2.0, tmid, nel, err) * dz;
-    const double k3 = he_step_rhs_group(SM + k * hs, a.ntile, q, sh, u0 + k2 / 2.0, tmid, nel, err) * dz;
-    const double k4 = he_step_rhs_group(SH + k * hs, a.ntile, q, sh, u0 + k3, tm1, nel, err) * dz;
-    const double u1 = u0 + 1.0 / 6.0 * (k1 + 2.0 * k2 + 2.0 * k3 + k4);
-    const RhoOut o = rho_group_at(SH + k * hs, a.ntile, q, sh, tm1, exp(u1), nel);
-    nel = o.ne, nh = o.nh, pel = o.pel, dens = o.dens, mw = o.mu;
-    if (o.err) err = o.err;
+    const double tm1 = (double)A(A_T, k), tmid = he_tmid(k, tm0, tm1);
+#pragma unroll
+    for (int m = 0; m < R::NS; ++m) {
+      m1[m] = pm1[m];
+      m2[m] = pm2[m];
+      k1a[m] = pk1[m];
+      k2a[m] = pk2[m];
+    }
+    const int kn = max(k - 1, 0);
+    g.load(SM + kn * hs, a.ntile, pm1, pm2);
+    g.load(SH + kn * hs, a.ntile, pk1, pk2);
+    const double s1 = rhs(h1, h2, u0, tm0) * dz;
+    R::invert(m2);
+    const double s2 = rhs(m1, m2, u0 + s1 / 2.0, tmid) * dz;
+    const double s3 = rhs(m1, m2, u0 + s2 / 2.0, tmid) * dz;
+    R::invert(k2a);
+    const double s4 = rhs(k1a, k2a, u0 + s3, tm1) * dz;
+    const double u1 = u0 + 1.0 / 6.0 * (s1 + 2.0 * s2 + 2.0 * s3 + s4);
+    const double pg = exp(u1);
+    const int e = g.solve(k1a, k2a, tm1, pg, nel, nh, pel, dens, mw);
+    if (e) err = e;
     if (wr) {
-      A(A_PG, k) = (float)exp(u1);
+      A(A_PG, k) = (float)pg;
       A(A_RHO, k) = (float)dens;
       A(A_PEL, k) = (float)pel;
       A(A_MU, k) = (float)mw;
       if (a.eos) a.eos[((long)nz + k) * a.ntile + cc] = nh;
     }
+#pragma unroll
+    for (int m = 0; m < R::NS; ++m) {
+      h1[m] = k1a[m];
+      h2[m] = k2a[m];
+    }
+    tm0 = tm1;
     u0 = u1;
   }
   if (a.eos && wr)
@@ -1076,8 +1141,7 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(const float* __restrict__ a
 // (normalization.f90:696-754): the EOS of every HSRA height warm-started
 // from the height below, as GET_RHO runs it there.  The Saha factors of all
 // heights and elements are independent (one thread each), the fixed point is
-// sequential in height (one group of RHO_G lanes, the fold in the
-// reference's order, so the iteration path is get_rho's bit for bit), and the
+// sequential in height (the 64 lanes of one wave), and the
 // opacities are independent again (one thread per height and region).
 __global__ void __launch_bounds__(256) hsra_saha_kernel(double* __restrict__ sb /*[387][92][4]*/) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1094,26 +1158,33 @@ __global__ void __launch_bounds__(256) hsra_saha_kernel(double* __restrict__ sb 
 
 __global__ void __launch_bounds__(64) hsra_rho_kernel(const double* __restrict__ sb, double* __restrict__ eos /*[2][387]*/,
                                                       int32_t* __restrict__ err_out /*[2]: code, first bad height*/) {
-  __shared__ double sh[RHO_ROW];
-  const int q = threadIdx.x;
-  if (q >= RHO_G) return;
+  using R = RhoGroup<64>;
+  const R g(threadIdx.x);
   double ne = 0.0;
   int err = ERR_OK, kbad = FZ_HSRA_LEN;
+  double n1[R::NS], n2[R::NS];
+  g.load(sb, 1, n1, n2);
   for (int k = 0; k < FZ_HSRA_LEN; ++k) {
-    const RhoOut o = rho_group_at(sb + (long)k * FZ_NELEM * 4, 1, q, sh, (double)fz_hsra_t[k],
-                                  (double)fz_hsra_pg[k], ne);
-    if (o.err) {
-      err = o.err;
+    double a1[R::NS], ia2[R::NS];
+#pragma unroll
+    for (int m = 0; m < R::NS; ++m) {
+      a1[m] = n1[m];
+      ia2[m] = n2[m];
+    }
+    g.load(sb + (long)min(k + 1, FZ_HSRA_LEN - 1) * FZ_NELEM * 4, 1, n1, n2);
+    R::invert(ia2);
+    double nh, pel, dens, mu;
+    err = g.solve(a1, ia2, (double)fz_hsra_t[k], (double)fz_hsra_pg[k], ne, nh, pel, dens, mu);
+    if (err) {
       kbad = k;
       break;
     }
-    ne = o.ne;
-    if (q == 0) {
-      eos[k] = o.ne;
-      eos[FZ_HSRA_LEN + k] = o.nh;
+    if (g.q == 0) {
+      eos[k] = ne;
+      eos[FZ_HSRA_LEN + k] = nh;
     }
   }
-  if (q == 0) {
+  if (g.q == 0) {
     err_out[0] = err;
     err_out[1] = kbad;
   }
@@ -1957,7 +2028,7 @@ static int launch_rt(fz_ctx* c, int rf_mode, const RtArgs& a, hipStream_t st, in
 // EOS takes N_H and n_e from that integration; with physics == false only the
 // hydrostatic integration runs (fz_hydrostatic_dev).
 // Microphysics tile when none is set: the electron-density fixed point is
-// sequential in height, one thread per column, so a tile should hold as many
+// sequential in height, a few lanes per column, so a tile should hold as many
 // columns as memory allows (up to a quarter of the free memory, at most
 // 64 GiB, for the Saha factors and the EOS buffers of every column).
 static int auto_mtile(fz_ctx* c, bool hydro) {
@@ -1970,6 +2041,19 @@ static int auto_mtile(fz_ctx* c, bool hydro) {
   const size_t m = budget / per_col;
   return (int)std::max<size_t>(4096, std::min<size_t>(m, 1 << 20));
 }
+
+// Lanes per column of the fixed-point kernels for a tile of n columns: as
+// many as keep about one wave per SIMD (1024), since a column's heights are a
+// chain and only more columns or more lanes fill the card; beyond, 16, whose
+// issue per column is lowest without spilling (8 lanes hold 12 elements each:
+// 262 registers).  64 heights, hydrostatic integration / forward without
+// response functions, ms:
+//   columns   64 lanes      32 lanes      16 lanes
+//      1024   0.57 / 0.54   0.59 / 0.54   0.70 / 0.58
+//      2048   0.88 / 0.65   0.68 / 0.60   0.79 / 0.65
+//      4096   1.49 / 0.95   1.09 / 0.83   0.98 / 0.82
+//     16384   5.76 / 3.60   3.88 / 2.33   3.26 / 2.07
+static int rho_lanes(int n) { return n <= 1024 ? 64 : n <= 3072 ? 32 : 16; }
 
 // the second stream and n ordering events of the overlapped forward
 static int ensure_aux(fz_ctx* c, int n) {
@@ -2025,13 +2109,18 @@ static int run_micro(fz_ctx* c, int ncol, float* d_atm, int32_t** status, bool d
       const long nmt = (long)(nz - 1) * a.ntile;
       hipLaunchKernelGGL(saha_mid_kernel, dim3((unsigned)((nmt + 255) / 256)), dim3(256), 0, st, a,
                          (double*)c->d_smid);
-      hipLaunchKernelGGL(he_rk4_group_kernel, dim3((unsigned)(((long)a.ntile * RHO_G + RHO_BLOCK - 1) / RHO_BLOCK)),
-                         dim3(RHO_BLOCK), 0,
-                         st, a, (const double*)c->d_smid);
+    }
+    const int gl = rho_lanes(a.ntile);
+    const dim3 gr((unsigned)(((long)a.ntile * gl + RHO_BLOCK - 1) / RHO_BLOCK)), gb(RHO_BLOCK);
+    const double* sm = (const double*)c->d_smid;
+    if (hydro) {
+      if (gl == 16) hipLaunchKernelGGL(he_rk4_group_kernel<16>, gr, gb, 0, st, a, sm);
+      else if (gl == 32) hipLaunchKernelGGL(he_rk4_group_kernel<32>, gr, gb, 0, st, a, sm);
+      else hipLaunchKernelGGL(he_rk4_group_kernel<64>, gr, gb, 0, st, a, sm);
     } else {
-      hipLaunchKernelGGL(rho_group_kernel, dim3((unsigned)(((long)a.ntile * RHO_G + RHO_BLOCK - 1) / RHO_BLOCK)),
-                         dim3(RHO_BLOCK), 0, st,
-                         a);
+      if (gl == 16) hipLaunchKernelGGL(rho_group_kernel<16>, gr, gb, 0, st, a);
+      else if (gl == 32) hipLaunchKernelGGL(rho_group_kernel<32>, gr, gb, 0, st, a);
+      else hipLaunchKernelGGL(rho_group_kernel<64>, gr, gb, 0, st, a);
     }
     if (physics) {
       if (a.der) hipLaunchKernelGGL(deriv_kernel, dim3((unsigned)((nkt + 255) / 256)), dim3(256), 0, st, a);

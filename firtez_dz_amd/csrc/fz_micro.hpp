@@ -57,17 +57,11 @@ __device__ __forceinline__ void partition(int elem, double T, double u[3], doubl
   partition_gen(elem, T, u, du);
 }
 
-// Saha factors of every element at one temperature (the quantities each
-// ION_CALC_* routine forms, chemical_equilibrium.f90:1601-1652).  Held in the
-// thread's private segment: lanes are interleaved there, so the per-element
-// loops below read them coalesced.
-struct Saha {
-  double a1[FZ_NELEM], a2[FZ_NELEM], da1[FZ_NELEM], da2[FZ_NELEM];
-};
-
-// The same four per-element rows read from a device buffer laid out
-// [height][element][4][column] (columns fastest), as the parallel Saha
-// kernel writes them: row q of element j at p[(j*4 + q) * stride].
+// Saha factors (the quantities each ION_CALC_* routine forms,
+// chemical_equilibrium.f90:1601-1652): a1, a2 and their T derivatives per
+// element, read from a device buffer laid out [height][element][4][column]
+// (columns fastest), as the parallel Saha kernel writes them: row q of
+// element j at p[(j*4 + q) * stride].
 struct SahaRow {
   const double* p;
   long st;
@@ -80,7 +74,7 @@ struct SahaView {
         da2{base + 3 * stride, 4 * stride} {}
 };
 
-// Saha factors of one element at temperature T (the loop body of saha_init)
+// Saha factors of one element at temperature T
 __device__ __forceinline__ void saha_element(int i, double T, double lam, double dlam, bool der, double& a1,
                                              double& a2, double& da1, double& da2) {
   double u[3], du[3];
@@ -98,29 +92,6 @@ __device__ __forceinline__ void saha_element(int i, double T, double lam, double
   }
 }
 
-__device__ inline void saha_init(Saha& s, double T, bool der) {
-  const double lam = g_c.csaha1 * pow(T, -1.5);
-  const double dlam = -3.0 / (2.0 * T);
-#pragma unroll 1
-  for (int i = 0; i < FZ_NELEM; ++i) {
-    double a1, a2, da1, da2;
-    saha_element(i, T, lam, dlam, der, a1, a2, da1, da2);
-    s.a1[i] = a1;
-    s.a2[i] = a2;
-    if (der) {
-      s.da1[i] = da1;
-      s.da2[i] = da2;
-    }
-  }
-}
-
-__device__ __forceinline__ void stages(double N, double ne, double a1, double a2,
-                                       double& ni, double& nii, double& niii) {
-  ni = N / (1.0 + (1.0 / (ne * a1)) * (1.0 + (1.0 / (ne * a2))));
-  nii = N / (ne * a1 + 1.0 + (1.0 / (ne * a2)));
-  niii = N / (1.0 + ne * a2 * (ne * a1 + 1.0));
-}
-
 // DERIVVAR scalars (derivvar.f90:16-24) needed downstream
 struct Deriv {
   double nh_T_pg, nh_T_rho, nh_pg_T, nh_rho_T;
@@ -128,48 +99,6 @@ struct Deriv {
 };
 
 enum : int { ERR_OK = 0, ERR_EOS = 1, ERR_NAN = 2, ERR_ION = 3, ERR_LAMBDA = 4 };
-
-// GET_RHO (chemical_equilibrium.f90:165-278).  ne: warm start in, result out.
-// pelec is the starting guess's electron pressure, as the reference returns.
-template <class S>
-__device__ inline int get_rho(const S& s, double T, double PG, double& ne, double& nh,
-                              double& pelec, double& dens, double& mu) {
-  const double kT = KBOL * T;
-  double n = ne;
-  if (n != n) n = 0.0;
-  if (n < 1.0) n = PG / (101.0 * kT);
-  pelec = n * kT;
-  if (pelec > PG) n = (PG * 0.5) / kT;
-  double err = 1.0, nnew = n, h = 0.0;
-  int iter = 1;
-  while (err > 1.0e-4 && iter <= 100 && h >= 0.0) {
-    const double nold = nnew;
-    h = (PG - nnew * kT) / (g_c.deno_sa * kT);
-    double ni, nii, niii;
-    stages(h * g_c.abfac[0], nnew, s.a1[0], s.a2[0], ni, nii, niii);
-    double est = niii - ni, s2 = 0.0, s3 = 0.0;
-#pragma unroll 7
-    for (int j = 1; j < FZ_NELEM; ++j) {
-      stages(h * g_c.abfac[j], nnew, s.a1[j], s.a2[j], ni, nii, niii);
-      s2 += nii;
-      s3 += niii;
-    }
-    est = est + s2 + s3;
-    nnew = (fmax(est, 0.0) + nold) / 2.0;
-    err = fabs((nnew - nold) / nnew);
-    ++iter;
-  }
-  if (iter >= 100 || h < 0.0) return ERR_EOS;
-  n = nnew;
-  h = (PG - n * kT) / (g_c.deno_sa * kT);
-  dens = h * g_c.deno_sam + n * MELE;
-  mu = ((dens * kT) / MAMU) * (1.0 / PG);
-  if (h != h || n != n) return ERR_NAN;
-  if (n < 0.0 || h <= 0.0) return ERR_EOS;
-  ne = n;
-  nh = h;
-  return ERR_OK;
-}
 
 // The four implicit-derivative solves of GET_DNHYDDTEMP
 // (chemical_equilibrium.f90:2008-2052), each a sum over the 92 elements of
@@ -179,8 +108,7 @@ __device__ inline int get_rho(const S& s, double T, double PG, double& ne, doubl
 // common denominator), and the reference's 1/g1, 1/g2, 1/g3 of GET_DNE_PG are
 // x y / D, y / D, 1 / D: one reciprocal per element instead of about twenty
 // FP64 divisions.  Same mathematics as the reference's expressions; the
-// values differ from them only in FP64 rounding (these are derivatives: the
-// EOS values themselves come from get_rho in the reference's operation order).
+// values differ from them only in FP64 rounding.
 template <class S>
 __device__ inline void eos_derivatives(const S& s, double T, double P, double RHO, double NE,
                                        Deriv& d) {
