@@ -45,25 +45,39 @@ constexpr int RF_CART_TBV = 4;
 constexpr int RT_WAVE = 64;   // wavelengths per radiative-transfer workgroup (one wave)
 constexpr int NATM = 12;
 enum { A_T = 0, A_PG, A_RHO, A_PEL, A_MU, A_BX, A_BY, A_BZ, A_VX, A_VY, A_VZ, A_TAU };
-enum { F_FLAG = 0, F_KC5 = 1, F_REG = 2 };
 
-// per-height record fields after the opacities: the field geometry (Geo,
-// seven floats) and 1/sqrt(T)
-constexpr int NGEO = 8;
+// Per-height record of a column, rec floats at micro[(k * ncol + col) * rec]:
+// a head of REC_HEAD floats, then per region REC_REG floats and REC_SLOT per
+// line of the region, each part a whole number of float4, so that a wave
+// copies the heights it needs next into LDS with 16-byte loads and every lane
+// reads them from there.  kappa_5000 is kept apart, [nz][ncol] after the
+// records (tau_kernel reads it along the columns).
+//   head    flag, T, 1/T, 1/sqrt(T) | v_z, |B|, sgf/2, cgf/4 | qf/2, qf/4, cg/2, sg |
+//           cos 2phi, sin 2phi, sg cg, line-optical-depth factor | d|B|/dB (3), d gamma/dB (3), d phi/dBx, dBy
+//           (sgf, cgf = 1 -+ cos^2 of the inclination; qf = sgf, 0 without a transverse field, whose frame is unturned)
+//   region  kappa_c and its three derivatives
+//   slot    kl, a, dkl/dT, da/dT | dkl/dPg, dkl/drho, da/dPg, da/drho | VoigtPoly (13) | 1/Doppler width,
+//           -1/(Doppler temperature), Doppler shift (mA)
+constexpr int REC_HEAD = 24, REC_REG = 4, REC_SLOT = 24;
 
 struct Cfg {
-  int nlines, nreg, nslot, numw, nz, nfield;
-  int fgeo0;            // first geometry field of the per-height record
+  int nlines, nreg, nslot, numw, nz;
+  int rec;              // floats of a per-height record
   LineConst line[MAXL];
   float dopfac[MAXL];   // Doppler width (mA) = dopfac * sqrt(T)
   float idopfac[MAXL];  // 1 / dopfac
   float vfac[MAXL];     // Doppler shift (mA) = vfac * v_z   (absorption_matrix.f90:1896)
   int reg_nblend[MAXR], reg_slot0[MAXR], reg_pix0[MAXR], reg_nwave[MAXR];
+  int reg_rec[MAXR];    // first float of the region in the per-height record
   double reg_wstart[MAXR], reg_wstep[MAXR], reg_l0main[MAXR];
   int slot_line[MAXS];
   float slot_bldiff[MAXS];
-  int comp0[MAXL], ntype[MAXL][3];   // components sorted sigma_r, pi, sigma_b
-  float comp_shift[MAXC], comp_str[MAXC];
+  // Zeeman components sorted sigma_r, pi, sigma_b (those of no strength left
+  // out): shift from the type's centre, strength and its products with the
+  // shift and its square; per type the strength-weighted centre and the sums
+  // of strength and strength * shift over sqrt(pi)
+  int comp0[MAXL], ntype[MAXL][3];
+  float4 comp[MAXC], type[MAXL][3];
   float dz_cm[MAXNZ];
   double zz[MAXNZ];    // heights in km, rounded through REAL(4) like MODEL(:,13)
   // radiative-transfer workgroups of one column: each covers up to RT_WAVE
@@ -87,13 +101,6 @@ struct Cfg {
   float xi_tf[MAXL];
 };
 __constant__ Cfg c_cfg;
-
-__device__ __forceinline__ int fslot(int s, int q) { return F_REG + 4 * c_cfg.nreg + 8 * s + q; }
-__device__ __forceinline__ int freg(int r, int q) { return F_REG + 4 * r + q; }
-__device__ __forceinline__ int fgeo(int q) { return c_cfg.fgeo0 + q; }
-// 1 / (N_H m_u MW) of a height whose opacities are formed, 0 where the height
-// is opaque (LINE OPTICAL DEPTH: KLINTAU = ETAI / N_H / m_u / MW)
-__device__ __forceinline__ int ftlf() { return c_cfg.fgeo0 + NGEO; }
 
 // ---------------------------------------------------------------- microphysics
 // FORWARD1D's per-height physics (forward.f90:911-1006) over a tile of
@@ -360,19 +367,27 @@ __global__ void __launch_bounds__(256) opac_kernel(MicroTile a) {
   const int k = (int)(t / a.ntile), ct = (int)(t - (long)k * a.ntile), col = a.col0 + ct;
   if (a.status[col] != 0) return;
   const long cs = a.ncol, ps = (long)nz * a.ncol;
-  auto M = [&](int f) -> float& { return a.micro[f * ps + k * cs + col]; };
+  float4* const R = reinterpret_cast<float4*>(a.micro + ((long)k * a.ncol + col) * c_cfg.rec);
+  const float* at = a.atm + k * cs + col;
+  const float Tf = at[A_T * ps], vz = at[A_VZ * ps], iT = 1.0f / Tf, rsT = rsqrtf(Tf);
   {
-    // FP32 field geometry and 1/sqrt(T) for the radiative transfer
-    const float* at = a.atm + k * cs + col;
-    const Geo g = geometry(at[A_BX * ps], at[A_BY * ps], at[A_BZ * ps]);
-    M(fgeo(0)) = g.B;
-    M(fgeo(1)) = g.cg;
-    M(fgeo(2)) = g.sg;
-    M(fgeo(3)) = g.sgf;
-    M(fgeo(4)) = g.cgf;
-    M(fgeo(5)) = g.c2p;
-    M(fgeo(6)) = g.s2p;
-    M(fgeo(7)) = rsqrtf(at[A_T * ps]);
+    // FP32 field geometry and the chain rule (|B|, gamma, phi) -> (Bx, By, Bz)
+    // for the radiative transfer.  With B = 0 every field derivative is zero,
+    // as in the reference (absorption_matrix.f90:1842-1866); with a vertical
+    // field the azimuth terms are dropped (the reference's d cos2phi / dBx is
+    // 0/0 there).
+    const float bx = at[A_BX * ps], by = at[A_BY * ps], bz = at[A_BZ * ps];
+    const Geo g = geometry(bx, by, bz);
+    const float bt2 = bx * bx + by * by, bt = sqrtf(bt2), B2 = g.B * g.B;
+    const bool hasB = g.B > 0.f, hasT = bt2 > 0.f;
+    const float iB = hasB ? 1.f / g.B : 0.f, iBt = hasT ? 1.f / (B2 * bt) : 0.f, ibt2 = hasT ? 1.f / bt2 : 0.f;
+    const float qf = hasT ? g.sgf : 0.f;
+    R[1] = {vz, g.B, 0.5f * g.sgf, 0.25f * g.cgf};
+    R[2] = {0.5f * qf, 0.25f * qf, 0.5f * g.cg, g.sg};
+    R[4] = {bx * iB, by * iB, bz * iB, bz * bx * iBt};
+    R[5] = {bz * by * iBt, hasB ? -bt / B2 : 0.f, -by * ibt2, bx * ibt2};
+    // the frame's angle; the line-optical-depth factor follows below
+    R[3] = {hasT ? g.c2p : 1.f, hasT ? g.s2p : 0.f, g.sg * g.cg, 0.f};
   }
   const double T = (double)a.atm[A_T * ps + k * cs + col], P = (double)a.atm[A_PG * ps + k * cs + col];
   const float rhof = a.atm[A_RHO * ps + k * cs + col];
@@ -397,35 +412,38 @@ __global__ void __launch_bounds__(256) opac_kernel(MicroTile a) {
   if (!err) {
     const double kc5 = kc[0] / nh * (1.0 / MAMU);
     const bool bnd = (k == 0) || (kc5 >= 2.0e10);     // forward.f90:884,931,971
-    M(F_FLAG) = bnd ? 1.0f : 0.0f;
-    M(F_KC5) = (float)kc5;
+    R[0] = {bnd ? 1.0f : 0.0f, Tf, iT, rsT};
+    a.micro[ps * c_cfg.rec + k * cs + col] = (float)kc5;
     // the opacities are formed wherever kc5 is below the threshold, the
     // bottom height included (its absorption matrix feeds LINE OPTICAL DEPTH,
     // forward.f90:931-968, while the transfer takes it as the boundary)
     const bool opaque = kc5 >= 2.0e10;
-    M(ftlf()) = opaque ? 0.f : (float)(1.0 / (nh * MAMU * (double)a.atm[A_MU * ps + k * cs + col]));
     if (opaque) return;
+    // 1 / (N_H m_u MW) (LINE OPTICAL DEPTH: KLINTAU = ETAI / N_H / m_u / MW; 0 where opaque)
+    R[3].w = (float)(1.0 / (nh * MAMU * (double)a.atm[A_MU * ps + k * cs + col]));
     for (int r = 0; r < c_cfg.nreg && !err; ++r) {
+      float4* Q = R + c_cfg.reg_rec[r] / 4;
       err = opac_cont(T, c_cfg.reg_l0main[r], ne, nh, d, a.der != 0, kc);
-      for (int q = 0; q < 4; ++q) M(freg(r, q)) = (float)kc[q];
-      for (int b = 0; b < c_cfg.reg_nblend[r] && !err; ++b) {
-        const int sl = c_cfg.reg_slot0[r] + b;
-        const LineConst& L = c_cfg.line[c_cfg.slot_line[sl]];
+      *Q++ = {(float)kc[0], (float)kc[1], (float)kc[2], (float)kc[3]};
+      for (int b = 0; b < c_cfg.reg_nblend[r] && !err; ++b, Q += REC_SLOT / 4) {
+        const int li = c_cfg.slot_line[c_cfg.reg_slot0[r] + b];
+        const LineConst& L = c_cfg.line[li];
         double kl[4] = {0, 0, 0, 0}, dm[4] = {0, 0, 0, 0};
         // the region's departure coefficients for every line of the region (forward.f90:949)
         const double bl = a.pop ? a.pop[((long)0 * nz + k) * c_cfg.nreg + r] : 1.0;
         const double bu = a.pop ? a.pop[((long)nz + k) * c_cfg.nreg + r] : 1.0;
-        const double Td = T + c_cfg.xi_t[c_cfg.slot_line[sl]];
+        const double Td = T + c_cfg.xi_t[li];
         err = opac_line(L, T, ne, nh, s, d, a.der != 0, kl, bl, bu, Td);
         damping(L, T, nh, d, a.der != 0, dm, Td);
-        M(fslot(sl, 0)) = (float)kl[0];
-        M(fslot(sl, 1)) = (float)dm[0];
-        M(fslot(sl, 2)) = (float)kl[1];
-        M(fslot(sl, 3)) = (float)kl[2];
-        M(fslot(sl, 4)) = (float)kl[3];
-        M(fslot(sl, 5)) = (float)dm[1];
-        M(fslot(sl, 6)) = (float)dm[2];
-        M(fslot(sl, 7)) = (float)dm[3];
+        const float rsd = c_cfg.xi_on ? rsqrtf(Tf + c_cfg.xi_tf[li]) : rsT;   // 1/sqrt(Doppler temperature)
+        float v[NVP];
+        voigt_poly((double)(float)dm[0], v);
+        Q[0] = {(float)kl[0], (float)dm[0], (float)kl[1], (float)dm[1]};
+        Q[1] = {(float)kl[2], (float)kl[3], (float)dm[2], (float)dm[3]};
+        Q[2] = {v[0], v[1], v[2], v[3]};
+        Q[3] = {v[4], v[5], v[6], v[7]};
+        Q[4] = {v[8], v[9], v[10], v[11]};
+        Q[5] = {v[12], c_cfg.idopfac[li] * rsd, c_cfg.xi_on ? -rsd * rsd : -iT, c_cfg.vfac[li] * vz};
       }
     }
   }
@@ -438,12 +456,13 @@ __global__ void __launch_bounds__(64) tau_kernel(MicroTile a) {
   const int nz = c_cfg.nz, col = a.col0 + ct;
   if (a.status[col] != 0) return;
   const long cs = a.ncol, ps = (long)nz * a.ncol;
+  const float* kc5 = a.micro + ps * c_cfg.rec;
   // log tau_5000 by the REAL(4) trapezoid of forward.f90:1000-1006 (z in km)
   float tau = 1e-9f;
   a.atm[A_TAU * ps + (nz - 1) * cs + col] = log10f(tau);
   for (int k = nz - 2; k >= 0; --k) {
-    const float x = (a.micro[F_KC5 * ps + k * cs + col] * a.atm[A_RHO * ps + k * cs + col] +
-                     a.micro[F_KC5 * ps + (k + 1) * cs + col] * a.atm[A_RHO * ps + (k + 1) * cs + col]) /
+    const float x = (kc5[k * cs + col] * a.atm[A_RHO * ps + k * cs + col] +
+                     kc5[(k + 1) * cs + col] * a.atm[A_RHO * ps + (k + 1) * cs + col]) /
                     2.0f;
     tau = (float)((double)tau + (double)x * ((c_cfg.zz[k + 1] - c_cfg.zz[k]) * 1000.0 * 100.0));
     a.atm[A_TAU * ps + k * cs + col] = log10f(tau);
@@ -601,6 +620,8 @@ struct RtArgs {
   float* jac;        // [ncol - jcol0][np][nz][4][numw]
   int jcol0;         // column of jac[0]
   float* scratch;    // [nz][4][ntile*numw]
+  int chunk;         // heights of the record that a wave holds in LDS at a time
+  int wcols;         // columns that a wave spans at most (1 unless packed)
   // per-pixel windows (items null: every column uses every wavelength)
   const RtItem* items;   // this launch's workgroups
   const int64_t* poff;   // [ncol+1] prefix of the pixels' wavelength counts: Stokes at 4*poff[col]
@@ -608,175 +629,156 @@ struct RtArgs {
   float* fs;             // FULL_STOKES [ncol][nz][4][numw] (Stokes after every height), or null
 };
 
-enum { D_T = 0, D_P, D_R, D_V, D_B, D_G, D_F, NDIR };
-
-// profile combination of the three component types (sigma_r, pi, sigma_b)
-// into (I,Q,U,V) (absorption_matrix.f90:1946-2230)
-struct Lin {
-  float I, Q, U, V;
-};
-__device__ __forceinline__ Lin lin(const Geo& g, float xr, float xp, float xb) {
-  const float qb = (0.5f * xp - 0.25f * (xr + xb)) * g.sgf;
-  return {0.5f * g.sgf * xp + 0.25f * g.cgf * (xr + xb), qb * g.c2p, qb * g.s2p, 0.5f * g.cg * (xr - xb)};
-}
-__device__ __forceinline__ Lin lin_dgamma(const Geo& g, float xr, float xp, float xb) {
-  const float dsgf = 2.f * g.sg * g.cg;   // d sin^2(gamma) / d gamma
-  const float qb = (0.5f * xp - 0.25f * (xr + xb)) * dsgf;
-  return {0.5f * dsgf * xp - 0.25f * dsgf * (xr + xb), qb * g.c2p, qb * g.s2p, -0.5f * g.sg * (xr - xb)};
-}
-__device__ __forceinline__ Lin lin_dphi(const Geo& g, float xr, float xp, float xb) {
-  const float qb = (0.5f * xp - 0.25f * (xr + xb)) * g.sgf;
-  return {0.f, -2.f * qb * g.s2p, 2.f * qb * g.c2p, 0.f};
-}
-
-// T, 1/T and 1/sqrt(T) (the inverse Doppler width of line li is
-// idopfac[li] / sqrt(T)), v_z and the field geometry of one height
-struct Layer {
-  float T, iT, rsT, vz;
-  Geo g;
+// The record of one (column, height) as the transfer reads it, from LDS or
+// from global memory (P: const float4* of either)
+template <class P>
+struct Rec {
+  P h, r;   // head, region
 };
 
-// propagation matrix without derivatives
-__device__ __forceinline__ void absorb(const RtArgs& a, int col, int k, int r, float wave, const Layer& ly,
-                                       float x7[7]) {
-  const long ps = (long)c_cfg.nz * a.ncol, cs = a.ncol;
-  const float* mic = a.micro + k * cs + col;
-  x7[0] = mic[freg(r, 0) * ps];
-  for (int c = 1; c < 7; ++c) x7[c] = 0.f;
-  for (int b = 0; b < c_cfg.reg_nblend[r]; ++b) {
-    const int sl = c_cfg.reg_slot0[r] + b, li = c_cfg.slot_line[sl];
-    const float kl = mic[fslot(sl, 0) * ps], dmp = mic[fslot(sl, 1) * ps];
-    const float rsd = c_cfg.xi_on ? rsqrtf(ly.T + c_cfg.xi_tf[li]) : ly.rsT;   // 1/sqrt(Doppler temperature)
-    const float idld = c_cfg.idopfac[li] * rsd;
-    const float base = (wave - c_cfg.slot_bldiff[sl] + c_cfg.vfac[li] * ly.vz) * idld;
-    const float bsc = ly.g.B * idld;
-    float hs[3], fs[3];
-    int m = c_cfg.comp0[li];
-    for (int t = 0; t < 3; ++t) {
-      float h = 0.f, f = 0.f;
-      const int n = c_cfg.ntype[li][t];
-      for (int j = 0; j < n; ++j, ++m) {
-        float H, F;
-        voigt(dmp, base + c_cfg.comp_shift[m] * bsc, H, F);
-        h += c_cfg.comp_str[m] * H;
-        f += c_cfg.comp_str[m] * F;
-      }
-      hs[t] = h;
-      fs[t] = f;
-    }
-    const Lin p = lin(ly.g, hs[0], hs[1], hs[2]), q = lin(ly.g, fs[0], fs[1], fs[2]);
-    x7[0] += kl * p.I;
-    x7[1] += kl * p.Q;
-    x7[2] += kl * p.U;
-    x7[3] += kl * p.V;
-    x7[4] += kl * q.Q;
-    x7[5] += kl * q.U;
-    x7[6] += kl * q.V;
-  }
-}
-
-// propagation matrix and its derivatives along the 7 internal directions
-// T|Pg, Pg|T, rho|T, v_z, |B|, inclination, azimuth (absorption_matrix.f90:1717-2642)
-__device__ __forceinline__ void absorb_der(const RtArgs& a, int col, int k, int r, float wave, const Layer& ly,
-                                           float x7[7], float dx[NDIR][7]) {
-  const long ps = (long)c_cfg.nz * a.ncol, cs = a.ncol;
-  const float* mic = a.micro + k * cs + col;
-  x7[0] = mic[freg(r, 0) * ps];
-  for (int c = 1; c < 7; ++c) x7[c] = 0.f;
-  for (int i = 0; i < NDIR; ++i)
-    for (int c = 0; c < 7; ++c) dx[i][c] = 0.f;
-  dx[D_T][0] = mic[freg(r, 1) * ps];
-  dx[D_P][0] = mic[freg(r, 2) * ps];
-  dx[D_R][0] = mic[freg(r, 3) * ps];
-  const float isp = 0.564189583547756f;   // 1/sqrt(pi)
-  for (int b = 0; b < c_cfg.reg_nblend[r]; ++b) {
-    const int sl = c_cfg.reg_slot0[r] + b, li = c_cfg.slot_line[sl];
-    const float kl = mic[fslot(sl, 0) * ps], dmp = mic[fslot(sl, 1) * ps];
-    const float dkl[3] = {mic[fslot(sl, 2) * ps], mic[fslot(sl, 3) * ps], mic[fslot(sl, 4) * ps]};
-    const float dda[3] = {mic[fslot(sl, 5) * ps], mic[fslot(sl, 6) * ps], mic[fslot(sl, 7) * ps]};
-    const float rsd = c_cfg.xi_on ? rsqrtf(ly.T + c_cfg.xi_tf[li]) : ly.rsT;   // 1/sqrt(Doppler temperature)
-    const float idld = c_cfg.idopfac[li] * rsd;
-    const float base = (wave - c_cfg.slot_bldiff[sl] + c_cfg.vfac[li] * ly.vz) * idld;
-    const float bsc = ly.g.B * idld;
-    // per component type: H, F, sum dH/du, dH/da, u*dH/du, u*dH/da, shift*dH/du, shift*dH/da
-    float S[8][3];
-    int m = c_cfg.comp0[li];
-    for (int t = 0; t < 3; ++t) {
-      float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-      const int n = c_cfg.ntype[li][t];
-      for (int j = 0; j < n; ++j, ++m) {
-        const float sh = c_cfg.comp_shift[m], st = c_cfg.comp_str[m];
-        const float u = base + sh * bsc;
-        float H, F;
-        voigt(dmp, u, H, F);
-        const float hu = 2.f * (dmp * F - u * H);            // dH/du
-        const float ha = 2.f * (dmp * H + u * F - isp);      // dH/da
-        acc[0] += st * H;
-        acc[1] += st * F;
-        acc[2] += st * hu;
-        acc[3] += st * ha;
-        acc[4] += st * hu * u;
-        acc[5] += st * ha * u;
-        acc[6] += st * hu * sh;
-        acc[7] += st * ha * sh;
-      }
-      for (int q = 0; q < 8; ++q) S[q][t] = acc[q];
-    }
-    const Geo& g = ly.g;
-    const Lin pH = lin(g, S[0][0], S[0][1], S[0][2]);
-    const Lin pF = lin(g, S[1][0], S[1][1], S[1][2]);
-    const Lin pHu = lin(g, S[2][0], S[2][1], S[2][2]);
-    const Lin pHa = lin(g, S[3][0], S[3][1], S[3][2]);
-    const Lin pHuu = lin(g, S[4][0], S[4][1], S[4][2]);
-    const Lin pHau = lin(g, S[5][0], S[5][1], S[5][2]);
-    const Lin pHb = lin(g, S[6][0], S[6][1], S[6][2]);
-    const Lin pHab = lin(g, S[7][0], S[7][1], S[7][2]);
-    const Lin gH = lin_dgamma(g, S[0][0], S[0][1], S[0][2]);
-    const Lin gF = lin_dgamma(g, S[1][0], S[1][1], S[1][2]);
-    const Lin fH = lin_dphi(g, S[0][0], S[0][1], S[0][2]);
-    const Lin fF = lin_dphi(g, S[1][0], S[1][1], S[1][2]);
-    // eta components use the H sums; rho components use the F sums, whose
-    // derivatives are dF/du = -dH/da and dF/da = dH/du for w = H + iF
-    const float e7[7] = {pH.I, pH.Q, pH.U, pH.V, pF.Q, pF.U, pF.V};
-    const float a7[7] = {pHa.I, pHa.Q, pHa.U, pHa.V, pHu.Q, pHu.U, pHu.V};      // d/da
-    const float u7[7] = {pHu.I, pHu.Q, pHu.U, pHu.V, -pHa.Q, -pHa.U, -pHa.V};  // d/du
-    const float uu7[7] = {pHuu.I, pHuu.Q, pHuu.U, pHuu.V, -pHau.Q, -pHau.U, -pHau.V};
-    const float b7[7] = {pHb.I, pHb.Q, pHb.U, pHb.V, -pHab.Q, -pHab.U, -pHab.V};
-    const float g7[7] = {gH.I, gH.Q, gH.U, gH.V, gF.Q, gF.U, gF.V};
-    const float f7[7] = {fH.I, fH.Q, fH.U, fH.V, fF.Q, fF.U, fF.V};
-    const float dudT = c_cfg.xi_on ? -0.5f * rsd * rsd : -0.5f * ly.iT;   // du/dT = -u/(2 T_Doppler)
-    const float dudv = c_cfg.vfac[li] * idld;
+// sums over the component types (sigma_r, pi, sigma_b) of one quantity: the
+// absorption profiles (h) and the dispersion profiles (f)
+struct Sums {
+  float h[3], f[3];
+};
+__device__ __forceinline__ void zero(Sums& x) {
 #pragma unroll
-    for (int c = 0; c < 7; ++c) {
-      x7[c] += kl * e7[c];
-      dx[D_T][c] += dkl[0] * e7[c] + kl * (dudT * uu7[c] + dda[0] * a7[c]);
-      dx[D_P][c] += dkl[1] * e7[c] + kl * dda[1] * a7[c];
-      dx[D_R][c] += dkl[2] * e7[c] + kl * dda[2] * a7[c];
-      dx[D_V][c] += kl * dudv * u7[c];
-      dx[D_B][c] += kl * idld * b7[c];
-      dx[D_G][c] += kl * g7[c];
-      dx[D_F][c] += kl * f7[c];
-    }
-  }
+  for (int t = 0; t < 3; ++t) x.h[t] = x.f[t] = 0.f;
 }
 
-__device__ __forceinline__ Layer load_layer(const RtArgs& a, int col, int k) {
-  const long ps = (long)c_cfg.nz * a.ncol, cs = a.ncol;
-  const float* at = a.atm + k * cs + col;
-  const float* mg = a.micro + k * cs + col;
-  Layer ly;
-  ly.T = at[A_T * ps];
-  ly.iT = 1.0f / ly.T;
-  ly.vz = at[A_VZ * ps];
-  ly.g.B = mg[fgeo(0) * ps];
-  ly.g.cg = mg[fgeo(1) * ps];
-  ly.g.sg = mg[fgeo(2) * ps];
-  ly.g.sgf = mg[fgeo(3) * ps];
-  ly.g.cgf = mg[fgeo(4) * ps];
-  ly.g.c2p = mg[fgeo(5) * ps];
-  ly.g.s2p = mg[fgeo(6) * ps];
-  ly.rsT = mg[fgeo(7) * ps];
-  return ly;
+// profile combination of the three types into the frame's five elements
+// (absorption_matrix.f90:1946-2230)
+struct Mix {
+  float i0, i1, q0, q1, v;   // I = i0 pi + i1 (r + b), q = q0 pi - q1 (r + b), V = v (r - b)
+};
+__device__ __forceinline__ Five mix(const Mix& m, const Sums& x) {
+  const float sh = x.h[0] + x.h[2], sf = x.f[0] + x.f[2];
+  return {fmaf(m.i0, x.h[1], m.i1 * sh), fmaf(m.q0, x.h[1], -(m.q1 * sh)), m.v * (x.h[0] - x.h[2]),
+          fmaf(m.q0, x.f[1], -(m.q1 * sf)), m.v * (x.f[0] - x.f[2])};
+}
+
+__device__ __forceinline__ VoigtPoly voigt_load(const float4& a, const float4& b, const float4& c, float d) {
+  return {{a.x, a.y, a.z, a.w, b.x, b.y}, {b.z, b.w, c.x, c.y, c.z, c.w, d}};
+}
+
+// Profile sums of region r's lines times kl dz at one height
+template <class P>
+__device__ __forceinline__ Sums absorb(P q, int r, float wave, float B, float dz) {
+  Sums X;
+  zero(X);
+  for (int b = 0; b < c_cfg.reg_nblend[r]; ++b, q += REC_SLOT / 4) {
+    const int sl = c_cfg.reg_slot0[r] + b, li = c_cfg.slot_line[sl];
+    const float4 q0 = q[0], q5 = q[5];
+    const VoigtPoly vp = voigt_load(q[2], q[3], q[4], q5.x);
+    const float kl = q0.x * dz;
+    const float base = (wave - c_cfg.slot_bldiff[sl] + q5.w) * q5.y, bsc = B * q5.y;
+    const float4* cm = c_cfg.comp + c_cfg.comp0[li];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      const float ut = fmaf(c_cfg.type[li][t].x, bsc, base);
+      const int n = c_cfg.ntype[li][t];
+      float h = 0.f, f = 0.f;
+      for (int j = 0; j < n; ++j, ++cm) {
+        float H, F;
+        voigt(vp, fmaf(cm->x, bsc, ut), H, F);
+        h = fmaf(cm->y, H, h);
+        f = fmaf(cm->y, F, f);
+      }
+      X.h[t] = fmaf(kl, h, X.h[t]);
+      X.f[t] = fmaf(kl, f, X.f[t]);
+    }
+  }
+  return X;
+}
+
+// The same with the derivatives along T|Pg, v_z, |B| and, with PR, Pg|T and
+// rho|T (absorption_matrix.f90:1717-2642).  With w = H + iF, dH/du = 2 (a F -
+// u H) = dF/da and dH/da = 2 (a H + u F - 1/sqrt(pi)) = -dF/du, and the
+// components of a type lie at u = ut + bsc delta: every derivative sum of
+// the type is a combination of the moments sum st delta^n (H, F), n = 0, 1, 2,
+// so a component costs its profile and six multiply-adds.
+template <bool PR, class P>
+__device__ __forceinline__ void absorb_der(P q, int r, float wave, float B, float dz, Sums& X, Sums& XT, Sums& XV,
+                                           Sums& XB, Sums& XP, Sums& XR) {
+  zero(X);
+  zero(XT);
+  zero(XV);
+  zero(XB);
+  if (PR) {
+    zero(XP);
+    zero(XR);
+  }
+  for (int b = 0; b < c_cfg.reg_nblend[r]; ++b, q += REC_SLOT / 4) {
+    const int sl = c_cfg.reg_slot0[r] + b, li = c_cfg.slot_line[sl];
+    const float4 q0 = q[0], q5 = q[5];
+    const VoigtPoly vp = voigt_load(q[2], q[3], q[4], q5.x);
+    const float a = q0.y, kl = q0.x * dz, dklT = q0.z * dz;
+    const float base = (wave - c_cfg.slot_bldiff[sl] + q5.w) * q5.y, bsc = B * q5.y;
+    // kl times twice the derivatives of u in T (over u), v_z and |B| (over
+    // the shift), and of a in T: the factor 2 of dH/du and dH/da
+    const float uT = kl * q5.z, uv = 2.f * kl * c_cfg.vfac[li] * q5.y, ub = 2.f * kl * q5.y, aT = 2.f * kl * q0.w;
+    float dklP = 0.f, dklR = 0.f, aP = 0.f, aR = 0.f;
+    if (PR) {
+      const float4 q1 = q[1];
+      dklP = q1.x * dz;
+      dklR = q1.y * dz;
+      aP = 2.f * kl * q1.z;
+      aR = 2.f * kl * q1.w;
+    }
+    const float4* cm = c_cfg.comp + c_cfg.comp0[li];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      const float4 ty = c_cfg.type[li][t];
+      const float ut = fmaf(ty.x, bsc, base);
+      const int n = c_cfg.ntype[li][t];
+      // half dH/du and dH/da summed over the type, and times u and the shift
+      float h0 = 0.f, f0 = 0.f, hu, ha, huu, hau, hb, hab;
+      if (n == 1) {
+        voigt(vp, ut, h0, f0);
+        hu = fmaf(a, f0, -(ut * h0));
+        ha = fmaf(a, h0, fmaf(ut, f0, -ty.y));
+        huu = ut * hu;
+        hau = ut * ha;
+        hb = ty.x * hu;
+        hab = ty.x * ha;
+        ++cm;
+      } else {
+        float h1 = 0.f, f1 = 0.f, h2 = 0.f, f2 = 0.f;
+        for (int j = 0; j < n; ++j, ++cm) {
+          float H, F;
+          voigt(vp, fmaf(cm->x, bsc, ut), H, F);
+          h0 = fmaf(cm->y, H, h0);
+          f0 = fmaf(cm->y, F, f0);
+          h1 = fmaf(cm->z, H, h1);
+          f1 = fmaf(cm->z, F, f1);
+          h2 = fmaf(cm->w, H, h2);
+          f2 = fmaf(cm->w, F, f2);
+        }
+        hu = fmaf(a, f0, -fmaf(ut, h0, bsc * h1));
+        ha = fmaf(a, h0, fmaf(ut, f0, fmaf(bsc, f1, -ty.y)));
+        const float hd = fmaf(a, f1, -fmaf(ut, h1, bsc * h2));
+        const float hc = fmaf(a, h1, fmaf(ut, f1, fmaf(bsc, f2, -ty.z)));
+        huu = fmaf(ut, hu, bsc * hd);
+        hau = fmaf(ut, ha, bsc * hc);
+        hb = fmaf(ty.x, hu, hd);
+        hab = fmaf(ty.x, ha, hc);
+      }
+      X.h[t] = fmaf(kl, h0, X.h[t]);
+      X.f[t] = fmaf(kl, f0, X.f[t]);
+      XT.h[t] = fmaf(dklT, h0, fmaf(uT, huu, fmaf(aT, ha, XT.h[t])));
+      XT.f[t] = fmaf(dklT, f0, fmaf(-uT, hau, fmaf(aT, hu, XT.f[t])));
+      XV.h[t] = fmaf(uv, hu, XV.h[t]);
+      XV.f[t] = fmaf(-uv, ha, XV.f[t]);
+      XB.h[t] = fmaf(ub, hb, XB.h[t]);
+      XB.f[t] = fmaf(-ub, hab, XB.f[t]);
+      if (PR) {
+        XP.h[t] = fmaf(dklP, h0, fmaf(aP, ha, XP.h[t]));
+        XP.f[t] = fmaf(dklP, f0, fmaf(aP, hu, XP.f[t]));
+        XR.h[t] = fmaf(dklR, h0, fmaf(aR, ha, XR.h[t]));
+        XR.f[t] = fmaf(dklR, f0, fmaf(aR, hu, XR.f[t]));
+      }
+    }
+  }
 }
 
 // LINE OPTICAL DEPTH (forward.f90:966-968, 1008-1015): per (column,
@@ -797,13 +799,14 @@ __global__ void __launch_bounds__(256) taulin_kernel(RtArgs a, float* __restrict
   const long ps = (long)nz * a.ncol, cs = a.ncol;
   float* o = out + (long)col * nz * numw + l;
   for (int k = 0; k < nz; ++k) {
-    const float fac = a.micro[ftlf() * ps + k * cs + col];
+    const float4* R = reinterpret_cast<const float4*>(a.micro + ((long)k * a.ncol + col) * c_cfg.rec);
+    const float fac = R[3].w;
     float kl = 0.f;
     if (fac != 0.f) {
-      const Layer ly = load_layer(a, col, k);
-      float x7[7];
-      absorb(a, col, k, r, wave, ly, x7);
-      kl = x7[0] * fac;
+      const float4* Q = R + c_cfg.reg_rec[r] / 4;
+      const float4 h1 = R[1];
+      const Sums X = absorb(Q + 1, r, wave, h1.y, 1.0f);
+      kl = (Q[0].x + fmaf(h1.z, X.h[1], h1.w * (X.h[0] + X.h[2]))) * fac;
     }
     o[(long)k * numw] = kl;
   }
@@ -818,6 +821,14 @@ __global__ void __launch_bounds__(256) taulin_kernel(RtArgs a, float* __restrict
   }
 }
 
+// bytes of LDS that a transfer wave fills with the records of its next heights
+constexpr size_t RT_LDS = 10 * 1024;
+
+// Radiative transfer, one lane per (column, wavelength), one wave per
+// workgroup.  Bound: the issue of FP32 operations (no packed FP32 in this
+// build), about 600 per height in pass 1 and 1400 in pass 2 for two lines with
+// 15 Zeeman components and five parameters.
+//
 // HE (HYDROSTATIC: yes, response functions on): the T response of height K
 // also carries the change of Pg below K through hydrostatic equilibrium,
 // dPg_i/dT_K = Pg_i (-mu_K m_u g dz_K / (k T_K^2)) (GET_HYD_DERIVATIVES), i.e.
@@ -831,88 +842,105 @@ __global__ void __launch_bounds__(256) taulin_kernel(RtArgs a, float* __restrict
 // PACK (one region, no per-pixel windows): the lanes of a launch run over
 // the flattened (column, wavelength) pairs of the tile, 64 to a wave, so no
 // lane idles when the wavelength count is not a multiple of 64 (112 = 64 +
-// 48 would leave 16 of 128 lanes idle per column); a wave then spans up to
-// two columns and reads their per-height quantities with vector loads.
+// 48 would leave 16 of 128 lanes idle per column); a wave then spans two or
+// more columns, each lane reading its own column's record from LDS.
 template <int RF, bool HE, bool PACK>
-__global__ void __launch_bounds__(RT_WAVE) rt_kernel(const float* __restrict__ atm, const float* __restrict__ micro,
-                                                     const float* __restrict__ gain, int32_t* __restrict__ status,
-                                                     float* __restrict__ stokes, float* __restrict__ jac,
-                                                     float* __restrict__ scratch, int ncol, int col0, int ntile,
-                                                     int jcol0, const RtItem* __restrict__ items,
-                                                     const int64_t* __restrict__ poff,
-                                                     const double* __restrict__ pop, float* __restrict__ fs) {
-  RtArgs a;
-  a.ncol = ncol;
-  a.col0 = col0;
-  a.ntile = ntile;
-  a.atm = atm;
-  a.micro = micro;
-  a.gain = gain;
-  a.status = status;
-  a.stokes = stokes;
-  a.jac = jac;
-  a.jcol0 = jcol0;
-  a.scratch = scratch;
-  a.items = items;
-  a.poff = poff;
-  a.pop = pop;
-  a.fs = fs;
+__global__ void __launch_bounds__(RT_WAVE) rt_kernel(RtArgs a) {
   // parameters: 5 spherical, 7 Cartesian, 8 with P0 (the top pressure)
   constexpr int NP = (RF == FZ_RF_SPHERICAL || RF == RF_CART_TBV)
                          ? 5
                          : (RF == FZ_RF_CARTESIAN ? 7 : (RF == FZ_RF_CARTESIAN_P0 ? 8 : 0));
   constexpr int NPL = RF == FZ_RF_CARTESIAN_P0 ? 7 : NP;    // parameters with a local response
-  const int numw = c_cfg.numw, nz = c_cfg.nz;
-  // workgroup -> (column, region, first wavelength); lane -> wavelength
-  int ct, r, l;
+  constexpr bool PR = RF == FZ_RF_CARTESIAN || RF == FZ_RF_CARTESIAN_P0;
+  constexpr bool HEX = HE && RF != 0;
+  extern __shared__ float4 lds[];
+  const int numw = c_cfg.numw, nz = c_cfg.nz, lane = (int)threadIdx.x;
+  // workgroup -> (column, region, first wavelength); lane -> wavelength.  A
+  // lane past the work repeats the last one without storing, so that the
+  // whole wave takes part in the copies to LDS.
+  bool live = true;
+  int ct, ct0, r, l;
   long sbase;        // the column's Stokes: stokes[sbase + s * snumw + lo]
   int snumw, lo;
   long t, nthr;      // lane slot and lane count of the tile (scratch rows)
   long jbase;        // the column's response functions: jac[jbase + ((p*nz + k)*4 + s)*snumw]
   if constexpr (PACK) {
-    const int g = (int)blockIdx.x * RT_WAVE + (int)threadIdx.x;
-    if (g >= a.ntile * numw) return;
+    const int g0 = (int)blockIdx.x * RT_WAVE, last = a.ntile * numw - 1;
+    live = g0 + lane <= last;
+    const int g = min(g0 + lane, last);
     ct = g / numw;
+    ct0 = g0 / numw;
     l = g - ct * numw;
     r = 0;
-    sbase = (long)(col0 + ct) * 4 * numw;
+    sbase = (long)(a.col0 + ct) * 4 * numw;
     snumw = numw;
     lo = l;
     t = g;
     nthr = (long)a.ntile * numw;
-    jbase = (long)(col0 + ct - a.jcol0) * NP * nz * 4 * numw + l;
-  } else if (items) {
+    jbase = (long)(a.col0 + ct - a.jcol0) * NP * nz * 4 * numw + l;
+  } else if (a.items) {
     // per-pixel windows: scratch and response functions are ragged too
-    const RtItem it = items[blockIdx.x];
-    if ((int)threadIdx.x >= it.n) return;
-    ct = it.col - col0;
+    const RtItem it = a.items[blockIdx.x];
+    live = lane < it.n;
+    const int i = min(lane, it.n - 1);
+    ct = ct0 = it.col - a.col0;
     r = it.r;
-    l = it.l0 + (int)threadIdx.x;
-    const int64_t p0 = poff[it.col], pt = poff[col0];
+    l = it.l0 + i;
+    const int64_t p0 = a.poff[it.col], pt = a.poff[a.col0];
     sbase = 4 * p0;
-    snumw = (int)(poff[it.col + 1] - p0);
-    lo = it.lout + (int)threadIdx.x;
+    snumw = (int)(a.poff[it.col + 1] - p0);
+    lo = it.lout + i;
     t = (p0 - pt) + lo;
-    nthr = poff[col0 + a.ntile] - pt;
-    jbase = (long)NP * nz * 4 * (p0 - poff[a.jcol0]) + lo;
+    nthr = a.poff[a.col0 + a.ntile] - pt;
+    jbase = (long)NP * nz * 4 * (p0 - a.poff[a.jcol0]) + lo;
   } else {
-    ct = (int)(blockIdx.x / (unsigned)c_cfg.nbpc);
+    ct = ct0 = (int)(blockIdx.x / (unsigned)c_cfg.nbpc);
     const int bc = (int)(blockIdx.x - (unsigned)ct * (unsigned)c_cfg.nbpc);
-    if ((int)threadIdx.x >= c_cfg.blk_n[bc]) return;
+    live = lane < c_cfg.blk_n[bc];
     r = c_cfg.blk_reg[bc];
-    l = c_cfg.blk_l0[bc] + (int)threadIdx.x;
-    sbase = (long)(col0 + ct) * 4 * numw;
+    l = c_cfg.blk_l0[bc] + min(lane, c_cfg.blk_n[bc] - 1);
+    sbase = (long)(a.col0 + ct) * 4 * numw;
     snumw = numw;
     lo = l;
     t = (long)ct * numw + l;
     nthr = (long)a.ntile * numw;
-    jbase = (long)(col0 + ct - a.jcol0) * NP * nz * 4 * numw + l;
+    jbase = (long)(a.col0 + ct - a.jcol0) * NP * nz * 4 * numw + l;
   }
   const int col = a.col0 + ct;
   if (a.status && a.status[col] != 0) {
-    for (int s = 0; s < 4; ++s) a.stokes[sbase + (long)s * snumw + lo] = __builtin_nanf("");
-    return;
+    if (live)
+      for (int s = 0; s < 4; ++s) a.stokes[sbase + (long)s * snumw + lo] = __builtin_nanf("");
+    live = false;
   }
+  if (__ballot(live) == 0) return;
+  // the wave's columns are ct0 .. ct0 + nc - 1
+  const int nc = PACK ? __builtin_amdgcn_readfirstlane(__shfl(ct, 63) - ct0 + 1) : 1;
+  const int rs4 = (REC_HEAD + REC_REG + REC_SLOT * c_cfg.reg_nblend[r]) / 4;   // float4 per (height, column) in LDS
+  const float4* grec = reinterpret_cast<const float4*>(a.micro);
+  const int rec4 = c_cfg.rec / 4, roff4 = (c_cfg.reg_rec[r] - REC_HEAD) / 4;
+  // heights k0 .. k0 + n - 1 of the wave's columns into LDS: half a wave per
+  // record (rs4 <= 32)
+  auto stage = [&](int k0, int n) {
+    __syncthreads();
+    const int f = lane & 31;
+    const int src = f + (f >= REC_HEAD / 4 ? roff4 : 0);
+    const int np = n * nc;
+    int h = 0, c = lane >> 5;
+    if (c >= nc) {
+      c -= nc;
+      ++h;
+    }
+    for (int p = lane >> 5; p < np; p += 2) {
+      if (f < rs4) lds[p * rs4 + f] = grec[((long)(k0 + h) * a.ncol + a.col0 + ct0 + c) * rec4 + src];
+      c += 2;
+      while (c >= nc) {
+        c -= nc;
+        ++h;
+      }
+    }
+    __syncthreads();
+  };
+  const float4* const mine = lds + (ct - ct0) * rs4;
   const double wd = c_cfg.reg_wstart[r] + c_cfg.reg_wstep[r] * (double)(l - c_cfg.reg_pix0[r]);
   const float wave = (float)wd;
   // Planck function constants (rtesolver.f90:1008-1035): S = c1 / (exp(c2/T) - 1)
@@ -920,7 +948,6 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(const float* __restrict__ a
   const float c1 = (float)(2.0 * HPLA * LIGHT * LIGHT / (lam * lam * lam * lam * lam));
   const float c2 = (float)(HPLA * LIGHT / (lam * KBOL));
   const long ps = (long)nz * a.ncol, cs = a.ncol;
-  constexpr bool HEX = HE && RF != 0;
   float I[4] = {0.f, 0.f, 0.f, 0.f};
   float Ahe[4] = {0.f, 0.f, 0.f, 0.f};
   float* scr = a.scratch + t;
@@ -932,69 +959,98 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(const float* __restrict__ a
   };
   // FULL_STOKES (forward.f90:980-983): the Stokes vector after every
   // height, times GAIN1D, at fs[((col * nz + k) * 4 + s) * numw + l]
-  float* fsp = a.fs ? a.fs + (long)(col0 + ct) * nz * 4 * snumw + lo : nullptr;
+  float* fsp = a.fs && live ? a.fs + (long)col * nz * 4 * snumw + lo : nullptr;
   auto store_fs = [&](int k) {
     if (!fsp) return;
 #pragma unroll
     for (int s = 0; s < 4; ++s) fsp[(long)(k * 4 + s) * snumw] = I[s] * a.gain[l * 4 + s];
   };
-  for (int k = 0; k < nz; ++k) {
-    const Layer ly = load_layer(a, col, k);
-    const float S = c1 * (1.0f / (depart(k) * expf(c2 * ly.iT) - 1.0f));
-    if (RF) {
+  // into the layer's frame (cos, sin of twice the azimuth) and back
+  auto turn = [](float c, float s, const float v[4], float o[4]) {
+    o[0] = v[0];
+    o[1] = fmaf(c, v[1], s * v[2]);
+    o[2] = fmaf(c, v[2], -(s * v[1]));
+    o[3] = v[3];
+  };
+  auto turn_back = [](float c, float s, float v[4]) {
+    const float q = fmaf(c, v[1], -(s * v[2])), u = fmaf(s, v[1], c * v[2]);
+    v[1] = q;
+    v[2] = u;
+  };
+  for (int k0 = 0; k0 < nz; k0 += a.chunk) {
+    const int n = min(a.chunk, nz - k0);
+    stage(k0, n);
+    for (int kk = 0; kk < n; ++kk) {
+      const int k = k0 + kk;
+      const float4* R = mine + kk * nc * rs4;
+      const float4 h0 = R[0];
+      const float S = c1 * (1.0f / (depart(k) * expf(c2 * h0.z) - 1.0f));
+      if (RF) {
+        if (live) {
 #pragma unroll
-      for (int s = 0; s < 4; ++s) scr[(long)(k * 4 + s) * sstr] = I[s];
-    }
-    if (a.micro[F_FLAG * ps + k * cs + col] != 0.f) {
-      I[0] = S; I[1] = 0.f; I[2] = 0.f; I[3] = 0.f;
-      store_fs(k);
-      continue;
-    }
-    float x7[7];
-    Evol E;
-    if constexpr (HEX) {
-      float dx[NDIR][7];
-      absorb_der(a, col, k, r, wave, ly, x7, dx);
-      const float dz = c_cfg.dz_cm[k];
-      evol_build<true>(x7, dz, E);
-      float v[4] = {I[0] - S, I[1], I[2], I[3]}, m4v[4], d2[4];
-      m4mul(E.e, E.r, E.s0, v, m4v);
-      evol_dir(E, dx[D_P], dz, v, m4v, d2);
-      float W[4];
-      const bool thin = E.O[0][0] > 1.0e-5f;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        W[i] = thin ? E.O[i][0] * Ahe[0] + E.O[i][1] * Ahe[1] + E.O[i][2] * Ahe[2] + E.O[i][3] * Ahe[3] : Ahe[i];
-      const float pg = a.atm[A_PG * ps + k * cs + col];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        scr[(long)((nz + k) * 4 + i) * sstr] = W[i];
-        if (thin) Ahe[i] = W[i] + d2[i] * pg;
+          for (int s = 0; s < 4; ++s) scr[(long)(k * 4 + s) * sstr] = I[s];
+        }
       }
-    } else {
-      absorb(a, col, k, r, wave, ly, x7);
-      evol_build<false>(x7, c_cfg.dz_cm[k], E);
+      if (h0.x != 0.f) {
+        I[0] = S; I[1] = 0.f; I[2] = 0.f; I[3] = 0.f;
+        store_fs(k);
+        continue;
+      }
+      const float4 h1 = R[1], h2 = R[2], h3 = R[3], rg = R[REC_HEAD / 4];
+      const float dz = c_cfg.dz_cm[k];
+      const Mix mx = {h1.z, h1.w, h2.x, h2.y, h2.z};
+      const float v[4] = {I[0] - S, I[1], I[2], I[3]};
+      float vf[4], dv[4];
+      turn(h3.x, h3.y, v, vf);
+      Evol E;
+      if constexpr (HEX) {
+        Sums X, XT, XV, XB, XP, XR;
+        absorb_der<true>(R + REC_HEAD / 4 + 1, r, wave, h1.y, dz, X, XT, XV, XB, XP, XR);
+        Five f = mix(mx, X), fp = mix(mx, XP);
+        f.I = fmaf(rg.x, dz, f.I);
+        fp.I = fmaf(rg.z, dz, fp.I);
+        evol_build<true>(f, E);
+        const Pieces w = evol_pieces(E, vf);
+        evol_apply(E, w, dv);
+        Grad G;
+        evol_grad(E, vf, w, G);
+        float d2[4], Af[4], W[4];
+        grad_dot(G, fp, d2);
+        turn_back(h3.x, h3.y, d2);
+        turn(h3.x, h3.y, Ahe, Af);
+        evol_apply(E, evol_pieces(E, Af), W);
+        turn_back(h3.x, h3.y, W);
+        const bool thin = fmaf(E.D4, E.s0, E.A) > 1.0e-5f;    // O_11
+        const float pg = a.atm[A_PG * ps + k * cs + col];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          W[i] = thin ? fmaf(E.A, Ahe[i], W[i]) : Ahe[i];
+          if (live) scr[(long)((nz + k) * 4 + i) * sstr] = W[i];
+          if (thin) Ahe[i] = W[i] + d2[i] * pg;
+        }
+      } else {
+        Five f = mix(mx, absorb(R + REC_HEAD / 4 + 1, r, wave, h1.y, dz));
+        f.I = fmaf(rg.x, dz, f.I);
+        evol_build<false>(f, E);
+        evol_apply(E, evol_pieces(E, vf), dv);
+      }
+      turn_back(h3.x, h3.y, dv);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) I[i] = fmaf(E.A, v[i], dv[i]) + (i == 0 ? S : 0.f);
+      store_fs(k);
     }
-    float In[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      In[i] = ((i == 0 ? 1.f : 0.f) - E.O[i][0]) * S + E.O[i][0] * I[0] + E.O[i][1] * I[1] + E.O[i][2] * I[2] +
-              E.O[i][3] * I[3];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) I[i] = In[i];
-    store_fs(k);
   }
   float gn[4];
 #pragma unroll
   for (int s = 0; s < 4; ++s) {
     gn[s] = a.gain[l * 4 + s];
-    a.stokes[sbase + (long)s * snumw + lo] = I[s] * gn[s];
+    if (live) a.stokes[sbase + (long)s * snumw + lo] = I[s] * gn[s];
   }
   // a non-finite Stokes vector comes from a non-finite profile, propagation
   // matrix or evolution operator, where the reference stops
   // (voigt.f:91-95, absorption_matrix.f90:1882-1889, rtesolver.f90:346-352)
-  if (a.status && !(__builtin_isfinite(I[0]) && __builtin_isfinite(I[1]) && __builtin_isfinite(I[2]) &&
-                    __builtin_isfinite(I[3])))
+  if (live && a.status && !(__builtin_isfinite(I[0]) && __builtin_isfinite(I[1]) && __builtin_isfinite(I[2]) &&
+                            __builtin_isfinite(I[3])))
     atomicMax(&a.status[col], (int32_t)ERR_NAN);
   if constexpr (RF != 0) {
     float acc[4][4];
@@ -1003,133 +1059,167 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(const float* __restrict__ a
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc[i][j] = (i == j) ? 1.f : 0.f;
     float* jb = a.jac + jbase;
-    for (int k = nz - 1; k >= 0; --k) {
-      float outv[NP][4];
-      const Layer ly = load_layer(a, col, k);
-      if (a.micro[F_FLAG * ps + k * cs + col] != 0.f) {
-        // boundary layer: no local response; layers below cannot reach the top
+    for (int k1 = nz; k1 > 0; k1 -= a.chunk) {
+      const int n = min(a.chunk, k1);
+      stage(k1 - n, n);
+      for (int kk = n - 1; kk >= 0; --kk) {
+        const int k = k1 - n + kk;
+        const float4* R = mine + kk * nc * rs4;
+        float outv[NP][4];
+        const float4 h0 = R[0];
+        if (h0.x != 0.f) {
+          // boundary layer: no local response; layers below cannot reach the top
 #pragma unroll
-        for (int p = 0; p < NP; ++p)
+          for (int p = 0; p < NP; ++p)
 #pragma unroll
-          for (int s = 0; s < 4; ++s) outv[p][s] = 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-      } else {
-        // S = c1 / (ex - 1), dS/dT = S (ex / (ex - 1)) (c2 / T) / T
-        const float x = c2 * ly.iT;
-        const float ex = depart(k) * expf(x);
-        const float iem1 = 1.0f / (ex - 1.0f);
-        const float S = c1 * iem1;
-        const float dS = S * (ex * iem1) * x * ly.iT;
-        float x7[7], dx[NDIR][7];
-        absorb_der(a, col, k, r, wave, ly, x7, dx);
-        Evol E;
-        const float dz = c_cfg.dz_cm[k];
-        evol_build<true>(x7, dz, E);
-        float v[4], m4v[4];
-#pragma unroll
-        for (int s = 0; s < 4; ++s) v[s] = scr[(long)(k * 4 + s) * sstr] - (s == 0 ? S : 0.f);
-        m4mul(E.e, E.r, E.s0, v, m4v);
-        float vo[4], m4vo[4];
-        if constexpr (HEX) {
-#pragma unroll
-          for (int s = 0; s < 4; ++s) vo[s] = (k == nz - 1 ? I[s] : scr[(long)((k + 1) * 4 + s) * sstr]) - (s == 0 ? S : 0.f);
-          m4mul(E.e, E.r, E.s0, vo, m4vo);
-        }
-        float loc[NDIR][4];
-        constexpr int dirs_sph[5] = {D_T, D_B, D_G, D_F, D_V};
-        constexpr int dirs_car[7] = {D_T, D_P, D_R, D_B, D_G, D_F, D_V};
-#pragma unroll
-        for (int q = 0; q < NPL; ++q) {
-          const int dd = (RF == FZ_RF_SPHERICAL || RF == RF_CART_TBV) ? dirs_sph[q] : dirs_car[q];
-          if (HEX && dd != D_T && dd != D_P) evol_dir(E, dx[dd], dz, vo, m4vo, loc[dd]);
-          else evol_dir(E, dx[dd], dz, v, m4v, loc[dd]);
-        }
-        // source-function term (1 - O) e0 dS/dT for T
-#pragma unroll
-        for (int i = 0; i < 4; ++i) loc[D_T][i] += ((i == 0 ? 1.f : 0.f) - E.O[i][0]) * dS;
-        if constexpr (HEX) {
-          const float mu = a.atm[A_MU * ps + k * cs + col];
-          const float gk = -mu * c_cfg.he_cte[k] * ly.iT * ly.iT;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) loc[D_T][i] += gk * scr[(long)((nz + k) * 4 + i) * sstr];
-        }
-        float lp[NPL][4];
-        if constexpr (RF == FZ_RF_SPHERICAL) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            lp[0][i] = loc[D_T][i];
-            lp[1][i] = loc[D_B][i];
-            lp[2][i] = loc[D_G][i];
-            lp[3][i] = loc[D_F][i];
-            lp[4][i] = loc[D_V][i];
-          }
-        } else {
-          // chain rule (|B|, gamma, phi) -> (Bx, By, Bz).  With B = 0 every
-          // field derivative is zero, as in the reference (absorption_matrix.f90:1842-1866);
-          // with a vertical field the azimuth terms are dropped (the reference's
-          // d cos2phi / dBx is 0/0 there).
-          const float* at = a.atm + k * cs + col;
-          const float bx = at[A_BX * ps], by = at[A_BY * ps], bz = at[A_BZ * ps];
-          const float bt2 = bx * bx + by * by, bt = sqrtf(bt2), B = ly.g.B, B2 = B * B;
-          const bool hasB = B > 0.f, hasT = bt2 > 0.f;
-          const float iB = hasB ? 1.f / B : 0.f, iBt = hasT ? 1.f / (B2 * bt) : 0.f, ibt2 = hasT ? 1.f / bt2 : 0.f;
-          const float dB[3] = {bx * iB, by * iB, bz * iB};
-          const float dG[3] = {bz * bx * iBt, bz * by * iBt, hasB ? -bt / B2 : 0.f};
-          const float dF[3] = {-by * ibt2, bx * ibt2, 0.f};
-          // slots T, (Pg, rho,) Bx, By, Bz, v_z
-          constexpr int o = RF == RF_CART_TBV ? 0 : 2;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            lp[0][i] = loc[D_T][i];
-            if constexpr (RF != RF_CART_TBV) {
-              lp[1][i] = loc[D_P][i];
-              lp[2][i] = loc[D_R][i];
-            }
-#pragma unroll
-            for (int j = 0; j < 3; ++j)
-              lp[1 + o + j][i] = dB[j] * loc[D_B][i] + dG[j] * loc[D_G][i] + dF[j] * loc[D_F][i];
-            lp[4 + o][i] = loc[D_V][i];
-          }
-        }
-#pragma unroll
-        for (int p = 0; p < NPL; ++p)
+            for (int s = 0; s < 4; ++s) outv[p][s] = 0.f;
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            outv[p][i] = acc[i][0] * lp[p][0] + acc[i][1] * lp[p][1] + acc[i][2] * lp[p][2] + acc[i][3] * lp[p][3];
-        if constexpr (RF == FZ_RF_CARTESIAN_P0) {
-          // P0 (forward.f90:543-545): the local response is 1 in every Stokes
-          // parameter; below the top it is propagated and then multiplied,
-          // component by component, by PG(K)/PG(NZ) and the propagated Pg|T
-          // response of the same height; the top layer keeps 1
-          if (k == nz - 1) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) outv[7][i] = 1.f;
-          } else {
-            const float ratio = a.atm[A_PG * ps + k * cs + col] / a.atm[A_PG * ps + (nz - 1) * cs + col];
+            for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+        } else {
+          const float4 h1 = R[1], h2 = R[2], h3 = R[3], rg = R[REC_HEAD / 4];
+          const float dz = c_cfg.dz_cm[k];
+          // S = c1 / (ex - 1), dS/dT = S (ex / (ex - 1)) (c2 / T) / T
+          const float x = c2 * h0.z;
+          const float ex = depart(k) * expf(x);
+          const float iem1 = 1.0f / (ex - 1.0f);
+          const float S = c1 * iem1;
+          const float dS = S * (ex * iem1) * x * h0.z;
+          const Mix mx = {h1.z, h1.w, h2.x, h2.y, h2.z};
+          Sums X, XT, XV, XB, XP, XR;
+          absorb_der<PR>(R + REC_HEAD / 4 + 1, r, wave, h1.y, dz, X, XT, XV, XB, XP, XR);
+          Five f = mix(mx, X);
+          f.I = fmaf(rg.x, dz, f.I);
+          Evol E;
+          evol_build<true>(f, E);
+          float v[4], vf[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-              outv[7][i] = (acc[i][0] + acc[i][1] + acc[i][2] + acc[i][3]) * ratio * outv[1][i];
+          for (int s = 0; s < 4; ++s) v[s] = scr[(long)(k * 4 + s) * sstr] - (s == 0 ? S : 0.f);
+          turn(h3.x, h3.y, v, vf);
+          // local responses in the frame: lp[0] = T, then (Pg, rho,) and the field's
+          float lp[NPL][4], lB[4], lG[4], lF[4];
+          constexpr int o = PR ? 2 : 0;
+          {
+            const Pieces w = evol_pieces(E, vf);
+            Grad G;
+            evol_grad(E, vf, w, G);
+            Five fd = mix(mx, XT);
+            fd.I = fmaf(rg.y, dz, fd.I);
+            grad_dot(G, fd, lp[0]);
+            if constexpr (PR) {
+              fd = mix(mx, XP);
+              fd.I = fmaf(rg.z, dz, fd.I);
+              grad_dot(G, fd, lp[1]);
+            }
+            if constexpr (HEX) {
+              float vo[4], vof[4];
+#pragma unroll
+              for (int s = 0; s < 4; ++s)
+                vo[s] = (k == nz - 1 ? I[s] : scr[(long)((k + 1) * 4 + s) * sstr]) - (s == 0 ? S : 0.f);
+              turn(h3.x, h3.y, vo, vof);
+              const Pieces wo = evol_pieces(E, vof);
+              evol_grad(E, vof, wo, G);
+              evol_azimuth(E, vof, wo, lF);
+            } else {
+              evol_azimuth(E, vf, w, lF);
+            }
+            if constexpr (PR) {
+              fd = mix(mx, XR);
+              fd.I = fmaf(rg.w, dz, fd.I);
+              grad_dot(G, fd, lp[2]);
+            }
+            grad_dot(G, mix(mx, XB), lB);
+            grad_dot(G, mix(mx, XV), lp[4 + o]);
+            // the inclination: I and q share their factor, d sin^2 = 2 sg cg
+            const Mix mg = {h3.z, -0.5f * h3.z, h3.z, 0.5f * h3.z, -0.5f * h2.w};
+            grad_dot(G, mix(mg, X), lG);
           }
+          // source-function term (1 - O) e0 dS/dT for T; O e0 in the frame
+          {
+            const float alx = -fmaf(E.ga, E.ex, E.gb * E.rx), alz = -fmaf(E.ga, E.ez, E.gb * E.rz);
+            lp[0][0] = fmaf(1.f - fmaf(E.D4, E.s0, E.A), dS, lp[0][0]);
+            lp[0][1] = fmaf(-alx, dS, lp[0][1]);
+            lp[0][2] = fmaf(E.D4 * E.cy, dS, lp[0][2]);
+            lp[0][3] = fmaf(-alz, dS, lp[0][3]);
+          }
+          if constexpr (HEX) {
+            const float mu = a.atm[A_MU * ps + k * cs + col];
+            const float gk = -mu * c_cfg.he_cte[k] * h0.z * h0.z;
+            float W[4], Wf[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) W[i] = scr[(long)((nz + k) * 4 + i) * sstr];
+            turn(h3.x, h3.y, W, Wf);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) lp[0][i] = fmaf(gk, Wf[i], lp[0][i]);
+          }
+          if constexpr (RF == FZ_RF_SPHERICAL) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              lp[1][i] = lB[i];
+              lp[2][i] = lG[i];
+              lp[3][i] = lF[i];
+            }
+          } else {
+            // chain rule (|B|, gamma, phi) -> (Bx, By, Bz)
+            const float4 h4 = R[4], h5 = R[5];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              lp[1 + o][i] = fmaf(h4.x, lB[i], fmaf(h4.w, lG[i], h5.z * lF[i]));
+              lp[2 + o][i] = fmaf(h4.y, lB[i], fmaf(h5.x, lG[i], h5.w * lF[i]));
+              lp[3 + o][i] = fmaf(h4.z, lB[i], h5.y * lG[i]);
+            }
+          }
+          // acc in the frame, the propagated responses, and the running
+          // product O_nz ... O_k = acc (A 1 + turned-back (O - A 1))
+          float na[4][4];
+          const float M11 = E.D4 * (fmaf(E.ex, E.ex, E.rx * E.rx) - E.s0), M33 = E.D4 * (fmaf(E.ez, E.ez, E.rz * E.rz) - E.s0);
+          const float M00 = E.D4 * E.s0, M02 = E.D4 * E.cy, M13 = E.D4 * fmaf(E.ex, E.ez, E.rx * E.rz);
+          const float M01 = -fmaf(E.ga, E.ex, E.gb * E.rx), M03 = -fmaf(E.ga, E.ez, E.gb * E.rz);
+          const float M12 = fmaf(E.ga, E.rz, -(E.gb * E.ez)), M23 = fmaf(E.ga, E.rx, -(E.gb * E.ex));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            float b[4];
+            turn(h3.x, h3.y, acc[i], b);
+#pragma unroll
+            for (int p = 0; p < NPL; ++p)
+              outv[p][i] = fmaf(b[0], lp[p][0], fmaf(b[1], lp[p][1], fmaf(b[2], lp[p][2], b[3] * lp[p][3])));
+            float m[4];
+            m[0] = fmaf(b[0], M00, fmaf(b[1], M01, fmaf(-b[2], M02, b[3] * M03)));
+            m[1] = fmaf(b[0], M01, fmaf(b[1], M11, fmaf(-b[2], M12, b[3] * M13)));
+            m[2] = fmaf(b[0], M02, fmaf(b[1], M12, fmaf(-b[2], M00, -(b[3] * M23))));
+            m[3] = fmaf(b[0], M03, fmaf(b[1], M13, fmaf(b[2], M23, b[3] * M33)));
+            turn_back(h3.x, h3.y, m);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) na[i][j] = fmaf(E.A, acc[i][j], m[j]);
+          }
+          if constexpr (RF == FZ_RF_CARTESIAN_P0) {
+            // P0 (forward.f90:543-545): the local response is 1 in every Stokes
+            // parameter; below the top it is propagated and then multiplied,
+            // component by component, by PG(K)/PG(NZ) and the propagated Pg|T
+            // response of the same height; the top layer keeps 1
+            if (k == nz - 1) {
+#pragma unroll
+              for (int i = 0; i < 4; ++i) outv[7][i] = 1.f;
+            } else {
+              const float ratio = a.atm[A_PG * ps + k * cs + col] / a.atm[A_PG * ps + (nz - 1) * cs + col];
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                outv[7][i] = (acc[i][0] + acc[i][1] + acc[i][2] + acc[i][3]) * ratio * outv[1][i];
+            }
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[i][j] = na[i][j];
         }
-        // running product O_nz ... O_k
-        float nacc[4][4];
+        if (live) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+          for (int p = 0; p < NP; ++p)
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
-            nacc[i][j] = acc[i][0] * E.O[0][j] + acc[i][1] * E.O[1][j] + acc[i][2] * E.O[2][j] + acc[i][3] * E.O[3][j];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) acc[i][j] = nacc[i][j];
+            for (int s = 0; s < 4; ++s) jb[((long)(p * nz + k) * 4 + s) * snumw] = outv[p][s] * gn[s];
+        }
       }
-#pragma unroll
-      for (int p = 0; p < NP; ++p)
-#pragma unroll
-        for (int s = 0; s < 4; ++s) jb[((long)(p * nz + k) * 4 + s) * snumw] = outv[p][s] * gn[s];
     }
   }
 }
@@ -1583,10 +1673,13 @@ static int zeeman_host(const fz_line& L, std::vector<float>& shift, std::vector<
   for (int t = 0; t < 3; ++t) {
     double sum = 0.0;
     for (double v : st[t]) sum += v;
-    ntype[t] = (int)st[t].size();
+    ntype[t] = 0;
     for (size_t i = 0; i < st[t].size(); ++i) {
+      // the pi component 0 -> 0 of a J = J transition has no strength
+      if (st[t][i] == 0.0) continue;
       shift.push_back((float)sh[t][i]);
       str.push_back((float)(st[t][i] / sum));
+      ++ntype[t];
     }
   }
   return 0;
@@ -1635,9 +1728,21 @@ int fz_configure(fz_ctx* c, const fz_line* lines, int nlines, const fz_region* r
     if (zeeman_host(L, shift, str, g.ntype[i]) != 0) return set_err(c, FZ_ECONFIG, "|Delta J| > 1");
   }
   if ((int)shift.size() > MAXC) return set_err(c, FZ_ECONFIG, "too many Zeeman components");
-  for (size_t i = 0; i < shift.size(); ++i) {
-    g.comp_shift[i] = shift[i];
-    g.comp_str[i] = str[i];
+  for (int i = 0; i < nlines; ++i) {
+    size_t m = (size_t)g.comp0[i];
+    for (int t = 0; t < 3; ++t) {
+      double c0 = 0.0, w = 0.0, w1 = 0.0;
+      for (int j = 0; j < g.ntype[i][t]; ++j) c0 += (double)str[m + j] * (double)shift[m + j];
+      const float cen = (float)c0;
+      for (int j = 0; j < g.ntype[i][t]; ++j, ++m) {
+        const float dl = (float)((double)shift[m] - (double)cen), st = str[m];
+        g.comp[m] = {dl, st, (float)((double)st * dl), (float)((double)st * dl * dl)};
+        w += (double)st;
+        w1 += (double)st * (double)dl;
+      }
+      const double isp = 0.564189583547756;   // 1/sqrt(pi)
+      g.type[i][t] = {cen, (float)(isp * w), (float)(isp * w1), 0.f};
+    }
   }
   int numw = 0, ns = 0;
   for (int r = 0; r < nreg; ++r) {
@@ -1669,8 +1774,11 @@ int fz_configure(fz_ctx* c, const fz_line* lines, int nlines, const fz_region* r
       g.blk_n[g.nbpc] = std::min(RT_WAVE, g.reg_pix0[r] + g.reg_nwave[r] - l0);
       ++g.nbpc;
     }
-  g.fgeo0 = F_REG + 4 * nreg + 8 * ns;
-  g.nfield = g.fgeo0 + NGEO + 1;      // + the line-optical-depth factor
+  g.rec = REC_HEAD;
+  for (int r = 0; r < nreg; ++r) {
+    g.reg_rec[r] = g.rec;
+    g.rec += REC_REG + REC_SLOT * g.reg_nblend[r];
+  }
   set_xi(g, matom, c->xi);
   // layer thickness uses the spacing to the next height, the top one the
   // spacing below (rtesolver.f90:439-443); z rounded to REAL(4) like MODEL(:,13)
@@ -1983,41 +2091,42 @@ static int rf_nparam(int rf_mode) {
          : 0;
 }
 
-static int launch_rt(fz_ctx* c, int rf_mode, const RtArgs& a, hipStream_t st, int nitems = 0) {
+static int launch_rt(fz_ctx* c, int rf_mode, RtArgs a, hipStream_t st, int nitems = 0) {
   if (a.items && nitems == 0) return FZ_OK;
+  const Cfg& g = c->cfg;
   // packed lanes for one region without windows (the HYDROSTATIC and P0
   // instances keep one region-uniform wave per 64 wavelengths)
-  const bool pack = !a.items && c->cfg.nreg == 1 && !c->hydro && rf_mode != FZ_RF_CARTESIAN_P0;
-  const unsigned npack = (unsigned)(((long)a.ntile * c->cfg.numw + RT_WAVE - 1) / RT_WAVE);
-  const dim3 grid(a.items ? (unsigned)nitems : pack ? npack : (unsigned)a.ntile * (unsigned)c->cfg.nbpc),
-      blk(RT_WAVE);
-#define FZ_RT_ARGS                                                                                               \
-  a.atm, a.micro, a.gain, a.status, a.stokes, a.jac, a.scratch, a.ncol, a.col0, a.ntile, a.jcol0, a.items, a.poff, \
-      c->pop_on ? c->d_pop : nullptr, a.fs
+  const bool pack = !a.items && g.nreg == 1 && !c->hydro && rf_mode != FZ_RF_CARTESIAN_P0;
+  const unsigned npack = (unsigned)(((long)a.ntile * g.numw + RT_WAVE - 1) / RT_WAVE);
+  const dim3 grid(a.items ? (unsigned)nitems : pack ? npack : (unsigned)a.ntile * (unsigned)g.nbpc), blk(RT_WAVE);
+  // a wave's share of LDS: as many heights of its columns' records as 10 KB
+  // hold (16 waves per CU), one at least
+  int nb = 0;
+  for (int r = 0; r < g.nreg; ++r) nb = std::max(nb, g.reg_nblend[r]);
+  a.wcols = pack ? std::min(a.ntile, 1 + (RT_WAVE - 1 + g.numw - 1) / g.numw) : 1;
+  const size_t per = sizeof(float) * (REC_HEAD + REC_REG + REC_SLOT * (size_t)nb) * a.wcols;
+  a.chunk = (int)std::max<size_t>(1, std::min<size_t>((size_t)std::min(16, g.nz), RT_LDS / per));
+  const size_t lds = per * a.chunk;
+  a.pop = c->pop_on ? c->d_pop : nullptr;
+#define FZ_RT(RF, HE, PK) hipLaunchKernelGGL((rt_kernel<RF, HE, PK>), grid, blk, lds, st, a)
   if (pack) {
-    if (rf_mode == FZ_RF_NONE) hipLaunchKernelGGL((rt_kernel<FZ_RF_NONE, false, true>), grid, blk, 0, st, FZ_RT_ARGS);
-    else if (rf_mode == FZ_RF_SPHERICAL)
-      hipLaunchKernelGGL((rt_kernel<FZ_RF_SPHERICAL, false, true>), grid, blk, 0, st, FZ_RT_ARGS);
-    else if (rf_mode == RF_CART_TBV)
-      hipLaunchKernelGGL((rt_kernel<RF_CART_TBV, false, true>), grid, blk, 0, st, FZ_RT_ARGS);
-    else hipLaunchKernelGGL((rt_kernel<FZ_RF_CARTESIAN, false, true>), grid, blk, 0, st, FZ_RT_ARGS);
+    if (rf_mode == FZ_RF_NONE) FZ_RT(FZ_RF_NONE, false, true);
+    else if (rf_mode == FZ_RF_SPHERICAL) FZ_RT(FZ_RF_SPHERICAL, false, true);
+    else if (rf_mode == RF_CART_TBV) FZ_RT(RF_CART_TBV, false, true);
+    else FZ_RT(FZ_RF_CARTESIAN, false, true);
   }
-  else if (rf_mode == FZ_RF_NONE) hipLaunchKernelGGL((rt_kernel<FZ_RF_NONE, false, false>), grid, blk, 0, st, FZ_RT_ARGS);
-  else if (!c->hydro && rf_mode == FZ_RF_SPHERICAL)
-    hipLaunchKernelGGL((rt_kernel<FZ_RF_SPHERICAL, false, false>), grid, blk, 0, st, FZ_RT_ARGS);
-  else if (!c->hydro && rf_mode == FZ_RF_CARTESIAN_P0)
-    hipLaunchKernelGGL((rt_kernel<FZ_RF_CARTESIAN_P0, false, false>), grid, blk, 0, st, FZ_RT_ARGS);
+  else if (rf_mode == FZ_RF_NONE) FZ_RT(FZ_RF_NONE, false, false);
+  else if (!c->hydro && rf_mode == FZ_RF_SPHERICAL) FZ_RT(FZ_RF_SPHERICAL, false, false);
+  else if (!c->hydro && rf_mode == FZ_RF_CARTESIAN_P0) FZ_RT(FZ_RF_CARTESIAN_P0, false, false);
   else if (rf_mode == RF_CART_TBV) {
     if (c->hydro) return set_err(c, FZ_ECONFIG, "reduced response set without HYDROSTATIC only");
-    hipLaunchKernelGGL((rt_kernel<RF_CART_TBV, false, false>), grid, blk, 0, st, FZ_RT_ARGS);
+    FZ_RT(RF_CART_TBV, false, false);
   }
-  else if (c->hydro && rf_mode == FZ_RF_CARTESIAN_P0)
-    hipLaunchKernelGGL((rt_kernel<FZ_RF_CARTESIAN_P0, true, false>), grid, blk, 0, st, FZ_RT_ARGS);
-  else if (!c->hydro) hipLaunchKernelGGL((rt_kernel<FZ_RF_CARTESIAN, false, false>), grid, blk, 0, st, FZ_RT_ARGS);
-  else if (rf_mode == FZ_RF_SPHERICAL)
-    hipLaunchKernelGGL((rt_kernel<FZ_RF_SPHERICAL, true, false>), grid, blk, 0, st, FZ_RT_ARGS);
-  else hipLaunchKernelGGL((rt_kernel<FZ_RF_CARTESIAN, true, false>), grid, blk, 0, st, FZ_RT_ARGS);
-#undef FZ_RT_ARGS
+  else if (c->hydro && rf_mode == FZ_RF_CARTESIAN_P0) FZ_RT(FZ_RF_CARTESIAN_P0, true, false);
+  else if (!c->hydro) FZ_RT(FZ_RF_CARTESIAN, false, false);
+  else if (rf_mode == FZ_RF_SPHERICAL) FZ_RT(FZ_RF_SPHERICAL, true, false);
+  else FZ_RT(FZ_RF_CARTESIAN, true, false);
+#undef FZ_RT
   HIPCHK(c, hipGetLastError());
   return FZ_OK;
 }
@@ -2179,7 +2288,7 @@ static int forward_impl(fz_ctx* c, int ncol, float* d_atm, int rf_mode, float* d
   HIPCHK(c, hipSetDevice(c->device));
   int r = upload_cfg(c);
   if (r) return r;
-  r = ensure(c, &c->d_micro, &c->micro_cap, sizeof(float) * (size_t)g.nfield * g.nz * ncol);
+  r = ensure(c, &c->d_micro, &c->micro_cap, sizeof(float) * (size_t)(g.rec + 1) * g.nz * ncol);
   if (r) return r;
   // columns per radiative-transfer launch: the configured tile, fewer where
   // its scratch would pass 48 GiB
@@ -2280,7 +2389,7 @@ int fz_line_tau_dev(fz_ctx* c, int ncol, float* d_atm, float* d_tau, int32_t* d_
   HIPCHK(c, hipSetDevice(c->device));
   int r = upload_cfg(c);
   if (r) return r;
-  r = ensure(c, &c->d_micro, &c->micro_cap, sizeof(float) * (size_t)g.nfield * g.nz * ncol);
+  r = ensure(c, &c->d_micro, &c->micro_cap, sizeof(float) * (size_t)(g.rec + 1) * g.nz * ncol);
   if (r) return r;
   r = run_micro(c, ncol, d_atm, &d_status, false, c->hydro, true, st);
   if (r) return r;
@@ -2763,7 +2872,7 @@ int fz_forward_nodes_dev(fz_ctx* c, int ncol, float* d_atm, float* d_stokes, flo
   HIPCHK(c, hipSetDevice(c->device));
   int r = upload_cfg(c);
   if (r) return r;
-  r = ensure(c, &c->d_micro, &c->micro_cap, sizeof(float) * (size_t)g.nfield * g.nz * ncol);
+  r = ensure(c, &c->d_micro, &c->micro_cap, sizeof(float) * (size_t)(g.rec + 1) * g.nz * ncol);
   if (r) return r;
   // the P0 slot is synthesised only when P0 is inverted; the Pg and rho
   // slots only when they are inverted or feed another response (P0, HYDROSTATIC)

@@ -1,64 +1,60 @@
 // FP32 per-(column, wavelength) radiative transfer pieces: Faraday-Voigt
-// profiles, the Zeeman-split propagation matrix and its derivatives, the
-// analytic evolution operator and its directional derivatives.
+// profiles, the evolution operator of a layer in the frame of its field and
+// the gradient of the operator's action.
 #pragma once
 #include <hip/hip_runtime.h>
 
 namespace fz {
 
-struct v3 {
-  float x, y, z;
+// Voigt H(a,u) and Faraday-Voigt L(a,u) = Re, Im of w(u + i a) with the
+// Hui, Armstrong & Wray (1978) 7/7 rational form in z = a - iu (voigt.f:17-98;
+// the coefficients are real, so H is even and L odd in u without |u|).  a > 0
+// always here (radiative damping is positive).  Both polynomials are expanded
+// about a, P(a - iu) = sum_j P^(j)(a)/j! (-iu)^j: even powers of u give the
+// real part, odd ones the imaginary part, as polynomials in u^2 with
+// coefficients of the height and line alone.  opac_kernel forms those in FP64
+// (VoigtPoly); a profile then takes 22 operations and a reciprocal, where
+// evaluating the polynomials at the complex point takes 40.  Largest FP32
+// error against FP64 for a = 1e-4 .. 30, |u| < 60: 2.4e-7 (2.6e-7 before).
+constexpr int NVP = 13;   // p0..p5, q0..q6; p6 and q7 are constants
+constexpr float VOIGT_A6 = .564189583562615f;
+
+struct VoigtPoly {
+  float p[6], q[7];
 };
-__device__ __forceinline__ v3 mk(float x, float y, float z) { return {x, y, z}; }
-__device__ __forceinline__ v3 operator+(v3 a, v3 b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
-__device__ __forceinline__ v3 operator-(v3 a, v3 b) { return {a.x - b.x, a.y - b.y, a.z - b.z}; }
-__device__ __forceinline__ v3 operator*(float s, v3 a) { return {s * a.x, s * a.y, s * a.z}; }
-__device__ __forceinline__ v3 operator-(v3 a) { return {-a.x, -a.y, -a.z}; }
-__device__ __forceinline__ float dot(v3 a, v3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
-__device__ __forceinline__ v3 cross(v3 a, v3 b) {
-  return {a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
+
+__device__ inline void voigt_poly(double a, float* v /*[NVP]*/) {
+  double P[7] = {122.607931777104326, 214.382388694706425, 181.928533092181549, 93.155580458138441,
+                 30.180142196210589, 5.912626209773153, .564189583562615};
+  double Q[8] = {122.60793177387535, 352.730625110963558, 457.334478783897737, 348.703917719495792,
+                 170.354001821091472, 53.992906912940207, 10.479857114260399, 1.0};
+  // Taylor coefficients about a by repeated synthetic division
+#pragma unroll
+  for (int j = 0; j < 6; ++j) {
+#pragma unroll
+    for (int k = 5; k >= j; --k) P[k] = fma(a, P[k + 1], P[k]);
+  }
+#pragma unroll
+  for (int j = 0; j < 7; ++j) {
+#pragma unroll
+    for (int k = 6; k >= j; --k) Q[k] = fma(a, Q[k + 1], Q[k]);
+  }
+#pragma unroll
+  for (int j = 0; j < 6; ++j) v[j] = (float)P[j];
+#pragma unroll
+  for (int j = 0; j < 7; ++j) v[6 + j] = (float)Q[j];
 }
 
-// Voigt H(a,u) and Faraday-Voigt L(a,u) = Re, Im of w(u + i a) with the
-// Hui, Armstrong & Wray (1978) 7/7 rational form in z = a - i|u|; L is odd
-// in u (voigt.f:17-98).  a > 0 always here (radiative damping is positive).
-// Both polynomials have real coefficients, so they are evaluated at the
-// complex point with Knuth's two-FMA recurrence on the quadratic
-// z^2 - 2 Re(z) z + |z|^2 (TAOCP vol. 2, 4.6.4): P(z) = p1 z + p0 after
-// p1 <- p0 + r p1, p0 <- c_k - s p1 with r = 2 Re z, s = |z|^2.
-__device__ __forceinline__ void voigt(float a, float u, float& H, float& F) {
-  const float A0 = 122.607931777104326f, A1 = 214.382388694706425f, A2 = 181.928533092181549f,
-              A3 = 93.155580458138441f, A4 = 30.180142196210589f, A5 = 5.912626209773153f,
-              A6 = .564189583562615f;
-  const float B0 = 122.60793177387535f, B1 = 352.730625110963558f, B2 = 457.334478783897737f,
-              B3 = 348.703917719495792f, B4 = 170.354001821091472f, B5 = 53.992906912940207f,
-              B6 = 10.479857114260399f;
-  const float v = fabsf(u);
-  const float x = a, y = -v;
-  const float r = 2.f * x, s = x * x + y * y;
-  float p1, p0, t;
-  // numerator A6 z^6 + ... + A0
-  p1 = A6;
-  p0 = A5;
-  t = p1; p1 = fmaf(r, t, p0); p0 = fmaf(-s, t, A4);
-  t = p1; p1 = fmaf(r, t, p0); p0 = fmaf(-s, t, A3);
-  t = p1; p1 = fmaf(r, t, p0); p0 = fmaf(-s, t, A2);
-  t = p1; p1 = fmaf(r, t, p0); p0 = fmaf(-s, t, A1);
-  t = p1; p1 = fmaf(r, t, p0); p0 = fmaf(-s, t, A0);
-  const float nr = fmaf(p1, x, p0), ni = p1 * y;
-  // denominator z^7 + B6 z^6 + ... + B0
-  float q1 = 1.f, q0 = B6;
-  t = q1; q1 = fmaf(r, t, q0); q0 = fmaf(-s, t, B5);
-  t = q1; q1 = fmaf(r, t, q0); q0 = fmaf(-s, t, B4);
-  t = q1; q1 = fmaf(r, t, q0); q0 = fmaf(-s, t, B3);
-  t = q1; q1 = fmaf(r, t, q0); q0 = fmaf(-s, t, B2);
-  t = q1; q1 = fmaf(r, t, q0); q0 = fmaf(-s, t, B1);
-  t = q1; q1 = fmaf(r, t, q0); q0 = fmaf(-s, t, B0);
-  const float dr = fmaf(q1, x, q0), di = q1 * y;
-  const float inv = __builtin_amdgcn_rcpf(fmaf(dr, dr, di * di));
-  H = fmaf(nr, dr, ni * di) * inv;
-  const float im = fmaf(ni, dr, -nr * di) * inv;
-  F = (u < 0.f) ? -im : im;
+__device__ __forceinline__ void voigt(const VoigtPoly& c, float u, float& H, float& F) {
+  const float s = u * u;
+  const float nr = fmaf(fmaf(fmaf(-VOIGT_A6, s, c.p[4]), s, -c.p[2]), s, c.p[0]);
+  const float ni = fmaf(fmaf(c.p[5], s, -c.p[3]), s, c.p[1]);             // Im P = -u ni
+  const float dr = fmaf(fmaf(fmaf(-c.q[6], s, c.q[4]), s, -c.q[2]), s, c.q[0]);
+  const float di = fmaf(fmaf(c.q[5] - s, s, -c.q[3]), s, c.q[1]);         // Im Q = -u di
+  const float sd = s * di;
+  const float inv = __builtin_amdgcn_rcpf(fmaf(dr, dr, sd * di));
+  H = fmaf(nr, dr, ni * sd) * inv;
+  F = (u * inv) * fmaf(nr, di, -(ni * dr));
 }
 
 // Field geometry of one height (absorption_matrix.f90:1800-1871): |B|,
@@ -92,18 +88,17 @@ __device__ __forceinline__ Geo geometry(float bx, float by, float bz) {
   return g;
 }
 
-// 4-vector helpers
-struct V4 {
-  float v[4];
+// Frame of a layer.  Every line and every direction but the azimuth moves Q
+// and U along (cos 2phi, sin 2phi), so in the (Q, U) axes turned by 2phi the
+// propagation matrix has five elements, (eta_I, eta_q, eta_V, rho_q, rho_V),
+// and the vectors e = (eta_q, 0, eta_V), r = (rho_q, 0, rho_V) no second
+// component.  Stokes vectors are turned into the frame, the operator's part
+// beyond A times the identity is applied there, and the result turned back;
+// the part A * 1 is applied unturned, so that a transparent layer does not
+// pick up the rounding of cos^2 + sin^2.
+struct Five {
+  float I, q, V, qF, VF;
 };
-
-// (P(a,w) v) for the matrix [[0,a1,a2,a3],[a1,0,w3,-w2],[a2,-w3,0,w1],[a3,w2,-w1,0]]
-__device__ __forceinline__ void pmul(v3 a, v3 w, const float* v, float* o) {
-  o[0] = a.x * v[1] + a.y * v[2] + a.z * v[3];
-  o[1] = a.x * v[0] + w.z * v[2] - w.y * v[3];
-  o[2] = a.y * v[0] - w.z * v[1] + w.x * v[3];
-  o[3] = a.z * v[0] + w.y * v[1] - w.x * v[2];
-}
 
 // Evolution operator of a constant-property layer, O = exp(-K dz), in the
 // closed form of Landi Degl'Innocenti & Landi Degl'Innocenti (1985)
@@ -112,6 +107,7 @@ __device__ __forceinline__ void pmul(v3 a, v3 w, const float* v, float* o) {
 // formed without cancellation (lambda1*lambda2 = |eta.rho|), and the
 // exp(-eta_I dz) factor is folded into cosh/sinh so nothing overflows.
 //   O = A*1 + P(alpha, omega) + D4 * M4raw
+// with alpha = -(ga e + gb r), omega = -(gb e - ga r).
 //
 // Near-degenerate polarisation eigenvalues.  The closed form divides by
 // th = sqrt(d^2 + 4 (e.r)^2) and by l1, l2; when th is small the terms of
@@ -123,257 +119,250 @@ __device__ __forceinline__ void pmul(v3 a, v3 w, const float* v, float* o) {
 //   D4 e^ei = (cosh l1 - cos l2)/th           = sum_{n>=1} H_{n-1} / (2n)!
 //   ga e^ei = (l1 sinh l1 + l2 sin l2)/th     = sum_n H_n / (2n+1)!
 //   gb e^ei = e.r (sinh l1/l1 - sin l2/l2)/th = e.r sum_{n>=1} H_{n-1} / (2n+1)!
-// where P_n = x^n + y^n and H_n = sum_{i<=n} x^i y^(n-i) both follow
-// F_n = d F_{n-1} + q F_{n-2} (P_0 = 2, H_0 = 1, F_1 = d), so the series and
-// their d- and q-derivatives need no square root and no division.  For
-// th < TH_SER the operator and its derivatives use these series (NSER terms,
-// truncation below 1e-11 at th = 2); the closed form is kept above, where
-// th is not small against s0 unless the layer is optically thick and
+// where H_n = sum_{i<=n} x^i y^(n-i) follows H_n = d H_{n-1} + q H_{n-2}
+// (H_0 = 1, H_1 = d) and P_n = x^n + y^n = 2 H_n - d H_{n-1}.  With
+// dP_n/dd = n H_{n-1}, dP_n/dq = n H_{n-2} and dH_n/dq = dH_{n-1}/dd (from
+// the generating functions) the d- and q-derivatives need one more recurrence,
+// H'_n = dH_n/dd, and those of A are the ga and gb series over 4.  For
+// th < TH_SER the operator and its derivatives use these series (terms below
+// NSER; |x|, |y| <= 2, truncation below 2e-10); the closed form is kept above,
+// where th is not small against s0 unless the layer is optically thick and
 // e^-ei removes it.
 constexpr float TH_SER = 2.0f;
-constexpr int NSER = 9;
-
-// Fields of one branch of the operator in a shared array (a lane takes one
-// branch; sharing keeps the register footprint of the struct that of one):
-// closed form: 1/l1 or 1/l2, 1/th, l1, l2, sign(e.r), C2, B3, and the
-// e^-ei cosh/sinh/cos/sin products; series: the d- and q-derivatives of the
-// A, D4, ga and gb series, the gb series and e^-ei.
-enum { W_IL = 0, W_ITH, W_L1, W_L2, W_SIG, W_C2, W_B3, W_CHE, W_SHE, W_CE, W_SE, NW };
-enum { W_AD = 0, W_AQ, W_DD, W_DQ, W_GD, W_GQ, W_BD, W_BQ, W_SB, W_EX };
+constexpr int NSER = 8;
 
 struct Evol {
-  float O[4][4];
-  v3 e, r;
-  float ei, th, d, er;
-  float A, D4, s0;
-  // al = -(ga e + gb r) and om = -(gb e - ga r)
-  float ga, gb;
-  bool ser;
-  float w[NW];
+  float ex, ez, rx, rz;        // e and r in the frame of the field
+  float A, D4, ga, gb, s0, cy; // cy: (e x r) along the second axis
+  // partial derivatives of A, D4, ga, gb in d and e.r (with DER)
+  float Ad, Ae, Dd, De, gad, gae, gbd, gbe;
 };
 
-// the four coefficient series of the comment above (times e^ei) and, with
-// DER, their partial derivatives in d and q
 template <bool DER>
-__device__ __forceinline__ void evol_series(float d, float q, float& A0, float& D0, float& G0, float& B0, Evol& E) {
-  // 1/k! for k = 0 .. 2 NSER
-  constexpr float IF[2 * NSER + 1] = {1.f, 1.f, 1.f / 2.f, 1.f / 6.f, 1.f / 24.f, 1.f / 120.f, 1.f / 720.f,
-                                      1.f / 5040.f, 1.f / 40320.f, 1.f / 362880.f, 1.f / 3628800.f,
-                                      1.f / 39916800.f, 1.f / 479001600.f, 1.f / 6227020800.f,
-                                      1.f / 87178291200.f, 1.f / 1307674368000.f, 1.f / 20922789888000.f,
-                                      1.f / 355687428096000.f, 1.f / 6402373705728000.f};
-  // F_n and its d-, q-derivatives for H (h*) and P (p*), n = 0 .. NSER - 1
-  float h0 = 1.f, h1 = d, hd0 = 0.f, hd1 = 1.f, hq0 = 0.f, hq1 = 0.f;
-  float p0 = 2.f, p1 = d, pd0 = 0.f, pd1 = 1.f, pq0 = 0.f, pq1 = 0.f;
-  A0 = 0.5f * p0;
-  D0 = 0.f;
-  G0 = h0 * IF[1];
-  B0 = 0.f;
-  float Ad = 0.f, Aq = 0.f, Dd = 0.f, Dq = 0.f, Gd = 0.f, Gq = 0.f, Bd = 0.f, Bq = 0.f;
-#pragma unroll
-  for (int n = 1; n < NSER; ++n) {
-    // terms with H_{n-1} (held in h0 ...) and P_n, H_n (held in p1, h1 ...)
-    A0 += 0.5f * p1 * IF[2 * n];
-    D0 += h0 * IF[2 * n];
-    G0 += h1 * IF[2 * n + 1];
-    B0 += h0 * IF[2 * n + 1];
-    if (DER) {
-      Ad += 0.5f * pd1 * IF[2 * n];
-      Aq += 0.5f * pq1 * IF[2 * n];
-      Dd += hd0 * IF[2 * n];
-      Dq += hq0 * IF[2 * n];
-      Gd += hd1 * IF[2 * n + 1];
-      Gq += hq1 * IF[2 * n + 1];
-      Bd += hd0 * IF[2 * n + 1];
-      Bq += hq0 * IF[2 * n + 1];
-    }
-    // advance to n + 1
-    const float h2 = d * h1 + q * h0, p2 = d * p1 + q * p0;
-    if (DER) {
-      const float hd2 = h1 + d * hd1 + q * hd0, hq2 = d * hq1 + h0 + q * hq0;
-      const float pd2 = p1 + d * pd1 + q * pd0, pq2 = d * pq1 + p0 + q * pq0;
-      hd0 = hd1;
-      hd1 = hd2;
-      hq0 = hq1;
-      hq1 = hq2;
-      pd0 = pd1;
-      pd1 = pd2;
-      pq0 = pq1;
-      pq1 = pq2;
-    }
-    h0 = h1;
-    h1 = h2;
-    p0 = p1;
-    p1 = p2;
-  }
-  if (DER) {
-    E.w[W_AD] = Ad;
-    E.w[W_AQ] = Aq;
-    E.w[W_DD] = Dd;
-    E.w[W_DQ] = Dq;
-    E.w[W_GD] = Gd;
-    E.w[W_GQ] = Gq;
-    E.w[W_BD] = Bd;
-    E.w[W_BQ] = Bq;
-  }
-}
-
-template <bool DER>
-__device__ __forceinline__ void evol_build(const float x7[7], float dz, Evol& E) {
-  E.ei = x7[0] * dz;
-  E.e = mk(x7[1] * dz, x7[2] * dz, x7[3] * dz);
-  E.r = mk(x7[4] * dz, x7[5] * dz, x7[6] * dz);
-  const float e2 = dot(E.e, E.e), r2 = dot(E.r, E.r);
-  E.er = dot(E.e, E.r);
-  E.d = e2 - r2;
+__device__ __forceinline__ void evol_build(const Five& f, Evol& E) {
+  // 1/k! for k = 0 .. 2 NSER - 1
+  constexpr float IF[2 * NSER] = {1.f, 1.f, 1.f / 2.f, 1.f / 6.f, 1.f / 24.f, 1.f / 120.f, 1.f / 720.f,
+                                  1.f / 5040.f, 1.f / 40320.f, 1.f / 362880.f, 1.f / 3628800.f,
+                                  1.f / 39916800.f, 1.f / 479001600.f, 1.f / 6227020800.f,
+                                  1.f / 87178291200.f, 1.f / 1307674368000.f};
+  E.ex = f.q;
+  E.ez = f.V;
+  E.rx = f.qF;
+  E.rz = f.VF;
+  const float e2 = fmaf(E.ex, E.ex, E.ez * E.ez), r2 = fmaf(E.rx, E.rx, E.rz * E.rz);
+  const float er = fmaf(E.ex, E.rx, E.ez * E.rz), d = e2 - r2;
+  E.s0 = 0.5f * (e2 + r2);
+  E.cy = fmaf(E.ez, E.rx, -(E.ex * E.rz));
   // hypot without its scaling unless the squares could overflow
-  E.th = (fabsf(E.d) < 1.0e18f && fabsf(E.er) < 1.0e18f) ? sqrtf(E.d * E.d + 4.0f * E.er * E.er)
-                                                          : hypotf(E.d, 2.0f * E.er);
-  E.ser = E.th < TH_SER;
-  if (E.ser) {
-    float A0, D0, G0, B0;
-    evol_series<DER>(E.d, E.er * E.er, A0, D0, G0, B0, E);
-    E.w[W_EX] = expf(-E.ei);
-    E.w[W_SB] = B0;
-    E.A = E.w[W_EX] * A0;
-    E.D4 = E.w[W_EX] * D0;
-    E.ga = E.w[W_EX] * G0;
-    E.gb = E.w[W_EX] * (E.er * B0);
-  } else {
-    float l1, l2;
-    if (E.d >= 0.f) {
-      l1 = sqrtf(0.5f * (E.th + E.d));
-      E.w[W_IL] = l1 > 0.f ? 1.0f / l1 : 0.f;
-      l2 = fabsf(E.er) * E.w[W_IL];
-    } else {
-      l2 = sqrtf(0.5f * (E.th - E.d));
-      E.w[W_IL] = 1.0f / l2;
-      l1 = fabsf(E.er) * E.w[W_IL];
+  const float th = (fabsf(d) < 1.0e18f && fabsf(er) < 1.0e18f) ? sqrtf(fmaf(d, d, 4.0f * er * er)) : hypotf(d, 2.0f * er);
+  const float ex = expf(-f.I);
+  if (th < TH_SER) {
+    const float q = er * er;
+    float h0 = 1.f, h1 = d, g0 = 0.f, g1 = 1.f, gm = 0.f;     // H_{n-1}, H_n, H'_{n-1}, H'_n, H'_{n-2}
+    float C = 1.f, G = 1.f, D = 0.f, B = 0.f;
+    float Dd = 0.f, Dq = 0.f, Gd = 0.f, Bd = 0.f, Bq = 0.f;
+#pragma unroll
+    for (int n = 1; n < NSER; ++n) {
+      C = fmaf(h1, IF[2 * n], C);
+      G = fmaf(h1, IF[2 * n + 1], G);
+      D = fmaf(h0, IF[2 * n], D);
+      B = fmaf(h0, IF[2 * n + 1], B);
+      if (DER) {
+        if (n > 1) {
+          Dd = fmaf(g0, IF[2 * n], Dd);
+          Bd = fmaf(g0, IF[2 * n + 1], Bd);
+        }
+        if (n > 2) {
+          Dq = fmaf(gm, IF[2 * n], Dq);
+          Bq = fmaf(gm, IF[2 * n + 1], Bq);
+        }
+        Gd = fmaf(g1, IF[2 * n + 1], Gd);
+        gm = g0;
+        const float g2 = fmaf(d, g1, fmaf(q, g0, h1));
+        g0 = g1;
+        g1 = g2;
+      }
+      const float h2 = fmaf(d, h1, q * h0);
+      h0 = h1;
+      h1 = h2;
     }
-    E.w[W_L1] = l1;
-    E.w[W_L2] = l2;
-    E.w[W_SIG] = E.er > 0.f ? 1.f : (E.er < 0.f ? -1.f : 0.f);
+    E.A = ex * fmaf(-0.5f * d, D, C);
+    E.D4 = ex * D;
+    E.ga = ex * G;
+    E.gb = ex * (er * B);
+    if (DER) {
+      const float er2 = 2.f * er;
+      E.Ad = 0.25f * E.ga;
+      E.Ae = (0.25f * er2) * (ex * B);
+      E.Dd = ex * Dd;
+      E.De = ex * (er2 * Dq);
+      E.gad = ex * Gd;
+      E.gae = ex * (er2 * Bd);
+      E.gbd = ex * (er * Bd);
+      E.gbe = ex * fmaf(er * er2, Bq, B);
+    }
+  } else {
+    float l1, l2, il;
+    const bool dp = d >= 0.f;
+    if (dp) {
+      l1 = sqrtf(0.5f * (th + d));
+      il = 1.0f / l1;
+      l2 = fabsf(er) * il;
+    } else {
+      l2 = sqrtf(0.5f * (th - d));
+      il = 1.0f / l2;
+      l1 = fabsf(er) * il;
+    }
+    const float sig = er > 0.f ? 1.f : (er < 0.f ? -1.f : 0.f);
+    float che, she;
     if (l1 < 40.f) {
       // cosh and sinh from one exponential; sinh by its Taylor series below
       // 0.5 (truncation 1e-11 relative), where E - 1/E would cancel
-      const float ex = expf(-E.ei);
       const float El = expf(l1), iEl = 1.0f / El;
       const float x2 = l1 * l1;
       const float shs = l1 * (1.f + x2 * (1.f / 6.f) * (1.f + x2 * (1.f / 20.f) * (1.f + x2 * (1.f / 42.f) * (1.f + x2 * (1.f / 72.f)))));
-      E.w[W_CHE] = ex * (0.5f * (El + iEl));
-      E.w[W_SHE] = ex * (l1 < 0.5f ? shs : 0.5f * (El - iEl));
+      che = ex * (0.5f * (El + iEl));
+      she = ex * (l1 < 0.5f ? shs : 0.5f * (El - iEl));
     } else {
-      const float p = expf(l1 - E.ei), m = expf(-l1 - E.ei);
-      E.w[W_CHE] = 0.5f * (p + m);
-      E.w[W_SHE] = 0.5f * (p - m);
+      const float p = expf(l1 - f.I), m = expf(-l1 - f.I);
+      che = 0.5f * (p + m);
+      she = 0.5f * (p - m);
     }
     float sn, cs;
     sincosf(l2, &sn, &cs);
-    const float ex = expf(-E.ei);
-    E.w[W_CE] = ex * cs;
-    E.w[W_SE] = ex * sn;
-    E.A = 0.5f * (E.w[W_CHE] + E.w[W_CE]);
-    const float ith = E.th > 0.f ? 1.0f / E.th : 0.f;
-    E.w[W_ITH] = ith;
-    E.w[W_C2] = E.w[W_SE] * ith;
-    E.w[W_B3] = E.w[W_SHE] * ith;
-    E.D4 = (E.w[W_CHE] - E.w[W_CE]) * ith;
+    const float ce = ex * cs, se = ex * sn;
+    const float ith = 1.0f / th;
+    const float C2 = se * ith, B3 = she * ith;
+    E.A = 0.5f * (che + ce);
+    E.D4 = (che - ce) * ith;
     // With a2 = l2 e - s l1 r, a3 = l1 e + s l2 r, w2 = -(s l1 e + l2 r) and
     // w3 = s l2 e - l1 r, the vectors al = -(C2 a2 + B3 a3) and
     // om = -(C2 w2 + B3 w3) take two scalars: ga = C2 l2 + B3 l1 and
     // gb = s (B3 l2 - C2 l1).
-    const float s = E.w[W_SIG];
-    E.ga = E.w[W_C2] * l2 + E.w[W_B3] * l1;
-    E.gb = s * (E.w[W_B3] * l2 - E.w[W_C2] * l1);
-  }
-  const v3 al = -(E.ga * E.e + E.gb * E.r);
-  const v3 om = -(E.gb * E.e - E.ga * E.r);
-  E.s0 = 0.5f * (e2 + r2);
-  const v3 c = cross(E.e, E.r);
-  const float D4 = E.D4;
-  const float ev[3] = {E.e.x, E.e.y, E.e.z}, rv[3] = {E.r.x, E.r.y, E.r.z};
-  const float alv[3] = {al.x, al.y, al.z}, cv[3] = {c.x, c.y, c.z};
-  E.O[0][0] = E.A + D4 * E.s0;
+    E.ga = C2 * l2 + B3 * l1;
+    E.gb = sig * (B3 * l2 - C2 * l1);
+    if (DER) {
+      // one pass per variable: dth, dl1, dl2 for a unit change of d, then of e.r
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    E.O[0][k + 1] = alv[k] + D4 * cv[k];
-    E.O[k + 1][0] = alv[k] - D4 * cv[k];
-    E.O[k + 1][k + 1] = E.A + D4 * (ev[k] * ev[k] + rv[k] * rv[k] - E.s0);
-  }
-  E.O[1][2] = om.z + D4 * (ev[0] * ev[1] + rv[0] * rv[1]);
-  E.O[2][1] = -om.z + D4 * (ev[0] * ev[1] + rv[0] * rv[1]);
-  E.O[1][3] = -om.y + D4 * (ev[0] * ev[2] + rv[0] * rv[2]);
-  E.O[3][1] = om.y + D4 * (ev[0] * ev[2] + rv[0] * rv[2]);
-  E.O[2][3] = om.x + D4 * (ev[1] * ev[2] + rv[1] * rv[2]);
-  E.O[3][2] = -om.x + D4 * (ev[1] * ev[2] + rv[1] * rv[2]);
-}
-
-// M4raw v and its pieces (c = e x r)
-__device__ __forceinline__ void m4mul(v3 e, v3 r, float s0, const float* v, float* o) {
-  const v3 c = cross(e, r);
-  const v3 vp = mk(v[1], v[2], v[3]);
-  const float ev = dot(e, vp), rv = dot(r, vp);
-  o[0] = s0 * v[0] + dot(c, vp);
-  o[1] = -c.x * v[0] + e.x * ev + r.x * rv - s0 * vp.x;
-  o[2] = -c.y * v[0] + e.y * ev + r.y * rv - s0 * vp.y;
-  o[3] = -c.z * v[0] + e.z * ev + r.z * rv - s0 * vp.z;
-}
-
-// Directional derivative (dO) v for a change (dx7 * dz) of the propagation
-// matrix; the reference forms the six partial derivatives of O explicitly
-// (rtesolver.f90:476-1002); here one direction costs one pass of this
-// function.
-__device__ __forceinline__ void evol_dir(const Evol& E, const float dx7[7], float dz, const float* v,
-                                         const float* m4v, float* out) {
-  const float dei = dx7[0] * dz;
-  const v3 de = mk(dx7[1] * dz, dx7[2] * dz, dx7[3] * dz);
-  const v3 dr = mk(dx7[4] * dz, dx7[5] * dz, dx7[6] * dz);
-  const float dd = 2.f * (dot(E.e, de) - dot(E.r, dr));
-  const float der = dot(de, E.r) + dot(E.e, dr);
-  float dA, dD4, dga, dgb;
-  if (E.ser) {
-    const float dq = 2.f * E.er * der;
-    dA = -dei * E.A + E.w[W_EX] * (E.w[W_AD] * dd + E.w[W_AQ] * dq);
-    dD4 = -dei * E.D4 + E.w[W_EX] * (E.w[W_DD] * dd + E.w[W_DQ] * dq);
-    dga = -dei * E.ga + E.w[W_EX] * (E.w[W_GD] * dd + E.w[W_GQ] * dq);
-    dgb = -dei * E.gb + E.w[W_EX] * (der * E.w[W_SB] + E.er * (E.w[W_BD] * dd + E.w[W_BQ] * dq));
-  } else {
-    float dth = 0.f, dl1 = 0.f, dl2 = 0.f, ith = 0.f;
-    if (E.th > 0.f) {
-      ith = E.w[W_ITH];
-      dth = (E.d * dd + 4.f * E.er * der) * ith;
-      if (E.d >= 0.f) {
-        dl1 = (dth + dd) * (0.25f * E.w[W_IL]);
-        dl2 = (E.w[W_SIG] * der - E.w[W_L2] * dl1) * E.w[W_IL];
-      } else {
-        dl2 = (dth - dd) * (0.25f * E.w[W_IL]);
-        dl1 = (E.w[W_SIG] * der - E.w[W_L1] * dl2) * E.w[W_IL];
+      for (int v = 0; v < 2; ++v) {
+        const float dd = v == 0 ? 1.f : 0.f, der = v == 0 ? 0.f : 1.f;
+        const float dth = (v == 0 ? d : 4.f * er) * ith;
+        float dl1, dl2;
+        if (dp) {
+          dl1 = (dth + dd) * (0.25f * il);
+          dl2 = (sig * der - l2 * dl1) * il;
+        } else {
+          dl2 = (dth - dd) * (0.25f * il);
+          dl1 = (sig * der - l1 * dl2) * il;
+        }
+        const float dA = 0.5f * (she * dl1 - se * dl2);
+        const float dC2 = (ce * dl2 - C2 * dth) * ith;
+        const float dB3 = (che * dl1 - B3 * dth) * ith;
+        const float dD = (she * dl1 + se * dl2 - E.D4 * dth) * ith;
+        const float dga = dC2 * l2 + C2 * dl2 + dB3 * l1 + B3 * dl1;
+        const float dgb = sig * (dB3 * l2 + B3 * dl2 - dC2 * l1 - C2 * dl1);
+        if (v == 0) {
+          E.Ad = dA; E.Dd = dD; E.gad = dga; E.gbd = dgb;
+        } else {
+          E.Ae = dA; E.De = dD; E.gae = dga; E.gbe = dgb;
+        }
       }
     }
-    dA = -dei * E.A + 0.5f * (E.w[W_SHE] * dl1 - E.w[W_SE] * dl2);
-    const float dC2 = -dei * E.w[W_C2] + (E.w[W_CE] * dl2 - E.w[W_C2] * dth) * ith;
-    const float dB3 = -dei * E.w[W_B3] + (E.w[W_CHE] * dl1 - E.w[W_B3] * dth) * ith;
-    dD4 = -dei * E.D4 + (E.w[W_SHE] * dl1 + E.w[W_SE] * dl2 - E.D4 * dth) * ith;
-    dga = dC2 * E.w[W_L2] + E.w[W_C2] * dl2 + dB3 * E.w[W_L1] + E.w[W_B3] * dl1;
-    dgb = E.w[W_SIG] * (dB3 * E.w[W_L2] + E.w[W_B3] * dl2 - dC2 * E.w[W_L1] - E.w[W_C2] * dl1);
   }
-  // d(al) = -(dga e + ga de + dgb r + gb dr), d(om) = -(dgb e + gb de - dga r - ga dr)
-  const v3 dal = -(dga * E.e + E.ga * de + dgb * E.r + E.gb * dr);
-  const v3 dom = -(dgb * E.e + E.gb * de - dga * E.r - E.ga * dr);
-  float p[4];
-  pmul(dal, dom, v, p);
-  // d(M4raw) v
-  const v3 vp = mk(v[1], v[2], v[3]);
-  const float ds0 = dot(E.e, de) + dot(E.r, dr);
-  const v3 dc = cross(de, E.r) + cross(E.e, dr);
-  const float ev = dot(E.e, vp), dev = dot(de, vp), rv = dot(E.r, vp), drv = dot(dr, vp);
-  float q[4];
-  q[0] = ds0 * v[0] + dot(dc, vp);
-  q[1] = -dc.x * v[0] + de.x * ev + E.e.x * dev + dr.x * rv + E.r.x * drv - ds0 * vp.x;
-  q[2] = -dc.y * v[0] + de.y * ev + E.e.y * dev + dr.y * rv + E.r.y * drv - ds0 * vp.y;
-  q[3] = -dc.z * v[0] + de.z * ev + E.e.z * dev + dr.z * rv + E.r.z * drv - ds0 * vp.z;
+}
+
+// The pieces of (O - A 1) v for a vector v in the frame: M4raw v, P(e, -r) v
+// and P(r, e) v, where P(a, w) = [[0,a1,a2,a3],[a1,0,w3,-w2],[a2,-w3,0,w1],[a3,w2,-w1,0]]
+struct Pieces {
+  float m4[4], p1[4], p2[4];   // p1[0] = e.v, p2[0] = r.v
+};
+
+__device__ __forceinline__ Pieces evol_pieces(const Evol& E, const float v[4]) {
+  Pieces w;
+  const float ev = fmaf(E.ex, v[1], E.ez * v[3]), rv = fmaf(E.rx, v[1], E.rz * v[3]);
+  w.m4[0] = fmaf(E.s0, v[0], E.cy * v[2]);
+  w.m4[1] = fmaf(E.ex, ev, fmaf(E.rx, rv, -(E.s0 * v[1])));
+  w.m4[2] = -fmaf(E.cy, v[0], E.s0 * v[2]);
+  w.m4[3] = fmaf(E.ez, ev, fmaf(E.rz, rv, -(E.s0 * v[3])));
+  w.p1[0] = ev;
+  w.p1[1] = fmaf(E.ex, v[0], -(E.rz * v[2]));
+  w.p1[2] = fmaf(E.rz, v[1], -(E.rx * v[3]));
+  w.p1[3] = fmaf(E.ez, v[0], E.rx * v[2]);
+  w.p2[0] = rv;
+  w.p2[1] = fmaf(E.rx, v[0], E.ez * v[2]);
+  w.p2[2] = fmaf(E.ex, v[3], -(E.ez * v[1]));
+  w.p2[3] = fmaf(E.rz, v[0], -(E.ex * v[2]));
+  return w;
+}
+
+// (O - A 1) v
+__device__ __forceinline__ void evol_apply(const Evol& E, const Pieces& w, float o[4]) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) out[i] = dA * v[i] + p[i] + dD4 * m4v[i] + E.D4 * q[i];
+  for (int i = 0; i < 4; ++i) o[i] = fmaf(E.D4, w.m4[i], -fmaf(E.ga, w.p1[i], E.gb * w.p2[i]));
+}
+
+// Gradient of O v in the five elements of the frame (columns I, q, V, qF, VF)
+// and, for the azimuth, the directional derivative itself.  The reference
+// forms the partial derivatives of O as matrices (rtesolver.f90:476-1002);
+// here the gradient of its action on one vector serves every direction, 20
+// operations each, where a directional derivative by itself took 200.
+struct Grad {
+  float g[5][4];
+};
+
+__device__ __forceinline__ void evol_grad(const Evol& E, const float v[4], const Pieces& w, Grad& G) {
+  float xd[4], xe[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    xd[i] = fmaf(E.Ad, v[i], fmaf(E.Dd, w.m4[i], -fmaf(E.gad, w.p1[i], E.gbd * w.p2[i])));
+    xe[i] = fmaf(E.Ae, v[i], fmaf(E.De, w.m4[i], -fmaf(E.gae, w.p1[i], E.gbe * w.p2[i])));
+    G.g[0][i] = -fmaf(E.A, v[i], fmaf(E.D4, w.m4[i], -fmaf(E.ga, w.p1[i], E.gb * w.p2[i])));
+  }
+  const float ev = w.p1[0], rv = w.p2[0];
+  const float ex = E.ex, ez = E.ez, rx = E.rx, rz = E.rz, D4 = E.D4, ga = E.ga, gb = E.gb;
+  const float ex2 = 2.f * ex, ez2 = 2.f * ez, rx2 = -2.f * rx, rz2 = -2.f * rz;
+  // d(M4raw) v of a unit change of e along the first axis is (ex v0 - rz v2,
+  // e.v, rz v0 - ex v2, ez v1 - ex v3), and so on
+  const float a02 = fmaf(ex, v[0], -(rz * v[2])), a13 = fmaf(ez, v[1], -(ex * v[3]));
+  const float b02 = fmaf(ez, v[0], rx * v[2]);
+  const float c02 = fmaf(rx, v[0], ez * v[2]), c13 = fmaf(rz, v[1], -(rx * v[3]));
+  const float d02 = fmaf(rz, v[0], -(ex * v[2]));
+  G.g[1][0] = fmaf(ex2, xd[0], fmaf(rx, xe[0], fmaf(D4, a02, -(ga * v[1]))));
+  G.g[1][1] = fmaf(ex2, xd[1], fmaf(rx, xe[1], fmaf(D4, ev, -(ga * v[0]))));
+  G.g[1][2] = fmaf(ex2, xd[2], fmaf(rx, xe[2], fmaf(D4, d02, -(gb * v[3]))));
+  G.g[1][3] = fmaf(ex2, xd[3], fmaf(rx, xe[3], fmaf(D4, a13, gb * v[2])));
+  G.g[2][0] = fmaf(ez2, xd[0], fmaf(rz, xe[0], fmaf(D4, b02, -(ga * v[3]))));
+  G.g[2][1] = fmaf(ez2, xd[1], fmaf(rz, xe[1], -fmaf(D4, a13, gb * v[2])));
+  G.g[2][2] = fmaf(ez2, xd[2], fmaf(rz, xe[2], fmaf(-D4, c02, gb * v[1])));
+  G.g[2][3] = fmaf(ez2, xd[3], fmaf(rz, xe[3], fmaf(D4, ev, -(ga * v[0]))));
+  G.g[3][0] = fmaf(rx2, xd[0], fmaf(ex, xe[0], fmaf(D4, c02, -(gb * v[1]))));
+  G.g[3][1] = fmaf(rx2, xd[1], fmaf(ex, xe[1], fmaf(D4, rv, -(gb * v[0]))));
+  G.g[3][2] = fmaf(rx2, xd[2], fmaf(ex, xe[2], fmaf(-D4, b02, ga * v[3])));
+  G.g[3][3] = fmaf(rx2, xd[3], fmaf(ex, xe[3], fmaf(D4, c13, -(ga * v[2]))));
+  G.g[4][0] = fmaf(rz2, xd[0], fmaf(ez, xe[0], fmaf(D4, d02, -(gb * v[3]))));
+  G.g[4][1] = fmaf(rz2, xd[1], fmaf(ez, xe[1], fmaf(-D4, c13, ga * v[2])));
+  G.g[4][2] = fmaf(rz2, xd[2], fmaf(ez, xe[2], fmaf(D4, a02, -(ga * v[1]))));
+  G.g[4][3] = fmaf(rz2, xd[3], fmaf(ez, xe[3], fmaf(D4, rv, -(gb * v[0]))));
+}
+
+// the directional derivative (dO) v for the change f of the five elements
+__device__ __forceinline__ void grad_dot(const Grad& G, const Five& f, float o[4]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    o[i] = fmaf(f.I, G.g[0][i],
+                fmaf(f.q, G.g[1][i], fmaf(f.V, G.g[2][i], fmaf(f.qF, G.g[3][i], f.VF * G.g[4][i]))));
+}
+
+// the derivative in the azimuth, which moves e and r along the frame's second
+// axis by twice their first component; every term carries that component, so
+// nothing cancels in a weak transverse field
+__device__ __forceinline__ void evol_azimuth(const Evol& E, const float v[4], const Pieces& w, float o[4]) {
+  const float alx = -fmaf(E.ga, E.ex, E.gb * E.rx), omx = fmaf(E.ga, E.rx, -(E.gb * E.ex));
+  const float t2 = fmaf(E.ex, E.ex, E.rx * E.rx), g = fmaf(E.ex, E.ez, E.rx * E.rz);
+  o[0] = 2.f * fmaf(alx, v[2], -(E.D4 * (E.cy * v[1])));
+  o[1] = 2.f * fmaf(E.D4, fmaf(E.cy, v[0], t2 * v[2]), -(omx * v[3]));
+  o[2] = 2.f * fmaf(E.D4, fmaf(E.ex, w.p1[0], E.rx * w.p2[0]), alx * v[0]);
+  o[3] = 2.f * fmaf(E.D4, g * v[2], omx * v[1]);
 }
 
 }  // namespace fz
