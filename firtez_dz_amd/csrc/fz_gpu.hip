@@ -821,6 +821,16 @@ __global__ void __launch_bounds__(256) taulin_kernel(RtArgs a, float* __restrict
   }
 }
 
+// a value that is the same in all lanes, in a scalar register
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ long uniform(int64_t x) {
+  const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)x);
+  return ((long)__builtin_amdgcn_readfirstlane((int)(x >> 32)) << 32) | lo;
+}
+
+// flags of a raw 32-bit buffer resource
+constexpr int RSRC_FLAGS = 0x00027000;
+
 // bytes of LDS that a transfer wave fills with the records of its next heights
 constexpr size_t RT_LDS = 10 * 1024;
 
@@ -862,39 +872,46 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(RtArgs a) {
   int ct, ct0, r, l;
   long sbase;        // the column's Stokes: stokes[sbase + s * snumw + lo]
   int snumw, lo;
-  long t, nthr;      // lane slot and lane count of the tile (scratch rows)
-  long jbase;        // the column's response functions: jac[jbase + ((p*nz + k)*4 + s)*snumw]
+  // scratch rows of nthr lanes and response functions: the wave's first
+  // element (t0, j0, wave-uniform) and the lane's distance from it, so that
+  // the accesses take a scalar base and a 32-bit offset
+  long t0, nthr, j0;
+  unsigned dt, dj;   // jac[j0 + dj + ((p*nz + k)*4 + s)*snumw]
   if constexpr (PACK) {
     const int g0 = (int)blockIdx.x * RT_WAVE, last = a.ntile * numw - 1;
     live = g0 + lane <= last;
     const int g = min(g0 + lane, last);
     ct = g / numw;
-    ct0 = g0 / numw;
+    ct0 = uniform(g0 / numw);
     l = g - ct * numw;
     r = 0;
     sbase = (long)(a.col0 + ct) * 4 * numw;
     snumw = numw;
     lo = l;
-    t = g;
+    t0 = g0;
+    dt = (unsigned)(g - g0);
     nthr = (long)a.ntile * numw;
-    jbase = (long)(a.col0 + ct - a.jcol0) * NP * nz * 4 * numw + l;
+    j0 = (long)(a.col0 + ct0 - a.jcol0) * NP * nz * 4 * numw;
+    dj = (unsigned)((ct - ct0) * NP * nz * 4 * numw + l);
   } else if (a.items) {
     // per-pixel windows: scratch and response functions are ragged too
     const RtItem it = a.items[blockIdx.x];
+    const int icol = uniform(it.col), lout = uniform(it.lout);
     live = lane < it.n;
     const int i = min(lane, it.n - 1);
-    ct = ct0 = it.col - a.col0;
-    r = it.r;
+    ct = ct0 = icol - a.col0;
+    r = uniform(it.r);
     l = it.l0 + i;
-    const int64_t p0 = a.poff[it.col], pt = a.poff[a.col0];
+    const long p0 = uniform(a.poff[icol]), pt = uniform(a.poff[a.col0]);
     sbase = 4 * p0;
-    snumw = (int)(a.poff[it.col + 1] - p0);
-    lo = it.lout + i;
-    t = (p0 - pt) + lo;
-    nthr = a.poff[a.col0 + a.ntile] - pt;
-    jbase = (long)NP * nz * 4 * (p0 - a.poff[a.jcol0]) + lo;
+    snumw = (int)(uniform(a.poff[icol + 1]) - p0);
+    lo = lout + i;
+    t0 = (p0 - pt) + lout;
+    dt = dj = (unsigned)i;
+    nthr = uniform(a.poff[a.col0 + a.ntile]) - pt;
+    j0 = (long)NP * nz * 4 * (p0 - uniform(a.poff[a.jcol0])) + lout;
   } else {
-    ct = ct0 = (int)(blockIdx.x / (unsigned)c_cfg.nbpc);
+    ct = ct0 = uniform((int)(blockIdx.x / (unsigned)c_cfg.nbpc));
     const int bc = (int)(blockIdx.x - (unsigned)ct * (unsigned)c_cfg.nbpc);
     live = lane < c_cfg.blk_n[bc];
     r = c_cfg.blk_reg[bc];
@@ -902,9 +919,10 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(RtArgs a) {
     sbase = (long)(a.col0 + ct) * 4 * numw;
     snumw = numw;
     lo = l;
-    t = (long)ct * numw + l;
+    t0 = (long)ct * numw + c_cfg.blk_l0[bc];
+    dt = dj = (unsigned)min(lane, c_cfg.blk_n[bc] - 1);
     nthr = (long)a.ntile * numw;
-    jbase = (long)(a.col0 + ct - a.jcol0) * NP * nz * 4 * numw + l;
+    j0 = (long)(a.col0 + ct - a.jcol0) * NP * nz * 4 * numw + c_cfg.blk_l0[bc];
   }
   const int col = a.col0 + ct;
   if (a.status && a.status[col] != 0) {
@@ -914,7 +932,7 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(RtArgs a) {
   }
   if (__ballot(live) == 0) return;
   // the wave's columns are ct0 .. ct0 + nc - 1
-  const int nc = PACK ? __builtin_amdgcn_readfirstlane(__shfl(ct, 63) - ct0 + 1) : 1;
+  const int nc = PACK ? uniform(__shfl(ct, 63) - ct0 + 1) : 1;
   const int rs4 = (REC_HEAD + REC_REG + REC_SLOT * c_cfg.reg_nblend[r]) / 4;   // float4 per (height, column) in LDS
   const float4* grec = reinterpret_cast<const float4*>(a.micro);
   const int rec4 = c_cfg.rec / 4, roff4 = (c_cfg.reg_rec[r] - REC_HEAD) / 4;
@@ -950,8 +968,24 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(RtArgs a) {
   const long ps = (long)nz * a.ncol, cs = a.ncol;
   float I[4] = {0.f, 0.f, 0.f, 0.f};
   float Ahe[4] = {0.f, 0.f, 0.f, 0.f};
-  float* scr = a.scratch + t;
-  const long sstr = nthr;
+  // row i of the pass-1 scratch and of the response functions
+  // rows of the pass-1 scratch (64 lanes from t0) and of the wave's response
+  // functions as buffers: the row is a scalar offset, the lane a 32-bit one
+  const unsigned dtb = 4u * dt, djb = 4u * dj;
+  auto scr = [&](int i) -> __amdgpu_buffer_rsrc_t {
+    return __builtin_amdgcn_make_buffer_rsrc(a.scratch + t0 + (long)i * nthr, 0, 4 * RT_WAVE, RSRC_FLAGS);
+  };
+  auto scr_store = [&](int i, float x) {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x), scr(i), dtb, 0, 0);
+  };
+  auto scr_load = [&](int i) -> float {
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(scr(i), dtb, 0, 0));
+  };
+  const __amdgpu_buffer_rsrc_t jbuf = __builtin_amdgcn_make_buffer_rsrc(
+      RF ? a.jac + j0 : nullptr, 0, 4 * nc * NP * nz * 4 * snumw, RSRC_FLAGS);
+  auto jac_store = [&](int i, float x) {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x), jbuf, djb, 4 * i * snumw, 0);
+  };
   // POPL/POPU of the wavelength's region at height k (SOURCE_FUNCTION,
   // rtesolver.f90:1030-1033): S = c1 / ((POPL/POPU) exp(c2/T) - 1)
   auto depart = [&](int k) -> float {
@@ -988,7 +1022,7 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(RtArgs a) {
       if (RF) {
         if (live) {
 #pragma unroll
-          for (int s = 0; s < 4; ++s) scr[(long)(k * 4 + s) * sstr] = I[s];
+          for (int s = 0; s < 4; ++s) scr_store(k * 4 + s, I[s]);
         }
       }
       if (h0.x != 0.f) {
@@ -1025,7 +1059,7 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(RtArgs a) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           W[i] = thin ? fmaf(E.A, Ahe[i], W[i]) : Ahe[i];
-          if (live) scr[(long)((nz + k) * 4 + i) * sstr] = W[i];
+          if (live) scr_store((nz + k) * 4 + i, W[i]);
           if (thin) Ahe[i] = W[i] + d2[i] * pg;
         }
       } else {
@@ -1053,31 +1087,32 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(RtArgs a) {
                             __builtin_isfinite(I[3])))
     atomicMax(&a.status[col], (int32_t)ERR_NAN);
   if constexpr (RF != 0) {
+    // O_nz ... O_{k+1}, its rows times GAIN1D (but for P0, whose response is
+    // a product of two propagated ones)
+    constexpr bool GACC = RF != FZ_RF_CARTESIAN_P0;
     float acc[4][4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = (i == j) ? 1.f : 0.f;
-    float* jb = a.jac + jbase;
+      for (int j = 0; j < 4; ++j) acc[i][j] = (i == j) ? (GACC ? gn[i] : 1.f) : 0.f;
     for (int k1 = nz; k1 > 0; k1 -= a.chunk) {
       const int n = min(a.chunk, k1);
       stage(k1 - n, n);
       for (int kk = n - 1; kk >= 0; --kk) {
         const int k = k1 - n + kk;
         const float4* R = mine + kk * nc * rs4;
-        float outv[NP][4];
         const float4 h0 = R[0];
         if (h0.x != 0.f) {
           // boundary layer: no local response; layers below cannot reach the top
-#pragma unroll
-          for (int p = 0; p < NP; ++p)
-#pragma unroll
-            for (int s = 0; s < 4; ++s) outv[p][s] = 0.f;
+          if (live)
+#pragma unroll 1
+            for (int i = 0; i < 4 * NP; ++i) jac_store(((i >> 2) * nz + k) * 4 + (i & 3), 0.f);
 #pragma unroll
           for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
         } else {
+          float outv[NP][4];
           const float4 h1 = R[1], h2 = R[2], h3 = R[3], rg = R[REC_HEAD / 4];
           const float dz = c_cfg.dz_cm[k];
           // S = c1 / (ex - 1), dS/dT = S (ex / (ex - 1)) (c2 / T) / T
@@ -1095,7 +1130,7 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(RtArgs a) {
           evol_build<true>(f, E);
           float v[4], vf[4];
 #pragma unroll
-          for (int s = 0; s < 4; ++s) v[s] = scr[(long)(k * 4 + s) * sstr] - (s == 0 ? S : 0.f);
+          for (int s = 0; s < 4; ++s) v[s] = scr_load(k * 4 + s) - (s == 0 ? S : 0.f);
           turn(h3.x, h3.y, v, vf);
           // local responses in the frame: lp[0] = T, then (Pg, rho,) and the field's
           float lp[NPL][4], lB[4], lG[4], lF[4];
@@ -1116,7 +1151,7 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(RtArgs a) {
               float vo[4], vof[4];
 #pragma unroll
               for (int s = 0; s < 4; ++s)
-                vo[s] = (k == nz - 1 ? I[s] : scr[(long)((k + 1) * 4 + s) * sstr]) - (s == 0 ? S : 0.f);
+                vo[s] = (k == nz - 1 ? I[s] : scr_load((k + 1) * 4 + s)) - (s == 0 ? S : 0.f);
               turn(h3.x, h3.y, vo, vof);
               const Pieces wo = evol_pieces(E, vof);
               evol_grad(E, vof, wo, G);
@@ -1148,7 +1183,7 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(RtArgs a) {
             const float gk = -mu * c_cfg.he_cte[k] * h0.z * h0.z;
             float W[4], Wf[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) W[i] = scr[(long)((nz + k) * 4 + i) * sstr];
+            for (int i = 0; i < 4; ++i) W[i] = scr_load((nz + k) * 4 + i);
             turn(h3.x, h3.y, W, Wf);
 #pragma unroll
             for (int i = 0; i < 4; ++i) lp[0][i] = fmaf(gk, Wf[i], lp[0][i]);
@@ -1212,12 +1247,12 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(RtArgs a) {
           for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int j = 0; j < 4; ++j) acc[i][j] = na[i][j];
-        }
-        if (live) {
+          if (live) {
 #pragma unroll
-          for (int p = 0; p < NP; ++p)
+            for (int p = 0; p < NP; ++p)
 #pragma unroll
-            for (int s = 0; s < 4; ++s) jb[((long)(p * nz + k) * 4 + s) * snumw] = outv[p][s] * gn[s];
+              for (int s = 0; s < 4; ++s) jac_store((p * nz + k) * 4 + s, GACC ? outv[p][s] : outv[p][s] * gn[s]);
+          }
         }
       }
     }
