@@ -2782,6 +2782,14 @@ int fz_set_inversion(fz_ctx* c, const fz_inversion* inv, int* ifreep, int* nfreq
   if (np == 0) return set_err(c, FZ_ECONFIG, "no parameter inverted");
   L.np = np;
   L.nparam = npar;
+  // the model columns that a step holds: the inverted ones, then log tau5
+  for (int p = 0; p < NATM; ++p) L.rowslot[p] = -1;
+  L.nheld = 0;
+  for (int ip = 0; ip < npar; ++ip) {
+    if (L.rowslot[L.mcol[ip]] < 0) L.rowslot[L.mcol[ip]] = L.nheld++;
+    L.mslot[ip] = L.rowslot[L.mcol[ip]];
+  }
+  L.rowslot[A_TAU] = L.nheld++;
   std::vector<double> colsum(np);
   c->kbeg.assign(np, 0);
   c->kend.assign(np, 0);

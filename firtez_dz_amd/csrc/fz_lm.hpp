@@ -4,13 +4,14 @@
 //                (CALCULATE_EQUIVALENT_DSYN, forward.f90:552-681): one thread
 //                per (pixel, spectral row), FP64 accumulation over the support
 //                of each node's hat function, REAL(4) store.
-//   lm_kernel  : one 256-thread workgroup per pixel, FP64 throughout except
-//                the REAL(4) model (GET_PERT_1D, get_dmodel.f90:1201-1244):
-//                chi^2 and accept/reject (:960-1032), lambda update
-//                (:917-956), Jacobian normalisation (:725-770), Gauss-Newton
-//                normal matrix and gradient streamed through LDS in chunks of
-//                64 spectral rows, damped pseudo-inverse by a parallel cyclic
-//                Jacobi eigen-decomposition in LDS (the symmetric form of the
+//   lm_kernel  : one wave per pixel (four beyond LM_MAXNP free parameters),
+//                FP64 throughout except the REAL(4) model (GET_PERT_1D,
+//                get_dmodel.f90:1201-1244): chi^2 and accept/reject
+//                (:960-1032), lambda update (:917-956), Jacobian
+//                normalisation (:725-770), Gauss-Newton normal matrix and
+//                gradient streamed through LDS in chunks of 32 spectral rows,
+//                damped pseudo-inverse by a parallel cyclic Jacobi
+//                eigen-decomposition in LDS (the symmetric form of the
 //                truncated SVD of lm.f90:61-133), and the limited
 //                perturbation applied through the node basis (:1715-2016).
 #pragma once
@@ -39,6 +40,9 @@ struct LmArgs {
   int par[8];                  // physical index 0..7 (T, Pg, rho, Bx, By, Bz, vz, P0)
   int slot[8];                 // response-function slot in the Cartesian per-height output
   int mcol[8];                 // model column
+  int mslot[8];                // its place among the pixel's columns in LDS (Pg and P0 share theirs)
+  int rowslot[12];             // place of each model row there (log tau5 last), -1: not held
+  int nheld;                   // columns held, log tau5 included
   int j0[8], nj[8];            // first free parameter, nodes
   int rowstk[4];               // Stokes index of each inverted Stokes block
   int regul, solver, node_expansion, pen_typ[8];
@@ -208,6 +212,18 @@ __global__ void __launch_bounds__(256) eqv_kernel(EqvArgs a) {
 }
 
 // ---------------------------------------------------------------- LM step
+// rows of a chunk in LDS: np normalised responses and the residual, padded to
+// a multiple of four doubles and to a stride that spreads the banks
+constexpr size_t lm_ldj(int np) { return (size_t)(np + 4) / 4 * 4 + 2; }
+// the normal matrix and the gradient (column np) in blocks of two rows by
+// four columns, those with an entry on or above the diagonal
+constexpr size_t lm_blocks(int np) {
+  size_t n = 0;
+  for (int i = 0; i < np; i += 2) n += (np + 4) / 4 - i / 4;
+  return n;
+}
+constexpr int LM_MAXHELD = 8;    // model columns of a pixel in LDS: seven inverted ones and log tau5
+
 template <int NT>
 __device__ __forceinline__ double block_sum(double v, double* red) {
   const int t = threadIdx.x;
@@ -222,6 +238,36 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
   return r;
 }
 
+// sum over a wave (every lane gets it) by the fixed tree of cross-lane moves,
+// and over a workgroup of NT threads
+__device__ __forceinline__ double wave_sum(double x) {
+  x = add_swap32(x);
+  x = add_swap16(x);
+  x += dpp64<0x128>(x);
+  x += dpp64<0xB1>(x);
+  x += dpp64<0x4E>(x);
+  return x + dpp64<0x141>(x);
+}
+template <int NT>
+__device__ __forceinline__ double team_sum(double v, double* red) {
+  v = wave_sum(v);
+  if constexpr (NT == 64) return v;
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double s = 0.0;
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) s += red[w];
+  return s;
+}
+
+// 1 / sqrt(x) for x of ordinary size
+__device__ __forceinline__ double rsq64(double x) {
+  double r = __builtin_amdgcn_rsq(x);
+  r = fma(0.5 * r, fma(-(x * r), r, 1.0), r);
+  return fma(0.5 * r, fma(-(x * r), r, 1.0), r);
+}
+
 // GET_IT_PENALTIES (get_dmodel.f90:1041-1197) by one thread: pen_res[np],
 // pen_hss[np*np] (row-major, block diagonal) from the model columns in LDS;
 // sm and pen are LDS work vectors of np entries.
@@ -232,7 +278,7 @@ __device__ void lm_penalties(const LmArgs& a, const float* mod, double* pen_res,
   for (int i = 0; i < np * np; ++i) pen_hss[i] = 0.0;
   for (int ip = 0; ip < a.nparam; ++ip) {
     const int p = a.par[ip], ji = a.j0[ip], jd = a.nj[ip];
-    const float* col = mod + a.mcol[ip] * nz;
+    const float* col = mod + a.mslot[ip] * nz;
     const double alp = sqrt(a.pen_alp[p] / (double)np);
     for (int j = 0; j < jd; ++j) {
       const double* cf = a.coefs + (long)(ji + j) * nz;
@@ -276,6 +322,23 @@ __device__ void lm_penalties(const LmArgs& a, const float* mod, double* pen_res,
   }
 }
 
+// The Jacobi rotation that clears a_pq: cs, sn with a reciprocal and two
+// reciprocal square roots where the entries' squares are of ordinary size
+// (the chain of one rotation is what a round waits for)
+__device__ __forceinline__ void jacobi_rotation(double app, double aqq, double apq, double& cs, double& sn) {
+  const double d = aqq - app, b = 2.0 * apq, h = fma(d, d, b * b);
+  double t;
+  if (h > 1.0e-280 && h < 1.0e280) {
+    t = (d >= 0.0 ? b : -b) * rcp64(fabs(d) + h * rsq64(h));
+    cs = rsq64(fma(t, t, 1.0));
+  } else {
+    const double th = d / b;
+    t = (th >= 0 ? 1.0 : -1.0) / (fabs(th) + sqrt(1.0 + th * th));
+    cs = 1.0 / sqrt(1.0 + t * t);
+  }
+  sn = t * cs;
+}
+
 // Damped solve of GET_PERTURBATION (lm.f90:137-204) on a symmetric matrix
 // A[np][ld] (ld = np + 1; rows up to np + (np & 1) zero-padded) and the
 // right-hand side g, by all NT threads of the workgroup; V must hold the
@@ -284,6 +347,12 @@ __device__ void lm_penalties(const LmArgs& a, const float* mod, double* pen_res,
 // svdtol * max dropped); solver 2: the CG iteration of
 // NEW_CALCULATE_DELTA_UBICGSTAB (lm.f90:375-453).  Work vectors: dv[np],
 // red[NT], rot[np + 1], nod[4 np].  Result in del[np]; A and V are destroyed.
+//
+// A round of the Jacobi sweep turns npe/2 disjoint pairs at once.  Each lane
+// takes one 2 x 2 block of A that two pairs share (the blocks above the
+// diagonal, mirrored on store) and applies both rotations to it, so A is read
+// and written once per round; V takes one rotation per pair and row.  Bound:
+// the latency of a round (the rotations' chain and two passes through LDS).
 template <int NT>
 __device__ void damped_solve(int solver, double svdtol, int np, double* A, double* V, const double* g,
                              double* dv, double* del, double* red, double* rot, double* nod) {
@@ -292,63 +361,94 @@ __device__ void damped_solve(int solver, double svdtol, int np, double* A, doubl
   const int npe = np + (np & 1);
   if (solver == 1) {
     const int half = npe / 2;
+    int* pq = reinterpret_cast<int*>(nod);                              // [half] the round's pairs
+    unsigned short* blk = reinterpret_cast<unsigned short*>(pq + half); // blocks (i1 <= i2), NT == 64
+    const int nblk = half * (half + 1) / 2;
+    if constexpr (NT == 64) {
+      for (int i = t; i < half; i += NT) {
+        int o = i * half - i * (i - 1) / 2;
+        for (int j = i; j < half; ++j) blk[o++] = (unsigned short)(i << 8 | j);
+      }
+    }
+    // the lane's first (pair, row) of V and its step from one to the next
+    const int vi0 = t / np, vk0 = t - vi0 * np, vdi = NT / np, vdk = NT - vdi * np;
     for (int sweep = 0; sweep < 60; ++sweep) {
       double o = 0.0, tt = 0.0;
-      for (int e = t; e < np * np; e += NT) {
-        const int i = e / np, j = e - i * np;
-        const double x = A[i * ld + j];
+      for (int i = vi0, k = vk0; i < np;) {
+        const double x = A[i * ld + k];
         tt += x * x;
-        if (i != j) o += x * x;
+        if (i != k) o += x * x;
+        i += vdi;
+        k += vdk;
+        if (k >= np) {
+          k -= np;
+          ++i;
+        }
       }
-      const double off = block_sum<NT>(o, red), tot = block_sum<NT>(tt, red);
+      const double off = team_sum<NT>(o, red), tot = team_sum<NT>(tt, red);
       if (off <= 1e-30 * tot || off == 0.0) break;
       for (int rnd = 0; rnd < npe - 1; ++rnd) {
         // pair i: players L[i], L[npe-1-i] with L = [0, (rnd+k)%(npe-1)+1 ...]
         for (int i = t; i < half; i += NT) {
-          const int p0 = (i == 0) ? 0 : ((rnd + i - 1) % (npe - 1)) + 1;
-          const int q0 = ((rnd + (npe - 1 - i) - 1) % (npe - 1)) + 1;
+          int x = rnd + i - 1, y = rnd + npe - 2 - i;
+          if (x >= npe - 1) x -= npe - 1;
+          if (y >= npe - 1) y -= npe - 1;
+          const int p0 = i == 0 ? 0 : x + 1, q0 = y + 1;
           const int p = min(p0, q0), q = max(p0, q0);
           double cs = 1.0, sn = 0.0;
           if (q < np) {
             const double apq = A[p * ld + q];
-            if (apq != 0.0) {
-              const double th = (A[q * ld + q] - A[p * ld + p]) / (2.0 * apq);
-              const double tq = (th >= 0 ? 1.0 : -1.0) / (fabs(th) + sqrt(1.0 + th * th));
-              cs = 1.0 / sqrt(1.0 + tq * tq);
-              sn = tq * cs;
-            }
+            if (apq != 0.0) jacobi_rotation(A[p * ld + p], A[q * ld + q], apq, cs, sn);
           }
           rot[2 * i] = cs;
           rot[2 * i + 1] = sn;
+          pq[i] = p | q << 16;
         }
         __syncthreads();
-        // columns of A and V: A <- A J, V <- V J
-        for (int e = t; e < half * npe; e += NT) {
-          const int i = e / npe, k = e - i * npe;
-          const int p0 = (i == 0) ? 0 : ((rnd + i - 1) % (npe - 1)) + 1;
-          const int q0 = ((rnd + (npe - 1 - i) - 1) % (npe - 1)) + 1;
-          const int p = min(p0, q0), q = max(p0, q0);
-          const double cs = rot[2 * i], sn = rot[2 * i + 1];
-          if (sn == 0.0 && cs == 1.0) continue;
-          const double akp = A[k * ld + p], akq = A[k * ld + q];
-          A[k * ld + p] = cs * akp - sn * akq;
-          A[k * ld + q] = sn * akp + cs * akq;
-          const double vkp = V[k * ld + p], vkq = V[k * ld + q];
-          V[k * ld + p] = cs * vkp - sn * vkq;
-          V[k * ld + q] = sn * vkp + cs * vkq;
+        // A <- J^T A J
+        auto turn = [&](int i1, int i2) {
+          const int w1 = pq[i1], w2 = pq[i2];
+          const int p1 = w1 & 0xffff, q1 = w1 >> 16, p2 = w2 & 0xffff, q2 = w2 >> 16;
+          const double c1 = rot[2 * i1], s1 = rot[2 * i1 + 1], c2 = rot[2 * i2], s2 = rot[2 * i2 + 1];
+          const double app = A[p1 * ld + p2], apq = A[p1 * ld + q2], aqp = A[q1 * ld + p2], aqq = A[q1 * ld + q2];
+          const double bpp = c2 * app - s2 * apq, bpq = s2 * app + c2 * apq;
+          const double bqp = c2 * aqp - s2 * aqq, bqq = s2 * aqp + c2 * aqq;
+          const double epp = c1 * bpp - s1 * bqp, epq = c1 * bpq - s1 * bqq;
+          const double eqp = s1 * bpp + c1 * bqp, eqq = s1 * bpq + c1 * bqq;
+          A[p1 * ld + p2] = epp;
+          A[p1 * ld + q2] = epq;
+          A[q1 * ld + p2] = eqp;
+          A[q1 * ld + q2] = eqq;
+          if (i1 != i2) {
+            A[p2 * ld + p1] = epp;
+            A[q2 * ld + p1] = epq;
+            A[p2 * ld + q1] = eqp;
+            A[q2 * ld + q1] = eqq;
+          }
+        };
+        if constexpr (NT == 64) {
+          for (int e = t; e < nblk; e += NT) turn(blk[e] >> 8, blk[e] & 255);
+        } else {
+          for (int e = t; e < half * half; e += NT) {
+            const int i1 = e / half, i2 = e - i1 * half;
+            if (i1 <= i2) turn(i1, i2);
+          }
         }
-        __syncthreads();
-        // rows of A: A <- J^T A
-        for (int e = t; e < half * npe; e += NT) {
-          const int i = e / npe, k = e - i * npe;
-          const int p0 = (i == 0) ? 0 : ((rnd + i - 1) % (npe - 1)) + 1;
-          const int q0 = ((rnd + (npe - 1 - i) - 1) % (npe - 1)) + 1;
-          const int p = min(p0, q0), q = max(p0, q0);
+        // V <- V J
+        for (int i = vi0, k = vk0; i < half;) {
+          const int w = pq[i], p = w & 0xffff, q = w >> 16;
           const double cs = rot[2 * i], sn = rot[2 * i + 1];
-          if (sn == 0.0 && cs == 1.0) continue;
-          const double apk = A[p * ld + k], aqk = A[q * ld + k];
-          A[p * ld + k] = cs * apk - sn * aqk;
-          A[q * ld + k] = sn * apk + cs * aqk;
+          if (q < np) {
+            const double vkp = V[k * ld + p], vkq = V[k * ld + q];
+            V[k * ld + p] = cs * vkp - sn * vkq;
+            V[k * ld + q] = sn * vkp + cs * vkq;
+          }
+          i += vdi;
+          k += vdk;
+          if (k >= np) {
+            k -= np;
+            ++i;
+          }
         }
         __syncthreads();
       }
@@ -464,10 +564,14 @@ __device__ void damped_solve(int solver, double svdtol, int np, double* A, doubl
 template <bool BIG>
 __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(LmArgs a) {
   constexpr int NT = BIG ? LM_BIG_THREADS : LM_THREADS;
-  extern __shared__ double smem_dyn[];
-  const int t = threadIdx.x;
-  const int row = a.row0 + (int)blockIdx.x;
-  double* smem = BIG ? a.work + (long)blockIdx.x * a.work_stride : smem_dyn;
+  extern __shared__ __align__(16) double smem_dyn[];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  // consecutive rows to one XCD (workgroups go round the eight of them), so
+  // that the lines of the model, a pixel's width each, meet in one L2
+  const int bid = (int)blockIdx.x, per = (int)gridDim.x / 8;
+  const int brow = bid < 8 * per ? (bid & 7) * per + (bid >> 3) : bid;
+  const int row = a.row0 + brow;
+  double* smem = BIG ? a.work + (long)brow * a.work_stride : smem_dyn;
   const int pix = a.pix_of ? a.pix_of[row] : row;
   if (a.done && a.done[pix] != 0) return;
   const int np = a.np, nz = a.nz;
@@ -491,42 +595,57 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
   };
   const int ld = np + 1;                       // LDS row stride of A and V
   const int npe = np + (np & 1);               // even size for the tournament ordering
+  const int ldj = (int)lm_ldj(np), nblk = (int)lm_blocks(np), nquad = (np + 4) / 4;
   // LDS carve-up
   double* A = smem;                            // [npe][ld]  (ld >= npe when np odd: ld = np+1 = npe)
-  double* V = A + npe * ld;
-  double* Jn = V + npe * ld;                   // [LM_CH][np]
-  double* rch = Jn + LM_CH * np;               // [LM_CH]
-  double* g = rch + LM_CH;                     // [np]
+  double* V = A + npe * ld;                    // [npe][ld], in the place of Jn once that is contracted
+  double* Jn = V;                              // [LM_CH][ldj]
+  double* g = V + max(npe * ld, LM_CH * ldj);  // [np]
   double* dv = g + np;                         // [np] eigenvalues / projections
   double* del = dv + np;                       // [np]
   double* red = del + np;                      // [NT]
-  double* rot = red + NT;              // [npe/2][2]
+  double* rot = red + NT;                      // [npe/2][2]
   double* nzp = rot + npe;                     // [nz]
   double* nod = nzp + nz;                      // [4][np] node work vectors
-  double* pen_res = nod + 4 * np;              // [np]
+  double* nrm = nod + 4 * np;                  // [np] PARAM_NORM of each free parameter
+  double* pen_res = nrm + np;                  // [np]
   double* pen_hss = pen_res + np;              // [np*np] (only when regularising)
-  float* mod = (float*)(pen_hss + (a.regul ? np * np : 0));   // [12][nz] current model
-  float* bum = mod + 12 * nz;                  // [nz]
+  float* mod = (float*)(pen_hss + (a.regul ? np * np : 0));   // [nheld][nz] current model
+  float* bum = mod + LM_MAXHELD * nz;          // [nz]
   float* ftmp = bum + nz;                      // [nz]
   int* izero = (int*)(ftmp + nz);              // [np] zeroed response columns
-  int* qtab = izero + np;                      // [ntri + np] (i << 16 | j) of each normal-matrix / gradient sum
+  int* btab = izero + np;                      // [nblk] (first row << 16 | first column) of each block
   __shared__ double s_sla[9];
-  __shared__ int s_accept, s_conv;
+  __shared__ int s_accept;
 
   const long ncol = a.ncol;
-  // ---- load the current model and the pixel's scalars
-  for (int i = t; i < 12 * nz; i += NT) mod[i] = a.atm[(long)i * ncol + pix];
+  const bool ext = a.gres != nullptr;
+  // ---- the pixel's model columns and scalars
+  auto load_model = [&](const float* src, float* copy) {
+    for (int p = 0; p < 12; ++p) {
+      const int sl = a.rowslot[p];
+      if (sl < 0 && !copy) continue;
+      for (int k = t; k < nz; k += NT) {
+        const float v = src[((long)p * nz + k) * ncol + pix];
+        if (sl >= 0) mod[sl * nz + k] = v;
+        if (copy) copy[((long)p * nz + k) * ncol + pix] = v;
+      }
+    }
+  };
+  load_model(a.atm, nullptr);
   if (t < 9) s_sla[t] = a.sla ? a.sla[(long)pix * 9 + t] : 0.0;
+  for (int ip = 0; ip < a.nparam; ++ip)
+    for (int j = t; j < a.nj[ip]; j += NT) nrm[a.j0[ip] + j] = c_lm_norm[a.par[ip]];
   // columns whose absolute sum overflows REAL(4) are zeroed (forward.f90:672-678)
   const float* ecur = a.eqv + o_ecur;
-  for (int j = t; j < np; j += NT) {
+  for (int j = wv; j < np; j += NT / 64) {
     float s = 0.f;
-    for (int f = 0; f < nf; ++f) s += fabsf(ecur[(long)j * nf + f]);
-    izero[j] = (s > 3.40282347e38f) ? 1 : 0;
+    for (int f = lane; f < nf; f += 64) s += fabsf(ecur[(long)j * nf + f]);
+    const double ws = wave_sum((double)s);
+    if (lane == 0) izero[j] = ws > (double)3.40282347e38f ? 1 : 0;
   }
   __syncthreads();
 
-  const bool ext = a.gres != nullptr;
   // ---- NEW_CALCULATE_CHI2 (get_dmodel.f90:960-1032)
   const double* obs = a.obs + o_obs;
   const float* stk = a.stokes + o_stk;
@@ -542,7 +661,7 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
     const double d = obs[f] - syn(f);
     part += d * d * isig(f);
   }
-  double chi = block_sum<NT>(part, red) / inu;
+  double chi = team_sum<NT>(part, red) / inu;
   if (a.regul) {
     if (t == 0) lm_penalties(a, mod, pen_res, pen_hss, nod, nod + np);
     __syncthreads();
@@ -555,16 +674,17 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
   const bool accept = s_accept != 0;
   double* bsyn = ext ? nullptr : a.best_syn + o_obs;
   float* ebest = ext ? nullptr : a.eqv_best + o_ebest;
+  const bool tobest = accept && !ext;
   if (ext) {
     // the caller keeps the best model; the step starts from atm
   } else if (accept) {
-    // best := current (model, equivalent response functions, synthesis)
-    for (int i = t; i < 12 * nz; i += NT) a.atm_best[(long)i * ncol + pix] = mod[i];
-    for (long i = t; i < (long)np * nf; i += NT) ebest[i] = izero[i / nf] ? 0.f : ecur[i];
+    // best := current (model and synthesis here, the equivalent response
+    // functions as they are read below)
+    load_model(a.atm, a.atm_best);
     for (int f = t; f < nf; f += NT) bsyn[f] = syn(f);
   } else {
     // current := best
-    for (int i = t; i < 12 * nz; i += NT) mod[i] = a.atm_best[(long)i * ncol + pix];
+    load_model(a.atm_best, a.atm);
   }
   __syncthreads();
   if (!accept && a.regul) {
@@ -601,59 +721,78 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
 
   // ---- normal matrix and gradient of the normalised problem
   //      J_n = J sqrt(w) / sqrt(nu) * PARAM_NORM,  r = (obs - best) sqrt(w) / sqrt(nu)
+  // Rows go to LDS in chunks, read along the spectrum; a lane sums blocks of
+  // two rows by four columns of [J_n | r]^T J_n, three 16-byte reads for eight
+  // products.  The block of the lane's own number stays in registers over the
+  // chunks, further ones (more than NT blocks) are summed in A.
   const float* jsrc = accept ? ecur : ebest;
-  const double snu = sqrt(inu);
-  const int ntri = np * (np + 1) / 2, nq = ntri + np;
-  // sums of the normal matrix (upper triangle, row-major) and of the
-  // gradient, accumulated in LDS over the chunks in row order
-  for (int q = t; q < nq; q += NT) {
-    int i, j;
-    if (q < ntri) {
-      int r = 0, base = 0;
-      while (q >= base + (np - r)) {
-        base += np - r;
-        ++r;
-      }
-      i = r;
-      j = r + (q - base);
-    } else {
-      i = q - ntri;
-      j = 0xffff;                              // gradient entry
-    }
-    qtab[q] = (i << 16) | j;
+  const double isnu = 1.0 / sqrt(inu);
+  for (int i = 2 * t; i < np; i += 2 * NT) {
+    int o = 0;
+    for (int m = 0; m < i; m += 2) o += nquad - m / 4;
+    for (int j = i / 4; j < nquad; ++j) btab[o++] = i << 16 | 4 * j;
   }
   for (int e = t; e < npe * ld; e += NT) A[e] = 0.0;
   for (int i = t; i < np; i += NT) g[i] = 0.0;
+  for (int e = t; e < LM_CH * ldj; e += NT) Jn[e] = 0.0;
   __syncthreads();
-  for (int f0 = 0; f0 < nf; f0 += LM_CH) {
-    const int nc = min(LM_CH, nf - f0);
-    for (int e = t; e < nc * np; e += NT) {
-      const int c = e / np, j = e - c * np;
-      const int f = f0 + c;
-      double v = (accept && izero[j]) ? 0.0 : (double)jsrc[(long)j * nf + f];
-      int ip = 0;
-      while (j >= a.j0[ip] + a.nj[ip]) ++ip;
-      Jn[c * np + j] = v * sqrt(isig(f)) / snu * (1.0 * c_lm_norm[a.par[ip]]);
-    }
-    for (int c = t; c < nc; c += NT) {
-      const int f = f0 + c;
-      rch[c] = (ext ? a.gres[o_obs + f] : obs[f] - bsyn[f]) * sqrt(isig(f)) / snu;
-    }
-    __syncthreads();
-    for (int q = t; q < nq; q += NT) {
-      const int i = qtab[q] >> 16, j = qtab[q] & 0xffff;
-      if (j != 0xffff) {
-        double s = A[i * ld + j];
-        for (int c = 0; c < nc; ++c) s += Jn[c * np + i] * Jn[c * np + j];
-        A[i * ld + j] = s;
-      } else {
-        double s = g[i];
-        for (int c = 0; c < nc; ++c) s += Jn[c * np + i] * rch[c];
-        g[i] = s;
+  auto add_block = [&](int w, const double (&acc)[2][4]) {
+    const int i0 = w >> 16, j0 = w & 0xffff;
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int i = i0 + r, j = j0 + c;
+        if (i >= np || j < i || j > np) continue;
+        if (j < np) A[i * ld + j] += acc[r][c];
+        else g[i] += acc[r][c];
       }
+  };
+  auto sum_block = [&](int w, double (&acc)[2][4]) {
+    const double* pi = Jn + (w >> 16);
+    const double* pj = Jn + (w & 0xffff);
+#pragma unroll 4
+    for (int c = 0; c < LM_CH; ++c) {
+      const double2 x = *reinterpret_cast<const double2*>(pi + c * ldj);
+      const double2 y0 = *reinterpret_cast<const double2*>(pj + c * ldj);
+      const double2 y1 = *reinterpret_cast<const double2*>(pj + c * ldj + 2);
+      acc[0][0] = fma(x.x, y0.x, acc[0][0]);
+      acc[0][1] = fma(x.x, y0.y, acc[0][1]);
+      acc[0][2] = fma(x.x, y1.x, acc[0][2]);
+      acc[0][3] = fma(x.x, y1.y, acc[0][3]);
+      acc[1][0] = fma(x.y, y0.x, acc[1][0]);
+      acc[1][1] = fma(x.y, y0.y, acc[1][1]);
+      acc[1][2] = fma(x.y, y1.x, acc[1][2]);
+      acc[1][3] = fma(x.y, y1.y, acc[1][3]);
     }
-    __syncthreads();
+  };
+  double own[2][4] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+  const int wown = t < nblk ? btab[t] : -1;
+  {
+    const int c = t & (LM_CH - 1), jg = t / LM_CH;
+    for (int f0 = 0; f0 < nf; f0 += LM_CH) {
+      const int f = f0 + c;
+      const bool in = f < nf;
+      const double w = in ? sqrt(isig(f)) * isnu : 0.0;
+      for (int j = jg; j < np; j += NT / LM_CH) {
+        float v = in ? jsrc[(long)j * nf + f] : 0.f;
+        if (accept && izero[j]) v = 0.f;
+        if (tobest && in) ebest[(long)j * nf + f] = v;
+        Jn[c * ldj + j] = (double)v * w * nrm[j];
+      }
+      if (jg == 0) Jn[c * ldj + np] = in ? (ext ? a.gres[o_obs + f] : obs[f] - bsyn[f]) * w : 0.0;
+      __syncthreads();
+      if (wown >= 0) sum_block(wown, own);
+      for (int q = t + NT; q < nblk; q += NT) {
+        double acc[2][4] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+        sum_block(btab[q], acc);
+        add_block(btab[q], acc);
+      }
+      __syncthreads();
+    }
   }
+  if (wown >= 0) add_block(wown, own);
+  __syncthreads();
   const double lam = s_sla[8];
   if (ext && a.hscale != 1.0) {
     for (int e = t; e < np * np; e += NT) {
@@ -677,10 +816,9 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
     }
   __syncthreads();
   for (int i = t; i < np; i += NT) A[i * ld + i] = A[i * ld + i] + A[i * ld + i] * lam;
-  for (int e = t; e < npe * ld; e += NT) {
-    const int i = e / ld, j = e - i * ld;
-    V[e] = (i == j) ? 1.0 : 0.0;
-  }
+  for (int e = t; e < npe * ld; e += NT) V[e] = 0.0;
+  __syncthreads();
+  for (int i = t; i < np; i += NT) V[i * ld + i] = 1.0;
   __syncthreads();
 
   // ---- damped solve (symmetric eigen-decomposition or CG)
@@ -698,29 +836,33 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
 
   // ---- LIMIT_PERTURBATION -> REARANGE_DA_MODEL -> SORT_DELTA_TO_ATMOSPHERE
   double* itd = nod;            // [np] scaled / limited node perturbation
-  double* avg = nod + np;       // [np] node means of the model
   double* sumv = nod + 2 * np;  // [np]
+  // node mean of a column: a wave per node, its lanes along the heights
+  auto node_mean = [&](const float* x, int j) -> double {
+    const double* cf = a.coefs + (long)j * nz;
+    double s = 0.0;
+    for (int k = lane; k < nz; k += 64) s = fma((double)x[k], cf[k], s);
+    return wave_sum(s) / a.colsum[j];
+  };
   for (int ip = 0; ip < a.nparam; ++ip) {
     const int p = a.par[ip], j0 = a.j0[ip], nj = a.nj[ip];
-    float* col = mod + a.mcol[ip] * nz;
+    float* col = mod + a.mslot[ip] * nz;
     const double factor = c_lm_norm[p], inf = c_lm_low[p], sup = c_lm_upp[p];
     const double absolute = c_lm_norm[p] * a.mpert;
     for (int k = t; k < nz; k += NT) bum[k] = col[k];
-    for (int j = t; j < nj; j += NT) {
-      const double* cf = a.coefs + (long)(j0 + j) * nz;
-      double s = 0.0;
-      for (int k = 0; k < nz; ++k) s = s + (double)col[k] * cf[k];
-      const double av = s / a.colsum[j0 + j];
+    for (int j = wv; j < nj; j += NT / 64) {
+      const double av = node_mean(col, j0 + j);
       double lim;
       if (absolute > 0) lim = fmax(absolute, fabs(a.mpert * av));
       else lim = fabs(a.mpert * av);
       if (av == 0) lim = absolute;
       double x = del[j0 + j] * factor;
       if (fabs(x) > lim) x = x / fabs(x) * lim;
-      itd[j] = x;
-      avg[j] = av;
-      sumv[j] = av + x;
-      del[j0 + j] = x;
+      if (lane == 0) {
+        itd[j] = x;
+        sumv[j] = av + x;
+        del[j0 + j] = x;
+      }
     }
     __syncthreads();
     for (int k = t; k < nz; k += NT) {
@@ -742,12 +884,12 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
         ftmp[k] = (float)nzp[k];
       }
       __syncthreads();
-      for (int j = t; j < nj; j += NT) {
-        const double* cf = a.coefs + (long)(j0 + j) * nz;
-        double s = 0.0;
-        for (int k = 0; k < nz; ++k) s = s + (double)ftmp[k] * cf[k];
-        itd[j] = s / a.colsum[j0 + j];
-        del[j0 + j] = itd[j];
+      for (int j = wv; j < nj; j += NT / 64) {
+        const double x = node_mean(ftmp, j0 + j);
+        if (lane == 0) {
+          itd[j] = x;
+          del[j0 + j] = x;
+        }
       }
       __syncthreads();
       for (int k = t; k < nz; k += NT) {
@@ -760,17 +902,27 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
       }
     }
     __syncthreads();
-    if (p == 0 && t == 0) {
-      // temperature tail rule in log tau5 (get_dmodel.f90:1970-1984)
-      const float* tau = mod + A_TAU * nz;
+    if (p == 0 && t < 64) {
+      // temperature tail rule in log tau5 (get_dmodel.f90:1970-1984), top
+      // down: damped above tllim, and below tulim the value of the height
+      // above, so of the nearest height above that does not take another's
+      const float* tau = mod + a.rowslot[A_TAU] * nz;
       const float tllim = -11.5f, tulim = 0.5f;
-      for (int k = nz - 1; k >= 0; --k) {
-        if (tau[k] < tllim) {
-          const float x = fabsf(tau[k] - tllim) / 0.5f;
-          col[k] = expf(-(x * x)) * col[k];
-        } else if (tau[k] > tulim) {
-          if (k + 1 < nz) col[k] = col[k + 1];
+      float carry = 0.f;
+      for (int kb = (nz - 1) / 64 * 64; kb >= 0; kb -= 64) {
+        const int k = kb + lane;
+        const bool in = k < nz;
+        const float tk = in ? tau[k] : 0.f;
+        float v = in ? col[k] : 0.f;
+        if (tk < tllim) {
+          const float x = fabsf(tk - tllim) / 0.5f;
+          v = expf(-(x * x)) * v;
         }
+        const unsigned long long keep = __ballot(in && (!(tk > tulim) || k == nz - 1)) >> lane;
+        const float from = __shfl(v, keep ? lane + __builtin_ctzll(keep) : lane);
+        if (in && tk > tulim && k != nz - 1) v = keep ? from : carry;
+        if (in) col[k] = v;
+        carry = __shfl(v, 0);
       }
     }
     __syncthreads();
@@ -778,8 +930,12 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
     __syncthreads();
   }
 
-  // ---- write back
-  for (int i = t; i < 12 * nz; i += NT) a.atm[(long)i * ncol + pix] = mod[i];
+  // ---- write back the inverted columns (the others are in place)
+  for (int p = 0; p < 12; ++p) {
+    const int sl = a.rowslot[p];
+    if (sl < 0 || p == A_TAU) continue;
+    for (int k = t; k < nz; k += NT) a.atm[((long)p * nz + k) * ncol + pix] = mod[sl * nz + k];
+  }
   if (t < 9 && a.sla) a.sla[(long)pix * 9 + t] = s_sla[t];
   if (a.delta)
     for (int i = t; i < np; i += NT) a.delta[(long)pix * np + i] = del[i];
@@ -789,10 +945,10 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
 // bytes of lm_kernel's work arrays (LDS, or the device-memory slice of one
 // pixel) for np free parameters, nz heights and nt threads
 inline size_t lm_lds_bytes(int np, int nz, bool regul, int nt) {
-  const int npe = np + (np & 1), ld = np + 1;
-  size_t d = (size_t)2 * npe * ld + (size_t)LM_CH * np + LM_CH + 3 * np + nt + npe + nz + 4 * np + np +
-             (regul ? (size_t)np * np : 0);
-  size_t f = (size_t)12 * nz + 2 * nz + np + (size_t)np * (np + 1) / 2 + np;   // floats + ints
+  const size_t npe = np + (np & 1), ld = np + 1;
+  const size_t d = npe * ld + std::max(npe * ld, LM_CH * lm_ldj(np)) + 3 * (size_t)np + nt + npe + nz + 4 * (size_t)np +
+                   2 * (size_t)np + (regul ? (size_t)np * np : 0);
+  const size_t f = (size_t)(LM_MAXHELD + 2) * nz + np + lm_blocks(np);   // floats + ints
   return d * 8 + f * 4;
 }
 

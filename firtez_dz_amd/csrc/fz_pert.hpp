@@ -104,7 +104,7 @@ inline size_t pert_work_doubles(int np, int nt) {
 template <bool BIG>
 __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) pert_solve_kernel(PertArgs a) {
   constexpr int NT = BIG ? LM_BIG_THREADS : LM_THREADS;
-  extern __shared__ double smem_dyn[];
+  extern __shared__ __align__(16) double smem_dyn[];
   double* smem = BIG ? a.work : smem_dyn;
   const int t = threadIdx.x;
   const int np = a.np, ld = np + 1, npe = np + (np & 1);
