@@ -23,6 +23,7 @@ constexpr int LM_MAXNP = 64;     // free parameters per pixel with the work arra
 // the barriers are cheap and a CU holds many pixels at once
 constexpr int LM_THREADS = 64;
 constexpr int LM_CH = 32;        // spectral rows per chunk of the normal matrix
+constexpr int LM_PF = 10;        // responses that a lane loads together
 // more free parameters (up to NZ nodes per parameter, the reference's
 // default): the same step with its work arrays in a per-pixel slice of
 // device memory, four waves per pixel
@@ -352,7 +353,10 @@ __device__ __forceinline__ void jacobi_rotation(double app, double aqq, double a
 // takes one 2 x 2 block of A that two pairs share (the blocks above the
 // diagonal, mirrored on store) and applies both rotations to it, so A is read
 // and written once per round; V takes one rotation per pair and row.  Bound:
-// the latency of a round (the rotations' chain and two passes through LDS).
+// the latency of a round, so a lane loads its block and its rows of V before
+// the rotations are formed (by the lanes of the diagonal blocks, from those
+// blocks) and one exchange through LDS hands the rotations out.  A round of 20
+// parameters took 1.3 us with the loads behind the exchange.
 template <int NT>
 __device__ void damped_solve(int solver, double svdtol, int np, double* A, double* V, const double* g,
                              double* dv, double* del, double* red, double* rot, double* nod) {
@@ -361,25 +365,66 @@ __device__ void damped_solve(int solver, double svdtol, int np, double* A, doubl
   const int npe = np + (np & 1);
   if (solver == 1) {
     const int half = npe / 2;
-    int* pq = reinterpret_cast<int*>(nod);                              // [half] the round's pairs
-    unsigned short* blk = reinterpret_cast<unsigned short*>(pq + half); // blocks (i1 <= i2), NT == 64
+    // pair i of a round: players L[i], L[npe-1-i] with L = [0, (rnd+k)%(npe-1)+1 ...]
+    auto pair = [&](int rnd, int i, int& p, int& q) {
+      int x = rnd + i - 1, y = rnd + npe - 2 - i;
+      if (x >= npe - 1) x -= npe - 1;
+      if (y >= npe - 1) y -= npe - 1;
+      const int p0 = i == 0 ? 0 : x + 1, q0 = y + 1;
+      p = min(p0, q0);
+      q = max(p0, q0);
+    };
+    // blocks (i1 <= i2): the diagonal ones first, then row by row (NT == 64:
+    // listed once in LDS; else found again for each)
     const int nblk = half * (half + 1) / 2;
+    unsigned short* blk = reinterpret_cast<unsigned short*>(nod);
     if constexpr (NT == 64) {
       for (int i = t; i < half; i += NT) {
-        int o = i * half - i * (i - 1) / 2;
-        for (int j = i; j < half; ++j) blk[o++] = (unsigned short)(i << 8 | j);
+        blk[i] = (unsigned short)(i << 8 | i);
+        int o = half + i * (half - 1) - i * (i - 1) / 2;
+        for (int j = i + 1; j < half; ++j) blk[o++] = (unsigned short)(i << 8 | j);
+      }
+      __syncthreads();
+    }
+    // V: NG lanes to a pair, each every NG-th row
+    const int ng = max(1, NT / half), vi0 = t / ng, vr = t - vi0 * ng, vstep = max(1, NT / ng);
+    auto turn = [&](double c1, double s1, double c2, double s2, double& app, double& apq, double& aqp, double& aqq) {
+      const double bpp = c2 * app - s2 * apq, bpq = s2 * app + c2 * apq;
+      const double bqp = c2 * aqp - s2 * aqq, bqq = s2 * aqp + c2 * aqq;
+      app = c1 * bpp - s1 * bqp;
+      apq = c1 * bpq - s1 * bqq;
+      aqp = s1 * bpp + c1 * bqp;
+      aqq = s1 * bpq + c1 * bqq;
+    };
+    auto put = [&](int i1, int i2, int p1, int q1, int p2, int q2, double app, double apq, double aqp, double aqq) {
+      A[p1 * ld + p2] = app;
+      A[p1 * ld + q2] = apq;
+      A[q1 * ld + p2] = aqp;
+      A[q1 * ld + q2] = aqq;
+      if (i1 != i2) {
+        A[p2 * ld + p1] = app;
+        A[q2 * ld + p1] = apq;
+        A[p2 * ld + q1] = aqp;
+        A[q2 * ld + q1] = aqq;
+      }
+    };
+    // the lane's first block
+    int j1 = -1, j2 = 0;
+    if constexpr (NT == 64) {
+      if (t < nblk) {
+        j1 = blk[t] >> 8;
+        j2 = blk[t] & 255;
       }
     }
-    // the lane's first (pair, row) of V and its step from one to the next
-    const int vi0 = t / np, vk0 = t - vi0 * np, vdi = NT / np, vdk = NT - vdi * np;
+    const int ei0 = t / np, ek0 = t - ei0 * np, edi = NT / np, edk = NT - edi * np;
     for (int sweep = 0; sweep < 60; ++sweep) {
       double o = 0.0, tt = 0.0;
-      for (int i = vi0, k = vk0; i < np;) {
+      for (int i = ei0, k = ek0; i < np;) {
         const double x = A[i * ld + k];
         tt += x * x;
         if (i != k) o += x * x;
-        i += vdi;
-        k += vdk;
+        i += edi;
+        k += edk;
         if (k >= np) {
           k -= np;
           ++i;
@@ -388,66 +433,86 @@ __device__ void damped_solve(int solver, double svdtol, int np, double* A, doubl
       const double off = team_sum<NT>(o, red), tot = team_sum<NT>(tt, red);
       if (off <= 1e-30 * tot || off == 0.0) break;
       for (int rnd = 0; rnd < npe - 1; ++rnd) {
-        // pair i: players L[i], L[npe-1-i] with L = [0, (rnd+k)%(npe-1)+1 ...]
+        int p1 = 0, q1 = 0, p2 = 0, q2 = 0;
+        double app = 0.0, apq = 0.0, aqp = 0.0, aqq = 0.0;
+        if (j1 >= 0) {
+          pair(rnd, j1, p1, q1);
+          pair(rnd, j2, p2, q2);
+          app = A[p1 * ld + p2];
+          apq = A[p1 * ld + q2];
+          aqp = A[q1 * ld + p2];
+          aqq = A[q1 * ld + q2];
+        }
+        int pv = 0, qv = 0;
+        const bool hasv = vi0 < half;
+        double vp[4], vq[4];
+        if (hasv) pair(rnd, vi0, pv, qv);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int k = vr + u * ng;
+          const bool in = hasv && k < np && qv < np;
+          vp[u] = in ? V[k * ld + pv] : 0.0;
+          vq[u] = in ? V[k * ld + qv] : 0.0;
+        }
         for (int i = t; i < half; i += NT) {
-          int x = rnd + i - 1, y = rnd + npe - 2 - i;
-          if (x >= npe - 1) x -= npe - 1;
-          if (y >= npe - 1) y -= npe - 1;
-          const int p0 = i == 0 ? 0 : x + 1, q0 = y + 1;
-          const int p = min(p0, q0), q = max(p0, q0);
+          int p, q;
+          pair(rnd, i, p, q);
           double cs = 1.0, sn = 0.0;
           if (q < np) {
-            const double apq = A[p * ld + q];
-            if (apq != 0.0) jacobi_rotation(A[p * ld + p], A[q * ld + q], apq, cs, sn);
+            // (NT == 64: block (i, i) is the lane's own)
+            const double bpp = NT == 64 ? app : A[p * ld + p], bqq = NT == 64 ? aqq : A[q * ld + q];
+            const double bpq = NT == 64 ? apq : A[p * ld + q];
+            if (bpq != 0.0) jacobi_rotation(bpp, bqq, bpq, cs, sn);
           }
           rot[2 * i] = cs;
           rot[2 * i + 1] = sn;
-          pq[i] = p | q << 16;
         }
         __syncthreads();
         // A <- J^T A J
-        auto turn = [&](int i1, int i2) {
-          const int w1 = pq[i1], w2 = pq[i2];
-          const int p1 = w1 & 0xffff, q1 = w1 >> 16, p2 = w2 & 0xffff, q2 = w2 >> 16;
-          const double c1 = rot[2 * i1], s1 = rot[2 * i1 + 1], c2 = rot[2 * i2], s2 = rot[2 * i2 + 1];
-          const double app = A[p1 * ld + p2], apq = A[p1 * ld + q2], aqp = A[q1 * ld + p2], aqq = A[q1 * ld + q2];
-          const double bpp = c2 * app - s2 * apq, bpq = s2 * app + c2 * apq;
-          const double bqp = c2 * aqp - s2 * aqq, bqq = s2 * aqp + c2 * aqq;
-          const double epp = c1 * bpp - s1 * bqp, epq = c1 * bpq - s1 * bqq;
-          const double eqp = s1 * bpp + c1 * bqp, eqq = s1 * bpq + c1 * bqq;
-          A[p1 * ld + p2] = epp;
-          A[p1 * ld + q2] = epq;
-          A[q1 * ld + p2] = eqp;
-          A[q1 * ld + q2] = eqq;
-          if (i1 != i2) {
-            A[p2 * ld + p1] = epp;
-            A[q2 * ld + p1] = epq;
-            A[p2 * ld + q1] = eqp;
-            A[q2 * ld + q1] = eqq;
-          }
+        if (j1 >= 0) {
+          turn(rot[2 * j1], rot[2 * j1 + 1], rot[2 * j2], rot[2 * j2 + 1], app, apq, aqp, aqq);
+          put(j1, j2, p1, q1, p2, q2, app, apq, aqp, aqq);
+        }
+        auto block = [&](int i1, int i2) {
+          pair(rnd, i1, p1, q1);
+          pair(rnd, i2, p2, q2);
+          app = A[p1 * ld + p2];
+          apq = A[p1 * ld + q2];
+          aqp = A[q1 * ld + p2];
+          aqq = A[q1 * ld + q2];
+          turn(rot[2 * i1], rot[2 * i1 + 1], rot[2 * i2], rot[2 * i2 + 1], app, apq, aqp, aqq);
+          put(i1, i2, p1, q1, p2, q2, app, apq, aqp, aqq);
         };
         if constexpr (NT == 64) {
-          for (int e = t; e < nblk; e += NT) turn(blk[e] >> 8, blk[e] & 255);
+          for (int e = t + NT; e < nblk; e += NT) block(blk[e] >> 8, blk[e] & 255);
         } else {
           for (int e = t; e < half * half; e += NT) {
             const int i1 = e / half, i2 = e - i1 * half;
-            if (i1 <= i2) turn(i1, i2);
+            if (i1 <= i2) block(i1, i2);
           }
         }
         // V <- V J
-        for (int i = vi0, k = vk0; i < half;) {
-          const int w = pq[i], p = w & 0xffff, q = w >> 16;
+        for (int i = vi0; i < half; i += vstep) {
+          if (i != vi0) pair(rnd, i, pv, qv);
           const double cs = rot[2 * i], sn = rot[2 * i + 1];
-          if (q < np) {
-            const double vkp = V[k * ld + p], vkq = V[k * ld + q];
-            V[k * ld + p] = cs * vkp - sn * vkq;
-            V[k * ld + q] = sn * vkp + cs * vkq;
-          }
-          i += vdi;
-          k += vdk;
-          if (k >= np) {
-            k -= np;
-            ++i;
+          for (int k0 = vr; k0 < np; k0 += 4 * ng) {
+            if (i != vi0 || k0 != vr) {
+#pragma unroll
+              for (int u = 0; u < 4; ++u) {
+                const int k = k0 + u * ng;
+                const bool in = k < np && qv < np;
+                vp[u] = in ? V[k * ld + pv] : 0.0;
+                vq[u] = in ? V[k * ld + qv] : 0.0;
+              }
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const int k = k0 + u * ng;
+              if (k < np && qv < np) {
+                V[k * ld + pv] = cs * vp[u] - sn * vq[u];
+                V[k * ld + qv] = sn * vp[u] + cs * vq[u];
+              }
+            }
           }
         }
         __syncthreads();
@@ -572,7 +637,7 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
   const int brow = bid < 8 * per ? (bid & 7) * per + (bid >> 3) : bid;
   const int row = a.row0 + brow;
   double* smem = BIG ? a.work + (long)brow * a.work_stride : smem_dyn;
-  const int pix = a.pix_of ? a.pix_of[row] : row;
+  const int pix = a.pix_of ? uniform(a.pix_of[row]) : row;
   if (a.done && a.done[pix] != 0) return;
   const int np = a.np, nz = a.nz;
   int nf = a.nfreq, numw = a.numw;
@@ -580,8 +645,8 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
   long o_ecur = (long)row * np * a.nfreq, o_ebest = (long)pix * np * a.nfreq;
   double inu = a.inu;
   if (a.poff) {
-    const int64_t p0 = a.poff[pix];
-    numw = (int)(a.poff[pix + 1] - p0);
+    const long p0 = uniform(a.poff[pix]);
+    numw = (int)(uniform(a.poff[pix + 1]) - p0);
     nf = a.nstk * numw;
     o_obs = (long)a.nstk * p0;
     o_stk = 4 * p0;
@@ -622,13 +687,15 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
   const bool ext = a.gres != nullptr;
   // ---- the pixel's model columns and scalars
   auto load_model = [&](const float* src, float* copy) {
-    for (int p = 0; p < 12; ++p) {
-      const int sl = a.rowslot[p];
-      if (sl < 0 && !copy) continue;
-      for (int k = t; k < nz; k += NT) {
-        const float v = src[((long)p * nz + k) * ncol + pix];
-        if (sl >= 0) mod[sl * nz + k] = v;
-        if (copy) copy[((long)p * nz + k) * ncol + pix] = v;
+    for (int k = t; k < nz; k += NT) {
+      float v[12];
+#pragma unroll
+      for (int p = 0; p < 12; ++p)
+        v[p] = a.rowslot[p] >= 0 || copy ? src[((long)p * nz + k) * ncol + pix] : 0.f;
+#pragma unroll
+      for (int p = 0; p < 12; ++p) {
+        if (a.rowslot[p] >= 0) mod[a.rowslot[p] * nz + k] = v[p];
+        if (copy) copy[((long)p * nz + k) * ncol + pix] = v[p];
       }
     }
   };
@@ -636,14 +703,7 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
   if (t < 9) s_sla[t] = a.sla ? a.sla[(long)pix * 9 + t] : 0.0;
   for (int ip = 0; ip < a.nparam; ++ip)
     for (int j = t; j < a.nj[ip]; j += NT) nrm[a.j0[ip] + j] = c_lm_norm[a.par[ip]];
-  // columns whose absolute sum overflows REAL(4) are zeroed (forward.f90:672-678)
   const float* ecur = a.eqv + o_ecur;
-  for (int j = wv; j < np; j += NT / 64) {
-    float s = 0.f;
-    for (int f = lane; f < nf; f += 64) s += fabsf(ecur[(long)j * nf + f]);
-    const double ws = wave_sum((double)s);
-    if (lane == 0) izero[j] = ws > (double)3.40282347e38f ? 1 : 0;
-  }
   __syncthreads();
 
   // ---- NEW_CALCULATE_CHI2 (get_dmodel.f90:960-1032)
@@ -657,6 +717,7 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
     return (double)stk[a.rowstk[b] * numw + l];
   };
   double part = 0.0;
+#pragma unroll 4
   for (int f = t; f < nf; f += NT) {
     const double d = obs[f] - syn(f);
     part += d * d * isig(f);
@@ -671,7 +732,7 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
   }
   if (t == 0) s_accept = (ext || chi < s_sla[2]) ? 1 : 0;
   __syncthreads();
-  const bool accept = s_accept != 0;
+  const bool accept = uniform(s_accept) != 0;
   double* bsyn = ext ? nullptr : a.best_syn + o_obs;
   float* ebest = ext ? nullptr : a.eqv_best + o_ebest;
   const bool tobest = accept && !ext;
@@ -732,10 +793,8 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
     for (int m = 0; m < i; m += 2) o += nquad - m / 4;
     for (int j = i / 4; j < nquad; ++j) btab[o++] = i << 16 | 4 * j;
   }
-  for (int e = t; e < npe * ld; e += NT) A[e] = 0.0;
-  for (int i = t; i < np; i += NT) g[i] = 0.0;
+  for (int j = t; j < np; j += NT) izero[j] = 0;
   for (int e = t; e < LM_CH * ldj; e += NT) Jn[e] = 0.0;
-  __syncthreads();
   auto add_block = [&](int w, const double (&acc)[2][4]) {
     const int i0 = w >> 16, j0 = w & 0xffff;
 #pragma unroll
@@ -766,21 +825,70 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
       acc[1][3] = fma(x.y, y1.y, acc[1][3]);
     }
   };
-  double own[2][4] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
-  const int wown = t < nblk ? btab[t] : -1;
-  {
+  // Columns whose absolute sum overflows REAL(4) are zeroed (forward.f90:672-678).
+  // The sum of nf < 1e8 values cannot overflow where none passes 1e30, so a
+  // first pass takes every column and notes whether one does; only then are
+  // the columns' sums formed and, where one overflows, the pass repeated.
+  for (int pass = 0; pass < 2; ++pass) {
+    for (int e = t; e < npe * ld; e += NT) A[e] = 0.0;
+    for (int i = t; i < np; i += NT) g[i] = 0.0;
+    __syncthreads();
+    double own[2][4] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+    const int wown = t < nblk ? btab[t] : -1;
+    bool large = false;
+    // the lane's responses of a chunk, LM_PF columns at a time loaded
+    // together and, for the first of them and the row's residual and weight,
+    // a chunk ahead: the loads of a chunk would otherwise wait for one another
+    // behind its stores
+    constexpr int S = NT / LM_CH;
     const int c = t & (LM_CH - 1), jg = t / LM_CH;
+    float pf[LM_PF];
+    double pw = 0.0, po = 0.0, pb = 0.0;
+    auto fetch = [&](int f, int jb, float (&v)[LM_PF]) {
+#pragma unroll
+      for (int u = 0; u < LM_PF; ++u) {
+        const int j = jb + S * u;
+        v[u] = f < nf && j < np ? jsrc[(unsigned)(j * nf + f)] : 0.f;
+      }
+    };
+    auto fetch_row = [&](int f) {
+      if (f >= nf) return;
+      pw = isig(f);
+      if (jg == 0) {
+        po = ext ? a.gres[o_obs + f] : obs[f];
+        pb = ext ? 0.0 : bsyn[f];
+      }
+    };
+    fetch_row(c);
+    fetch(c, jg, pf);
     for (int f0 = 0; f0 < nf; f0 += LM_CH) {
       const int f = f0 + c;
       const bool in = f < nf;
-      const double w = in ? sqrt(isig(f)) * isnu : 0.0;
-      for (int j = jg; j < np; j += NT / LM_CH) {
-        float v = in ? jsrc[(long)j * nf + f] : 0.f;
-        if (accept && izero[j]) v = 0.f;
-        if (tobest && in) ebest[(long)j * nf + f] = v;
-        Jn[c * ldj + j] = (double)v * w * nrm[j];
+      const double w = in ? sqrt(pw) * isnu : 0.0;
+      asm volatile("" ::: "memory");   // the columns' norms stay in LDS
+      for (int jb = jg; jb < np; jb += S * LM_PF) {
+        float v[LM_PF];
+        if (jb == jg) {
+#pragma unroll
+          for (int u = 0; u < LM_PF; ++u) v[u] = pf[u];
+        } else {
+          fetch(f, jb, v);
+        }
+#pragma unroll
+        for (int u = 0; u < LM_PF; ++u) {
+          const int j = jb + S * u;
+          if (j >= np) break;
+          large = large || fabsf(v[u]) > 1.0e30f;
+          if (pass && izero[j]) v[u] = 0.f;
+          if (tobest && in) ebest[(unsigned)(j * nf + f)] = v[u];
+          Jn[c * ldj + j] = (double)v[u] * w * nrm[j];
+        }
       }
-      if (jg == 0) Jn[c * ldj + np] = in ? (ext ? a.gres[o_obs + f] : obs[f] - bsyn[f]) * w : 0.0;
+      if (jg == 0) Jn[c * ldj + np] = in ? (po - pb) * w : 0.0;
+      if (f0 + LM_CH < nf) {
+        fetch_row(f + LM_CH);
+        fetch(f + LM_CH, jg, pf);
+      }
       __syncthreads();
       if (wown >= 0) sum_block(wown, own);
       for (int q = t + NT; q < nblk; q += NT) {
@@ -790,8 +898,18 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
       }
       __syncthreads();
     }
+    if (wown >= 0) add_block(wown, own);
+    if (pass || !accept || !__syncthreads_or(large)) break;
+    bool over = false;
+    for (int j = wv; j < np; j += NT / 64) {
+      float s = 0.f;
+      for (int f = lane; f < nf; f += 64) s += fabsf(ecur[(long)j * nf + f]);
+      const bool z = wave_sum((double)s) > (double)3.40282347e38f;
+      if (lane == 0) izero[j] = z ? 1 : 0;
+      over = over || z;
+    }
+    if (!__syncthreads_or(over)) break;
   }
-  if (wown >= 0) add_block(wown, own);
   __syncthreads();
   const double lam = s_sla[8];
   if (ext && a.hscale != 1.0) {
@@ -840,9 +958,10 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
   // node mean of a column: a wave per node, its lanes along the heights
   auto node_mean = [&](const float* x, int j) -> double {
     const double* cf = a.coefs + (long)j * nz;
+    const double cs = a.colsum[j];
     double s = 0.0;
     for (int k = lane; k < nz; k += 64) s = fma((double)x[k], cf[k], s);
-    return wave_sum(s) / a.colsum[j];
+    return wave_sum(s) / cs;
   };
   for (int ip = 0; ip < a.nparam; ++ip) {
     const int p = a.par[ip], j0 = a.j0[ip], nj = a.nj[ip];
@@ -931,6 +1050,7 @@ __global__ void __launch_bounds__(BIG ? LM_BIG_THREADS : LM_THREADS) lm_kernel(L
   }
 
   // ---- write back the inverted columns (the others are in place)
+#pragma unroll 1
   for (int p = 0; p < 12; ++p) {
     const int sl = a.rowslot[p];
     if (sl < 0 || p == A_TAU) continue;
