@@ -79,6 +79,13 @@ struct Cfg {
   // of strength and strength * shift over sqrt(pi)
   int comp0[MAXL], ntype[MAXL][3];
   float4 comp[MAXC], type[MAXL][3];
+  // what the transfer needs of a slot's line, together: the scalar loads of a
+  // layer then wait once
+  struct SlotRt {
+    int comp0, n[3];
+    float bldiff, vfac, pad[2];
+    float4 type[3];
+  } slot_rt[MAXS];
   float dz_cm[MAXNZ];
   double zz[MAXNZ];    // heights in km, rounded through REAL(4) like MODEL(:,13)
   // radiative-transfer workgroups of one column: each covers up to RT_WAVE
@@ -141,8 +148,9 @@ __global__ void __launch_bounds__(256) saha_kernel(MicroTile a) {
   const double lam = g_c.csaha1 * pow(T, -1.5);
   const double dlam = -3.0 / (2.0 * T);
   double* o = a.sbuf + (long)k * FZ_NELEM * 4 * a.ntile + ct;
+  const int per = (FZ_NELEM + gridDim.y - 1) / gridDim.y;   // elements of this workgroup
 #pragma unroll 1
-  for (int i = 0; i < FZ_NELEM; ++i) {
+  for (int i = blockIdx.y * per; i < min(FZ_NELEM, (int)(blockIdx.y + 1) * per); ++i) {
     double a1, a2, da1, da2;
     saha_element(i, T, lam, dlam, a.der != 0, a1, a2, da1, da2);
     o[(long)(i * 4 + 0) * a.ntile] = a1;
@@ -461,12 +469,26 @@ __global__ void __launch_bounds__(64) tau_kernel(MicroTile a) {
   // log tau_5000 by the REAL(4) trapezoid of forward.f90:1000-1006 (z in km)
   float tau = 1e-9f;
   a.atm[A_TAU * ps + (nz - 1) * cs + col] = log10f(tau);
-  for (int k = nz - 2; k >= 0; --k) {
-    const float x = (kc5[k * cs + col] * a.atm[A_RHO * ps + k * cs + col] +
-                     kc5[(k + 1) * cs + col] * a.atm[A_RHO * ps + (k + 1) * cs + col]) /
-                    2.0f;
-    tau = (float)((double)tau + (double)x * ((c_cfg.zz[k + 1] - c_cfg.zz[k]) * 1000.0 * 100.0));
-    a.atm[A_TAU * ps + k * cs + col] = log10f(tau);
+  // eight heights' loads together: the trapezoid is a chain, its terms are not
+  float xn = kc5[(nz - 1) * cs + col] * a.atm[A_RHO * ps + (nz - 1) * cs + col];
+  for (int k0 = nz - 2; k0 >= 0; k0 -= 8) {
+    float q[8], r[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int k = max(k0 - i, 0);
+      q[i] = kc5[k * cs + col];
+      r[i] = a.atm[A_RHO * ps + k * cs + col];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int k = k0 - i;
+      if (k < 0) break;
+      const float xk = q[i] * r[i];
+      const float x = (xk + xn) / 2.0f;
+      tau = (float)((double)tau + (double)x * ((c_cfg.zz[k + 1] - c_cfg.zz[k]) * 1000.0 * 100.0));
+      a.atm[A_TAU * ps + k * cs + col] = log10f(tau);
+      xn = xk;
+    }
   }
 }
 
@@ -491,8 +513,9 @@ __global__ void __launch_bounds__(256) saha_mid_kernel(MicroTile a, double* __re
   const double T = he_tmid(k, tm0, tm1);
   const double lam = g_c.csaha1 * pow(T, -1.5);
   double* o = smid + (long)k * FZ_NELEM * 4 * a.ntile + ct;
+  const int per = (FZ_NELEM + gridDim.y - 1) / gridDim.y;
 #pragma unroll 1
-  for (int i = 0; i < FZ_NELEM; ++i) {
+  for (int i = blockIdx.y * per; i < min(FZ_NELEM, (int)(blockIdx.y + 1) * per); ++i) {
     double a1, a2, da1, da2;
     saha_element(i, T, lam, 0.0, false, a1, a2, da1, da2);
     o[(long)(i * 4 + 0) * a.ntile] = a1;
@@ -668,22 +691,34 @@ __device__ __forceinline__ Sums absorb(P q, int r, float wave, float B, float dz
   Sums X;
   zero(X);
   for (int b = 0; b < c_cfg.reg_nblend[r]; ++b, q += REC_SLOT / 4) {
-    const int sl = c_cfg.reg_slot0[r] + b, li = c_cfg.slot_line[sl];
+    const Cfg::SlotRt sc = c_cfg.slot_rt[c_cfg.reg_slot0[r] + b];
     const float4 q0 = q[0], q5 = q[5];
     const VoigtPoly vp = voigt_load(q[2], q[3], q[4], q5.x);
     const float kl = q0.x * dz;
-    const float base = (wave - c_cfg.slot_bldiff[sl] + q5.w) * q5.y, bsc = B * q5.y;
-    const float4* cm = c_cfg.comp + c_cfg.comp0[li];
+    const float base = (wave - sc.bldiff + q5.w) * q5.y, bsc = B * q5.y;
+    const float4* cm = c_cfg.comp + sc.comp0;
 #pragma unroll
     for (int t = 0; t < 3; ++t) {
-      const float ut = fmaf(c_cfg.type[li][t].x, bsc, base);
-      const int n = c_cfg.ntype[li][t];
+      const float ut = fmaf(sc.type[t].x, bsc, base);
+      const int n = sc.n[t];
       float h = 0.f, f = 0.f;
-      for (int j = 0; j < n; ++j, ++cm) {
+      // two components at a time: one wait for their constants and two
+      // independent profiles
+      int j = 0;
+      for (; j + 2 <= n; j += 2, cm += 2) {
+        const float4 ca = cm[0], cb = cm[1];
+        float H, F, H2, F2;
+        voigt(vp, fmaf(ca.x, bsc, ut), H, F);
+        voigt(vp, fmaf(cb.x, bsc, ut), H2, F2);
+        h = fmaf(cb.y, H2, fmaf(ca.y, H, h));
+        f = fmaf(cb.y, F2, fmaf(ca.y, F, f));
+      }
+      if (j < n) {
         float H, F;
         voigt(vp, fmaf(cm->x, bsc, ut), H, F);
         h = fmaf(cm->y, H, h);
         f = fmaf(cm->y, F, f);
+        ++cm;
       }
       X.h[t] = fmaf(kl, h, X.h[t]);
       X.f[t] = fmaf(kl, f, X.f[t]);
@@ -710,14 +745,14 @@ __device__ __forceinline__ void absorb_der(P q, int r, float wave, float B, floa
     zero(XR);
   }
   for (int b = 0; b < c_cfg.reg_nblend[r]; ++b, q += REC_SLOT / 4) {
-    const int sl = c_cfg.reg_slot0[r] + b, li = c_cfg.slot_line[sl];
+    const Cfg::SlotRt sc = c_cfg.slot_rt[c_cfg.reg_slot0[r] + b];
     const float4 q0 = q[0], q5 = q[5];
     const VoigtPoly vp = voigt_load(q[2], q[3], q[4], q5.x);
     const float a = q0.y, kl = q0.x * dz, dklT = q0.z * dz;
-    const float base = (wave - c_cfg.slot_bldiff[sl] + q5.w) * q5.y, bsc = B * q5.y;
+    const float base = (wave - sc.bldiff + q5.w) * q5.y, bsc = B * q5.y;
     // kl times twice the derivatives of u in T (over u), v_z and |B| (over
     // the shift), and of a in T: the factor 2 of dH/du and dH/da
-    const float uT = kl * q5.z, uv = 2.f * kl * c_cfg.vfac[li] * q5.y, ub = 2.f * kl * q5.y, aT = 2.f * kl * q0.w;
+    const float uT = kl * q5.z, uv = 2.f * kl * sc.vfac * q5.y, ub = 2.f * kl * q5.y, aT = 2.f * kl * q0.w;
     float dklP = 0.f, dklR = 0.f, aP = 0.f, aR = 0.f;
     if (PR) {
       const float4 q1 = q[1];
@@ -726,12 +761,12 @@ __device__ __forceinline__ void absorb_der(P q, int r, float wave, float B, floa
       aP = 2.f * kl * q1.z;
       aR = 2.f * kl * q1.w;
     }
-    const float4* cm = c_cfg.comp + c_cfg.comp0[li];
+    const float4* cm = c_cfg.comp + sc.comp0;
 #pragma unroll
     for (int t = 0; t < 3; ++t) {
-      const float4 ty = c_cfg.type[li][t];
+      const float4 ty = sc.type[t];
       const float ut = fmaf(ty.x, bsc, base);
-      const int n = c_cfg.ntype[li][t];
+      const int n = sc.n[t];
       // half dH/du and dH/da summed over the type, and times u and the shift
       float h0 = 0.f, f0 = 0.f, hu, ha, huu, hau, hb, hab;
       if (n == 1) {
@@ -745,15 +780,29 @@ __device__ __forceinline__ void absorb_der(P q, int r, float wave, float B, floa
         ++cm;
       } else {
         float h1 = 0.f, f1 = 0.f, h2 = 0.f, f2 = 0.f;
-        for (int j = 0; j < n; ++j, ++cm) {
+        int j = 0;
+        for (; j + 2 <= n; j += 2, cm += 2) {
+          const float4 ca = cm[0], cb = cm[1];
+          float H, F, H2, F2;
+          voigt(vp, fmaf(ca.x, bsc, ut), H, F);
+          voigt(vp, fmaf(cb.x, bsc, ut), H2, F2);
+          h0 = fmaf(cb.y, H2, fmaf(ca.y, H, h0));
+          f0 = fmaf(cb.y, F2, fmaf(ca.y, F, f0));
+          h1 = fmaf(cb.z, H2, fmaf(ca.z, H, h1));
+          f1 = fmaf(cb.z, F2, fmaf(ca.z, F, f1));
+          h2 = fmaf(cb.w, H2, fmaf(ca.w, H, h2));
+          f2 = fmaf(cb.w, F2, fmaf(ca.w, F, f2));
+        }
+        if (j < n) {
+          const float4 ca = *cm++;
           float H, F;
-          voigt(vp, fmaf(cm->x, bsc, ut), H, F);
-          h0 = fmaf(cm->y, H, h0);
-          f0 = fmaf(cm->y, F, f0);
-          h1 = fmaf(cm->z, H, h1);
-          f1 = fmaf(cm->z, F, f1);
-          h2 = fmaf(cm->w, H, h2);
-          f2 = fmaf(cm->w, F, f2);
+          voigt(vp, fmaf(ca.x, bsc, ut), H, F);
+          h0 = fmaf(ca.y, H, h0);
+          f0 = fmaf(ca.y, F, f0);
+          h1 = fmaf(ca.z, H, h1);
+          f1 = fmaf(ca.z, F, f1);
+          h2 = fmaf(ca.w, H, h2);
+          f2 = fmaf(ca.w, F, f2);
         }
         hu = fmaf(a, f0, -fmaf(ut, h0, bsc * h1));
         ha = fmaf(a, h0, fmaf(ut, f0, fmaf(bsc, f1, -ty.y)));
@@ -1893,6 +1942,17 @@ int fz_configure(fz_ctx* c, const fz_line* lines, int nlines, const fz_region* r
       g.blk_n[g.nbpc] = std::min(RT_WAVE, g.reg_pix0[r] + g.reg_nwave[r] - l0);
       ++g.nbpc;
     }
+  for (int sl = 0; sl < ns; ++sl) {
+    const int li = g.slot_line[sl];
+    Cfg::SlotRt& q = g.slot_rt[sl];
+    q.comp0 = g.comp0[li];
+    q.bldiff = g.slot_bldiff[sl];
+    q.vfac = g.vfac[li];
+    for (int t = 0; t < 3; ++t) {
+      q.n[t] = g.ntype[li][t];
+      q.type[t] = g.type[li][t];
+    }
+  }
   g.rec = REC_HEAD;
   for (int r = 0; r < nreg; ++r) {
     g.reg_rec[r] = g.rec;
@@ -2276,6 +2336,15 @@ static int auto_mtile(fz_ctx* c, bool hydro) {
   return (int)std::max<size_t>(4096, std::min<size_t>(m, 1 << 20));
 }
 
+// Grid of the Saha kernels over n (height, column) pairs: the 92 elements are
+// shared out over up to 46 workgroups where the pairs alone do not give every
+// SIMD two waves (one workgroup per pair block takes 80 us for a single
+// column, the partition functions of all elements being a chain).
+static dim3 saha_grid(long n) {
+  const unsigned nb = (unsigned)((n + 255) / 256);
+  return dim3(nb, std::max(1u, std::min(46u, 512u / nb)));
+}
+
 // Lanes per column of the fixed-point kernels for a tile of n columns: as
 // many as keep about one wave per SIMD (1024), since a column's heights are a
 // chain and only more columns or more lanes fill the card; beyond, 16, whose
@@ -2338,11 +2407,10 @@ static int run_micro(fz_ctx* c, int ncol, float* d_atm, int32_t** status, bool d
     a.status = stv;
     a.pop = c->pop_on ? c->d_pop : nullptr;
     const long nkt = (long)nz * a.ntile;
-    hipLaunchKernelGGL(saha_kernel, dim3((unsigned)((nkt + 255) / 256)), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(saha_kernel, saha_grid(nkt), dim3(256), 0, st, a);
     if (hydro) {
       const long nmt = (long)(nz - 1) * a.ntile;
-      hipLaunchKernelGGL(saha_mid_kernel, dim3((unsigned)((nmt + 255) / 256)), dim3(256), 0, st, a,
-                         (double*)c->d_smid);
+      hipLaunchKernelGGL(saha_mid_kernel, saha_grid(nmt), dim3(256), 0, st, a, (double*)c->d_smid);
     }
     const int gl = rho_lanes(a.ntile);
     const dim3 gr((unsigned)(((long)a.ntile * gl + RHO_BLOCK - 1) / RHO_BLOCK)), gb(RHO_BLOCK);
