@@ -1646,41 +1646,37 @@ struct MlpState {
   long np = 0;
   long woff[8] = {0}, boff[8] = {0};
   int din[8] = {0}, dout[8] = {0};
+  MlpShape shape;           // the same, and where the parameters are, for the kernels
   float *w = nullptr, *g = nullptr, *m1 = nullptr, *m2 = nullptr;
-  bf16* wb = nullptr;
+  bf16* wb = nullptr;       // each W_l and its transpose
   float* norms = nullptr;   // xmean[nin], xstd[nin], tmean[nout], tstd[nout]
   double* pinv = nullptr;   // [nj][nz] least-squares node fit
   double* coefs = nullptr;  // [nz][nj] hat basis
-  long step = 0;
-  int cap = 0;              // rows the work buffers hold
-  bf16* X = nullptr;
-  bf16* act = nullptr;      // [nl][cap][nh]
-  float* Y = nullptr;       // [cap][nout]
-  float* dYf = nullptr;
-  bf16* dYb = nullptr;
-  float* dZf[2] = {nullptr, nullptr};
-  bf16* dZb[2] = {nullptr, nullptr};
-  float* partial = nullptr;
   float* loss = nullptr;
+  long step = 0;
+  int cap = 0;              // rows the work buffers hold; with the gradient's, gcap
+  int gcap = 0;
+  bf16 *X = nullptr, *XT = nullptr;
+  bf16 *act = nullptr, *actT = nullptr;   // [nl] of frag_size(cap, nh)
+  bf16 *dZ = nullptr, *dZT = nullptr;     // two of the widest layer; every layer's
+  float *csum = nullptr, *partial = nullptr;
+  size_t act_stride() const { return frag_size(cap, nh); }
+  size_t dzt_stride() const { return frag_size(std::max(nh, nout), cap); }
+  size_t csum_stride() const { return (size_t)pad32(cap) / 16 * pad32(std::max(nh, nout)); }
   void release() {
-    void* ps[] = {w, g, m1, m2, wb, norms, pinv, coefs, X, act, Y, dYf, dYb, dZf[0], dZf[1], dZb[0], dZb[1],
-                  partial, loss};
+    release_work();
+    void* ps[] = {w, g, m1, m2, wb, norms, pinv, coefs, loss};
     for (void* q : ps)
       if (q) (void)hipFree(q);
     *this = MlpState();
   }
   void release_work() {
-    void* ps[] = {X, act, Y, dYf, dYb, dZf[0], dZf[1], dZb[0], dZb[1], partial};
+    void* ps[] = {X, XT, act, actT, dZ, dZT, csum, partial};
     for (void* q : ps)
       if (q) (void)hipFree(q);
-    X = nullptr;
-    act = nullptr;
-    Y = dYf = nullptr;
-    dYb = nullptr;
-    dZf[0] = dZf[1] = nullptr;
-    dZb[0] = dZb[1] = nullptr;
-    partial = nullptr;
-    cap = 0;
+    X = XT = act = actT = dZ = dZT = nullptr;
+    csum = partial = nullptr;
+    cap = gcap = 0;
   }
 };
 
@@ -4270,134 +4266,178 @@ uint64_t splitmix64(uint64_t& x) {
   return z ^ (z >> 31);
 }
 
-int mlp_work(fz_ctx* c, int n) {
+// Work buffers for n rows of the forward pass and, with grad, of the gradient.
+int mlp_work(fz_ctx* c, int n, bool grad) {
   MlpState& M = c->mlp;
-  if (M.cap >= n) return FZ_OK;
+  if ((grad ? M.gcap : M.cap) >= n) return FZ_OK;
   M.release_work();
-  const size_t r = (size_t)n;
-  const int nmax = std::max(M.nh, std::max(M.nin, M.nout));
-  bool ok = hipMalloc(&M.X, sizeof(bf16) * r * M.nin) == hipSuccess &&
-            hipMalloc(&M.act, sizeof(bf16) * r * M.nh * M.nl) == hipSuccess &&
-            hipMalloc(&M.Y, sizeof(float) * r * M.nout) == hipSuccess &&
-            hipMalloc(&M.dYf, sizeof(float) * r * M.nout) == hipSuccess &&
-            hipMalloc(&M.dYb, sizeof(bf16) * r * M.nout) == hipSuccess &&
-            hipMalloc(&M.partial, sizeof(float) * ((r * M.nout + 255) / 256 + 1)) == hipSuccess;
-  for (int i = 0; i < 2 && ok; ++i)
-    ok = hipMalloc(&M.dZf[i], sizeof(float) * r * nmax) == hipSuccess &&
-         hipMalloc(&M.dZb[i], sizeof(bf16) * r * nmax) == hipSuccess;
+  M.cap = n;
+  bool ok = hipMalloc(&M.X, sizeof(bf16) * frag_size(n, M.nin)) == hipSuccess &&
+            hipMalloc(&M.act, sizeof(bf16) * M.act_stride() * M.nl) == hipSuccess;
+  if (grad)
+    ok = ok && hipMalloc(&M.XT, sizeof(bf16) * frag_size(M.nin, n)) == hipSuccess &&
+         hipMalloc(&M.actT, sizeof(bf16) * frag_size(M.nh, n) * M.nl) == hipSuccess &&
+         hipMalloc(&M.dZ, sizeof(bf16) * 2 * frag_size(n, std::max(M.nh, M.nout))) == hipSuccess &&
+         hipMalloc(&M.dZT, sizeof(bf16) * M.dzt_stride() * (M.nl + 1)) == hipSuccess &&
+         hipMalloc(&M.csum, sizeof(float) * M.csum_stride() * (M.nl + 1)) == hipSuccess &&
+         hipMalloc(&M.partial, sizeof(float) * 4 * (pad32(n) / 32) * (pad32(M.nout) / 32)) == hipSuccess;
   if (!ok) {
     M.release_work();
     return set_err(c, FZ_ENOMEM, "device allocation failed (network work buffers)");
   }
-  M.cap = n;
+  if (grad) M.gcap = n;
   return FZ_OK;
 }
 
-void mlp_gemm(const GemmArgs& g, hipStream_t st) {
-  const dim3 grid((unsigned)((g.N + MLP_TN - 1) / MLP_TN), (unsigned)((g.M + MLP_TM - 1) / MLP_TM));
-  hipLaunchKernelGGL(mlp_gemm_kernel, grid, dim3(256), 0, st, g);
-}
-
-GemmArgs gemm0() {
+// A product of the network: D[m][n], A [N][K] and B [M][K] in operand order
+GemmArgs mlp_gemm(const bf16* A, const bf16* B, int M, int N, int K) {
   GemmArgs g;
   memset(&g, 0, sizeof(g));
+  g.A = A;
+  g.B = B;
+  g.M = M;
+  g.N = N;
+  g.ks = pad32(K) / 32;
+  g.tn = pad32(N) / 32;
   return g;
 }
 
-// forward pass of n rows already in M.X; the output (standardised) in M.Y
-void mlp_forward_rows(MlpState& M, int n, hipStream_t st) {
-  for (int l = 0; l <= M.nl; ++l) {
-    GemmArgs g = gemm0();
-    g.M = n;
-    g.N = M.dout[l];
-    g.K = M.din[l];
-    g.A = l == 0 ? M.X : M.act + (size_t)(l - 1) * M.cap * M.nh;
-    g.sam = M.din[l];
-    g.sak = 1;
-    g.B = M.wb + M.woff[l];
-    g.sbn = M.din[l];
-    g.sbk = 1;
+template <int MODE>
+void mlp_layer(GemmArgs g, const LossArgs& ls, hipStream_t st) {
+  const long m64 = (g.M + 63) / 64, n64 = (g.N + 63) / 64;
+  if (MODE != MLP_LOSS && m64 * n64 >= 512) {
+    g.tn = (int)n64;
+    hipLaunchKernelGGL((mlp_layer_kernel<MODE, 2>), dim3((unsigned)(m64 * n64)), dim3(256), 0, st, g, ls);
+  } else {
+    hipLaunchKernelGGL((mlp_layer_kernel<MODE, 1>), dim3((unsigned)(pad32(g.M) / 32 * g.tn)), dim3(256), 0, st, g, ls);
+  }
+}
+
+// Forward pass of n rows already in M.X: the hidden layers (with their
+// transposes for the gradient) and, when y is given, the output (standardised).
+void mlp_forward_rows(MlpState& M, int n, float* y, bool grad, hipStream_t st) {
+  const LossArgs none = {};
+  for (int l = 0; l < M.nl + (y ? 1 : 0); ++l) {
+    GemmArgs g = mlp_gemm(M.wb + M.shape.wb[l], l == 0 ? M.X : M.act + (l - 1) * M.act_stride(), n, M.dout[l],
+                          M.din[l]);
     g.bias = M.w + M.boff[l];
     if (l < M.nl) {
-      g.relu = 1;
-      g.Cb = M.act + (size_t)l * M.cap * M.nh;
-      g.sbm2 = M.dout[l];
-      g.sbn2 = 1;
+      g.Cb = M.act + l * M.act_stride();
+      if (grad) g.CbT = M.actT + l * frag_size(M.nh, M.cap);
+      mlp_layer<MLP_HIDDEN>(g, none, st);
     } else {
-      g.Cf = M.Y;
-      g.scm = M.nout;
-      g.scn = 1;
+      g.Cf = y;
+      mlp_layer<MLP_OUT>(g, none, st);
     }
-    mlp_gemm(g, st);
   }
 }
 
-// loss and gradient of the parameters into M.g for n rows (targets t, rows
-// gathered by idx when given); the mean squared error into M.loss[0]
-void mlp_backward_rows(MlpState& M, int n, const float* d_t, const int32_t* d_idx, hipStream_t st) {
+// Output layer, loss and gradient of the parameters for n rows (targets t,
+// rows gathered by idx when given): the mean squared error into loss[0].
+void mlp_backward_rows(MlpState& M, int n, const float* d_t, const int32_t* d_idx, float* loss, float* grad,
+                       hipStream_t st) {
   const float* tmean = M.norms + 2 * M.nin;
-  const float* tstd = tmean + M.nout;
-  const long ne = (long)n * M.nout;
-  const unsigned nb = (unsigned)((ne + 255) / 256);
-  hipLaunchKernelGGL(mlp_loss_kernel, dim3(nb), dim3(256), 0, st, n, M.nout, (const float*)M.Y, d_t, d_idx, tmean,
-                     tstd, M.dYf, M.dYb, M.partial);
-  hipLaunchKernelGGL(mlp_reduce_kernel, dim3(1), dim3(256), 0, st, (int)nb, (const float*)M.partial, (float)ne, M.loss);
-  const float* cf = M.dYf;
-  const bf16* cb = M.dYb;
-  int buf = 0;
+  LossArgs ls = {d_t, tmean, tmean + M.nout, d_idx, M.partial};
+  DwArgs dw;
+  memset(&dw, 0, sizeof(dw));
+  const bf16* dz = nullptr;
   for (int l = M.nl; l >= 0; --l) {
-    const bf16* ain = l == 0 ? M.X : M.act + (size_t)(l - 1) * M.cap * M.nh;
-    const int di = M.din[l], dO = M.dout[l];
-    GemmArgs g = gemm0();   // dW_l[o][k] = sum_m dZ[m][o] A_in[m][k]
-    g.M = dO;
-    g.N = di;
-    g.K = n;
-    g.A = cb;
-    g.sam = 1;
-    g.sak = dO;
-    g.B = ain;
-    g.sbn = 1;
-    g.sbk = di;
-    g.Cf = M.g + M.woff[l];
-    g.scm = di;
-    g.scn = 1;
-    mlp_gemm(g, st);
-    hipLaunchKernelGGL(mlp_colsum_kernel, dim3((unsigned)((dO + 255) / 256)), dim3(256), 0, st, n, dO, cf,
-                       M.g + M.boff[l]);
-    if (l == 0) break;
-    GemmArgs h = gemm0();   // dA_in[m][k] = sum_o dZ[m][o] W_l[o][k], times ReLU'(A_in)
-    h.M = n;
-    h.N = di;
-    h.K = dO;
-    h.A = cb;
-    h.sam = dO;
-    h.sak = 1;
-    h.B = M.wb + M.woff[l];
-    h.sbn = 1;
-    h.sbk = di;
-    h.mask = ain;
-    h.smm = di;
-    h.smn = 1;
-    h.Cf = M.dZf[buf];
-    h.scm = di;
-    h.scn = 1;
-    h.Cb = M.dZb[buf];
-    h.sbm2 = di;
-    h.sbn2 = 1;
-    mlp_gemm(h, st);
-    cf = M.dZf[buf];
-    cb = M.dZb[buf];
-    buf ^= 1;
+    bf16* out = M.dZ + (l & 1) * frag_size(M.cap, std::max(M.nh, M.nout));
+    bf16* outT = M.dZT + l * M.dzt_stride();
+    GemmArgs g;
+    if (l == M.nl)         // Y = A W^T + b and dY from it
+      g = mlp_gemm(M.wb + M.shape.wb[l], M.act + (l - 1) * M.act_stride(), n, M.dout[l], M.din[l]);
+    else                   // dZ_l[m][k] = sum_o dZ_(l+1)[m][o] W_(l+1)[o][k], times ReLU'
+      g = mlp_gemm(M.wb + M.shape.wt[l + 1], dz, n, M.dout[l], M.dout[l + 1]);
+    g.bias = M.w + M.boff[l];
+    g.mask = l < M.nl ? M.act + l * M.act_stride() : nullptr;
+    g.Cb = out;
+    g.CbT = outT;
+    g.csum = M.csum + l * M.csum_stride();
+    if (l == M.nl)
+      mlp_layer<MLP_LOSS>(g, ls, st);
+    else
+      mlp_layer<MLP_DACT>(g, ls, st);
+    dz = out;
+    // dW_l[o][k] = sum_m dZ_l[m][o] A_l[m][k]
+    GemmArgs& h = dw.g[l];
+    h = mlp_gemm(l == 0 ? M.XT : M.actT + (l - 1) * frag_size(M.nh, M.cap), outT, M.dout[l], M.din[l], n);
+    h.Cf = grad + M.woff[l];
+    dw.csum[l] = g.csum;
+    dw.bg[l] = grad + M.boff[l];
   }
+  dw.n = M.nl + 1;
+  dw.nparts = pad32(n) / 16;
+  int nb = 0;
+  for (int l = 0; l <= M.nl; ++l) {
+    dw.g[l].tile0 = nb;
+    nb += pad32(M.dout[l]) / 32 * dw.g[l].tn;
+  }
+  for (int l = 0; l <= M.nl; ++l) {
+    dw.blk0[l] = nb;
+    nb += (M.dout[l] + 15) / 16;
+  }
+  dw.loss_blk = nb;
+  dw.nloss = 4 * (pad32(n) / 32) * (pad32(M.nout) / 32);
+  dw.lpart = M.partial;
+  dw.lscale = (float)((long)n * M.nout);
+  dw.loss = loss;
+  hipLaunchKernelGGL(mlp_dw_kernel, dim3((unsigned)(nb + 1)), dim3(256), 0, st, dw);
 }
 
-int mlp_input(fz_ctx* c, int n, const float* d_x, const double* d_xd, const int32_t* d_idx, hipStream_t st) {
+int mlp_input(fz_ctx* c, int n, const float* d_x, const double* d_xd, const int32_t* d_idx, bool grad,
+              hipStream_t st) {
   MlpState& M = c->mlp;
-  const long ne = (long)n * M.nin;
-  hipLaunchKernelGGL(mlp_input_kernel, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, st, n, M.nin, d_x, d_xd,
-                     d_idx, (const float*)M.norms, (const float*)(M.norms + M.nin), M.X);
+  const size_t np = frag_size(n, M.nin) / 8 * (grad ? 2 : 1);
+  hipLaunchKernelGGL(mlp_input_kernel, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, st, n, M.nin, d_x, d_xd,
+                     d_idx, (const float*)M.norms, (const float*)(M.norms + M.nin), M.X, grad ? M.XT : nullptr);
   HIPCHK(c, hipGetLastError());
   return FZ_OK;
+}
+
+// Bytes of LDS of mlp_infer_kernel for tiles of R rows
+size_t mlp_infer_lds(const MlpState& M, int R) {
+  const size_t pitch = std::max(pad32(M.nin), pad32(M.nh)) + 8;
+  return std::max(sizeof(bf16) * R * pitch, sizeof(float) * 2 * R * M.nout);
+}
+
+constexpr size_t MLP_LDS = 144 * 1024;
+
+template <int MF>
+int mlp_infer_launch(fz_ctx* c, const InferArgs& a, hipStream_t st) {
+  const size_t lds = mlp_infer_lds(c->mlp, 16 * MF);
+  HIPCHK(c, hipFuncSetAttribute((const void*)mlp_infer_kernel<MF>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)MLP_LDS));
+  hipLaunchKernelGGL((mlp_infer_kernel<MF>), dim3((unsigned)((a.n + 16 * MF - 1) / (16 * MF))), dim3(512), lds, st,
+                     c->mlp.shape, a);
+  HIPCHK(c, hipGetLastError());
+  return FZ_OK;
+}
+
+// All layers in one launch, where the network fits the kernel (widest layer
+// and LDS): 16 rows a workgroup while these fill no more than the chip, else 32, else
+// 64, so that the weights are read through as few CUs' ports as keep all busy.
+bool mlp_infer_fits(const MlpState& M) { return M.nh <= MLP_INFER_NH && mlp_infer_lds(M, 16) <= MLP_LDS; }
+
+int mlp_infer(fz_ctx* c, int n, const float* d_x, const double* d_xd, float* d_y, float* d_atm, hipStream_t st) {
+  MlpState& M = c->mlp;
+  InferArgs a;
+  a.n = n;
+  a.pitch = std::max(pad32(M.nin), pad32(M.nh)) + 8;
+  a.xf = d_x;
+  a.xd = d_xd;
+  a.mean = M.norms;
+  a.sdev = M.norms + M.nin;
+  a.tmean = M.norms + 2 * M.nin;
+  a.tstd = a.tmean + M.nout;
+  a.w = M.w;
+  a.wb = M.wb;
+  a.y = d_y;
+  a.coefs = M.coefs;
+  a.atm = d_atm;
+  if (n > 8192 && mlp_infer_lds(M, 64) <= MLP_LDS) return mlp_infer_launch<4>(c, a, st);
+  if (n > 4096 && mlp_infer_lds(M, 32) <= MLP_LDS) return mlp_infer_launch<2>(c, a, st);
+  return mlp_infer_launch<1>(c, a, st);
 }
 
 }  // namespace
@@ -4427,6 +4467,24 @@ int fz_mlp_create(fz_ctx* c, int nin, int nhidden, int nlayers, int nodes, uint6
     off += M.dout[l];
   }
   M.np = off;
+  size_t nwb = 0;
+  MlpShape& S = M.shape;
+  memset(&S, 0, sizeof(S));
+  S.nl = nlayers;
+  S.nin = nin;
+  S.nout = M.nout;
+  S.nj = nodes;
+  S.nz = M.nz;
+  for (int l = 0; l <= nlayers; ++l) {
+    S.din[l] = M.din[l];
+    S.dout[l] = M.dout[l];
+    S.woff[l] = M.woff[l];
+    S.boff[l] = M.boff[l];
+    S.wb[l] = (long)nwb;
+    nwb += frag_size(M.dout[l], M.din[l]);
+    S.wt[l] = (long)nwb;
+    nwb += frag_size(M.din[l], M.dout[l]);
+  }
   // He-uniform weights for ReLU layers (bound sqrt(6 / fan_in)), the output
   // layer scaled by 1/4; zero biases
   std::vector<float> w(off, 0.f);
@@ -4438,7 +4496,7 @@ int fz_mlp_create(fz_ctx* c, int nin, int nhidden, int nlayers, int nodes, uint6
   }
   bool ok = hipMalloc(&M.w, sizeof(float) * off) == hipSuccess && hipMalloc(&M.g, sizeof(float) * off) == hipSuccess &&
             hipMalloc(&M.m1, sizeof(float) * off) == hipSuccess &&
-            hipMalloc(&M.m2, sizeof(float) * off) == hipSuccess && hipMalloc(&M.wb, sizeof(bf16) * off) == hipSuccess &&
+            hipMalloc(&M.m2, sizeof(float) * off) == hipSuccess && hipMalloc(&M.wb, sizeof(bf16) * nwb) == hipSuccess &&
             hipMalloc(&M.norms, sizeof(float) * 2 * (nin + M.nout)) == hipSuccess &&
             hipMalloc(&M.pinv, sizeof(double) * nodes * M.nz) == hipSuccess &&
             hipMalloc(&M.coefs, sizeof(double) * nodes * M.nz) == hipSuccess &&
@@ -4451,8 +4509,9 @@ int fz_mlp_create(fz_ctx* c, int nin, int nhidden, int nlayers, int nodes, uint6
   HIPCHK(c, hipMemset(M.m1, 0, sizeof(float) * off));
   HIPCHK(c, hipMemset(M.m2, 0, sizeof(float) * off));
   HIPCHK(c, hipMemset(M.g, 0, sizeof(float) * off));
-  hipLaunchKernelGGL(mlp_to_bf16_kernel, dim3((unsigned)((off + 255) / 256)), dim3(256), 0, 0, off, (const float*)M.w,
-                     M.wb);
+  HIPCHK(c, hipMemset(M.wb, 0, sizeof(bf16) * nwb));   // the padding of K stays zero
+  hipLaunchKernelGGL(mlp_to_bf16_kernel, dim3((unsigned)((off + 255) / 256)), dim3(256), 0, 0, off, S,
+                     (const float*)M.w, M.wb);
   HIPCHK(c, hipGetLastError());
   std::vector<float> nrm(2 * (nin + M.nout));
   for (int i = 0; i < nin; ++i) {
@@ -4541,7 +4600,7 @@ int fz_mlp_set_params(fz_ctx* c, const float* params) {
   HIPCHK(c, hipMemcpy(M.w, params, sizeof(float) * M.np, hipMemcpyHostToDevice));
   HIPCHK(c, hipMemcpy(M.norms, params + M.np, sizeof(float) * 2 * (M.nin + M.nout), hipMemcpyHostToDevice));
   hipLaunchKernelGGL(mlp_to_bf16_kernel, dim3((unsigned)((M.np + 255) / 256)), dim3(256), 0, 0, M.np,
-                     (const float*)M.w, M.wb);
+                     M.shape, (const float*)M.w, M.wb);
   HIPCHK(c, hipGetLastError());
   HIPCHK(c, hipMemset(M.m1, 0, sizeof(float) * M.np));
   HIPCHK(c, hipMemset(M.m2, 0, sizeof(float) * M.np));
@@ -4578,17 +4637,16 @@ int fz_mlp_forward_dev(fz_ctx* c, int n, const float* d_x, const double* d_xd, f
   MlpState& M = c->mlp;
   hipStream_t st = (hipStream_t)stream;
   HIPCHK(c, hipSetDevice(c->device));
+  if (mlp_infer_fits(M)) return mlp_infer(c, n, d_x, d_xd, d_y, nullptr, st);
   const int chunk = 65536;
-  int r = mlp_work(c, std::min(n, chunk));
+  int r = mlp_work(c, std::min(n, chunk), false);
   if (r) return r;
   for (int r0 = 0; r0 < n; r0 += M.cap) {
     const int nr = std::min(M.cap, n - r0);
     r = mlp_input(c, nr, d_x ? d_x + (size_t)r0 * M.nin : nullptr, d_xd ? d_xd + (size_t)r0 * M.nin : nullptr,
-                  nullptr, st);
+                  nullptr, false, st);
     if (r) return r;
-    mlp_forward_rows(M, nr, st);
-    HIPCHK(c, hipMemcpyAsync(d_y + (size_t)r0 * M.nout, M.Y, sizeof(float) * nr * M.nout, hipMemcpyDeviceToDevice,
-                             st));
+    mlp_forward_rows(M, nr, d_y + (size_t)r0 * M.nout, false, st);
   }
   HIPCHK(c, hipGetLastError());
   return FZ_OK;
@@ -4600,14 +4658,12 @@ int fz_mlp_gradient_dev(fz_ctx* c, int n, const float* d_x, const float* d_t, co
   MlpState& M = c->mlp;
   hipStream_t st = (hipStream_t)stream;
   HIPCHK(c, hipSetDevice(c->device));
-  int r = mlp_work(c, n);
+  int r = mlp_work(c, n, true);
   if (r) return r;
-  r = mlp_input(c, n, d_x, nullptr, d_idx, st);
+  r = mlp_input(c, n, d_x, nullptr, d_idx, true, st);
   if (r) return r;
-  mlp_forward_rows(M, n, st);
-  mlp_backward_rows(M, n, d_t, d_idx, st);
-  if (d_loss) HIPCHK(c, hipMemcpyAsync(d_loss, M.loss, sizeof(float), hipMemcpyDeviceToDevice, st));
-  if (d_grad) HIPCHK(c, hipMemcpyAsync(d_grad, M.g, sizeof(float) * M.np, hipMemcpyDeviceToDevice, st));
+  mlp_forward_rows(M, n, nullptr, true, st);
+  mlp_backward_rows(M, n, d_t, d_idx, d_loss ? d_loss : M.loss, d_grad ? d_grad : M.g, st);
   HIPCHK(c, hipGetLastError());
   return FZ_OK;
 }
@@ -4622,7 +4678,7 @@ int fz_mlp_train_step_dev(fz_ctx* c, int n, const float* d_x, const float* d_t, 
   const float c1 = (float)(1.0 - std::pow((double)b1, (double)M.step));
   const float c2 = (float)(1.0 - std::pow((double)b2, (double)M.step));
   hipLaunchKernelGGL(mlp_adam_kernel, dim3((unsigned)((M.np + 255) / 256)), dim3(256), 0, (hipStream_t)stream, M.np,
-                     M.w, (const float*)M.g, M.m1, M.m2, M.wb, lr, b1, b2, 1e-8f, c1, c2);
+                     M.shape, M.w, (const float*)M.g, M.m1, M.m2, M.wb, lr, b1, b2, 1e-8f, c1, c2);
   HIPCHK(c, hipGetLastError());
   return FZ_OK;
 }
@@ -4633,11 +4689,17 @@ int fz_learned_init_dev(fz_ctx* c, int ncol, const double* d_obs, float* d_atm, 
   MlpState& M = c->mlp;
   hipStream_t st = (hipStream_t)stream;
   HIPCHK(c, hipSetDevice(c->device));
+  if (mlp_infer_fits(M)) {
+    const int r = mlp_infer(c, ncol, nullptr, d_obs, nullptr, d_atm, st);
+    if (r) return r;
+    HIPCHK(c, hipStreamSynchronize(st));
+    return FZ_OK;
+  }
   DevBuf y;
   HIPCHK(c, hipMalloc(&y.p, sizeof(float) * (size_t)ncol * M.nout));
   int r = fz_mlp_forward_dev(c, ncol, nullptr, d_obs, (float*)y.p, stream);
   if (r) return r;
-  hipLaunchKernelGGL(mlp_decode_kernel, dim3((unsigned)((ncol + 127) / 128)), dim3(128), 0, st, ncol, M.nz, M.nj,
+  hipLaunchKernelGGL(mlp_decode_kernel, dim3((unsigned)((ncol + 31) / 32)), dim3(256), 0, st, M.shape, ncol,
                      (const float*)y.p, (const float*)(M.norms + 2 * M.nin), (const float*)(M.norms + 2 * M.nin + M.nout),
                      (const double*)M.coefs, d_atm);
   HIPCHK(c, hipGetLastError());
