@@ -138,25 +138,34 @@ struct MicroTile {
   const double* pop;
 };
 
+// The Saha factors of every (height, column), one thread each, all lanes of a
+// wave at the same element; with DER their T derivatives too (without
+// them those rows are neither written nor read).
+// Bounds: with DER the writes (2944 B per height and column), without them the FP64
+// issue about as much as the writes.  The partition functions' derivatives, four
+// divisions and two general exponentials per element, and the rows of zeros left out
+// where nothing reads them: 82944 columns x 96 heights 5.5 -> 2.75 ms; with DER
+// 36864 x 96 take 2.15 ms before and after.
+template <bool DER>
 __global__ void __launch_bounds__(256) saha_kernel(MicroTile a) {
   const int nz = c_cfg.nz;
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (long)nz * a.ntile) return;
   const int k = (int)(t / a.ntile), ct = (int)(t - (long)k * a.ntile);
   const long cs = a.ncol, ps = (long)nz * a.ncol;
-  const double T = (double)a.atm[A_T * ps + k * cs + a.col0 + ct];
-  const double lam = g_c.csaha1 * pow(T, -1.5);
-  const double dlam = -3.0 / (2.0 * T);
+  const SahaT s((double)a.atm[A_T * ps + k * cs + a.col0 + ct]);
   double* o = a.sbuf + (long)k * FZ_NELEM * 4 * a.ntile + ct;
   const int per = (FZ_NELEM + gridDim.y - 1) / gridDim.y;   // elements of this workgroup
 #pragma unroll 1
   for (int i = blockIdx.y * per; i < min(FZ_NELEM, (int)(blockIdx.y + 1) * per); ++i) {
     double a1, a2, da1, da2;
-    saha_element(i, T, lam, dlam, a.der != 0, a1, a2, da1, da2);
+    saha_element<DER>(i, s, a1, a2, da1, da2);
     o[(long)(i * 4 + 0) * a.ntile] = a1;
     o[(long)(i * 4 + 1) * a.ntile] = a2;
-    o[(long)(i * 4 + 2) * a.ntile] = da1;
-    o[(long)(i * 4 + 3) * a.ntile] = da2;
+    if constexpr (DER) {
+      o[(long)(i * 4 + 2) * a.ntile] = da1;
+      o[(long)(i * 4 + 3) * a.ntile] = da2;
+    }
   }
 }
 
@@ -181,12 +190,6 @@ __global__ void __launch_bounds__(256) saha_kernel(MicroTile a) {
 // column that this replaces: hydrostatic integration of 16 columns x 64
 // heights 8.9 -> 0.55 ms, of 9216 x 96 heights 26.9 -> 2.2 ms; the forward's
 // fixed point of 82944 columns x 96 heights 24.4 -> 6.5 ms.
-__device__ __forceinline__ double rcp64(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  r = fma(fma(-x, r, 1.0), r, r);
-  return fma(fma(-x, r, 1.0), r, r);
-}
-
 template <int CTRL>
 __device__ __forceinline__ double dpp64(double x) {
   const int lo = __double2loint(x), hi = __double2hiint(x);
@@ -369,7 +372,10 @@ __global__ void __launch_bounds__(256) deriv_kernel(MicroTile a) {
   a.deriv[7 * ds + o] = d.ne_rho_T;
 }
 
-__global__ void __launch_bounds__(256) opac_kernel(MicroTile a) {
+// Bound by its FP64 chains and their latency: limited to 256 registers (22 of them
+// then spill, outside the loops) two waves share a SIMD instead of one: 82944
+// columns x 96 heights 2.65 -> 2.15 ms, with response functions 36864 x 96 1.57 -> 1.27 ms.
+__global__ void __launch_bounds__(256, 2) opac_kernel(MicroTile a) {
   const int nz = c_cfg.nz;
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (long)nz * a.ntile) return;
@@ -510,14 +516,13 @@ __global__ void __launch_bounds__(256) saha_mid_kernel(MicroTile a, double* __re
   const long cs = a.ncol, ps = (long)nz * a.ncol;
   const double tm0 = (double)a.atm[A_T * ps + (k + 1) * cs + a.col0 + ct];
   const double tm1 = (double)a.atm[A_T * ps + k * cs + a.col0 + ct];
-  const double T = he_tmid(k, tm0, tm1);
-  const double lam = g_c.csaha1 * pow(T, -1.5);
+  const SahaT s(he_tmid(k, tm0, tm1));
   double* o = smid + (long)k * FZ_NELEM * 4 * a.ntile + ct;
   const int per = (FZ_NELEM + gridDim.y - 1) / gridDim.y;
 #pragma unroll 1
   for (int i = blockIdx.y * per; i < min(FZ_NELEM, (int)(blockIdx.y + 1) * per); ++i) {
     double a1, a2, da1, da2;
-    saha_element(i, T, lam, 0.0, false, a1, a2, da1, da2);
+    saha_element<false>(i, s, a1, a2, da1, da2);
     o[(long)(i * 4 + 0) * a.ntile] = a1;
     o[(long)(i * 4 + 1) * a.ntile] = a2;
   }
@@ -1403,10 +1408,9 @@ __global__ void __launch_bounds__(256) hsra_saha_kernel(double* __restrict__ sb 
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= FZ_HSRA_LEN * FZ_NELEM) return;
   const int k = t / FZ_NELEM, i = t - k * FZ_NELEM;
-  const double T = (double)fz_hsra_t[k];
-  const double lam = g_c.csaha1 * pow(T, -1.5);
+  const SahaT s((double)fz_hsra_t[k]);
   double a1, a2, da1, da2;
-  saha_element(i, T, lam, -3.0 / (2.0 * T), false, a1, a2, da1, da2);
+  saha_element<false>(i, s, a1, a2, da1, da2);
   double* o = sb + ((long)k * FZ_NELEM + i) * 4;
   o[0] = a1;
   o[1] = a2;
@@ -2491,7 +2495,10 @@ static int run_micro(fz_ctx* c, int ncol, float* d_atm, int32_t** status, bool d
     a.status = stv;
     a.pop = c->pop_on ? c->d_pop : nullptr;
     const long nkt = (long)nz * a.ntile;
-    hipLaunchKernelGGL(saha_kernel, saha_grid(nkt), dim3(256), 0, st, a);
+    if (a.der)
+      hipLaunchKernelGGL(saha_kernel<true>, saha_grid(nkt), dim3(256), 0, st, a);
+    else
+      hipLaunchKernelGGL(saha_kernel<false>, saha_grid(nkt), dim3(256), 0, st, a);
     if (hydro) {
       const long nmt = (long)(nz - 1) * a.ntile;
       hipLaunchKernelGGL(saha_mid_kernel, saha_grid(nmt), dim3(256), 0, st, a, (double*)c->d_smid);

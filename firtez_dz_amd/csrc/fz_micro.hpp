@@ -11,6 +11,43 @@
 
 #define FZ_DATA_QUAL static __constant__
 #include "fz_atomdata.h"
+
+namespace fz {
+
+__device__ __forceinline__ double rcp64(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.0), r, r);
+  return fma(fma(-x, r, 1.0), r, r);
+}
+
+// exp(x) for |x| <= 700: x = k ln 2 + r, |r| <= ln 2 / 2, ln 2 in two parts (the
+// first with 32 bits, so that k times it is exact), and the Taylor series of exp(r) to
+// r^13 (remainder below 2^-57 of it): within 0.9 ulp over 10^7 arguments.
+__device__ __forceinline__ double exp64(double x) {
+  const double k = rint(x * 1.4426950408889634);
+  const double r = fma(-k, 1.9082149292705877e-10, fma(-k, 0.6931471803691238, x));
+  double p = 1.6059043836821613e-10;                // 1 / 13!
+  p = fma(p, r, 2.0876756987868099e-9);
+  p = fma(p, r, 2.5052108385441719e-8);
+  p = fma(p, r, 2.7557319223985891e-7);
+  p = fma(p, r, 2.7557319223985893e-6);
+  p = fma(p, r, 2.4801587301587302e-5);
+  p = fma(p, r, 1.9841269841269841e-4);
+  p = fma(p, r, 1.3888888888888889e-3);
+  p = fma(p, r, 8.3333333333333333e-3);
+  p = fma(p, r, 4.1666666666666667e-2);
+  p = fma(p, r, 1.6666666666666667e-1);
+  p = fma(p, r, 0.5);
+  p = fma(p, r, 1.0);
+  p = fma(p, r, 1.0);
+  return ldexp(p, (int)k);
+}
+
+}  // namespace fz
+
+// quotients of the partition functions' derivatives: within an ulp
+#define PF_DIV(x, y) ((x) * rcp64(y))
+#define PF_EXP(x) exp(x)
 #include "fz_partition_gen.h"
 
 namespace fz {
@@ -74,21 +111,30 @@ struct SahaView {
         da2{base + 3 * stride, 4 * stride} {}
 };
 
-// Saha factors of one element at temperature T
-__device__ __forceinline__ void saha_element(int i, double T, double lam, double dlam, bool der, double& a1,
-                                             double& a2, double& da1, double& da2) {
+// What the Saha factors need of a temperature, once for all elements
+struct SahaT {
+  double T, X, Y, iT, lam, dlam, cT;
+  __device__ __forceinline__ explicit SahaT(double t)
+      : T(t), X(log(5040.0 / t)), Y(1.0e-3 * t), iT(1.0 / t), lam(0.5 * g_c.csaha1 * pow(t, -1.5)),
+        dlam(-3.0 / (2.0 * t)), cT(g_c.csaha2 / t) {}
+};
+
+// Saha factors of one element (and their T derivatives)
+template <bool DER>
+__device__ __forceinline__ void saha_element(int i, const SahaT& s, double& a1, double& a2, double& da1, double& da2) {
   double u[3], du[3];
-  partition(i, T, u, du);
-  double e1 = g_c.csaha2 * fz_xi[i] / T, e2 = g_c.csaha2 * fz_xii[i] / T;
-  e1 = fmax(fmin(e1, 650.0), -650.0);
-  e2 = fmax(fmin(e2, 650.0), -650.0);
-  a1 = (u[0] / (2.0 * u[1])) * lam * exp(e1);
-  a2 = (u[1] / (2.0 * u[2])) * lam * exp(e2);
-  da1 = da2 = 0.0;
-  if (der) {
-    const double T2 = T * T;
-    da1 = a1 * (du[0] - du[1] + dlam + (-g_c.csaha2 * fz_xi[i] / T2));
-    da2 = a2 * (du[1] - du[2] + dlam + (-g_c.csaha2 * fz_xii[i] / T2));
+  if constexpr (DER)
+    partition_at(i, s.T, s.X, s.Y, -s.iT, u, du);
+  else
+    partition_values(i, s.T, s.X, s.Y, u);
+  const double x1 = s.cT * fz_xi[i], x2 = s.cT * fz_xii[i];
+  const double e1 = fmax(fmin(x1, 650.0), -650.0);
+  const double e2 = fmax(fmin(x2, 650.0), -650.0);
+  a1 = u[0] * s.lam * rcp64(u[1]) * exp64(e1);
+  a2 = u[1] * s.lam * rcp64(u[2]) * exp64(e2);
+  if constexpr (DER) {
+    da1 = a1 * (du[0] - du[1] + s.dlam - x1 * s.iT);
+    da2 = a2 * (du[1] - du[2] + s.dlam - x2 * s.iT);
   }
 }
 

@@ -4,8 +4,11 @@ program per element) turned into straight-line device code: one out-of-line
 function per element, dispatched by a switch on the (wave-uniform) element
 index.  The operations and their order are those of the programs, FP
 contraction is off, and conditional assignments stay selects, so the results
-are those of the stack-program interpreter bit for bit; what goes away is the
-interpreter's per-opcode dispatch and its register-indexed stack.
+are those of the stack-program interpreter bit for bit where PF_DIV and PF_EXP
+are the plain division and exponential (as they are unless the includer
+defines them); what goes away is the interpreter's per-opcode dispatch and its
+register-indexed stack.  Each element has a second function without the
+derivatives.
 
   python firtez_dz_amd/csrc/gen_partition.py     (rewrites fz_partition_gen.h)
 """
@@ -57,14 +60,14 @@ def element_code(ops, args, consts):
         elif name == "NEG":
             stack.append(tmp("-%s" % stack.pop()))
         elif name == "EXP":
-            stack.append(tmp("exp(%s)" % stack.pop()))
+            stack.append(tmp("PF_EXP(%s)" % stack.pop()))
         elif name == "SEL":
             c, old, nw = stack.pop(), stack.pop(), stack.pop()
             stack.append(tmp("(%s != 0.0) ? %s : %s" % (c, nw, old)))
         else:
             y, x = stack.pop(), stack.pop()
             expr = {
-                "ADD": "%s + %s", "SUB": "%s - %s", "MUL": "%s * %s", "DIV": "%s / %s",
+                "ADD": "%s + %s", "SUB": "%s - %s", "MUL": "%s * %s", "DIV": "PF_DIV(%s, %s)",
                 "MAX": "(%s > %s) ? {x} : {y}", "AMAX1": "pf_amax1(%s, %s)",
                 "GT": "(%s > %s) ? 1.0 : 0.0", "LT": "(%s < %s) ? 1.0 : 0.0", "LE": "(%s <= %s) ? 1.0 : 0.0",
                 "GE": "(%s >= %s) ? 1.0 : 0.0", "NE": "(%s != %s) ? 1.0 : 0.0", "EQ": "(%s == %s) ? 1.0 : 0.0",
@@ -77,6 +80,17 @@ def element_code(ops, args, consts):
             stack.append(tmp(expr))
     assert not stack, stack
     return lines
+
+
+def without_derivatives(lines):
+    """The lines that the partition functions themselves need."""
+    need, out = {"vUI", "vUII", "vUIII"}, []
+    for ln in reversed(lines):
+        name, expr = re.match(r"(?:const double )?(\w+) = (.*);$", ln).groups()
+        if name in need:
+            out.append(ln)
+            need.update(re.findall(r"\b(?:v[A-Z]+|t\d+)\b", expr))
+    return out[::-1]
 
 
 def main():
@@ -95,9 +109,14 @@ def main():
            "  const float fx = (float)x, fy = (float)y;",
            "  return (double)(fx > fy ? fx : fy);",
            "}", "",
+           "#ifndef PF_DIV",
+           "#define PF_DIV(x, y) ((x) / (y))",
+           "#define PF_EXP(x) exp(x)",
+           "#endif", "",
            "// One function per element (kept out of line: inlined into one switch the",
            "// 92 bodies are scheduled together and the register demand explodes).",
-           "struct PfOut { double u[3], du[3]; };"]
+           "struct PfOut { double u[3], du[3]; };",
+           "struct PfVal { double u[3]; };"]
     for e in range(nelem):
         body = element_code(ops[start[e]:start[e + 1]], args[start[e]:start[e + 1]], consts)
         out += ["__device__ __noinline__ PfOut pf_elem_%d(double vT, double vX, double vY, double vDX) {" % e,
@@ -106,9 +125,24 @@ def main():
                 "  (void)vT; (void)vX; (void)vY; (void)vDX;"]
         out += ["  " + ln for ln in body]
         out += ["  return PfOut{{vUI, vUII, vUIII}, {vDUI, vDUII, vDUIII}};", "}", ""]
+        out += ["__device__ __noinline__ PfVal pf_value_%d(double vT, double vX, double vY) {" % e,
+                "#pragma clang fp contract(off)",
+                "  double vUI = 0.0, vUII = 0.0, vUIII = 0.0;",
+                "  (void)vT; (void)vX; (void)vY;"]
+        out += ["  " + ln for ln in without_derivatives(body)]
+        out += ["  return PfVal{{vUI, vUII, vUIII}};", "}", ""]
+    out += ["// The same without derivatives, vX = log(5040 / T) and vY = 1e-3 T given",
+            "__device__ __forceinline__ void partition_values(int elem, double vT, double vX, double vY, double u[3]) {",
+            "  PfVal r = {{0.0, 0.0, 0.0}};",
+            "  switch (elem) {"]
+    for e in range(nelem):
+        out.append("    case %d: r = pf_value_%d(vT, vX, vY); break;" % (e, e))
+    out += ["    default: break;", "  }",
+            "  u[0] = r.u[0]; u[1] = r.u[1]; u[2] = r.u[2];",
+            "}", ""]
     out += ["// U_I, U_II, U_III and their d ln U / dT at T for element elem (0-based)",
-            "__device__ __forceinline__ void partition_gen(int elem, double T, double u[3], double du[3]) {",
-            "  const double vT = T, vX = log(5040.0 / T), vY = 1.0e-3 * T, vDX = -1.0 / T;",
+            "__device__ __forceinline__ void partition_at(int elem, double vT, double vX, double vY, double vDX, double u[3],",
+            "                                             double du[3]) {",
             "  PfOut r = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};",
             "  switch (elem) {"]
     for e in range(nelem):
@@ -116,6 +150,9 @@ def main():
     out += ["    default: break;", "  }",
             "  u[0] = r.u[0]; u[1] = r.u[1]; u[2] = r.u[2];",
             "  du[0] = r.du[0]; du[1] = r.du[1]; du[2] = r.du[2];",
+            "}", "",
+            "__device__ __forceinline__ void partition_gen(int elem, double T, double u[3], double du[3]) {",
+            "  partition_at(elem, T, log(5040.0 / T), 1.0e-3 * T, -1.0 / T, u, du);",
             "}", "", "}  // namespace fz", ""]
     with open(OUT, "w") as fh:
         fh.write("\n".join(out))
