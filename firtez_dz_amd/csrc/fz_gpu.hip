@@ -928,6 +928,14 @@ constexpr size_t RT_LDS = 10 * 1024;
 // LDS.  437 columns x 81 heights in three regions of 77 wavelengths, seven
 // responses with hydrostatic equilibrium: 1.46 ms with a column per wave, 0.94 packed.
 //
+// NW (packed launches of few waves): a team of NW waves has the wave's 64
+// lanes' layers in turn, NW at a time.  Absorption, evolution operator and local responses,
+// nine tenths of the work, do not depend on the neighbouring layers; the step
+// of the Stokes vector (pass 1) and of the running product (pass 2) go from wave to
+// wave through LDS.  The same operations on the same values: the same bits.
+// One column of 64 heights and 112 wavelengths: synthesis 0.32 -> 0.22 ms with its
+// microphysics, with five responses 0.61 -> 0.34 ms (where the line lies: launch_rt).
+//
 // NODES (RF_CART_TBV): the responses are contracted with the node basis as
 // they are formed instead of going to memory per height.  Going down, a slot
 // feeds the FP64 sums of two nodes; where the lower one's support ends the
@@ -935,8 +943,9 @@ constexpr size_t RT_LDS = 10 * 1024;
 // waves per SIMD instead of three, which the issue-bound transfer bears:
 // forward and contraction of 128x128x64 columns 10.2 -> 7.9 ms against
 // responses stored per height (9.4 GB) and read again by eqv_kernel.
-template <int RF, bool HE, bool PACK, bool NODES = false>
-__global__ void __launch_bounds__(RT_WAVE) rt_kernel(RtArgs a, NodeArgs nd, const NodeTab* __restrict__ ntab) {
+template <int RF, bool HE, bool PACK, bool NODES = false, int NW = 1>
+__global__ void __launch_bounds__(RT_WAVE * NW) rt_kernel(RtArgs a, NodeArgs nd, const NodeTab* __restrict__ ntab) {
+#pragma clang fp contract(off)
   // parameters: 5 spherical, 7 Cartesian, 8 with P0 (the top pressure)
   constexpr int NP = (RF == FZ_RF_SPHERICAL || RF == RF_CART_TBV)
                          ? 5
@@ -945,7 +954,11 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(RtArgs a, NodeArgs nd, cons
   constexpr bool PR = RF == FZ_RF_CARTESIAN || RF == FZ_RF_CARTESIAN_P0;
   constexpr bool HEX = HE && RF != 0;
   extern __shared__ float4 lds[];
-  const int numw = c_cfg.numw, nz = c_cfg.nz, lane = (int)threadIdx.x;
+  // a team's running Stokes vector (and Ahe) and its running product
+  __shared__ float xi[NW > 1 ? 8 : 1][RT_WAVE], xa[NW > 1 && RF != 0 ? 16 : 1][RT_WAVE];
+  __shared__ float xo[NW > 1 && NODES ? NW : 1][20][RT_WAVE];   // responses of a team's layers
+  const int numw = c_cfg.numw, nz = c_cfg.nz, lane = (int)threadIdx.x & (RT_WAVE - 1);
+  const int wv = NW > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : 0;
   // workgroup -> (column, region, first wavelength); lane -> wavelength.  A
   // lane past the work repeats the last one without storing, so that the
   // whole wave takes part in the copies to LDS.
@@ -1017,7 +1030,7 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(RtArgs a, NodeArgs nd, cons
   if constexpr (NODES)
     eqv = nd.eqv + (a.items ? (long)nd.np * nd.nstk * (sbase / 4) : (long)col * nd.np * nd.nstk * snumw) + lo;
   if (a.status && a.status[col] != 0) {
-    if (live) {
+    if (live && wv == 0) {
       for (int s = 0; s < 4; ++s) a.stokes[sbase + (long)s * snumw + lo] = __builtin_nanf("");
       if constexpr (NODES)
         for (int i = 0; i < nd.np * nd.nstk; ++i) eqv[(long)i * snumw] = 0.f;
@@ -1037,14 +1050,14 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(RtArgs a, NodeArgs nd, cons
     const int f = lane & 31;
     const int src = f + (f >= REC_HEAD / 4 ? roff4 : 0);
     const int np = n * nc;
-    int h = 0, c = lane >> 5;
-    if (c >= nc) {
+    int h = 0, c = 2 * wv + (lane >> 5);
+    while (c >= nc) {
       c -= nc;
       ++h;
     }
-    for (int p = lane >> 5; p < np; p += 2) {
+    for (int p = 2 * wv + (lane >> 5); p < np; p += 2 * NW) {
       if (f < rs4) lds[p * rs4 + f] = grec[((long)(k0 + h) * a.ncol + a.col0 + ct0 + c) * rec4 + src];
-      c += 2;
+      c += 2 * NW;
       while (c >= nc) {
         c -= nc;
         ++h;
@@ -1105,79 +1118,131 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(RtArgs a, NodeArgs nd, cons
     v[1] = q;
     v[2] = u;
   };
+  // Pass 1, bottom to top.  What of a layer does not depend on the light
+  // (form) and the step through it (pass).
+  struct Layer {
+    Evol E;
+    Five fp;
+    float S;
+  };
+  auto form = [&](int k, const float4* R, Layer& Y) {
+    const float4 h1 = R[1], h2 = R[2], rg = R[REC_HEAD / 4];
+    const float dz = c_cfg.dz_cm[k];
+    const Mix mx = {h1.z, h1.w, h2.x, h2.y, h2.z};
+    Five f;
+    if constexpr (HEX) {
+      Sums X, XT, XV, XB, XP, XR;
+      absorb_der<true>(R + REC_HEAD / 4 + 1, r, wave, h1.y, dz, X, XT, XV, XB, XP, XR);
+      f = mix(mx, X);
+      Y.fp = mix(mx, XP);
+      Y.fp.I = fmaf(rg.z, dz, Y.fp.I);
+    } else {
+      f = mix(mx, absorb(R + REC_HEAD / 4 + 1, r, wave, h1.y, dz));
+    }
+    f.I = fmaf(rg.x, dz, f.I);
+    evol_build<HEX>(f, Y.E);
+  };
+  auto pass = [&](int k, const float4& h3, const Layer& Y) {
+    const Evol& E = Y.E;
+    const float v[4] = {I[0] - Y.S, I[1], I[2], I[3]};
+    float vf[4], dv[4];
+    turn(h3.x, h3.y, v, vf);
+    const Pieces w = evol_pieces(E, vf);
+    evol_apply(E, w, dv);
+    if constexpr (HEX) {
+      Grad G;
+      evol_grad(E, vf, w, G);
+      float d2[4], Af[4], W[4];
+      grad_dot(G, Y.fp, d2);
+      turn_back(h3.x, h3.y, d2);
+      turn(h3.x, h3.y, Ahe, Af);
+      evol_apply(E, evol_pieces(E, Af), W);
+      turn_back(h3.x, h3.y, W);
+      const bool thin = fmaf(E.D4, E.s0, E.A) > 1.0e-5f;    // O_11
+      const float pg = a.atm[A_PG * ps + k * cs + col];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        W[i] = thin ? fmaf(E.A, Ahe[i], W[i]) : Ahe[i];
+        if (live) scr_store((nz + k) * 4 + i, W[i]);
+        if (thin) Ahe[i] = fmaf(d2[i], pg, W[i]);
+      }
+    }
+    turn_back(h3.x, h3.y, dv);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) I[i] = fmaf(E.A, v[i], dv[i]) + (i == 0 ? Y.S : 0.f);
+  };
+  auto keep = [&](int k) {
+    if (RF && live) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) scr_store(k * 4 + s, I[s]);
+    }
+  };
+  if constexpr (NW > 1) {
+    if (wv == 0)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) xi[i][lane] = 0.f;
+  }
   for (int k0 = 0; k0 < nz; k0 += a.chunk) {
     const int n = min(a.chunk, nz - k0);
     stage(k0, n);
-    for (int kk = 0; kk < n; ++kk) {
-      const int k = k0 + kk;
-      const float4* R = mine + kk * nc * rs4;
-      const float4 h0 = R[0];
-      const float S = c1 * (1.0f / (depart(k) * expf(c2 * h0.z) - 1.0f));
-      if (RF) {
-        if (live) {
-#pragma unroll
-          for (int s = 0; s < 4; ++s) scr_store(k * 4 + s, I[s]);
+    for (int kb = 0; kb < n; kb += NW) {
+      const int kk = kb + wv, k = k0 + kk;
+      const bool has = NW == 1 || kk < n;
+      const float4* R = mine + (has ? kk : 0) * nc * rs4;
+      const float4 h0 = R[0], h3 = R[3];
+      Layer Y;
+      Y.S = c1 * (1.0f / (depart(has ? k : 0) * expf(c2 * h0.z) - 1.0f));
+      if constexpr (NW == 1) {
+        keep(k);
+        if (h0.x != 0.f) {
+          I[0] = Y.S; I[1] = 0.f; I[2] = 0.f; I[3] = 0.f;
+        } else {
+          form(k, R, Y);
+          pass(k, h3, Y);
         }
-      }
-      if (h0.x != 0.f) {
-        I[0] = S; I[1] = 0.f; I[2] = 0.f; I[3] = 0.f;
         store_fs(k);
-        continue;
-      }
-      const float4 h1 = R[1], h2 = R[2], h3 = R[3], rg = R[REC_HEAD / 4];
-      const float dz = c_cfg.dz_cm[k];
-      const Mix mx = {h1.z, h1.w, h2.x, h2.y, h2.z};
-      const float v[4] = {I[0] - S, I[1], I[2], I[3]};
-      float vf[4], dv[4];
-      turn(h3.x, h3.y, v, vf);
-      Evol E;
-      if constexpr (HEX) {
-        Sums X, XT, XV, XB, XP, XR;
-        absorb_der<true>(R + REC_HEAD / 4 + 1, r, wave, h1.y, dz, X, XT, XV, XB, XP, XR);
-        Five f = mix(mx, X), fp = mix(mx, XP);
-        f.I = fmaf(rg.x, dz, f.I);
-        fp.I = fmaf(rg.z, dz, fp.I);
-        evol_build<true>(f, E);
-        const Pieces w = evol_pieces(E, vf);
-        evol_apply(E, w, dv);
-        Grad G;
-        evol_grad(E, vf, w, G);
-        float d2[4], Af[4], W[4];
-        grad_dot(G, fp, d2);
-        turn_back(h3.x, h3.y, d2);
-        turn(h3.x, h3.y, Ahe, Af);
-        evol_apply(E, evol_pieces(E, Af), W);
-        turn_back(h3.x, h3.y, W);
-        const bool thin = fmaf(E.D4, E.s0, E.A) > 1.0e-5f;    // O_11
-        const float pg = a.atm[A_PG * ps + k * cs + col];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          W[i] = thin ? fmaf(E.A, Ahe[i], W[i]) : Ahe[i];
-          if (live) scr_store((nz + k) * 4 + i, W[i]);
-          if (thin) Ahe[i] = W[i] + d2[i] * pg;
-        }
       } else {
-        Five f = mix(mx, absorb(R + REC_HEAD / 4 + 1, r, wave, h1.y, dz));
-        f.I = fmaf(rg.x, dz, f.I);
-        evol_build<false>(f, E);
-        evol_apply(E, evol_pieces(E, vf), dv);
-      }
-      turn_back(h3.x, h3.y, dv);
+        if (has && h0.x == 0.f) form(k, R, Y);
+#pragma unroll 1
+        for (int i = 0; i < NW; ++i) {
+          if (i == wv && has) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) I[i] = fmaf(E.A, v[i], dv[i]) + (i == 0 ? S : 0.f);
-      store_fs(k);
+            for (int s = 0; s < 4; ++s) {
+              I[s] = xi[s][lane];
+              if (HEX) Ahe[s] = xi[4 + s][lane];
+            }
+            keep(k);
+            if (h0.x != 0.f) {
+              I[0] = Y.S; I[1] = 0.f; I[2] = 0.f; I[3] = 0.f;
+            } else {
+              pass(k, h3, Y);
+            }
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+              xi[s][lane] = I[s];
+              if (HEX) xi[4 + s][lane] = Ahe[s];
+            }
+            store_fs(k);
+          }
+          __syncthreads();
+        }
+      }
     }
+  }
+  if constexpr (NW > 1) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) I[s] = xi[s][lane];
   }
   float gn[4];
 #pragma unroll
   for (int s = 0; s < 4; ++s) {
     gn[s] = a.gain[l * 4 + s];
-    if (live) a.stokes[sbase + (long)s * snumw + lo] = I[s] * gn[s];
+    if (live && wv == 0) a.stokes[sbase + (long)s * snumw + lo] = I[s] * gn[s];
   }
   // a non-finite Stokes vector comes from a non-finite profile, propagation
   // matrix or evolution operator, where the reference stops
   // (voigt.f:91-95, absorption_matrix.f90:1882-1889, rtesolver.f90:346-352)
-  if (live && a.status && !(__builtin_isfinite(I[0]) && __builtin_isfinite(I[1]) && __builtin_isfinite(I[2]) &&
+  if (live && wv == 0 && a.status && !(__builtin_isfinite(I[0]) && __builtin_isfinite(I[1]) && __builtin_isfinite(I[2]) &&
                             __builtin_isfinite(I[3])))
     atomicMax(&a.status[col], (int32_t)ERR_NAN);
   if constexpr (RF != 0) {
@@ -1189,205 +1254,285 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(RtArgs a, NodeArgs nd, cons
     for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc[i][j] = (i == j) ? (GACC ? gn[i] : 1.f) : 0.f;
-    double nlo[NODES ? 5 : 1][4], nhi[NODES ? 5 : 1][4];   // sums of nodes jl, jl + 1
+    // sums of nodes jl, jl + 1 of a slot (a team's wave keeps those of one Stokes
+    // parameter, with eight waves of some slots)
+    constexpr int NST = NW > 1 ? 1 : 4;
+    double nlo[NODES ? 5 : 1][NST], nhi[NODES ? 5 : 1][NST];
     int jl[5];
-    auto store_node = [&](int p, int j, const double (&x)[4]) {
+    const int st0 = NW > 1 ? wv & 3 : 0;
+    auto owned = [&](int p) { return NW <= 4 || (p < 3) == (wv < 4); };
+    auto store_node = [&](int p, int j, const double (&x)[NST]) {
       if (!live || j > nd.last[p]) return;
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (nd.blk[i] >= 0) eqv[((long)j * nd.nstk + nd.blk[i]) * snumw] = (float)x[i];
+      for (int i = 0; i < NST; ++i)
+        if (nd.blk[st0 + i] >= 0) eqv[((long)j * nd.nstk + nd.blk[st0 + i]) * snumw] = (float)x[i];
+    };
+    // a slot's nodes whose support ends above height k are complete
+    auto next_node = [&](int p, int k) {
+      const int w = ntab[k * 5 + p].node;
+      while (w >= 0 && jl[p] > w) {
+        store_node(p, jl[p] + 1, nhi[p]);
+#pragma unroll
+        for (int i = 0; i < NST; ++i) {
+          nhi[p][i] = nlo[p][i];
+          nlo[p][i] = 0.0;
+        }
+        --jl[p];
+      }
     };
     if constexpr (NODES) {
 #pragma unroll
       for (int p = 0; p < 5; ++p) {
         jl[p] = nd.last[p];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) nlo[p][i] = nhi[p][i] = 0.0;
+        for (int i = 0; i < NST; ++i) nlo[p][i] = nhi[p][i] = 0.0;
       }
     }
-    for (int k1 = nz; k1 > 0; k1 -= a.chunk) {
-      const int n = min(a.chunk, k1);
-      stage(k1 - n, n);
-      for (int kk = n - 1; kk >= 0; --kk) {
-        const int k = k1 - n + kk;
-        const float4* R = mine + kk * nc * rs4;
-        const float4 h0 = R[0];
-        if constexpr (NODES) {
+    // Pass 2, top to bottom.  A layer's local responses in the frame (local: lp[0] =
+    // T, then (Pg, rho,) and the field's), the running product (extend) with the row
+    // vectors b of acc in the frame, and the propagated responses (emit).
+    auto local = [&](int k, const float4* R, const float4& h0, Evol& E, float (&lp)[NPL][4]) {
+                const float4 h1 = R[1], h2 = R[2], h3 = R[3], rg = R[REC_HEAD / 4];
+                const float dz = c_cfg.dz_cm[k];
+                // S = c1 / (ex - 1), dS/dT = S (ex / (ex - 1)) (c2 / T) / T
+                const float x = c2 * h0.z;
+                const float ex = depart(k) * expf(x);
+                const float iem1 = 1.0f / (ex - 1.0f);
+                const float S = c1 * iem1;
+                const float dS = S * (ex * iem1) * x * h0.z;
+                const Mix mx = {h1.z, h1.w, h2.x, h2.y, h2.z};
+                Sums X, XT, XV, XB, XP, XR;
+                absorb_der<PR>(R + REC_HEAD / 4 + 1, r, wave, h1.y, dz, X, XT, XV, XB, XP, XR);
+                Five f = mix(mx, X);
+                f.I = fmaf(rg.x, dz, f.I);
+                evol_build<true>(f, E);
+                float v[4], vf[4];
 #pragma unroll
-          for (int p = 0; p < 5; ++p) {
-            const int w = ntab[k * 5 + p].node;
-            while (w >= 0 && jl[p] > w) {
-              store_node(p, jl[p] + 1, nhi[p]);
+                for (int s = 0; s < 4; ++s) v[s] = scr_load(k * 4 + s) - (s == 0 ? S : 0.f);
+                turn(h3.x, h3.y, v, vf);
+                // local responses in the frame: lp[0] = T, then (Pg, rho,) and the field's
+                float lB[4], lG[4], lF[4];
+                constexpr int o = PR ? 2 : 0;
+                {
+                  const Pieces w = evol_pieces(E, vf);
+                  Grad G;
+                  evol_grad(E, vf, w, G);
+                  Five fd = mix(mx, XT);
+                  fd.I = fmaf(rg.y, dz, fd.I);
+                  grad_dot(G, fd, lp[0]);
+                  if constexpr (PR) {
+                    fd = mix(mx, XP);
+                    fd.I = fmaf(rg.z, dz, fd.I);
+                    grad_dot(G, fd, lp[1]);
+                  }
+                  if constexpr (HEX) {
+                    float vo[4], vof[4];
 #pragma unroll
-              for (int i = 0; i < 4; ++i) {
-                nhi[p][i] = nlo[p][i];
-                nlo[p][i] = 0.0;
-              }
-              --jl[p];
-            }
+                    for (int s = 0; s < 4; ++s)
+                      vo[s] = (k == nz - 1 ? I[s] : scr_load((k + 1) * 4 + s)) - (s == 0 ? S : 0.f);
+                    turn(h3.x, h3.y, vo, vof);
+                    const Pieces wo = evol_pieces(E, vof);
+                    evol_grad(E, vof, wo, G);
+                    evol_azimuth(E, vof, wo, lF);
+                  } else {
+                    evol_azimuth(E, vf, w, lF);
+                  }
+                  if constexpr (PR) {
+                    fd = mix(mx, XR);
+                    fd.I = fmaf(rg.w, dz, fd.I);
+                    grad_dot(G, fd, lp[2]);
+                  }
+                  grad_dot(G, mix(mx, XB), lB);
+                  grad_dot(G, mix(mx, XV), lp[4 + o]);
+                  // the inclination: I and q share their factor, d sin^2 = 2 sg cg
+                  const Mix mg = {h3.z, -0.5f * h3.z, h3.z, 0.5f * h3.z, -0.5f * h2.w};
+                  grad_dot(G, mix(mg, X), lG);
+                }
+                // source-function term (1 - O) e0 dS/dT for T; O e0 in the frame
+                {
+                  const float alx = -fmaf(E.ga, E.ex, E.gb * E.rx), alz = -fmaf(E.ga, E.ez, E.gb * E.rz);
+                  lp[0][0] = fmaf(1.f - fmaf(E.D4, E.s0, E.A), dS, lp[0][0]);
+                  lp[0][1] = fmaf(-alx, dS, lp[0][1]);
+                  lp[0][2] = fmaf(E.D4 * E.cy, dS, lp[0][2]);
+                  lp[0][3] = fmaf(-alz, dS, lp[0][3]);
+                }
+                if constexpr (HEX) {
+                  const float mu = a.atm[A_MU * ps + k * cs + col];
+                  const float gk = -mu * c_cfg.he_cte[k] * h0.z * h0.z;
+                  float W[4], Wf[4];
+#pragma unroll
+                  for (int i = 0; i < 4; ++i) W[i] = scr_load((nz + k) * 4 + i);
+                  turn(h3.x, h3.y, W, Wf);
+#pragma unroll
+                  for (int i = 0; i < 4; ++i) lp[0][i] = fmaf(gk, Wf[i], lp[0][i]);
+                }
+                if constexpr (RF == FZ_RF_SPHERICAL) {
+#pragma unroll
+                  for (int i = 0; i < 4; ++i) {
+                    lp[1][i] = lB[i];
+                    lp[2][i] = lG[i];
+                    lp[3][i] = lF[i];
+                  }
+                } else {
+                  // chain rule (|B|, gamma, phi) -> (Bx, By, Bz)
+                  const float4 h4 = R[4], h5 = R[5];
+#pragma unroll
+                  for (int i = 0; i < 4; ++i) {
+                    lp[1 + o][i] = fmaf(h4.x, lB[i], fmaf(h4.w, lG[i], h5.z * lF[i]));
+                    lp[2 + o][i] = fmaf(h4.y, lB[i], fmaf(h5.x, lG[i], h5.w * lF[i]));
+                    lp[3 + o][i] = fmaf(h4.z, lB[i], h5.y * lG[i]);
+                  }
+                }
+    };
+    // the running product O_nz ... O_k = acc (A 1 + turned-back (O - A 1))
+    auto extend = [&](const float4& h3, const Evol& E, float (&b)[4][4]) {
+      const float M11 = E.D4 * (fmaf(E.ex, E.ex, E.rx * E.rx) - E.s0), M33 = E.D4 * (fmaf(E.ez, E.ez, E.rz * E.rz) - E.s0);
+      const float M00 = E.D4 * E.s0, M02 = E.D4 * E.cy, M13 = E.D4 * fmaf(E.ex, E.ez, E.rx * E.rz);
+      const float M01 = -fmaf(E.ga, E.ex, E.gb * E.rx), M03 = -fmaf(E.ga, E.ez, E.gb * E.rz);
+      const float M12 = fmaf(E.ga, E.rz, -(E.gb * E.ez)), M23 = fmaf(E.ga, E.rx, -(E.gb * E.ex));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        turn(h3.x, h3.y, acc[i], b[i]);
+        float m[4];
+        m[0] = fmaf(b[i][0], M00, fmaf(b[i][1], M01, fmaf(-b[i][2], M02, b[i][3] * M03)));
+        m[1] = fmaf(b[i][0], M01, fmaf(b[i][1], M11, fmaf(-b[i][2], M12, b[i][3] * M13)));
+        m[2] = fmaf(b[i][0], M02, fmaf(b[i][1], M12, fmaf(-b[i][2], M00, -(b[i][3] * M23))));
+        m[3] = fmaf(b[i][0], M03, fmaf(b[i][1], M13, fmaf(b[i][2], M23, b[i][3] * M33)));
+        turn_back(h3.x, h3.y, m);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(E.A, acc[i][j], m[j]);
+      }
+    };
+    // above[i]: sum of row i of acc above the layer (for P0)
+    auto emit = [&](int k, const float (&lp)[NPL][4], const float (&b)[4][4], const float (&above)[4]) {
+      float outv[NP][4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int p = 0; p < NPL; ++p)
+          outv[p][i] = fmaf(b[i][0], lp[p][0], fmaf(b[i][1], lp[p][1], fmaf(b[i][2], lp[p][2], b[i][3] * lp[p][3])));
+      if constexpr (RF == FZ_RF_CARTESIAN_P0) {
+        // P0 (forward.f90:543-545): the local response is 1 in every Stokes
+        // parameter; below the top it is propagated and then multiplied,
+        // component by component, by PG(K)/PG(NZ) and the propagated Pg|T
+        // response of the same height; the top layer keeps 1
+        if (k == nz - 1) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) outv[7][i] = 1.f;
+        } else {
+          const float ratio = a.atm[A_PG * ps + k * cs + col] / a.atm[A_PG * ps + (nz - 1) * cs + col];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) outv[7][i] = above[i] * ratio * outv[1][i];
+        }
+      }
+      if constexpr (NODES && NW > 1) {
+#pragma unroll
+        for (int p = 0; p < 5; ++p)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) xo[wv][p * 4 + i][lane] = outv[p][i];
+      } else if constexpr (NODES) {
+#pragma unroll
+        for (int p = 0; p < 5; ++p) {
+          const double c0 = ntab[k * 5 + p].c0, c1 = ntab[k * 5 + p].c1;
+#pragma unroll
+          for (int i = 0; i < NST; ++i) {
+            const double x = (double)outv[p][i];
+            nlo[p][i] = fma(x, c0, nlo[p][i]);
+            nhi[p][i] = fma(x, c1, nhi[p][i]);
           }
         }
-        if (h0.x != 0.f) {
-          // boundary layer: no local response; layers below cannot reach the top
-          if (!NODES && live)
+      } else if (live) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+#pragma unroll
+          for (int s = 0; s < 4; ++s) jac_store((p * nz + k) * 4 + s, GACC ? outv[p][s] : outv[p][s] * gn[s]);
+      }
+    };
+    auto row_sums = [&](float (&above)[4]) {
+      if constexpr (RF == FZ_RF_CARTESIAN_P0)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) above[i] = acc[i][0] + acc[i][1] + acc[i][2] + acc[i][3];
+    };
+    // boundary layer: no local response; layers below cannot reach the top
+    auto blank = [&](int k) {
+      if constexpr (NODES && NW > 1) {
+#pragma unroll
+        for (int i = 0; i < 20; ++i) xo[wv][i][lane] = 0.f;
+      }
+      if (!NODES && live)
 #pragma unroll 1
-            for (int i = 0; i < 4 * NP; ++i) jac_store(((i >> 2) * nz + k) * 4 + (i & 3), 0.f);
+        for (int i = 0; i < 4 * NP; ++i) jac_store(((i >> 2) * nz + k) * 4 + (i & 3), 0.f);
+    };
+    if constexpr (NW > 1) {
+      if (wv == 0)
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 16; ++i) xa[i][lane] = acc[i >> 2][i & 3];
+    }
+    for (int k0 = (nz - 1) / a.chunk * a.chunk; k0 >= 0; k0 -= a.chunk) {
+      const int n = min(a.chunk, nz - k0);
+      stage(k0, n);
+      for (int kb = (n - 1) / NW * NW; kb >= 0; kb -= NW) {
+        const int kk = kb + wv, k = k0 + kk;
+        const bool has = NW == 1 || kk < n;
+        const float4* R = mine + (has ? kk : 0) * nc * rs4;
+        const float4 h0 = R[0];
+        if constexpr (NODES && NW == 1) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-        } else {
-          float outv[NP][4];
-          const float4 h1 = R[1], h2 = R[2], h3 = R[3], rg = R[REC_HEAD / 4];
-          const float dz = c_cfg.dz_cm[k];
-          // S = c1 / (ex - 1), dS/dT = S (ex / (ex - 1)) (c2 / T) / T
-          const float x = c2 * h0.z;
-          const float ex = depart(k) * expf(x);
-          const float iem1 = 1.0f / (ex - 1.0f);
-          const float S = c1 * iem1;
-          const float dS = S * (ex * iem1) * x * h0.z;
-          const Mix mx = {h1.z, h1.w, h2.x, h2.y, h2.z};
-          Sums X, XT, XV, XB, XP, XR;
-          absorb_der<PR>(R + REC_HEAD / 4 + 1, r, wave, h1.y, dz, X, XT, XV, XB, XP, XR);
-          Five f = mix(mx, X);
-          f.I = fmaf(rg.x, dz, f.I);
-          Evol E;
-          evol_build<true>(f, E);
-          float v[4], vf[4];
+          for (int p = 0; p < 5; ++p) next_node(p, k);
+        }
+        Evol E;
+        float lp[NPL][4], b[4][4], above[4] = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (NW == 1) {
+          if (h0.x != 0.f) {
+            blank(k);
 #pragma unroll
-          for (int s = 0; s < 4; ++s) v[s] = scr_load(k * 4 + s) - (s == 0 ? S : 0.f);
-          turn(h3.x, h3.y, v, vf);
-          // local responses in the frame: lp[0] = T, then (Pg, rho,) and the field's
-          float lp[NPL][4], lB[4], lG[4], lF[4];
-          constexpr int o = PR ? 2 : 0;
-          {
-            const Pieces w = evol_pieces(E, vf);
-            Grad G;
-            evol_grad(E, vf, w, G);
-            Five fd = mix(mx, XT);
-            fd.I = fmaf(rg.y, dz, fd.I);
-            grad_dot(G, fd, lp[0]);
-            if constexpr (PR) {
-              fd = mix(mx, XP);
-              fd.I = fmaf(rg.z, dz, fd.I);
-              grad_dot(G, fd, lp[1]);
-            }
-            if constexpr (HEX) {
-              float vo[4], vof[4];
-#pragma unroll
-              for (int s = 0; s < 4; ++s)
-                vo[s] = (k == nz - 1 ? I[s] : scr_load((k + 1) * 4 + s)) - (s == 0 ? S : 0.f);
-              turn(h3.x, h3.y, vo, vof);
-              const Pieces wo = evol_pieces(E, vof);
-              evol_grad(E, vof, wo, G);
-              evol_azimuth(E, vof, wo, lF);
-            } else {
-              evol_azimuth(E, vf, w, lF);
-            }
-            if constexpr (PR) {
-              fd = mix(mx, XR);
-              fd.I = fmaf(rg.w, dz, fd.I);
-              grad_dot(G, fd, lp[2]);
-            }
-            grad_dot(G, mix(mx, XB), lB);
-            grad_dot(G, mix(mx, XV), lp[4 + o]);
-            // the inclination: I and q share their factor, d sin^2 = 2 sg cg
-            const Mix mg = {h3.z, -0.5f * h3.z, h3.z, 0.5f * h3.z, -0.5f * h2.w};
-            grad_dot(G, mix(mg, X), lG);
-          }
-          // source-function term (1 - O) e0 dS/dT for T; O e0 in the frame
-          {
-            const float alx = -fmaf(E.ga, E.ex, E.gb * E.rx), alz = -fmaf(E.ga, E.ez, E.gb * E.rz);
-            lp[0][0] = fmaf(1.f - fmaf(E.D4, E.s0, E.A), dS, lp[0][0]);
-            lp[0][1] = fmaf(-alx, dS, lp[0][1]);
-            lp[0][2] = fmaf(E.D4 * E.cy, dS, lp[0][2]);
-            lp[0][3] = fmaf(-alz, dS, lp[0][3]);
-          }
-          if constexpr (HEX) {
-            const float mu = a.atm[A_MU * ps + k * cs + col];
-            const float gk = -mu * c_cfg.he_cte[k] * h0.z * h0.z;
-            float W[4], Wf[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) W[i] = scr_load((nz + k) * 4 + i);
-            turn(h3.x, h3.y, W, Wf);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) lp[0][i] = fmaf(gk, Wf[i], lp[0][i]);
-          }
-          if constexpr (RF == FZ_RF_SPHERICAL) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              lp[1][i] = lB[i];
-              lp[2][i] = lG[i];
-              lp[3][i] = lF[i];
-            }
+            for (int i = 0; i < 16; ++i) acc[i >> 2][i & 3] = 0.f;
           } else {
-            // chain rule (|B|, gamma, phi) -> (Bx, By, Bz)
-            const float4 h4 = R[4], h5 = R[5];
+            local(k, R, h0, E, lp);
+            row_sums(above);
+            extend(R[3], E, b);
+            emit(k, lp, b, above);
+          }
+        } else {
+          const float4 h3 = R[3];
+          if (has && h0.x == 0.f) local(k, R, h0, E, lp);
+#pragma unroll 1
+          for (int i = NW - 1; i >= 0; --i) {
+            if (i == wv && has) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              lp[1 + o][i] = fmaf(h4.x, lB[i], fmaf(h4.w, lG[i], h5.z * lF[i]));
-              lp[2 + o][i] = fmaf(h4.y, lB[i], fmaf(h5.x, lG[i], h5.w * lF[i]));
-              lp[3 + o][i] = fmaf(h4.z, lB[i], h5.y * lG[i]);
+              for (int j = 0; j < 16; ++j) acc[j >> 2][j & 3] = xa[j][lane];
+              row_sums(above);
+              if (h0.x != 0.f) {
+#pragma unroll
+                for (int j = 0; j < 16; ++j) acc[j >> 2][j & 3] = 0.f;
+              } else {
+                extend(h3, E, b);
+              }
+#pragma unroll
+              for (int j = 0; j < 16; ++j) xa[j][lane] = acc[j >> 2][j & 3];
             }
+            __syncthreads();
           }
-          // acc in the frame, the propagated responses, and the running
-          // product O_nz ... O_k = acc (A 1 + turned-back (O - A 1))
-          float na[4][4];
-          const float M11 = E.D4 * (fmaf(E.ex, E.ex, E.rx * E.rx) - E.s0), M33 = E.D4 * (fmaf(E.ez, E.ez, E.rz * E.rz) - E.s0);
-          const float M00 = E.D4 * E.s0, M02 = E.D4 * E.cy, M13 = E.D4 * fmaf(E.ex, E.ez, E.rx * E.rz);
-          const float M01 = -fmaf(E.ga, E.ex, E.gb * E.rx), M03 = -fmaf(E.ga, E.ez, E.gb * E.rz);
-          const float M12 = fmaf(E.ga, E.rz, -(E.gb * E.ez)), M23 = fmaf(E.ga, E.rx, -(E.gb * E.ex));
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            float b[4];
-            turn(h3.x, h3.y, acc[i], b);
-#pragma unroll
-            for (int p = 0; p < NPL; ++p)
-              outv[p][i] = fmaf(b[0], lp[p][0], fmaf(b[1], lp[p][1], fmaf(b[2], lp[p][2], b[3] * lp[p][3])));
-            float m[4];
-            m[0] = fmaf(b[0], M00, fmaf(b[1], M01, fmaf(-b[2], M02, b[3] * M03)));
-            m[1] = fmaf(b[0], M01, fmaf(b[1], M11, fmaf(-b[2], M12, b[3] * M13)));
-            m[2] = fmaf(b[0], M02, fmaf(b[1], M12, fmaf(-b[2], M00, -(b[3] * M23))));
-            m[3] = fmaf(b[0], M03, fmaf(b[1], M13, fmaf(b[2], M23, b[3] * M33)));
-            turn_back(h3.x, h3.y, m);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) na[i][j] = fmaf(E.A, acc[i][j], m[j]);
+          if (has) {
+            if (h0.x != 0.f)
+              blank(k);
+            else
+              emit(k, lp, b, above);
           }
-          if constexpr (RF == FZ_RF_CARTESIAN_P0) {
-            // P0 (forward.f90:543-545): the local response is 1 in every Stokes
-            // parameter; below the top it is propagated and then multiplied,
-            // component by component, by PG(K)/PG(NZ) and the propagated Pg|T
-            // response of the same height; the top layer keeps 1
-            if (k == nz - 1) {
-#pragma unroll
-              for (int i = 0; i < 4; ++i) outv[7][i] = 1.f;
-            } else {
-              const float ratio = a.atm[A_PG * ps + k * cs + col] / a.atm[A_PG * ps + (nz - 1) * cs + col];
-#pragma unroll
-              for (int i = 0; i < 4; ++i)
-                outv[7][i] = (acc[i][0] + acc[i][1] + acc[i][2] + acc[i][3]) * ratio * outv[1][i];
-            }
-          }
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = na[i][j];
           if constexpr (NODES) {
+            __syncthreads();
+#pragma unroll 1
+            for (int q = min(NW, n - kb) - 1; q >= 0; --q) {
+              const int kq = k0 + kb + q;
 #pragma unroll
-            for (int p = 0; p < 5; ++p) {
-              const double c0 = ntab[k * 5 + p].c0, c1 = ntab[k * 5 + p].c1;
-#pragma unroll
-              for (int i = 0; i < 4; ++i) {
-                const double x = (double)outv[p][i];
-                nlo[p][i] = fma(x, c0, nlo[p][i]);
-                nhi[p][i] = fma(x, c1, nhi[p][i]);
+              for (int p = 0; p < 5; ++p) {
+                if (!owned(p)) continue;
+                next_node(p, kq);
+                const double x = (double)xo[q][p * 4 + st0][lane];
+                nlo[p][0] = fma(x, ntab[kq * 5 + p].c0, nlo[p][0]);
+                nhi[p][0] = fma(x, ntab[kq * 5 + p].c1, nhi[p][0]);
               }
             }
-          } else if (live) {
-#pragma unroll
-            for (int p = 0; p < NP; ++p)
-#pragma unroll
-              for (int s = 0; s < 4; ++s) jac_store((p * nz + k) * 4 + s, GACC ? outv[p][s] : outv[p][s] * gn[s]);
           }
         }
       }
@@ -1395,7 +1540,7 @@ __global__ void __launch_bounds__(RT_WAVE) rt_kernel(RtArgs a, NodeArgs nd, cons
     if constexpr (NODES) {
 #pragma unroll
       for (int p = 0; p < 5; ++p) {
-        if (nd.last[p] < 0) continue;
+        if (nd.last[p] < 0 || !owned(p)) continue;
         store_node(p, jl[p] + 1, nhi[p]);
         store_node(p, jl[p], nlo[p]);
       }
@@ -1555,7 +1700,6 @@ __device__ __forceinline__ void lsf_tiles(const float* __restrict__ x, const flo
                                           f32x4* acc) {
 #pragma unroll
   for (int g = 0; g < NT; ++g) acc[g] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
   for (int k = 0; k < n4; k += 4) {
     const float a = x[k];
 #pragma unroll
@@ -2383,38 +2527,50 @@ static int launch_rt(fz_ctx* c, int rf_mode, RtArgs a, hipStream_t st, int nitem
   a.wcols = std::min(a.ntile, 1 + (RT_WAVE - 1 + nmin - 1) / nmin);
   const bool pack = !a.items && 16L * a.wcols * npar * g.nz * g.numw < (1L << 31);
   if (!pack) a.wcols = 1;
-  const dim3 grid(a.items ? (unsigned)nitems : pack ? (unsigned)npack : (unsigned)a.ntile * (unsigned)g.nbpc),
-      blk(RT_WAVE);
+  const dim3 grid(a.items ? (unsigned)nitems : pack ? (unsigned)npack : (unsigned)a.ntile * (unsigned)g.nbpc);
   // a wave's share of LDS: as many heights of its columns' records as 10 KB
   // hold (16 waves per CU), one at least
   const size_t per = sizeof(float) * (REC_HEAD + REC_REG + REC_SLOT * (size_t)nb) * a.wcols;
   a.chunk = (int)std::max<size_t>(1, std::min<size_t>((size_t)std::min(16, g.nz), RT_LDS / per));
+  // Teams while one wave per 64 lanes leaves SIMDs without a wave, for the
+  // synthesis always (its tail and its records in LDS gain from them):
+  // ms with 8 / 4 / 1 waves, 64 heights: 64 columns x 120 wavelengths, 5
+  // responses 0.42 / 0.47 / 0.74; 400 columns 0.65 / 0.55 / 0.80; 1600 columns 1.74 / 1.36 / 1.30;
+  // node responses of 256 x 112 0.76 / 0.70 / 0.94, of 1024 x 112 1.52 / 1.23 / 1.14;
+  // synthesis of 64 x 112 0.27 / 0.28 / 0.37, of 4096 x 112 1.05 / 0.98 / 1.05.
+  int team = 1;
+  if (pack || nd) {
+    if (grid.x <= 256 && per * 8 <= 16384) team = 8;
+    else if ((grid.x <= 1024 || rf_mode == FZ_RF_NONE) && per * 4 <= 16384) team = 4;
+  }
+  if (team > 1) a.chunk = (int)std::min<size_t>(16, 16384 / per) / team * team;
   const size_t lds = per * a.chunk;
   a.pop = c->pop_on ? c->d_pop : nullptr;
   const NodeArgs nodes = nd ? *nd : NodeArgs();
-#define FZ_RT(RF, HE, PK) \
-  hipLaunchKernelGGL((rt_kernel<RF, HE, PK>), grid, blk, lds, st, a, nodes, (const NodeTab*)nullptr)
-  if (nd) {
-    if (pack)
-      hipLaunchKernelGGL((rt_kernel<RF_CART_TBV, false, true, true>), grid, blk, lds, st, a, nodes, (const NodeTab*)c->d_nodetab);
-    else
-      hipLaunchKernelGGL((rt_kernel<RF_CART_TBV, false, false, true>), grid, blk, lds, st, a, nodes,
-                         (const NodeTab*)c->d_nodetab);
-    HIPCHK(c, hipGetLastError());
-    return FZ_OK;
-  }
+#define FZ_RT(RF, HE, PK, ND, NW) \
+  hipLaunchKernelGGL((rt_kernel<RF, HE, PK, ND, NW>), grid, dim3(RT_WAVE * NW), lds, st, a, nodes, \
+                     (const NodeTab*)c->d_nodetab)
+#define FZ_RTT(RF, HE, PK, ND) \
+  do { \
+    if (team == 8) FZ_RT(RF, HE, PK, ND, 8); \
+    else if (team == 4) FZ_RT(RF, HE, PK, ND, 4); \
+    else FZ_RT(RF, HE, PK, ND, 1); \
+  } while (0)
 #define FZ_RTP(RF, HE) \
   do { \
-    if (pack) FZ_RT(RF, HE, true); \
-    else FZ_RT(RF, HE, false); \
+    if (pack) FZ_RTT(RF, HE, true, false); \
+    else FZ_RT(RF, HE, false, false, 1); \
   } while (0)
-  if (rf_mode == FZ_RF_NONE) FZ_RTP(FZ_RF_NONE, false);
+  if (nd && pack) FZ_RTT(RF_CART_TBV, false, true, true);
+  else if (nd) FZ_RTT(RF_CART_TBV, false, false, true);
+  else if (rf_mode == FZ_RF_NONE) FZ_RTP(FZ_RF_NONE, false);
   else if (!c->hydro && rf_mode == FZ_RF_SPHERICAL) FZ_RTP(FZ_RF_SPHERICAL, false);
   else if (!c->hydro && rf_mode == FZ_RF_CARTESIAN_P0) FZ_RTP(FZ_RF_CARTESIAN_P0, false);
   else if (c->hydro && rf_mode == FZ_RF_CARTESIAN_P0) FZ_RTP(FZ_RF_CARTESIAN_P0, true);
   else if (!c->hydro) FZ_RTP(FZ_RF_CARTESIAN, false);
   else if (rf_mode == FZ_RF_SPHERICAL) FZ_RTP(FZ_RF_SPHERICAL, true);
   else FZ_RTP(FZ_RF_CARTESIAN, true);
+#undef FZ_RTT
 #undef FZ_RTP
 #undef FZ_RT
   HIPCHK(c, hipGetLastError());

@@ -131,6 +131,10 @@ struct Five {
 constexpr float TH_SER = 2.0f;
 constexpr int NSER = 8;
 
+// (From here on, and in the transfer kernel, the multiply-adds are written out: what
+// else the compiler would join could differ between the kernel's instances, whose
+// results are the same bits.)
+#pragma clang fp contract(off)
 struct Evol {
   float ex, ez, rx, rz;        // e and r in the frame of the field
   float A, D4, ga, gb, s0, cy; // cy: (e x r) along the second axis
@@ -220,7 +224,7 @@ __device__ __forceinline__ void evol_build(const Five& f, Evol& E) {
       // 0.5 (truncation 1e-11 relative), where E - 1/E would cancel
       const float El = expf(l1), iEl = 1.0f / El;
       const float x2 = l1 * l1;
-      const float shs = l1 * (1.f + x2 * (1.f / 6.f) * (1.f + x2 * (1.f / 20.f) * (1.f + x2 * (1.f / 42.f) * (1.f + x2 * (1.f / 72.f)))));
+      const float shs = l1 * fmaf(x2 * (1.f / 6.f), fmaf(x2 * (1.f / 20.f), fmaf(x2 * (1.f / 42.f), fmaf(x2, 1.f / 72.f, 1.f), 1.f), 1.f), 1.f);
       che = ex * (0.5f * (El + iEl));
       she = ex * (l1 < 0.5f ? shs : 0.5f * (El - iEl));
     } else {
@@ -239,8 +243,8 @@ __device__ __forceinline__ void evol_build(const Five& f, Evol& E) {
     // w3 = s l2 e - l1 r, the vectors al = -(C2 a2 + B3 a3) and
     // om = -(C2 w2 + B3 w3) take two scalars: ga = C2 l2 + B3 l1 and
     // gb = s (B3 l2 - C2 l1).
-    E.ga = C2 * l2 + B3 * l1;
-    E.gb = sig * (B3 * l2 - C2 * l1);
+    E.ga = fmaf(C2, l2, B3 * l1);
+    E.gb = sig * fmaf(B3, l2, -(C2 * l1));
     if (DER) {
       // one pass per variable: dth, dl1, dl2 for a unit change of d, then of e.r
 #pragma unroll
@@ -250,17 +254,17 @@ __device__ __forceinline__ void evol_build(const Five& f, Evol& E) {
         float dl1, dl2;
         if (dp) {
           dl1 = (dth + dd) * (0.25f * il);
-          dl2 = (sig * der - l2 * dl1) * il;
+          dl2 = fmaf(-l2, dl1, sig * der) * il;
         } else {
           dl2 = (dth - dd) * (0.25f * il);
-          dl1 = (sig * der - l1 * dl2) * il;
+          dl1 = fmaf(-l1, dl2, sig * der) * il;
         }
-        const float dA = 0.5f * (she * dl1 - se * dl2);
-        const float dC2 = (ce * dl2 - C2 * dth) * ith;
-        const float dB3 = (che * dl1 - B3 * dth) * ith;
-        const float dD = (she * dl1 + se * dl2 - E.D4 * dth) * ith;
-        const float dga = dC2 * l2 + C2 * dl2 + dB3 * l1 + B3 * dl1;
-        const float dgb = sig * (dB3 * l2 + B3 * dl2 - dC2 * l1 - C2 * dl1);
+        const float dA = 0.5f * fmaf(she, dl1, -(se * dl2));
+        const float dC2 = fmaf(ce, dl2, -(C2 * dth)) * ith;
+        const float dB3 = fmaf(che, dl1, -(B3 * dth)) * ith;
+        const float dD = fmaf(she, dl1, fmaf(se, dl2, -(E.D4 * dth))) * ith;
+        const float dga = fmaf(dC2, l2, fmaf(C2, dl2, fmaf(dB3, l1, B3 * dl1)));
+        const float dgb = sig * fmaf(dB3, l2, fmaf(B3, dl2, -fmaf(dC2, l1, C2 * dl1)));
         if (v == 0) {
           E.Ad = dA; E.Dd = dD; E.gad = dga; E.gbd = dgb;
         } else {
@@ -364,5 +368,7 @@ __device__ __forceinline__ void evol_azimuth(const Evol& E, const float v[4], co
   o[2] = 2.f * fmaf(E.D4, fmaf(E.ex, w.p1[0], E.rx * w.p2[0]), alx * v[0]);
   o[3] = 2.f * fmaf(E.D4, g * v[2], omx * v[1]);
 }
+
+#pragma clang fp contract(fast)
 
 }  // namespace fz
