@@ -1672,8 +1672,8 @@ __global__ void soa_to_cube(const float* __restrict__ src, float* __restrict__ d
 #include "fz_lm.hpp"
 #include "fz_pert.hpp"
 #include "fz_invert.hpp"
-#include "fz_psf.hpp"
 #include "fz_mlp.hpp"
+#include "fz_psf.hpp"
 
 namespace fz {
 // Spectral line-spread function (MLSF) on rows of numw floats (Stokes rows,
@@ -1920,6 +1920,8 @@ struct fz_ctx {
   std::vector<double> h_psf;
   int psf_npx = 0, psf_npy = 0;
   float* d_taps = nullptr;
+  bf16* d_tapfrag = nullptr;  // the taps as matrix operands (both directions), where these are in range
+  bool taps_split = false;
   int taps_nx = 0, taps_ny = 0, taps_rx = 0, taps_ry = 0, taps_ntx = 0;
   double taps_sq = 0.0;   // sum of the squared taps
 };
@@ -2045,6 +2047,7 @@ void fz_destroy(fz_ctx* c) {
   if (c->d_pert) (void)hipFree(c->d_pert);
   if (c->d_pstage) (void)hipFree(c->d_pstage);
   if (c->d_taps) (void)hipFree(c->d_taps);
+  if (c->d_tapfrag) (void)hipFree(c->d_tapfrag);
   c->mlp.release();
   for (int i = 0; i < 3; ++i)
     if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
@@ -2318,9 +2321,44 @@ static int psf_taps(fz_ctx* c, int nx, int ny) {
     }
   HIPCHK(c, hipSetDevice(c->device));
   if (c->d_taps) (void)hipFree(c->d_taps);
+  if (c->d_tapfrag) (void)hipFree(c->d_tapfrag);
   c->d_taps = nullptr;
+  c->d_tapfrag = nullptr;
   HIPCHK(c, hipMalloc(&c->d_taps, sizeof(float) * t.size()));
   HIPCHK(c, hipMemcpy(c->d_taps, t.data(), sizeof(float) * t.size(), hipMemcpyHostToDevice));
+  // Operands of psf_split_kernel: [direction][u][x tile][step][part][lane][8], tap t of
+  // output i of the x tile at input k = 16 tile + i + t.  Sixteen taps and fewer are left
+  // to the vector units: the matrix cores' work does not get less below 2 rx + 1 = 32
+  // (ms, vector units / matrix cores, 112 maps of 256 x 256: 9 x 9 taps 0.067 / 0.071,
+  // 15 x 15 0.089 / 0.092, 17 x 17 0.131 / 0.087; 64 maps, 63 x 63 0.61 / 0.29).
+  c->taps_split = ntx > 16;
+  for (float v : t)
+    if (v != 0.f && !(std::fabs(v) > 0x1p-100f && std::fabs(v) < 0x1p100f)) c->taps_split = false;
+  if (c->taps_split) {
+    const int ks = ntx > 32 ? 3 : 2;
+    std::vector<uint16_t> f((size_t)2 * nu * 2 * ks * 3 * 512);
+    auto part = [](float& v) {   // the nearest BF16 of v, taken off it
+      uint32_t b;
+      memcpy(&b, &v, 4);
+      b = (b + 0x7fffu + ((b >> 16) & 1u)) & 0xffff0000u;
+      float h;
+      memcpy(&h, &b, 4);
+      v -= h;
+      return (uint16_t)(b >> 16);
+    };
+    for (int du = 0; du < 2 * nu; ++du)
+      for (int xt = 0; xt < 2; ++xt)
+        for (int s = 0; s < ks; ++s)
+          for (int lane = 0; lane < 64; ++lane)
+            for (int j = 0; j < 8; ++j) {
+              const int tt = 32 * s + 8 * (lane >> 4) + j - 16 * xt - (lane & 15);
+              float v = tt >= 0 && tt <= 2 * rx ? t[(size_t)du * ntx + tt] : 0.f;
+              for (int p = 0; p < 3; ++p)
+                f[((((size_t)du * 2 + xt) * ks + s) * 3 + p) * 512 + lane * 8 + j] = part(v);
+            }
+    HIPCHK(c, hipMalloc(&c->d_tapfrag, sizeof(uint16_t) * f.size()));
+    HIPCHK(c, hipMemcpy(c->d_tapfrag, f.data(), sizeof(uint16_t) * f.size(), hipMemcpyHostToDevice));
+  }
   c->taps_nx = nx;
   c->taps_ny = ny;
   c->taps_rx = rx;
@@ -2328,6 +2366,18 @@ static int psf_taps(fz_ctx* c, int nx, int ny) {
   c->taps_ntx = ntx;
   c->taps_sq = sq;
   return FZ_OK;
+}
+
+template <int KS, int YT>
+static void launch_psf_split(fz_ctx* c, const PsfArgs& a, int adjoint, hipStream_t st) {
+  const int ntx = c->taps_ntx, ty = 32 * YT, nu = 2 * a.ry + 1;
+  const size_t lds = std::max(sizeof(bf16) * 3 * (ty + 2 * a.ry) * (32 * KS + 8),
+                              sizeof(float) * (PSF_TX + ntx - 1) * (PSF_TY + 2 * a.ry));
+  (void)hipFuncSetAttribute((const void*)psf_split_kernel<KS, YT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            144 * 1024);
+  const dim3 grid((unsigned)((a.ny + ty - 1) / ty), (unsigned)((a.nx + PSF_TX - 1) / PSF_TX), (unsigned)a.nmaps);
+  hipLaunchKernelGGL((psf_split_kernel<KS, YT>), grid, dim3(256), lds, st, a,
+                     (const bf16*)c->d_tapfrag + (adjoint ? (size_t)nu * 2 * KS * 3 * 512 : 0), ntx);
 }
 
 static void launch_psf(fz_ctx* c, int nx, int ny, int nmaps, const float* in, float* out, int adjoint, hipStream_t st) {
@@ -2342,6 +2392,15 @@ static void launch_psf(fz_ctx* c, int nx, int ny, int nmaps, const float* in, fl
   a.taps = c->d_taps + (adjoint ? (size_t)(2 * a.ry + 1) * ntx : 0);
   a.in = in;
   a.out = out;
+  if (c->taps_split) {
+    // 128 y a workgroup, 64 where that covers the map with fewer
+    const bool wide = (ny + 127) / 128 * 2 <= (ny + 63) / 64;
+    if (ntx <= 32)
+      wide ? launch_psf_split<2, 4>(c, a, adjoint, st) : launch_psf_split<2, 2>(c, a, adjoint, st);
+    else
+      wide ? launch_psf_split<3, 4>(c, a, adjoint, st) : launch_psf_split<3, 2>(c, a, adjoint, st);
+    return;
+  }
   const size_t lds = sizeof(float) * (PSF_TX + ntx - 1) * (PSF_TY + 2 * a.ry);
   const dim3 grid((unsigned)((ny + PSF_TY - 1) / PSF_TY), (unsigned)((nx + PSF_TX - 1) / PSF_TX), (unsigned)nmaps);
   switch (ntx) {

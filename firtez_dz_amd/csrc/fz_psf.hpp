@@ -8,12 +8,14 @@
 // a circular convolution,
 //   out(y, x) = sum_{dy, dx} PSF(Y0 + dy, X0 + dx) in(y - dy mod NY, x - dx mod NX).
 // Here the same sum is formed directly (a 31 x 31 PSF is 961 taps per
-// output; 1.04 ms for 448 maps of 256 x 256 on MI355X), which needs no FFT
-// library and keeps the result exact to FP32 summation.  The adjoint (the transpose
+// output), which needs no FFT library and keeps the result exact to FP32
+// summation: psf_split_kernel on the matrix cores, psf_conv_kernel on the
+// vector units for PSFs of up to 16 pixels in x and taps outside the range of the
+// former.  The adjoint (the transpose
 // of the convolution, used for the gradient of the coupled chi^2) is the
 // correlation out(y, x) = sum PSF(Y0 + dy, X0 + dx) in(y + dy, x + dx).
 //
-// Layout: maps channel-major, map m at in[m * npix + col] with
+// psf_conv_kernel: maps channel-major, map m at in[m * npix + col] with
 // col = y + ny * x (the cube's column order), so a map is an nx x ny image
 // with y contiguous.  One workgroup of four waves computes a 32 (x) x 64 (y)
 // output tile of one map: the lanes of a wave take 64 consecutive y, and
@@ -92,6 +94,172 @@ __global__ void __launch_bounds__(256) psf_conv_kernel(PsfArgs a) {
   for (int i = 0; i < PSF_OX; ++i) {
     const int x = x0 + xw + i;
     if (x < a.nx) dst[(long)x * a.ny] = acc[i];
+  }
+}
+
+// The same tile (64 columns from y0) with the tap count at run time, by all
+// 256 threads: the sums of psf_conv_kernel in its order.
+__device__ __forceinline__ void psf_direct(const PsfArgs& a, int ntx, int x0, int y0, const float* __restrict__ src,
+                                           float* __restrict__ dst, float* tile) {
+  const int rows = PSF_TX + ntx - 1, cols = PSF_TY + 2 * a.ry;
+  __syncthreads();
+  for (int e = threadIdx.x; e < rows * cols; e += 256) {
+    const int i = e / cols, j = e - i * cols;
+    int x = (x0 - a.rx + i) % a.nx;
+    if (x < 0) x += a.nx;
+    int y = (y0 - a.ry + j) % a.ny;
+    if (y < 0) y += a.ny;
+    tile[e] = src[(long)x * a.ny + y];
+  }
+  __syncthreads();
+  const int ty = threadIdx.x & 63, xw = (threadIdx.x >> 6) * PSF_OX;
+  float acc[PSF_OX];
+#pragma unroll
+  for (int i = 0; i < PSF_OX; ++i) acc[i] = 0.f;
+  for (int u = 0; u <= 2 * a.ry; ++u) {
+    const float* colp = tile + xw * cols + ty + u;
+    float v[2 * PSF_OX - 1];
+#pragma unroll
+    for (int j = 0; j < PSF_OX - 1; ++j) v[j] = colp[j * cols];
+    for (int t0 = 0; t0 < ntx; t0 += PSF_OX) {
+#pragma unroll
+      for (int j = PSF_OX - 1; j < 2 * PSF_OX - 1; ++j) v[j] = colp[(t0 + j) * cols];
+#pragma unroll
+      for (int t = 0; t < PSF_OX; ++t)
+#pragma unroll
+        for (int i = 0; i < PSF_OX; ++i) acc[i] = fmaf(a.taps[u * ntx + t0 + t], v[i + t], acc[i]);
+#pragma unroll
+      for (int j = 0; j < PSF_OX - 1; ++j) v[j] = v[j + PSF_OX];
+    }
+  }
+  const int y = y0 + ty;
+#pragma unroll
+  for (int i = 0; i < PSF_OX; ++i)
+    if (y < a.ny && x0 + xw + i < a.nx) dst[(long)(x0 + xw + i) * a.ny + y] = acc[i];
+}
+
+// The convolution on the matrix cores.  Inputs and taps are split into three BF16
+// parts each (8 + 8 + 8 bits: x = hi + mid + lo exactly), and six of the nine
+// products of parts are summed in FP32; the three left out are below 2^-24 of
+// the product.  For a tap row u the outputs of 32 x are a banded Toeplitz matrix of the
+// taps (two 16 x (32 KS) operands, in operand order from memory, the same for
+// every tile) times the strip of 32 + 2 rx inputs, which lies in LDS with x contiguous
+// so that 16 y and 32 x are one operand at any row y + u.
+//
+// A workgroup has 32 x and 32 YT y of one map: of its four waves two have
+// half the y each, two the even and two the odd tap rows, added at the end.  Per tap row
+// a wave reads 6 KS tap operands (a row ahead) and 3 KS YT input operands for
+// 12 KS YT MFMAs.  Bound: these, (2 rx + 1) / (32 KS) of whose products are taps.
+// Error against 64 bits (448 maps of 256 x 256, 31 x 31 taps): 1.6e-7 of the
+// result, with the vector units' sums 4.7e-7; time 0.49 ms for 0.97.
+//
+// A tile with an input that is not finite, beyond 2^120 or, not being zero,
+// below 2^-100, where the parts would leave BF16's range, takes psf_direct.
+template <int KS, int YT>
+__global__ void __launch_bounds__(256) psf_split_kernel(PsfArgs a, const bf16* __restrict__ frag, int ntx) {
+  extern __shared__ __attribute__((aligned(16))) char psf_lds[];
+  __shared__ int flag[4];
+  constexpr int XP = 32 * KS + 8, TY = 32 * YT;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int lr = lane & 15, lg = lane >> 4;
+  const int x0 = blockIdx.y * PSF_TX, y0 = blockIdx.x * TY;
+  const int rows = TY + 2 * a.ry, nk = PSF_TX + 2 * a.rx, nu = 2 * a.ry + 1;
+  const float* src = a.in + (long)blockIdx.z * a.npix;
+  float* dst = a.out + (long)blockIdx.z * a.npix;
+  bf16* plane = reinterpret_cast<bf16*>(psf_lds);
+  const int ps = rows * XP;
+  bool bad = false;
+  for (int e = threadIdx.x; e < rows * 4 * KS; e += 256) {
+    const int g = e / rows, j = e - g * rows;
+    // (rx < nx, ry < ny; small maps go round more than once)
+    int y = y0 - a.ry + j, x = x0 - a.rx + 8 * g;
+    y += y < 0 ? a.ny : 0;
+    x += x < 0 ? a.nx : 0;
+    while (y >= a.ny) y -= a.ny;
+    while (x >= a.nx) x -= a.nx;
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      v[i] = 8 * g + i < nk ? src[(long)x * a.ny + y] : 0.f;
+      x = x + 1 == a.nx ? 0 : x + 1;
+    }
+    bf16x8 p0, p1, p2;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const unsigned b = __float_as_uint(v[i]) & 0x7fffffffu;
+      bad |= b > 0x7b800000u || (b != 0 && b < 0x0d800000u);
+      p0[i] = (bf16)v[i];
+      const float r = v[i] - (float)p0[i];
+      p1[i] = (bf16)r;
+      p2[i] = (bf16)(r - (float)p1[i]);
+    }
+    bf16* o = plane + j * XP + 8 * g;
+    *reinterpret_cast<bf16x8*>(o) = p0;
+    *reinterpret_cast<bf16x8*>(o + ps) = p1;
+    *reinterpret_cast<bf16x8*>(o + 2 * ps) = p2;
+  }
+  const bool any = __ballot(bad) != 0;
+  if (lane == 0) flag[wave] = any;
+  __syncthreads();
+  if (flag[0] | flag[1] | flag[2] | flag[3]) {
+    for (int h = 0; h < TY; h += PSF_TY)
+      psf_direct(a, ntx, x0, y0 + h, src, dst, reinterpret_cast<float*>(psf_lds));
+    return;
+  }
+  f32x4 acc[2][YT];
+#pragma unroll
+  for (int i = 0; i < 2 * YT; ++i) acc[i & 1][i >> 1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  const int yb = (wave & 1) * 16 * YT;
+  const bf16x8* F = reinterpret_cast<const bf16x8*>(frag) + lane;
+  constexpr int NF = 6 * KS;     // tap operands of a row: [x tile][step][part]
+  bf16x8 t[NF];
+#pragma unroll
+  for (int i = 0; i < NF; ++i) t[i] = F[(min(wave >> 1, nu - 1) * NF + i) * 64];
+  for (int u = wave >> 1; u < nu; u += 2) {
+    bf16x8 n[NF];
+    const int un = min(u + 2, nu - 1);
+#pragma unroll
+    for (int i = 0; i < NF; ++i) n[i] = F[(un * NF + i) * 64];
+    __builtin_amdgcn_sched_barrier(0);   // keeps the loads here, a row ahead
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+#pragma unroll
+      for (int yt = 0; yt < YT; ++yt) {
+        const bf16* b = plane + (yb + 16 * yt + lr + u) * XP + 32 * s + 8 * lg;
+        const bf16x8 b0 = *reinterpret_cast<const bf16x8*>(b), b1 = *reinterpret_cast<const bf16x8*>(b + ps),
+                     b2 = *reinterpret_cast<const bf16x8*>(b + 2 * ps);
+#pragma unroll
+        for (int xt = 0; xt < 2; ++xt) {
+          const bf16x8 *c = t + (xt * KS + s) * 3;
+          f32x4 d = acc[xt][yt];
+          d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[0], b2, d, 0, 0, 0);
+          d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[2], b0, d, 0, 0, 0);
+          d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[1], b1, d, 0, 0, 0);
+          d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[0], b1, d, 0, 0, 0);
+          d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[1], b0, d, 0, 0, 0);
+          d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[0], b0, d, 0, 0, 0);
+          acc[xt][yt] = d;
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NF; ++i) t[i] = n[i];
+  }
+  // the odd rows' sums to the waves of the even ones
+  f32x4* red = reinterpret_cast<f32x4*>(psf_lds);
+  __syncthreads();
+  if (wave >= 2)
+#pragma unroll
+    for (int i = 0; i < 2 * YT; ++i) red[((wave & 1) * 2 * YT + i) * 64 + lane] = acc[i & 1][i >> 1];
+  __syncthreads();
+  if (wave >= 2) return;
+#pragma unroll
+  for (int i = 0; i < 2 * YT; ++i) {
+    const f32x4 d = acc[i & 1][i >> 1] + red[(wave * 2 * YT + i) * 64 + lane];
+    const int y = y0 + yb + 16 * (i >> 1) + lr, x = x0 + 16 * (i & 1) + 4 * lg;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (y < a.ny && x + q < a.nx) dst[(long)(x + q) * a.ny + y] = d[q];
   }
 }
 
