@@ -317,16 +317,21 @@ __global__ void __launch_bounds__(256) mlp_input_kernel(int n, int nin, const fl
   const size_t f = t >> 6;
   const int r = (int)(f / steps) * 16 + (lane & 15), k0 = (int)(f % steps) * 32 + 8 * (lane >> 4);
   bf16x8 v;
+  // (one type per loop, so that the eight loads are in flight together)
+  auto fill = [&](const auto* x) {
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int m = tr ? k0 + j : r, i = tr ? r : k0 + j;
-    float x = 0.f;
-    if (m < n && i < nin) {
-      const long row = idx ? (long)idx[m] : (long)m;
-      x = ((xf ? xf[row * nin + i] : (float)xd[row * nin + i]) - mean[i]) / sdev[i];
+    for (int j = 0; j < 8; ++j) {
+      const int m = tr ? k0 + j : r, i = tr ? r : k0 + j;
+      const int mc = min(m, n - 1), ic = min(i, nin - 1);
+      const long row = idx ? (long)idx[mc] : (long)mc;
+      const float e = ((float)x[row * nin + ic] - mean[ic]) / sdev[ic];
+      v[j] = (bf16)(m < n && i < nin ? e : 0.f);
     }
-    v[j] = (bf16)x;
-  }
+  };
+  if (xf)
+    fill(xf);
+  else
+    fill(xd);
   reinterpret_cast<bf16x8*>(tr ? XT : X)[t] = v;
 }
 
@@ -441,7 +446,9 @@ __device__ __forceinline__ void mlp_decode(const MlpShape& S, int R, int c0, int
   const int c = threadIdx.x % R;
   if (c0 + c >= ncol) return;
   const size_t cs = (size_t)S.nz * ncol;
-  for (int k = threadIdx.x / R; k < S.nz; k += blockDim.x / R) {
+  // with 64 columns the height is the wave's: the basis comes through scalar loads
+  for (int k = R == 64 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64) : (int)threadIdx.x / R; k < S.nz;
+       k += blockDim.x / R) {
     double T = 0.0, X = 0.0, Y = 0.0, Z = 0.0, V = 0.0;
     for (int j = 0; j < nj; ++j) {
       const double w = coefs[k * nj + j];
@@ -480,7 +487,7 @@ __global__ void __launch_bounds__(256) mlp_decode_kernel(MlpShape S, int ncol, c
 // the output fragments w, w + 8, w + 16 and w + 24 of 16.  Bounded by the weights' way
 // into a CU (64 B per cycle: 11 us for the 1.5 MB of 448-512-512-512-20) and by
 // the inputs from memory.  Layer by layer, with activations in
-// memory, inputs and decoding apart, 16384 rows of 448 took 210 us in kernels, here 63.
+// memory, inputs and decoding apart, 16384 rows of 448 took 210 us in kernels, here 53.
 // y [n][nout] or, when atm is given, the initial model.
 struct InferArgs {
   int n, pitch;
@@ -504,23 +511,39 @@ __global__ void __launch_bounds__(512) mlp_infer_kernel(MlpShape S, InferArgs a)
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int lr = lane & 15, lg = lane >> 4, pitch = a.pitch;
   const int c0 = (int)blockIdx.x * R;
-  // inputs: wave w standardises rows w, w + 8, ...; eight rows' loads in flight
-  {
+  // inputs: wave w standardises rows w, w + 8, ..., the loads of all its rows in
+  // flight (one at a time, as a choice of the type at each load makes them, 16384 rows
+  // took 63 us in all instead of 53)
+  auto inputs = [&](const auto* x) {
     const int nin = S.nin, np = pad32(nin);
-    constexpr int U = R / 8;
-    for (int i = lane; i < np; i += 64) {
-      const bool in = i < nin;
-      const float mu = in ? a.mean[i] : 0.f, sd = in ? a.sdev[i] : 1.f;
-      float v[U];
+    constexpr int U = R / 8, V = 2;
+    for (int i0 = lane; i0 < np; i0 += 64 * V) {
+      auto v = [&](int q, int u) {
+        return x[(size_t)min(c0 + wave + 8 * u, a.n - 1) * nin + min(i0 + 64 * q, nin - 1)];
+      };
+      decltype(v(0, 0)) w[V][U];
+      float mu[V], sd[V];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const size_t o = (size_t)min(c0 + wave + 8 * u, a.n - 1) * nin + min(i, nin - 1);
-        v[u] = a.xf ? a.xf[o] : (float)a.xd[o];
+      for (int q = 0; q < V; ++q) {
+        mu[q] = a.mean[min(i0 + 64 * q, nin - 1)];
+        sd[q] = a.sdev[min(i0 + 64 * q, nin - 1)];
+#pragma unroll
+        for (int u = 0; u < U; ++u) w[q][u] = v(q, u);
       }
 #pragma unroll
-      for (int u = 0; u < U; ++u) act[(wave + 8 * u) * pitch + i] = (bf16)(in ? (v[u] - mu) / sd : 0.f);
+      for (int q = 0; q < V; ++q) {
+        const int i = i0 + 64 * q;
+        if (i >= np) break;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          act[(wave + 8 * u) * pitch + i] = (bf16)(i < nin ? ((float)w[q][u] - mu[q]) / sd[q] : 0.f);
+      }
     }
-  }
+  };
+  if (a.xf)
+    inputs(a.xf);
+  else
+    inputs(a.xd);
   __syncthreads();
   for (int l = 0; l <= S.nl; ++l) {
     const int N = S.dout[l], nfr = pad32(N) >> 4, ks = pad32(S.din[l]) >> 5;
