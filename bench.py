@@ -341,8 +341,8 @@ def main():
     # roofline of the dominant kernel (radiative transfer), HIP-event timed
     rt_avg_ms = float(np.mean(rt_ms))
     nlaunch = (ncol + args.tile - 1) // args.tile
-    ncomp = 16
-    fl = flops.per_column_lambda(args.nz, 2, ncomp, npar)
+    ncomp = 15          # 12 of Fe I 6301.5 (without the pi component of no strength) + the triplet 6302.5
+    fl = flops.per_column_lambda(args.nz, 2, ncomp, npar, ntriplet=1)
     # per launch: the tile's columns x wavelengths x flop, over the average launch time
     launch_ms = rt_avg_ms / nlaunch
     # HBM bytes of rt_kernel<1> per column of this workload (nz = 96, 112

@@ -121,7 +121,7 @@ __constant__ Cfg c_cfg;
 //   rho_group_kernel  16 to 64 lanes per column, heights bottom->top: only the
 //                warm-started electron-density fixed point (GET_RHO), reading
 //                the factors from sbuf -> rho, mu, Pe and (n_e, N_H) per height
-//   opac_kernel  one thread per (height, column): implicit EOS derivatives,
+//   deriv_kernel, opac_kernel  one thread per (height, column): EOS derivatives,
 //                continuum and line opacity, damping -> the per-height record
 //   tau_kernel   one thread per column: the REAL(4) log tau5 trapezoid
 // FP64 throughout; the fixed point keeps the reference's iteration path

@@ -1,6 +1,7 @@
 // Per-pixel Levenberg-Marquardt step of the FIRTEZ-dz inversion on the GPU.
 //
-//   eqv_kernel : node contraction of the per-height response functions
+//   eqv_kernel : node contraction of the per-height response functions where
+//                rt_kernel does not form it (Pg, rho, P0, HYDROSTATIC)
 //                (CALCULATE_EQUIVALENT_DSYN, forward.f90:552-681): one thread
 //                per (pixel, spectral row), FP64 accumulation over the support
 //                of each node's hat function, REAL(4) store.

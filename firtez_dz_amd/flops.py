@@ -7,56 +7,67 @@ hardware reciprocal = 1 each.  Loads/stores, selects, comparisons and integer
 index arithmetic are not counted.  The counts are per non-boundary layer.
 They were tallied by hand from the source of each device function (the
 names below follow csrc/fz_rt.hpp and rt_kernel); change them together with
-the kernel.  Response-function directions that a mode does not store are
-not formed by the kernel (the compiler drops them), so the per-line
-derivative work depends on the parameter set.
+the kernel.  The evolution operator is counted in its series form, which nearly
+all layers take.
 """
 from __future__ import annotations
 
 # per Zeeman component
-VOIGT = 66           # Hui 7/7 rational: r, s (4); 5 + 6 two-FMA rounds (44); real/imag parts (6);
-                     # |den|^2 (3), reciprocal (1), H and L (8)
-COMP_FWD = 2 + VOIGT + 4              # u, profile, 2 accumulations (absorb)
-COMP_DER = 2 + VOIGT + 4 + 5 + 20     # u, profile, dH/du, dH/da, 8 accumulations (absorb_der)
+VOIGT = 36           # u^2 (1); numerator 6 + 4, denominator 6 + 5 + 1, |den|^2 (3), reciprocal (1), H (4), F (5)
+COMP_FWD = 2 + VOIGT + 4              # u, 2 accumulations (absorb)
+COMP_DER = 2 + VOIGT + 12             # u, 6 moments (absorb_der)
+# per component type (sigma_r, pi, sigma_b) of a line
+TYPE_FWD = 2 + 4                      # u of the type's centre, 2 accumulations
+TYPE_SUM = 32                         # dH/du, dH/da and their products with u and the shift from the moments
+TYPE_SUM_ONE = 11                     # the same of a type with one component
+TYPE_ACC = 24                         # value, T, v, |B| of absorption and dispersion
+TYPE_ACC_PR = 16                      # Pg and rho
 # per line
-LINE_SETUP = 5                        # inverse Doppler width (from the stored 1/sqrt(T)), shift, field scale
-LINE_FWD = LINE_SETUP + 2 * 14 + 14   # 2 lin() combinations, 7 accumulations
-LIN_ALL = 8 * 14 + 2 * 15 + 2 * 8     # 8 lin(), 2 lin_dgamma(), 2 lin_dphi() combinations
-# accumulation into the 7 propagation-matrix elements per direction formed
-ACC = {"value": 2, "T": 7, "Pg": 5, "rho": 5, "v": 2, "B": 2, "gamma": 2, "phi": 2}
-DIRS = {5: ("T", "v", "B", "gamma", "phi"), 7: ("T", "Pg", "rho", "v", "B", "gamma", "phi")}
+LINE_FWD = 5                          # kappa_l dz, shift, Doppler scale, field scale
+LINE_DER = 14
+LINE_DER_PR = 6
 # per layer
-GEOMETRY = 0          # |B|, inclination and azimuth terms: formed by opac_kernel, read from the record
-SOURCE = 6            # 1/T, c2/T, exp, -1, reciprocal, x c1
-SOURCE_DER = 11       # the same and dS/dT = S (ex/(ex-1)) (c2/T) / T
-EVOL_BUILD = 155                      # evol_build: scaling, eigen-parameters, exponentials, sin/cos, O
-FORMAL = 40                           # I_k = (1-O) S + O I_{k-1}
-M4V = 46                              # v = I_in - S, M4raw v
-EVOL_DIR = 257                        # evol_dir: one directional derivative (dO) v
-SOURCE_TERM = 12                      # (1-O) e0 dS/dT
+MIX = 15 + 2                          # the five elements from the types' sums, with the continuum
+SOURCE = 6                            # c2/T, exp, departure, -1, reciprocal, x c1
+SOURCE_DER = 10                       # the same and dS/dT = S (ex/(ex-1)) (c2/T) / T
+TURN = 6                              # into the layer's frame or back
+EVOL_BUILD = 107                      # evol_build (series form): invariants, exp, four series, coefficients
+EVOL_BUILD_DER = 103                  # their derivatives
+PIECES = 40                           # evol_pieces
+APPLY = 20                            # evol_apply
+FORMAL = 1 + 2 * TURN + PIECES + APPLY + 9   # I_k = S + O (I_(k-1) - S)
+GRAD = 218                            # evol_grad
+GRAD_DOT = 36
+AZIMUTH = 36
+INCLINATION = 3 + MIX - 2 + GRAD_DOT
+SOURCE_TERM = 18                      # (1-O) e0 dS/dT
+CHAIN = 52                            # (|B|, inclination, azimuth) -> (Bx, By, Bz)
+EXTEND = 28 + 4 * (2 * TURN + 28 + 8) # ACC in the frame, ACC <- ACC . O_k
 PROPAGATE_PER_PARAM = 28              # ACC . local response
-ACC_UPDATE = 112                      # ACC <- ACC . O_k
-STORE_SCALE = 4                       # x GAIN1D per stored parameter
 
 
-def line_der(nparam: int) -> int:
-    acc = 7 * (ACC["value"] + sum(ACC[d] for d in DIRS[nparam]))
-    return LINE_SETUP + LIN_ALL + 2 + acc
-
-
-def per_layer(nlines: int, ncomp: int, nparam: int, chain: int = 0) -> dict:
-    fwd = GEOMETRY + SOURCE + nlines * LINE_FWD + ncomp * COMP_FWD + EVOL_BUILD + FORMAL
+def per_layer(nlines: int, ncomp: int, nparam: int, ntriplet: int = 0) -> dict:
+    """ntriplet: how many of the lines have one component per type."""
+    ntype = 3 * nlines
+    # a one-component type takes its centre's u
+    ncu = ncomp - 3 * ntriplet
+    fwd = (SOURCE + nlines * LINE_FWD + ncomp * COMP_FWD + ntype * TYPE_FWD + MIX + EVOL_BUILD + FORMAL)
     der = 0
     if nparam:
-        der = (GEOMETRY + SOURCE_DER + nlines * line_der(nparam) + ncomp * COMP_DER + EVOL_BUILD + M4V
-               + nparam * (EVOL_DIR + PROPAGATE_PER_PARAM + STORE_SCALE) + SOURCE_TERM + ACC_UPDATE + chain)
+        pr = nparam == 7
+        der = (SOURCE_DER + nlines * (LINE_DER + (LINE_DER_PR if pr else 0))
+               + ncomp * VOIGT + ncu * (COMP_DER - VOIGT)
+               + ntype * (2 + TYPE_ACC + (TYPE_ACC_PR if pr else 0))
+               + 3 * (nlines - ntriplet) * TYPE_SUM + 3 * ntriplet * TYPE_SUM_ONE
+               + MIX + EVOL_BUILD + EVOL_BUILD_DER + 1 + TURN + PIECES + GRAD
+               + (3 + (2 if pr else 0)) * (MIX + GRAD_DOT) + AZIMUTH + INCLINATION
+               + SOURCE_TERM + (CHAIN if pr else 0) + EXTEND + nparam * PROPAGATE_PER_PARAM)
     return {"pass1": fwd, "pass2": der, "total": fwd + der}
 
 
-def per_column_lambda(nz: int, nlines: int, ncomp: int, nparam: int) -> float:
+def per_column_lambda(nz: int, nlines: int, ncomp: int, nparam: int, ntriplet: int = 0) -> float:
     """FLOPs per (column, wavelength) over nz layers (boundary layer excluded)."""
-    chain = 3 * 4 * 5 if nparam == 7 else 0
-    return (nz - 1) * per_layer(nlines, ncomp, nparam, chain)["total"]
+    return (nz - 1) * per_layer(nlines, ncomp, nparam, ntriplet)["total"]
 
 
 # bytes that must cross HBM per (column, wavelength): the Jacobian and Stokes
