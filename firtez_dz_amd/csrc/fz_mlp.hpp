@@ -340,7 +340,8 @@ __device__ __forceinline__ void mlp_put(const MlpShape& S, long i, float v, bf16
   int l = 0;
   while (l < S.nl && i >= S.woff[l + 1]) ++l;
   if (i >= S.boff[l]) return;
-  const int e = (int)(i - S.woff[l]), o = e / S.din[l], k = e - o * S.din[l];
+  const long e = i - S.woff[l];
+  const int o = (int)(e / S.din[l]), k = (int)(e - (long)o * S.din[l]);
   const bf16 b = (bf16)v;
   wb[S.wb[l] + frag_at(o, k, pad32(S.din[l]) >> 5)] = b;
   wb[S.wt[l] + frag_at(k, o, pad32(S.dout[l]) >> 5)] = b;
