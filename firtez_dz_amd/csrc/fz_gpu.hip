@@ -2327,7 +2327,7 @@ static int psf_taps(fz_ctx* c, int nx, int ny) {
   HIPCHK(c, hipMalloc(&c->d_taps, sizeof(float) * t.size()));
   HIPCHK(c, hipMemcpy(c->d_taps, t.data(), sizeof(float) * t.size(), hipMemcpyHostToDevice));
   // Operands of psf_split_kernel: [direction][u][x tile][step][part][lane][8], tap t of
-  // output i of the x tile at input k = 16 tile + i + t.  Sixteen taps and fewer are left
+  // output i of the 32 at input k = i + t.  Sixteen taps and fewer are left
   // to the vector units: the matrix cores' work does not get less below 2 rx + 1 = 32
   // (ms, vector units / matrix cores, 112 maps of 256 x 256: 9 x 9 taps 0.067 / 0.071,
   // 15 x 15 0.089 / 0.092, 17 x 17 0.131 / 0.087; 64 maps, 63 x 63 0.61 / 0.29).
@@ -2347,15 +2347,16 @@ static int psf_taps(fz_ctx* c, int nx, int ny) {
       return (uint16_t)(b >> 16);
     };
     for (int du = 0; du < 2 * nu; ++du)
-      for (int xt = 0; xt < 2; ++xt)
-        for (int s = 0; s < ks; ++s)
-          for (int lane = 0; lane < 64; ++lane)
-            for (int j = 0; j < 8; ++j) {
-              const int tt = 32 * s + 8 * (lane >> 4) + j - 16 * xt - (lane & 15);
-              float v = tt >= 0 && tt <= 2 * rx ? t[(size_t)du * ntx + tt] : 0.f;
-              for (int p = 0; p < 3; ++p)
-                f[((((size_t)du * 2 + xt) * ks + s) * 3 + p) * 512 + lane * 8 + j] = part(v);
-            }
+      for (int tt = 0; tt <= 2 * rx; ++tt) {
+        float v = t[(size_t)du * ntx + tt];
+        for (int p = 0; p < 3; ++p) {
+          const uint16_t h = part(v);
+          for (int i = 0; i < 32; ++i) {   // output i of 32, input k = i + tt
+            const int k = i + tt, xt = i >> 4, lane = (i & 15) + 16 * ((k >> 3) & 3);
+            f[((((size_t)du * 2 + xt) * ks + (k >> 5)) * 3 + p) * 512 + lane * 8 + (k & 7)] = h;
+          }
+        }
+      }
     HIPCHK(c, hipMalloc(&c->d_tapfrag, sizeof(uint16_t) * f.size()));
     HIPCHK(c, hipMemcpy(c->d_tapfrag, f.data(), sizeof(uint16_t) * f.size(), hipMemcpyHostToDevice));
   }
