@@ -2320,6 +2320,9 @@ static int psf_taps(fz_ctx* c, int nx, int ny) {
       sq += (double)v * (double)v;
     }
   HIPCHK(c, hipSetDevice(c->device));
+  // no map size holds until every table is there: a failed allocation below
+  // leaves the next call to cut the taps again
+  c->taps_nx = c->taps_ny = 0;
   if (c->d_taps) (void)hipFree(c->d_taps);
   if (c->d_tapfrag) (void)hipFree(c->d_tapfrag);
   c->d_taps = nullptr;

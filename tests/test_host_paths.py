@@ -1,0 +1,54 @@
+"""Host code of the library on a machine without a GPU (tests/hostdouble): what
+it launches and holds after allocations fail, and with maps at the limits of
+the card.  Each case runs in an interpreter of its own."""
+import ctypes
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIB = os.path.join(ROOT, "firtez_dz_amd", "libfirtez_gpu.so")
+
+
+def case_psf_failed_operands():
+    """A failed allocation while the taps are cut for another map size leaves
+    no state that a later convolution would launch with missing operands."""
+    import numpy as np
+    d = hostdouble.load()
+    ctx = d.gpu.Context(0)
+    ctx.set_psf(np.full((31, 31), 1.0 / 961.0))
+    d.watch["psf_"] = lambda x: (x.name, x.arg(1, ctypes.c_void_p).value if "split" in x.name else None)
+    maps = d.malloc(4 * 2 * 128 * 128)
+    out = d.malloc(4 * 2 * 128 * 128)
+
+    def convolve(n):
+        return ctx.lib.fz_psf_convolve_dev(ctx.h, n, n, 2, maps, out, 0, None)
+
+    assert convolve(64) == 0
+    for fail in range(3):           # taps, operands, nothing
+        d.lib.double_fail_after(fail)
+        rc = convolve(70)
+        assert (rc != 0) == (fail < 2), (fail, rc)
+        d.lib.double_fail_after(-1)
+        for n in (64, 70, 64):
+            assert convolve(n) == 0
+    assert len(d.seen) == 11 and all("psf_split" in n and frag for n, frag in d.seen), d.seen
+
+
+CASES = [n[5:] for n in list(globals()) if n.startswith("case_")]
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_host(case):
+    if not os.path.exists(LIB):
+        pytest.skip("library not built")
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), case], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+if __name__ == "__main__":
+    sys.path[:0] = [ROOT, os.path.join(ROOT, "tests")]
+    import hostdouble
+    globals()["case_" + sys.argv[1]]()
