@@ -1029,7 +1029,21 @@ __global__ void __launch_bounds__(RT_WAVE * NW) rt_kernel(RtArgs a, NodeArgs nd,
   float* eqv = nullptr;
   if constexpr (NODES)
     eqv = nd.eqv + (a.items ? (long)nd.np * nd.nstk * (sbase / 4) : (long)col * nd.np * nd.nstk * snumw) + lo;
-  if (a.status && a.status[col] != 0) {
+  // Another workgroup of the column may set its status during this launch (below):
+  // a team takes its first wave's reading, so that its waves agree on what they do.
+  bool failed;
+  if constexpr (NW > 1) {
+    __shared__ unsigned long long bad;
+    if (wv == 0) {
+      const unsigned long long m = __ballot(a.status && a.status[col] != 0);
+      if (lane == 0) bad = m;
+    }
+    __syncthreads();
+    failed = (bad >> lane) & 1;
+  } else {
+    failed = a.status && a.status[col] != 0;
+  }
+  if (failed) {
     if (live && wv == 0) {
       for (int s = 0; s < 4; ++s) a.stokes[sbase + (long)s * snumw + lo] = __builtin_nanf("");
       if constexpr (NODES)

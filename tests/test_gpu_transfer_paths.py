@@ -85,3 +85,35 @@ def test_contraction_against_general_path(gpu_ctx, cpu, nodes, invstk, ncol):
             assert np.all(np.abs(eqv[:, j0 + j] - ref) <= tol), (name, j)
         j0 += nodes[name]
     assert j0 == np_
+
+
+@pytest.mark.parametrize("ncol,mode", [(3, gpu.RF_NONE), (3, gpu.RF_SPHERICAL), (40, gpu.RF_CARTESIAN),
+                                       (120, gpu.RF_SPHERICAL)])
+def test_column_that_fails_in_one_region(gpu_ctx, ncol, mode):
+    """A column whose profiles overflow in one region only (1e9 G, a line without Zeeman
+    splitting in the other) is flagged.  Workgroups of its other region that start later than
+    that return NaN, the others the region's own result, a whole team either way; the
+    other columns, some of whose lanes share its waves, keep their bits."""
+    import torch
+    ls = lines.setup([((4,), 150, -600.0, 8.0), ((5,), 150, -600.0, 8.0)])
+    for k, v in dict(sl=2.0, ll=3.0, jl=1.0, su=2.0, lu=2.0, ju=0.0).items():     # 5F1 - 5D0: g = 0
+        setattr(ls.lines[ls.regions[0].lines[0]], k, v)
+    one = lines.LineSetup([ls.lines[ls.regions[0].lines[0]]], [lines.Region([0], 150, -600.0, 8.0)])
+    d = cube(gpu_ctx, ls, ncol, 33)
+    d[7, :, 1] = 1e9
+    good = [i for i in range(ncol) if i != 1]
+    st, jac, status = gpu_ctx.forward_torch(d.clone(), mode)
+    sg, jg, s0 = gpu_ctx.forward_torch(d[:, :, good].contiguous(), mode)
+    torch.cuda.synchronize()
+    assert int(s0.max()) == 0 and status.tolist() == [2 if i == 1 else 0 for i in range(ncol)]
+    assert torch.equal(st[good], sg) and (jac is None or torch.equal(jac[good], jg))
+    assert bool(torch.isnan(st[1, :, 150:]).all())
+    gain = gpu_ctx.gain_hsra()
+    gpu_ctx.configure(one, np.arange(33) * (1200.0 / 33))
+    gpu_ctx.set_gain(gain[:, :150])
+    s1, _, st1 = gpu_ctx.forward_torch(d[:, :, 1:2].contiguous(), gpu.RF_NONE)
+    assert int(st1.max()) == 0
+    got, ref = st[1, :, :150], s1[0]
+    nan = torch.isnan(got)
+    assert torch.equal(got[~nan], ref[~nan])
+    assert torch.equal(nan, nan[:1].expand_as(nan))       # all four Stokes parameters of a wavelength
