@@ -97,3 +97,17 @@ def test_taps_outside_the_split(gpu_ctx):
     got = run(gpu_ctx, psf, maps, False)
     ref, mag = reference(psf, maps, False)
     assert np.all(np.abs(got - ref) <= (21 * 7 + 8) * 2.0 ** -24 * mag)
+
+
+@pytest.mark.parametrize("ein,etap", [(-98, 0), (-90, -30), (-60, -60), (-95, -45), (-98, -98)])
+def test_small_products(gpu_ctx, ein, etap):
+    """Operands inside the split's range whose products, or the products of
+    their parts, are subnormal: as exact as sums of FP32 products."""
+    rng = np.random.default_rng(4)
+    psf = rng.uniform(0.6, 1.0, (31, 9)) * 2.0 ** etap
+    maps = (rng.uniform(0.6, 1.0, (2, 64, 70)) * rng.choice([-1.0, 1.0], (2, 64, 70)) * 2.0 ** ein)
+    maps = maps.astype(np.float32).astype(np.float64)
+    got = run(gpu_ctx, psf, maps, False)
+    ref, mag = reference(psf, maps, False)
+    # the bound of ordinary operands, and a rounding at the subnormal spacing for each of six products a tap
+    assert np.all(np.abs(got - ref) <= (31 * 9 + 8) * 2.0 ** -24 * mag + 6 * 31 * 9 * 2.0 ** -149)
