@@ -1824,29 +1824,38 @@ struct MlpState {
   double* coefs = nullptr;  // [nz][nj] hat basis
   float* loss = nullptr;
   long step = 0;
-  int cap = 0;              // rows the work buffers hold; with the gradient's, gcap
-  int gcap = 0;
-  bf16 *X = nullptr, *XT = nullptr;
-  bf16 *act = nullptr, *actT = nullptr;   // [nl] of frag_size(cap, nh)
+  // work buffers of the forward pass for cap rows, and what the gradient needs besides for
+  // gcap; each only grows, so that batches of different sizes in turn allocate nothing
+  int cap = 0, gcap = 0;
+  bf16 *X = nullptr, *act = nullptr;      // act: [nl] of frag_size(cap, nh)
+  bf16 *XT = nullptr, *actT = nullptr;
   bf16 *dZ = nullptr, *dZT = nullptr;     // two of the widest layer; every layer's
   float *csum = nullptr, *partial = nullptr;
   size_t act_stride() const { return frag_size(cap, nh); }
-  size_t dzt_stride() const { return frag_size(std::max(nh, nout), cap); }
-  size_t csum_stride() const { return (size_t)pad32(cap) / 16 * pad32(std::max(nh, nout)); }
+  size_t actt_stride() const { return frag_size(nh, gcap); }
+  size_t dz_stride() const { return frag_size(gcap, std::max(nh, nout)); }
+  size_t dzt_stride() const { return frag_size(std::max(nh, nout), gcap); }
+  size_t csum_stride() const { return (size_t)pad32(gcap) / 16 * pad32(std::max(nh, nout)); }
   void release() {
-    release_work();
+    release_forward();
+    release_gradient();
     void* ps[] = {w, g, m1, m2, wb, norms, pinv, coefs, loss};
     for (void* q : ps)
       if (q) (void)hipFree(q);
     *this = MlpState();
   }
-  void release_work() {
-    void* ps[] = {X, XT, act, actT, dZ, dZT, csum, partial};
-    for (void* q : ps)
+  void release_forward() {
+    for (void* q : {(void*)X, (void*)act})
       if (q) (void)hipFree(q);
-    X = XT = act = actT = dZ = dZT = nullptr;
+    X = act = nullptr;
+    cap = 0;
+  }
+  void release_gradient() {
+    for (void* q : {(void*)XT, (void*)actT, (void*)dZ, (void*)dZT, (void*)csum, (void*)partial})
+      if (q) (void)hipFree(q);
+    XT = actT = dZ = dZT = nullptr;
     csum = partial = nullptr;
-    cap = gcap = 0;
+    gcap = 0;
   }
 };
 
@@ -4526,24 +4535,26 @@ uint64_t splitmix64(uint64_t& x) {
 // Work buffers for n rows of the forward pass and, with grad, of the gradient.
 int mlp_work(fz_ctx* c, int n, bool grad) {
   MlpState& M = c->mlp;
-  if ((grad ? M.gcap : M.cap) >= n) return FZ_OK;
-  M.release_work();
-  M.cap = n;
-  bool ok = hipMalloc(&M.X, sizeof(bf16) * frag_size(n, M.nin)) == hipSuccess &&
-            hipMalloc(&M.act, sizeof(bf16) * M.act_stride() * M.nl) == hipSuccess;
-  if (grad)
-    ok = ok && hipMalloc(&M.XT, sizeof(bf16) * frag_size(M.nin, n)) == hipSuccess &&
-         hipMalloc(&M.actT, sizeof(bf16) * frag_size(M.nh, n) * M.nl) == hipSuccess &&
-         hipMalloc(&M.dZ, sizeof(bf16) * 2 * frag_size(n, std::max(M.nh, M.nout))) == hipSuccess &&
+  bool ok = true;
+  if (M.cap < n) {
+    M.release_forward();
+    M.cap = n;
+    ok = hipMalloc(&M.X, sizeof(bf16) * frag_size(n, M.nin)) == hipSuccess &&
+         hipMalloc(&M.act, sizeof(bf16) * M.act_stride() * M.nl) == hipSuccess;
+    if (!ok) M.release_forward();
+  }
+  if (ok && grad && M.gcap < n) {
+    M.release_gradient();
+    M.gcap = n;
+    ok = hipMalloc(&M.XT, sizeof(bf16) * frag_size(M.nin, n)) == hipSuccess &&
+         hipMalloc(&M.actT, sizeof(bf16) * M.actt_stride() * M.nl) == hipSuccess &&
+         hipMalloc(&M.dZ, sizeof(bf16) * 2 * M.dz_stride()) == hipSuccess &&
          hipMalloc(&M.dZT, sizeof(bf16) * M.dzt_stride() * (M.nl + 1)) == hipSuccess &&
          hipMalloc(&M.csum, sizeof(float) * M.csum_stride() * (M.nl + 1)) == hipSuccess &&
          hipMalloc(&M.partial, sizeof(float) * 4 * (pad32(n) / 32) * (pad32(M.nout) / 32)) == hipSuccess;
-  if (!ok) {
-    M.release_work();
-    return set_err(c, FZ_ENOMEM, "device allocation failed (network work buffers)");
+    if (!ok) M.release_gradient();
   }
-  if (grad) M.gcap = n;
-  return FZ_OK;
+  return ok ? FZ_OK : set_err(c, FZ_ENOMEM, "device allocation failed (network work buffers)");
 }
 
 // A product of the network: D[m][n], A [N][K] and B [M][K] in operand order
@@ -4580,7 +4591,7 @@ void mlp_forward_rows(MlpState& M, int n, float* y, bool grad, hipStream_t st) {
     g.bias = M.w + M.boff[l];
     if (l < M.nl) {
       g.Cb = M.act + l * M.act_stride();
-      if (grad) g.CbT = M.actT + l * frag_size(M.nh, M.cap);
+      if (grad) g.CbT = M.actT + l * M.actt_stride();
       mlp_layer<MLP_HIDDEN>(g, none, st);
     } else {
       g.Cf = y;
@@ -4599,7 +4610,7 @@ void mlp_backward_rows(MlpState& M, int n, const float* d_t, const int32_t* d_id
   memset(&dw, 0, sizeof(dw));
   const bf16* dz = nullptr;
   for (int l = M.nl; l >= 0; --l) {
-    bf16* out = M.dZ + (l & 1) * frag_size(M.cap, std::max(M.nh, M.nout));
+    bf16* out = M.dZ + (l & 1) * M.dz_stride();
     bf16* outT = M.dZT + l * M.dzt_stride();
     GemmArgs g;
     if (l == M.nl)         // Y = A W^T + b and dY from it
@@ -4618,7 +4629,7 @@ void mlp_backward_rows(MlpState& M, int n, const float* d_t, const int32_t* d_id
     dz = out;
     // dW_l[o][k] = sum_m dZ_l[m][o] A_l[m][k]
     GemmArgs& h = dw.g[l];
-    h = mlp_gemm(l == 0 ? M.XT : M.actT + (l - 1) * frag_size(M.nh, M.cap), outT, M.dout[l], M.din[l], n);
+    h = mlp_gemm(l == 0 ? M.XT : M.actT + (l - 1) * M.actt_stride(), outT, M.dout[l], M.din[l], n);
     h.Cf = grad + M.woff[l];
     dw.csum[l] = g.csum;
     dw.bg[l] = grad + M.boff[l];

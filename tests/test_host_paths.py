@@ -37,6 +37,27 @@ def case_psf_failed_operands():
     assert len(d.seen) == 11 and all("psf_split" in n and frag for n, frag in d.seen), d.seen
 
 
+def case_network_buffers_only_grow():
+    """Training batches between forward passes of a large map allocate
+    nothing once both sizes have been seen, in either order."""
+    import numpy as np
+    from firtez_dz_amd import lines
+    d = hostdouble.load()
+    ctx = d.gpu.Context(0)
+    ctx.configure(lines.fe6301_6302(nwave=16), np.arange(32) * 30.0)
+    x = d.malloc(1 << 30)
+    for sizes in ((5000, 100), (100, 5000), (70000, 70000)):
+        ctx.mlp_create(64, 513, 2, 3)
+        def both():
+            assert ctx.lib.fz_mlp_forward_dev(ctx.h, sizes[0], x, None, x, None) == 0
+            assert ctx.lib.fz_mlp_gradient_dev(ctx.h, sizes[1], x, x, None, x, x, None) == 0
+        both()
+        n, held = d.lib.double_mallocs(), d.lib.double_held()
+        for _ in range(3):
+            both()
+        assert (d.lib.double_mallocs(), d.lib.double_held()) == (n, held), sizes
+
+
 CASES = [n[5:] for n in list(globals()) if n.startswith("case_")]
 
 
