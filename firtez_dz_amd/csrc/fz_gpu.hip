@@ -2588,6 +2588,13 @@ static size_t rt_scratch_per_lane(const fz_ctx* c, int rf_mode) {
   return nz * (c->hydro ? 8 : 4);
 }
 
+// columns of one radiative-transfer launch: the configured tile, at most as many as
+// keep its lanes (rounded up to waves) below 2^29, so that the kernel's lane
+// numbers and the launch's work-items, four times as many with teams, stay within 32 bits
+static int rt_tile(const fz_ctx* c, int ncol) {
+  return std::min(std::min(c->tile, ncol), (1 << 29) / (RT_WAVE * c->cfg.nbpc));
+}
+
 static int rf_nparam(int rf_mode) {
   return rf_mode == FZ_RF_SPHERICAL ? 5
          : rf_mode == FZ_RF_CARTESIAN ? 7
@@ -2836,7 +2843,7 @@ static int forward_impl(fz_ctx* c, int ncol, float* d_atm, int rf_mode, float* d
   // columns per radiative-transfer launch: the configured tile, fewer where
   // its scratch would pass 48 GiB
   const size_t per_col = sizeof(float) * rt_scratch_per_lane(c, rf_mode) * g.numw;
-  int tile = std::min(c->tile, ncol);
+  int tile = rt_tile(c, ncol);
   if (per_col) tile = (int)std::max<size_t>(1, std::min<size_t>((size_t)tile, ((size_t)48 << 30) / per_col));
   if (rf_mode != FZ_RF_NONE) {
     r = ensure(c, &c->d_scratch, &c->scratch_cap, per_col * tile);
@@ -3449,7 +3456,7 @@ int fz_forward_nodes_dev(fz_ctx* c, int ncol, float* d_atm, float* d_stokes, flo
   // wavelengths of its columns: ragged with per-pixel windows)
   const size_t per_w = sizeof(float) * ((size_t)nslot * g.nz * 4 + rt_scratch_per_lane(c, rf));
   const size_t budget = (size_t)24 << 30;
-  int tile = std::min(c->tile, ncol);
+  int tile = rt_tile(c, ncol);
   size_t wmax = 0;
   for (;;) {
     wmax = 0;

@@ -58,6 +58,38 @@ def case_network_buffers_only_grow():
         assert (d.lib.double_mallocs(), d.lib.double_held()) == (n, held), sizes
 
 
+class RtArgs(ctypes.Structure):     # the first members of the transfer's argument
+    _fields_ = [("ncol", ctypes.c_int), ("col0", ctypes.c_int), ("ntile", ctypes.c_int)]
+
+
+def case_transfer_indices_in_32_bits():
+    """A transfer launch numbers its lanes in 32 bits and its work-items fit
+    the launch, whatever tile is set; the launches cover the map once."""
+    import numpy as np
+    from firtez_dz_amd import gpu, lines
+    d = hostdouble.load()
+    ctx = d.gpu.Context(0)
+    d.watch["rt_kernel"] = lambda x: (x.arg(0, RtArgs), x.grid * x.block)
+    for widths, ncol, nodes in (((8192,), 262144, False), ((1024,) * 8, 262145, False), ((1,), 4000000, False),
+                                ((8192,), 262144, True)):
+        ctx.configure(lines.setup([((4,), n, -1.0 * n, 2.0) for n in widths]), np.arange(2) * 30.0)
+        ctx._check(ctx.lib.fz_set_tile(ctx.h, 1 << 24, 64), "tile")
+        atm, stokes = d.malloc(12 * 2 * 4 * ncol), d.malloc(16 * ctx.numw * ncol)
+        d.seen.clear()
+        if nodes:
+            ctx.set_inversion(gpu.inversion({"T": 1}))
+            assert ctx.lib.fz_forward_nodes_dev(ctx.h, ncol, atm, stokes, stokes, None, None) == 0
+        else:
+            assert ctx.lib.fz_forward_dev(ctx.h, ncol, atm, gpu.RF_NONE, stokes, None, None, None) == 0
+        d.free(atm)
+        d.free(stokes)
+        col = 0
+        for a, items in d.seen:
+            assert a.col0 == col and a.ntile > 0 and a.ntile * max(widths) + 64 < 2 ** 31 and items < 2 ** 32
+            col += a.ntile
+        assert col == ncol
+
+
 CASES = [n[5:] for n in list(globals()) if n.startswith("case_")]
 
 
