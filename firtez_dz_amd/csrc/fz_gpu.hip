@@ -47,11 +47,12 @@ constexpr int RT_WAVE = 64;   // wavelengths per radiative-transfer workgroup (o
 constexpr int NATM = 12;
 enum { A_T = 0, A_PG, A_RHO, A_PEL, A_MU, A_BX, A_BY, A_BZ, A_VX, A_VY, A_VZ, A_TAU };
 
-// Per-height record of a column, rec floats at micro[(k * ncol + col) * rec]:
+// Per-height record of a column, rec floats at micro[(k * rncol + col - rcol0) * rec]
+// (columns rcol0 .. rcol0 + rncol - 1 are held):
 // a head of REC_HEAD floats, then per region REC_REG floats and REC_SLOT per
 // line of the region, each part a whole number of float4, so that a wave
 // copies the heights it needs next into LDS with 16-byte loads and every lane
-// reads them from there.  kappa_5000 is kept apart, [nz][ncol] after the
+// reads them from there.  kappa_5000 is kept apart, [nz][rncol] after the
 // records (tau_kernel reads it along the columns).
 //   head    flag, T, 1/T, 1/sqrt(T) | v_z, |B|, sgf/2, cgf/4 | qf/2, qf/4, cg/2, sg |
 //           cos 2phi, sin 2phi, sg cg, line-optical-depth factor | d|B|/dB (3), d gamma/dB (3), d phi/dBx, dBy
@@ -128,6 +129,7 @@ __constant__ Cfg c_cfg;
 // (stopping rule 1e-4, warm start).
 struct MicroTile {
   int ncol, col0, ntile, der;
+  int rcol0, rncol;   // columns held in micro
   float* atm;
   float* micro;
   double* sbuf;    // [nz][92][4][ntile]
@@ -382,7 +384,7 @@ __global__ void __launch_bounds__(256, 2) opac_kernel(MicroTile a) {
   const int k = (int)(t / a.ntile), ct = (int)(t - (long)k * a.ntile), col = a.col0 + ct;
   if (a.status[col] != 0) return;
   const long cs = a.ncol, ps = (long)nz * a.ncol;
-  float4* const R = reinterpret_cast<float4*>(a.micro + ((long)k * a.ncol + col) * c_cfg.rec);
+  float4* const R = reinterpret_cast<float4*>(a.micro + ((long)k * a.rncol + col - a.rcol0) * c_cfg.rec);
   const float* at = a.atm + k * cs + col;
   const float Tf = at[A_T * ps], vz = at[A_VZ * ps], iT = 1.0f / Tf, rsT = rsqrtf(Tf);
   {
@@ -428,7 +430,7 @@ __global__ void __launch_bounds__(256, 2) opac_kernel(MicroTile a) {
     const double kc5 = kc[0] / nh * (1.0 / MAMU);
     const bool bnd = (k == 0) || (kc5 >= 2.0e10);     // forward.f90:884,931,971
     R[0] = {bnd ? 1.0f : 0.0f, Tf, iT, rsT};
-    a.micro[ps * c_cfg.rec + k * cs + col] = (float)kc5;
+    a.micro[(long)nz * a.rncol * c_cfg.rec + (long)k * a.rncol + col - a.rcol0] = (float)kc5;
     // the opacities are formed wherever kc5 is below the threshold, the
     // bottom height included (its absorption matrix feeds LINE OPTICAL DEPTH,
     // forward.f90:931-968, while the transfer takes it as the boundary)
@@ -471,18 +473,19 @@ __global__ void __launch_bounds__(64) tau_kernel(MicroTile a) {
   const int nz = c_cfg.nz, col = a.col0 + ct;
   if (a.status[col] != 0) return;
   const long cs = a.ncol, ps = (long)nz * a.ncol;
-  const float* kc5 = a.micro + ps * c_cfg.rec;
+  const float* kc5 = a.micro + (long)nz * a.rncol * c_cfg.rec + col - a.rcol0;
+  const long rs = a.rncol;
   // log tau_5000 by the REAL(4) trapezoid of forward.f90:1000-1006 (z in km)
   float tau = 1e-9f;
   a.atm[A_TAU * ps + (nz - 1) * cs + col] = log10f(tau);
   // eight heights' loads together: the trapezoid is a chain, its terms are not
-  float xn = kc5[(nz - 1) * cs + col] * a.atm[A_RHO * ps + (nz - 1) * cs + col];
+  float xn = kc5[(nz - 1) * rs] * a.atm[A_RHO * ps + (nz - 1) * cs + col];
   for (int k0 = nz - 2; k0 >= 0; k0 -= 8) {
     float q[8], r[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int k = max(k0 - i, 0);
-      q[i] = kc5[k * cs + col];
+      q[i] = kc5[k * rs];
       r[i] = a.atm[A_RHO * ps + k * cs + col];
     }
 #pragma unroll
@@ -641,6 +644,7 @@ struct RtArgs {
   int ncol;          // columns in the whole cube (strides of atm/micro)
   int col0;          // first column of this launch
   int ntile;         // columns in this launch
+  int rcol0, rncol;  // columns held in micro
   const float* atm;
   const float* micro;
   const float* gain; // [numw][4]
@@ -854,7 +858,7 @@ __global__ void __launch_bounds__(256) taulin_kernel(RtArgs a, float* __restrict
   const long ps = (long)nz * a.ncol, cs = a.ncol;
   float* o = out + (long)col * nz * numw + l;
   for (int k = 0; k < nz; ++k) {
-    const float4* R = reinterpret_cast<const float4*>(a.micro + ((long)k * a.ncol + col) * c_cfg.rec);
+    const float4* R = reinterpret_cast<const float4*>(a.micro + ((long)k * a.rncol + col - a.rcol0) * c_cfg.rec);
     const float fac = R[3].w;
     float kl = 0.f;
     if (fac != 0.f) {
@@ -1056,6 +1060,7 @@ __global__ void __launch_bounds__(RT_WAVE * NW) rt_kernel(RtArgs a, NodeArgs nd,
   const int nc = PACK ? uniform(__shfl(ct, 63) - ct0 + 1) : 1;
   const int rs4 = (REC_HEAD + REC_REG + REC_SLOT * c_cfg.reg_nblend[r]) / 4;   // float4 per (height, column) in LDS
   const float4* grec = reinterpret_cast<const float4*>(a.micro);
+  const int rc0 = a.col0 + ct0 - a.rcol0;
   const int rec4 = c_cfg.rec / 4, roff4 = (c_cfg.reg_rec[r] - REC_HEAD) / 4;
   // heights k0 .. k0 + n - 1 of the wave's columns into LDS: half a wave per
   // record (rs4 <= 32)
@@ -1070,7 +1075,7 @@ __global__ void __launch_bounds__(RT_WAVE * NW) rt_kernel(RtArgs a, NodeArgs nd,
       ++h;
     }
     for (int p = 2 * wv + (lane >> 5); p < np; p += 2 * NW) {
-      if (f < rs4) lds[p * rs4 + f] = grec[((long)(k0 + h) * a.ncol + a.col0 + ct0 + c) * rec4 + src];
+      if (f < rs4) lds[p * rs4 + f] = grec[((long)(k0 + h) * a.rncol + rc0 + c) * rec4 + src];
       c += 2 * NW;
       while (c >= nc) {
         c -= nc;
@@ -2670,7 +2675,24 @@ static int launch_rt(fz_ctx* c, int rf_mode, RtArgs a, hipStream_t st, int nitem
   return FZ_OK;
 }
 
-// Microphysics over all columns, tile by tile; status[ncol] receives each
+// Columns whose records are held at a time: all of them, or, where these would
+// pass a third of the memory that is free or holds records already, as many
+// as that third takes; a larger map is then worked through in slabs of so many
+// columns (microphysics and transfer of one after the other).  A record is 308
+// bytes per height with two lines, 30 KB per column of 96 heights.
+static int record_slab(const fz_ctx* c, int ncol) {
+  const size_t per = sizeof(float) * (size_t)(c->cfg.rec + 1) * c->cfg.nz, held = c->micro_cap / per;
+  size_t freeb = 0, totb = 0;
+  if (held >= (size_t)ncol || hipMemGetInfo(&freeb, &totb) != hipSuccess) return ncol;
+  const size_t n = std::max(held, (freeb + c->micro_cap) / 3 / per);
+  return (int)std::max<size_t>(1, std::min<size_t>(n, (size_t)ncol));
+}
+
+static int ensure_records(fz_ctx* c, int slab) {
+  return ensure(c, &c->d_micro, &c->micro_cap, sizeof(float) * (size_t)(c->cfg.rec + 1) * c->cfg.nz * slab);
+}
+
+// Microphysics of columns cbeg .. cend - 1, tile by tile; status[ncol] receives each
 // column's FZ_E* code (the caller's array, or the context's own).  With
 // hydro, Pg is first re-integrated from the top (forward.f90:891-906) and the
 // EOS takes N_H and n_e from that integration; with physics == false only the
@@ -2724,8 +2746,7 @@ static int ensure_aux(fz_ctx* c, int n) {
 }
 
 static int run_micro(fz_ctx* c, int ncol, float* d_atm, int32_t** status, bool der, bool hydro, bool physics,
-                     hipStream_t st, int cbeg = 0, int cend = -1) {
-  if (cend < 0) cend = ncol;
+                     hipStream_t st, int cbeg, int cend, int rcol0, int rncol) {
   const int nz = c->cfg.nz;
   int32_t* stv = *status;
   if (!stv) {
@@ -2753,6 +2774,8 @@ static int run_micro(fz_ctx* c, int ncol, float* d_atm, int32_t** status, bool d
     a.col0 = c0;
     a.ntile = std::min(mt, cend - c0);
     a.der = (der && physics) ? 1 : 0;
+    a.rcol0 = rcol0;
+    a.rncol = rncol;
     a.atm = d_atm;
     a.micro = c->d_micro;
     a.sbuf = (double*)c->d_sbuf;
@@ -2838,19 +2861,20 @@ static int forward_impl(fz_ctx* c, int ncol, float* d_atm, int rf_mode, float* d
   HIPCHK(c, hipSetDevice(c->device));
   int r = upload_cfg(c);
   if (r) return r;
-  r = ensure(c, &c->d_micro, &c->micro_cap, sizeof(float) * (size_t)(g.rec + 1) * g.nz * ncol);
-  if (r) return r;
   // columns per radiative-transfer launch: the configured tile, fewer where
-  // its scratch would pass 48 GiB
+  // its scratch would pass 48 GiB; whole tiles to a slab of records
   const size_t per_col = sizeof(float) * rt_scratch_per_lane(c, rf_mode) * g.numw;
-  int tile = rt_tile(c, ncol);
+  int slab = record_slab(c, ncol), tile = std::min(rt_tile(c, ncol), slab);
   if (per_col) tile = (int)std::max<size_t>(1, std::min<size_t>((size_t)tile, ((size_t)48 << 30) / per_col));
+  if (slab < ncol) slab = slab / tile * tile;
+  r = ensure_records(c, slab);
+  if (r) return r;
   if (rf_mode != FZ_RF_NONE) {
     r = ensure(c, &c->d_scratch, &c->scratch_cap, per_col * tile);
     if (r) return r;
   }
   const int ntiles = (ncol + tile - 1) / tile;
-  const bool ovl = c->overlap && ntiles > 1 && !c->win_on;
+  const bool ovl = c->overlap && ntiles > 1 && !c->win_on && slab == ncol;
   if (c->prof) HIPCHK(c, hipEventRecord(c->ev[0], st));
   if (ovl) {
     // the microphysics of RT tile i+1 runs on the second stream while tile
@@ -2868,45 +2892,53 @@ static int forward_impl(fz_ctx* c, int ncol, float* d_atm, int rf_mode, float* d
     HIPCHK(c, hipStreamWaitEvent(c->aux, c->tev[0], 0));
     for (int i = 0; i < ntiles; ++i) {
       r = run_micro(c, ncol, d_atm, &d_status, rf_mode != FZ_RF_NONE, c->hydro, true, c->aux, i * tile,
-                    std::min(ncol, (i + 1) * tile));
+                    std::min(ncol, (i + 1) * tile), 0, ncol);
       if (r) return r;
       HIPCHK(c, hipEventRecord(c->tev[i + 1], c->aux));
     }
-  } else {
-    r = run_micro(c, ncol, d_atm, &d_status, rf_mode != FZ_RF_NONE, c->hydro, true, st);
-    if (r) return r;
   }
-  if (ovl) HIPCHK(c, hipStreamWaitEvent(st, c->tev[1], 0));
-  // with the overlap, "microphysics" is the first tile's, which nothing hides
-  if (c->prof) HIPCHK(c, hipEventRecord(c->ev[1], st));
   c->rt_launches = 0;
-  for (int c0 = 0; c0 < ncol; c0 += tile) {
-    if (ovl && c0 > 0) HIPCHK(c, hipStreamWaitEvent(st, c->tev[c0 / tile + 1], 0));
-    RtArgs a;
-    a.ncol = ncol;
-    a.col0 = c0;
-    a.ntile = std::min(tile, ncol - c0);
-    a.atm = d_atm;
-    a.micro = c->d_micro;
-    a.gain = c->d_gain;
-    a.status = d_status;
-    a.stokes = d_stokes;
-    a.jac = d_jac;
-    a.jcol0 = 0;
-    a.scratch = c->d_scratch;
-    a.items = nullptr;
-    a.poff = nullptr;
-    a.fs = d_full;
-    int nit = 0;
-    if (c->win_on) {
-      a.items = c->d_items + c->h_item_first[c0];
-      a.poff = c->d_poff;
-      nit = c->h_item_first[c0 + a.ntile] - c->h_item_first[c0];
+  for (int s0 = 0; s0 < ncol; s0 += slab) {
+    const int s1 = std::min(ncol, s0 + slab);
+    if (!ovl) {
+      r = run_micro(c, ncol, d_atm, &d_status, rf_mode != FZ_RF_NONE, c->hydro, true, st, s0, s1, s0, slab);
+      if (r) return r;
+    } else {
+      HIPCHK(c, hipStreamWaitEvent(st, c->tev[1], 0));
     }
-    r = launch_rt(c, rf_mode, a, st, nit);
-    if (r) return r;
-    HIPCHK(c, hipGetLastError());
-    c->rt_launches++;
+    // with the overlap, "microphysics" is the first tile's, which nothing
+    // hides, and with several slabs the first one's
+    if (c->prof && s0 == 0) HIPCHK(c, hipEventRecord(c->ev[1], st));
+    for (int c0 = s0; c0 < s1; c0 += tile) {
+      if (ovl && c0 > 0) HIPCHK(c, hipStreamWaitEvent(st, c->tev[c0 / tile + 1], 0));
+      RtArgs a;
+      a.ncol = ncol;
+      a.col0 = c0;
+      a.ntile = std::min(tile, s1 - c0);
+      a.rcol0 = s0;
+      a.rncol = slab;
+      a.atm = d_atm;
+      a.micro = c->d_micro;
+      a.gain = c->d_gain;
+      a.status = d_status;
+      a.stokes = d_stokes;
+      a.jac = d_jac;
+      a.jcol0 = 0;
+      a.scratch = c->d_scratch;
+      a.items = nullptr;
+      a.poff = nullptr;
+      a.fs = d_full;
+      int nit = 0;
+      if (c->win_on) {
+        a.items = c->d_items + c->h_item_first[c0];
+        a.poff = c->d_poff;
+        nit = c->h_item_first[c0 + a.ntile] - c->h_item_first[c0];
+      }
+      r = launch_rt(c, rf_mode, a, st, nit);
+      if (r) return r;
+      HIPCHK(c, hipGetLastError());
+      c->rt_launches++;
+    }
   }
   r = run_lsf(c, d_stokes, (long)ncol * 4, st);
   if (r) return r;
@@ -2939,21 +2971,25 @@ int fz_line_tau_dev(fz_ctx* c, int ncol, float* d_atm, float* d_tau, int32_t* d_
   HIPCHK(c, hipSetDevice(c->device));
   int r = upload_cfg(c);
   if (r) return r;
-  r = ensure(c, &c->d_micro, &c->micro_cap, sizeof(float) * (size_t)(g.rec + 1) * g.nz * ncol);
+  const int slab = record_slab(c, ncol);
+  r = ensure_records(c, slab);
   if (r) return r;
-  r = run_micro(c, ncol, d_atm, &d_status, false, c->hydro, true, st);
-  if (r) return r;
-  RtArgs a = {};
-  a.ncol = ncol;
-  a.col0 = 0;
-  a.ntile = ncol;
-  a.atm = d_atm;
-  a.micro = c->d_micro;
-  a.gain = c->d_gain;
-  a.status = d_status;
-  const long n = (long)ncol * g.numw;
-  hipLaunchKernelGGL(taulin_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, d_tau);
-  HIPCHK(c, hipGetLastError());
+  for (int s0 = 0; s0 < ncol; s0 += slab) {
+    RtArgs a = {};
+    a.ncol = ncol;
+    a.col0 = a.rcol0 = s0;
+    a.ntile = std::min(slab, ncol - s0);
+    a.rncol = slab;
+    r = run_micro(c, ncol, d_atm, &d_status, false, c->hydro, true, st, s0, s0 + a.ntile, s0, slab);
+    if (r) return r;
+    a.atm = d_atm;
+    a.micro = c->d_micro;
+    a.gain = c->d_gain;
+    a.status = d_status;
+    const long n = (long)a.ntile * g.numw;
+    hipLaunchKernelGGL(taulin_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, d_tau);
+    HIPCHK(c, hipGetLastError());
+  }
   return FZ_OK;
 }
 
@@ -3131,7 +3167,7 @@ int fz_hydrostatic_dev(fz_ctx* c, int ncol, float* d_atm, int32_t* d_status, voi
   HIPCHK(c, hipSetDevice(c->device));
   int r = upload_cfg(c);
   if (r) return r;
-  r = run_micro(c, ncol, d_atm, &d_status, false, true, false, (hipStream_t)stream);
+  r = run_micro(c, ncol, d_atm, &d_status, false, true, false, (hipStream_t)stream, 0, ncol, 0, ncol);
   return r;
 }
 
@@ -3442,8 +3478,6 @@ int fz_forward_nodes_dev(fz_ctx* c, int ncol, float* d_atm, float* d_stokes, flo
   HIPCHK(c, hipSetDevice(c->device));
   int r = upload_cfg(c);
   if (r) return r;
-  r = ensure(c, &c->d_micro, &c->micro_cap, sizeof(float) * (size_t)(g.rec + 1) * g.nz * ncol);
-  if (r) return r;
   // the P0 slot is synthesised only when P0 is inverted; the Pg and rho
   // slots only when they are inverted or feed another response (P0, HYDROSTATIC)
   const bool p0 = c->lm_p0;
@@ -3456,7 +3490,7 @@ int fz_forward_nodes_dev(fz_ctx* c, int ncol, float* d_atm, float* d_stokes, flo
   // wavelengths of its columns: ragged with per-pixel windows)
   const size_t per_w = sizeof(float) * ((size_t)nslot * g.nz * 4 + rt_scratch_per_lane(c, rf));
   const size_t budget = (size_t)24 << 30;
-  int tile = rt_tile(c, ncol);
+  int slab = record_slab(c, ncol), tile = std::min(rt_tile(c, ncol), slab);
   size_t wmax = 0;
   for (;;) {
     wmax = 0;
@@ -3467,6 +3501,9 @@ int fz_forward_nodes_dev(fz_ctx* c, int ncol, float* d_atm, float* d_stokes, flo
     if (wmax * per_w <= budget || tile == 1) break;
     tile = std::max(1, (int)((double)tile * (double)budget / (double)(wmax * per_w)));
   }
+  if (slab < ncol) slab = slab / tile * tile;
+  r = ensure_records(c, slab);
+  if (r) return r;
   r = ensure(c, &c->d_scratch, &c->scratch_cap, sizeof(float) * rt_scratch_per_lane(c, rf) * wmax);
   if (r) return r;
   if (nslot) {
@@ -3474,9 +3511,6 @@ int fz_forward_nodes_dev(fz_ctx* c, int ncol, float* d_atm, float* d_stokes, flo
     if (r) return r;
   }
   if (c->prof) HIPCHK(c, hipEventRecord(c->ev[0], st));
-  r = run_micro(c, ncol, d_atm, &d_status, true, c->hydro, true, st);
-  if (r) return r;
-  if (c->prof) HIPCHK(c, hipEventRecord(c->ev[1], st));
   c->rt_launches = 0;
   EqvArgs e;
   e.nz = g.nz;
@@ -3510,11 +3544,19 @@ int fz_forward_nodes_dev(fz_ctx* c, int ncol, float* d_atm, float* d_stokes, flo
   for (int p = 0; p < 5; ++p) nd.last[p] = -1;
   for (int ip = 0; ip < e.nparam; ++ip)
     if (tbv) nd.last[TBV_SLOT[c->lm.par[ip]]] = e.j0[ip] + e.nj[ip] - 1;
-  for (int c0 = 0; c0 < ncol; c0 += tile) {
+  for (int c0 = 0, s0 = 0; c0 < ncol; c0 += tile) {
+    if (c0 % slab == 0) {
+      s0 = c0;
+      r = run_micro(c, ncol, d_atm, &d_status, true, c->hydro, true, st, s0, std::min(ncol, s0 + slab), s0, slab);
+      if (r) return r;
+      if (c->prof && s0 == 0) HIPCHK(c, hipEventRecord(c->ev[1], st));
+    }
     RtArgs a;
     a.ncol = ncol;
     a.col0 = c0;
     a.ntile = std::min(tile, ncol - c0);
+    a.rcol0 = s0;
+    a.rncol = slab;
     a.atm = d_atm;
     a.micro = c->d_micro;
     a.gain = c->d_gain;

@@ -35,6 +35,7 @@ class Double:
         self.watch = {}
         self.seen = []
         lib.double_held.restype = ctypes.c_size_t
+        lib.double_size.restype, lib.double_size.argtypes = ctypes.c_size_t, [ctypes.c_void_p]
         lib.double_mallocs.restype = ctypes.c_long
         lib.double_fail_after.argtypes = [ctypes.c_long]
         lib.double_budget.argtypes = [ctypes.c_size_t]

@@ -61,6 +61,12 @@ int hipFree(void* p) {
   return p ? 1 : 0;
 }
 
+size_t double_size(const void* p) {
+  for (int i = 0; i < nmem; ++i)
+    if (mem[i].p == p) return mem[i].n;
+  return 0;
+}
+
 /* copies of tables are made, whole maps are not */
 static int copy(void* d, const void* s, size_t n) {
   if (n <= ((size_t)64 << 20)) memcpy(d, s, n);

@@ -59,7 +59,12 @@ def case_network_buffers_only_grow():
 
 
 class RtArgs(ctypes.Structure):     # the first members of the transfer's argument
-    _fields_ = [("ncol", ctypes.c_int), ("col0", ctypes.c_int), ("ntile", ctypes.c_int)]
+    _fields_ = [(n, ctypes.c_int) for n in ("ncol", "col0", "ntile", "rcol0", "rncol")]
+
+
+class MicroTile(ctypes.Structure):  # and of the microphysics'
+    _fields_ = ([(n, ctypes.c_int) for n in ("ncol", "col0", "ntile", "der", "rcol0", "rncol")] +
+                [("atm", ctypes.c_void_p), ("micro", ctypes.c_void_p)])
 
 
 def case_transfer_indices_in_32_bits():
@@ -88,6 +93,49 @@ def case_transfer_indices_in_32_bits():
             assert a.col0 == col and a.ntile > 0 and a.ntile * max(widths) + 64 < 2 ** 31 and items < 2 ** 32
             col += a.ntile
         assert col == ncol
+
+
+def case_maps_whose_records_exceed_the_memory():
+    """Twelve million columns of 96 heights: model, profiles and the rest fit
+    the card, the records of all columns (355 GB) do not.  Every column's
+    records are written before they are read, inside their buffer."""
+    import numpy as np
+    from firtez_dz_amd import gpu, lines
+    d = hostdouble.load()
+    nz, ncol = 96, 12000000
+    ctx = d.gpu.Context(0)
+    d.watch = {"opac_kernel": lambda x: ("w", x.arg(0, MicroTile)), "tau_kernel": lambda x: ("w", x.arg(0, MicroTile)),
+               "rt_kernel": lambda x: ("r", x.arg(0, RtArgs)), "taulin": lambda x: ("r", x.arg(0, RtArgs))}
+    atm = d.malloc(12 * nz * 4 * ncol)
+    for call in ("synthesis", "nodes", "pressure", "line_tau", "small"):
+        if call == "small":
+            ncol = 300
+        ctx.configure(lines.fe6301_6302(nwave=2 if call == "line_tau" else 56), np.arange(nz) * 15.0)
+        out = d.malloc(4 * ncol * (nz * 2 if call == "line_tau" else 4 * 56))
+        eqv = d.malloc(4 * ncol * 4 * 56) if call in ("nodes", "pressure") else None
+        d.seen.clear()
+        if eqv:
+            ctx.set_inversion(gpu.inversion({"T": 1} if call == "nodes" else {"Pg": 1}))
+            rc = ctx.lib.fz_forward_nodes_dev(ctx.h, ncol, atm, out, eqv, None, None)
+            d.free(eqv)
+        elif call == "line_tau":
+            rc = ctx.lib.fz_line_tau_dev(ctx.h, ncol, atm, out, None, None)
+        else:
+            rc = ctx.lib.fz_forward_dev(ctx.h, ncol, atm, gpu.RF_NONE, out, None, None, None)
+        assert rc == 0, (call, ctx.lib.fz_last_error(ctx.h))
+        d.free(out)
+        held, done, written = (0, 0), 0, 0      # held: the columns now in the records
+        for kind, a in d.seen:
+            lo, hi = a.rcol0, a.rcol0 + a.rncol
+            assert a.ncol == ncol and lo <= a.col0 and a.col0 + a.ntile <= hi
+            if kind == "w":
+                assert d.lib.double_size(a.micro) >= 77 * 4 * nz * a.rncol
+                held = (min(held[0], a.col0) if held[0] >= lo else a.col0, a.col0 + a.ntile)
+                written = max(written, a.col0 + a.ntile)
+            else:
+                assert held[0] <= a.col0 and a.col0 + a.ntile <= held[1] and a.col0 == done, call
+                done += a.ntile
+        assert done == written == ncol, call
 
 
 CASES = [n[5:] for n in list(globals()) if n.startswith("case_")]
