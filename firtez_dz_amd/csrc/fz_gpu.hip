@@ -3301,6 +3301,7 @@ int fz_set_inversion(fz_ctx* c, const fz_inversion* inv, int* ifreep, int* nfreq
   if (!c->configured) return set_err(c, FZ_ECONFIG, "fz_configure first");
   const int nz = c->cfg.nz, numw = c->cfg.numw;
   LmArgs& L = c->lm;
+  c->inv_set = false;   // until every table is there
   L = LmArgs();
   L.nz = nz;
   L.numw = numw;
@@ -3469,6 +3470,8 @@ int fz_forward_nodes_dev(fz_ctx* c, int ncol, float* d_atm, float* d_stokes, flo
                          void* stream) {
   if (!c || !c->configured || ncol < 1 || !d_atm || !d_stokes || !d_eqv) return FZ_EARG;
   if (!c->inv_set) return set_err(c, FZ_ECONFIG, "fz_set_inversion first");
+  if (c->lm.nz != c->cfg.nz || c->lm.numw != c->cfg.numw)
+    return set_err(c, FZ_ECONFIG, "heights or wavelengths changed since fz_set_inversion");
   if (c->win_on) {
     if (ncol != c->win_ncol) return set_err(c, FZ_EARG, "column count differs from fz_set_windows");
     if (c->cfg.lsf_on) return set_err(c, FZ_ECONFIG, "per-pixel windows and an LSF together are not supported");

@@ -138,6 +138,47 @@ def case_maps_whose_records_exceed_the_memory():
         assert done == written == ncol, call
 
 
+def case_inversion_that_was_not_set():
+    """After a refused or failed fz_set_inversion nothing is launched from
+    what it left half set; the next one that succeeds holds again."""
+    import numpy as np
+    from firtez_dz_amd import gpu, lines
+    d = hostdouble.load()
+    ctx = d.gpu.Context(0)
+    ctx.configure(lines.fe6301_6302(nwave=16), np.arange(32) * 30.0)
+    atm, out, eqv = (d.malloc(1 << 24) for _ in range(3))
+    good = gpu.inversion({"T": 4, "Bz": 2, "vz": 1})
+    d.watch["rt_kernel"] = lambda x: x.name
+
+    def forward():
+        return ctx.lib.fz_forward_nodes_dev(ctx.h, 10, atm, out, eqv, None, None)
+
+    for bad in (gpu.inversion({"T": 4, "vz": 33}), gpu.inversion({"T": 4}, invstk=(0, 0, 0, 0)),
+                gpu.inversion({"T": 4}, solver=9)) + (None,) * 6:
+        ctx.set_inversion(good)
+        assert forward() == 0
+        n = len(d.seen)
+        if bad is None:     # tables: coefficients, sums, nodes, two of the pairs, the transfer's
+            d.lib.double_fail_after(case_inversion_that_was_not_set.fail)
+            case_inversion_that_was_not_set.fail += 1
+        try:
+            ctx.set_inversion(bad or good)
+            raise AssertionError("accepted")
+        except gpu.FzError:
+            pass
+        d.lib.double_fail_after(-1)
+        assert forward() != 0 and len(d.seen) == n
+    ctx.set_inversion(good)
+    assert forward() == 0
+    # the tables are those of one height and wavelength grid
+    for nwave, nz, same in ((16, 40, False), (17, 32, False), (16, 32, True)):
+        ctx.configure(lines.fe6301_6302(nwave=nwave), np.arange(nz) * 30.0)
+        n = len(d.seen)
+        assert (forward() == 0) == same and (len(d.seen) > n) == same
+
+
+case_inversion_that_was_not_set.fail = 0
+
 CASES = [n[5:] for n in list(globals()) if n.startswith("case_")]
 
 
