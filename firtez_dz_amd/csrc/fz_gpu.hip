@@ -4957,7 +4957,12 @@ int fz_mlp_forward_dev(fz_ctx* c, int n, const float* d_x, const double* d_xd, f
   MlpState& M = c->mlp;
   hipStream_t st = (hipStream_t)stream;
   HIPCHK(c, hipSetDevice(c->device));
-  if (mlp_infer_fits(M)) return mlp_infer(c, n, d_x, d_xd, d_y, nullptr, st);
+  // (one launch reads some rows after it has written others: outputs in the place of
+  // inputs go by layers, whose first takes every row)
+  const char *x = d_x ? (const char*)d_x : (const char*)d_xd, *y = (const char*)d_y;
+  const bool apart = y + sizeof(float) * (size_t)n * M.nout <= x ||
+                     x + (d_x ? sizeof(float) : sizeof(double)) * (size_t)n * M.nin <= y;
+  if (apart && mlp_infer_fits(M)) return mlp_infer(c, n, d_x, d_xd, d_y, nullptr, st);
   const int chunk = 65536;
   int r = mlp_work(c, std::min(n, chunk), false);
   if (r) return r;

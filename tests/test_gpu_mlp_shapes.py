@@ -95,3 +95,18 @@ def test_training_after_larger_and_smaller_batches(gpu_ctx):
     l1, g1 = gpu_ctx.mlp_gradient_torch(x[:45].contiguous(), t[:45].contiguous())
     npar = g0.numel() - 2 * (100 + nout)
     assert torch.equal(l0, l1) and torch.equal(g0[:npar], g1[:npar])
+
+
+@pytest.mark.parametrize("nin", [100, 448])
+def test_outputs_in_the_place_of_inputs(gpu_ctx, nin):
+    """The forward pass with its output at the start of its input gives the
+    bits of one apart from it."""
+    import ctypes
+    import torch
+    p, nout, rng = make(gpu_ctx, nin, 200, 2, 4)
+    x = torch.from_numpy(rng.normal(0.3, 0.15, (5000, nin)).astype(np.float32)).cuda()
+    ref = gpu_ctx.mlp_forward_torch(x)
+    q = ctypes.c_void_p(x.data_ptr())
+    assert gpu_ctx.lib.fz_mlp_forward_dev(gpu_ctx.h, 5000, q, None, q, None) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(x.reshape(-1)[:5000 * nout].reshape(5000, nout), ref)

@@ -177,6 +177,26 @@ def case_inversion_that_was_not_set():
         assert (forward() == 0) == same and (len(d.seen) > n) == same
 
 
+def case_network_outputs_over_its_inputs():
+    """The forward pass of all layers in one launch is not taken where its
+    outputs would overwrite inputs that other workgroups have yet to read."""
+    import numpy as np
+    from firtez_dz_amd import lines
+    d = hostdouble.load()
+    ctx = d.gpu.Context(0)
+    ctx.configure(lines.fe6301_6302(nwave=16), np.arange(32) * 30.0)
+    ctx.mlp_create(64, 100, 2, 3)
+    d.watch["mlp_"] = lambda x: "infer" in x.name
+    n, p = 1000, d.malloc(1 << 22)
+    base = p + (1 << 20)
+    for x, xd, nx in ((base, None, 4 * 64 * n), (None, base, 8 * 64 * n)):
+        for y, one in ((base, False), (base + 4, False), (base + nx - 4, False), (base + nx, True),
+                       (base - 4 * 15 * n, True), (base - 4 * 15 * n + 4, False)):
+            d.seen.clear()
+            assert ctx.lib.fz_mlp_forward_dev(ctx.h, n, x, xd, y, None) == 0
+            assert d.seen == [True] if one else not any(d.seen), (y - base, d.seen)
+
+
 case_inversion_that_was_not_set.fail = 0
 
 CASES = [n[5:] for n in list(globals()) if n.startswith("case_")]
