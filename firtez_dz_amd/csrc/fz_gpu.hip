@@ -654,7 +654,6 @@ struct RtArgs {
   int jcol0;         // column of jac[0]
   float* scratch;    // [nz][4][ntile*numw]
   int chunk;         // heights of the record that a wave holds in LDS at a time
-  int wcols;         // columns that a wave spans at most (1 unless packed)
   // per-pixel windows (items null: every column uses every wavelength)
   const RtItem* items;   // this launch's workgroups
   const int64_t* poff;   // [ncol+1] prefix of the pixels' wavelength counts: Stokes at 4*poff[col]
@@ -2622,13 +2621,13 @@ static int launch_rt(fz_ctx* c, int rf_mode, RtArgs a, hipStream_t st, int nitem
     nmin = std::min(nmin, g.reg_nwave[r]);
     nb = std::max(nb, g.reg_nblend[r]);
   }
-  a.wcols = std::min(a.ntile, 1 + (RT_WAVE - 1 + nmin - 1) / nmin);
-  const bool pack = !a.items && 16L * a.wcols * npar * g.nz * g.numw < (1L << 31);
-  if (!pack) a.wcols = 1;
+  int wcols = std::min(a.ntile, 1 + (RT_WAVE - 1 + nmin - 1) / nmin);   // columns that a packed wave spans at most
+  const bool pack = !a.items && 16L * wcols * npar * g.nz * g.numw < (1L << 31);
+  if (!pack) wcols = 1;
   const dim3 grid(a.items ? (unsigned)nitems : pack ? (unsigned)npack : (unsigned)a.ntile * (unsigned)g.nbpc);
   // a wave's share of LDS: as many heights of its columns' records as 10 KB
   // hold (16 waves per CU), one at least
-  const size_t per = sizeof(float) * (REC_HEAD + REC_REG + REC_SLOT * (size_t)nb) * a.wcols;
+  const size_t per = sizeof(float) * (REC_HEAD + REC_REG + REC_SLOT * (size_t)nb) * wcols;
   a.chunk = (int)std::max<size_t>(1, std::min<size_t>((size_t)std::min(16, g.nz), RT_LDS / per));
   // Teams while one wave per 64 lanes leaves SIMDs without a wave, for the
   // synthesis always (its tail and its records in LDS gain from them):

@@ -1,8 +1,9 @@
 """The transfer's launch forms against each other and against the general path.
 
-  * teams of waves (few columns) give the bits of one wave per 64 lanes (many
-    columns): the same columns synthesised alone, in a small and in a large
-    cube, heights beside multiples of the team's size;
+  * teams of waves (few columns, or no response functions) give the bits of one
+    wave per 64 lanes (many columns, or per-pixel windows): the same columns
+    synthesised alone, in a small and in a large cube, heights beside multiples
+    of the team's size;
   * the node contraction within the transfer against the per-height
     Cartesian responses contracted on the host in 64 bits, for one node up to
     one per height, subsets of parameters and of Stokes parameters.
@@ -34,10 +35,16 @@ def test_teams_give_the_bits_of_one_wave(gpu_ctx, nz, mode, he):
     import torch
     ls = lines.setup([((4, 5), 100, -624.0, 22.0), ((2,), 29, -300.0, 20.0)])
     try:
-        d = cube(gpu_ctx, ls, 700, nz, he=he)      # 1094 + 318 waves: one each
+        d = cube(gpu_ctx, ls, 700, nz, he=he)
+        # with response functions 1094 + 318 packed waves are no teams; a packed
+        # synthesis always is one, per-pixel windows (here of every wavelength) are not
+        if mode == gpu.RF_NONE:
+            gpu_ctx.set_windows(np.tile(np.array([[0, 100], [0, 29]], np.int32), (700, 1, 1)))
         st, jac, status = gpu_ctx.forward_torch(d.clone(), mode)
+        gpu_ctx.set_windows(None)
+        st = st.reshape(700, 4, 129)
         assert int(status.max()) == 0 and bool(torch.isfinite(st).all())
-        for n in (1, 5, 300):                      # 8, 8 and 4 waves
+        for n in (1, 5, 300) + ((700,) if mode == gpu.RF_NONE else ()):     # 8, 8 and 4 waves
             s1, j1, _ = gpu_ctx.forward_torch(d[:, :, :n].contiguous(), mode)
             assert torch.equal(s1, st[:n]), n
             if jac is not None:
