@@ -1942,14 +1942,15 @@ struct fz_ctx {
   float* d_pstage = nullptr;
   size_t pstage_cap = 0;
   MlpState mlp;
-  // spatial PSF of the coupled inversion: PSF(NPY, NPX) as given, and the
-  // taps of the last map size it was cut for
+  // spatial PSF of the coupled inversion: PSF(NPY, NPX) as given, and its
+  // tap tables, made at the first convolution with it
   std::vector<double> h_psf;
   int psf_npx = 0, psf_npy = 0;
   float* d_taps = nullptr;
-  bf16* d_tapfrag = nullptr;  // the taps as matrix operands (both directions), where these are in range
-  bool taps_split = false;
-  int taps_nx = 0, taps_ny = 0, taps_rx = 0, taps_ry = 0, taps_ntx = 0;
+  size_t taps_cap = 0;
+  bf16* d_tapfrag = nullptr;  // behind the taps: these as matrix operands (both directions), where in range
+  bool taps_ok = false, taps_split = false;
+  int taps_rx = 0, taps_ry = 0, taps_ntx = 0;
   double taps_sq = 0.0;   // sum of the squared taps
 };
 
@@ -1968,6 +1969,8 @@ static int set_err(fz_ctx* c, int code, const std::string& msg) {
     hipError_t e_ = (x);                                                                 \
     if (e_ != hipSuccess) return set_err((c), FZ_EHIP, std::string(#x ": ") + hipGetErrorString(e_)); \
   } while (0)
+
+static int ensure(fz_ctx* c, float** p, size_t* cap, size_t bytes);
 
 // rows of numw floats through the LSF (no-op when it is off)
 static int run_lsf(fz_ctx* c, float* d_rows, long nrows, hipStream_t st) {
@@ -2074,7 +2077,6 @@ void fz_destroy(fz_ctx* c) {
   if (c->d_pert) (void)hipFree(c->d_pert);
   if (c->d_pstage) (void)hipFree(c->d_pstage);
   if (c->d_taps) (void)hipFree(c->d_taps);
-  if (c->d_tapfrag) (void)hipFree(c->d_tapfrag);
   c->mlp.release();
   for (int i = 0; i < 3; ++i)
     if (c->ev[i]) (void)hipEventDestroy(c->ev[i]);
@@ -2305,7 +2307,7 @@ int fz_set_psf(fz_ctx* c, const double* psf, int npy, int npx) {
   if (!psf) {
     c->h_psf.clear();
     c->psf_npx = c->psf_npy = 0;
-    c->taps_nx = c->taps_ny = 0;
+    c->taps_ok = false;
     return FZ_OK;
   }
   if (npx < 1 || npy < 1 || npx / 2 > PSF_RMAX || npy / 2 > PSF_RMAX)
@@ -2318,20 +2320,20 @@ int fz_set_psf(fz_ctx* c, const double* psf, int npy, int npx) {
   c->h_psf.assign(psf, psf + (size_t)npx * npy);
   c->psf_npx = npx;
   c->psf_npy = npy;
-  c->taps_nx = c->taps_ny = 0;
+  c->taps_ok = false;
   return FZ_OK;
 }
 
 }  // extern "C"
 
-// the taps of the PSF for an nx x ny map (READ_PSF's central part of
-// half-widths NPX/2, NPY/2 around (NPY/2 + 1, NPX/2 + 1)); the periodic sum
-// needs 2 r + 1 <= n along each axis
+// the taps of the PSF (READ_PSF's central part of half-widths NPX/2, NPY/2
+// around (NPY/2 + 1, NPX/2 + 1)) for an nx x ny map: the tables do not depend on
+// the map, whose periodic sum needs 2 r + 1 <= n along each axis
 static int psf_taps(fz_ctx* c, int nx, int ny) {
   if (c->h_psf.empty()) return set_err(c, FZ_ECONFIG, "no PSF set (fz_set_psf)");
-  if (c->taps_nx == nx && c->taps_ny == ny && c->d_taps) return FZ_OK;
   const int rx = c->psf_npx / 2, ry = c->psf_npy / 2;
   if (2 * rx + 1 > nx || 2 * ry + 1 > ny) return set_err(c, FZ_ECONFIG, "PSF wider than the map");
+  if (c->taps_ok) return FZ_OK;
   const int x0 = c->psf_npx / 2, y0 = c->psf_npy / 2, nu = 2 * ry + 1;
   const int ntx = (2 * rx + 1 + 7) / 8 * 8;
   // two tap tables [nu][ntx] in the kernel's window order: the convolution's
@@ -2346,56 +2348,35 @@ static int psf_taps(fz_ctx* c, int nx, int ny) {
       t[(size_t)nu * ntx + (size_t)(ry + dy) * ntx + (rx + dx)] = v;
       sq += (double)v * (double)v;
     }
-  HIPCHK(c, hipSetDevice(c->device));
-  // no map size holds until every table is there: a failed allocation below
-  // leaves the next call to cut the taps again
-  c->taps_nx = c->taps_ny = 0;
-  if (c->d_taps) (void)hipFree(c->d_taps);
-  if (c->d_tapfrag) (void)hipFree(c->d_tapfrag);
-  c->d_taps = nullptr;
-  c->d_tapfrag = nullptr;
-  HIPCHK(c, hipMalloc(&c->d_taps, sizeof(float) * t.size()));
-  HIPCHK(c, hipMemcpy(c->d_taps, t.data(), sizeof(float) * t.size(), hipMemcpyHostToDevice));
-  // Operands of psf_split_kernel: [direction][u][x tile][step][part][lane][8], tap t of
-  // output i of the 32 at input k = i + t.  Sixteen taps and fewer are left
-  // to the vector units: the matrix cores' work does not get less below 2 rx + 1 = 32
-  // (ms, vector units / matrix cores, 112 maps of 256 x 256: 9 x 9 taps 0.067 / 0.071,
-  // 15 x 15 0.089 / 0.092, 17 x 17 0.131 / 0.087; 64 maps, 63 x 63 0.61 / 0.29).
-  c->taps_split = ntx > 16;
+  // Sixteen taps and fewer are left to the vector units: the matrix cores' work
+  // does not get less below 2 rx + 1 = 32 (ms, vector units / matrix cores, 112
+  // maps of 256 x 256: 9 x 9 taps 0.067 / 0.071, 15 x 15 0.089 / 0.092, 17 x 17
+  // 0.131 / 0.087; 64 maps, 63 x 63 0.61 / 0.29).
+  bool split = ntx > 16;
   for (float v : t)
-    if (v != 0.f && !(std::fabs(v) > 0x1p-100f && std::fabs(v) < 0x1p100f)) c->taps_split = false;
-  if (c->taps_split) {
-    const int ks = ntx > 32 ? 3 : 2;
-    std::vector<uint16_t> f((size_t)2 * nu * 2 * ks * 3 * 512);
-    auto part = [](float& v) {   // the nearest BF16 of v, taken off it
-      uint32_t b;
-      memcpy(&b, &v, 4);
-      b = (b + 0x7fffu + ((b >> 16) & 1u)) & 0xffff0000u;
-      float h;
-      memcpy(&h, &b, 4);
-      v -= h;
-      return (uint16_t)(b >> 16);
-    };
-    for (int du = 0; du < 2 * nu; ++du)
-      for (int tt = 0; tt <= 2 * rx; ++tt) {
-        float v = t[(size_t)du * ntx + tt];
-        for (int p = 0; p < 3; ++p) {
-          const uint16_t h = part(v);
-          for (int i = 0; i < 32; ++i) {   // output i of 32, input k = i + tt
-            const int k = i + tt, xt = i >> 4, lane = (i & 15) + 16 * ((k >> 3) & 3);
-            f[((((size_t)du * 2 + xt) * ks + (k >> 5)) * 3 + p) * 512 + lane * 8 + (k & 7)] = h;
-          }
-        }
-      }
-    HIPCHK(c, hipMalloc(&c->d_tapfrag, sizeof(uint16_t) * f.size()));
-    HIPCHK(c, hipMemcpy(c->d_tapfrag, f.data(), sizeof(uint16_t) * f.size(), hipMemcpyHostToDevice));
+    if (v != 0.f && !(std::fabs(v) > 0x1p-100f && std::fabs(v) < 0x1p100f)) split = false;
+  // taps, then operands: [direction][u][x tile][step][part][lane][8]
+  const int ks = ntx > 32 ? 3 : 2, npiece = split ? 2 * nu * 2 * ks * 3 * 64 : 0;
+  const size_t off = (sizeof(float) * t.size() + 255) / 256 * 256;
+  HIPCHK(c, hipSetDevice(c->device));
+  // convolutions with the tables of another PSF may be running
+  HIPCHK(c, hipDeviceSynchronize());
+  int r = ensure(c, &c->d_taps, &c->taps_cap, off + sizeof(bf16) * 8 * npiece);
+  if (r) return r;
+  c->d_tapfrag = reinterpret_cast<bf16*>(reinterpret_cast<char*>(c->d_taps) + off);
+  HIPCHK(c, hipMemcpy(c->d_taps, t.data(), sizeof(float) * t.size(), hipMemcpyHostToDevice));
+  if (split) {
+    hipLaunchKernelGGL(psf_operand_kernel, dim3((unsigned)((npiece + 255) / 256)), dim3(256), 0, 0,
+                       (const float*)c->d_taps, npiece, ks, ntx, c->d_tapfrag);
+    HIPCHK(c, hipGetLastError());
+    HIPCHK(c, hipStreamSynchronize(0));   // before a convolution on any stream
   }
-  c->taps_nx = nx;
-  c->taps_ny = ny;
   c->taps_rx = rx;
   c->taps_ry = ry;
   c->taps_ntx = ntx;
   c->taps_sq = sq;
+  c->taps_split = split;
+  c->taps_ok = true;
   return FZ_OK;
 }
 

@@ -263,6 +263,34 @@ __global__ void __launch_bounds__(256) psf_split_kernel(PsfArgs a, const bf16* _
   }
 }
 
+// Operands of psf_split_kernel from the taps [direction, u][ntx], a lane's
+// eight k (16 bytes) per thread: tap t of output i of the 32 is at input k = i + t,
+// its parts as the kernel splits its inputs.  A new PSF and its first convolution
+// (4 maps of 64 x 64) took 250 us for 31 x 31 taps and 880 for 63 x 63 when the host
+// built and copied these 0.8 and 2.3 MB, and take 51 and 71.
+__global__ void __launch_bounds__(256) psf_operand_kernel(const float* __restrict__ taps, int npiece, int ks, int ntx,
+                                                          bf16* __restrict__ frag) {
+  const int e = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (e >= npiece) return;
+  int q = e >> 6;
+  const int lane = e & 63, part = q % 3;
+  q /= 3;
+  const int s = q % ks;
+  q /= ks;
+  const int i = 16 * (q & 1) + (lane & 15), k0 = 32 * s + 8 * (lane >> 4), du = q >> 1;
+  bf16x8 o;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int t = k0 + j - i;
+    const float v = t >= 0 && t < ntx ? taps[du * ntx + t] : 0.f;
+    const bf16 p0 = (bf16)v;
+    const float r = v - (float)p0;
+    const bf16 p1 = (bf16)r;
+    o[j] = part == 0 ? p0 : part == 1 ? p1 : (bf16)(r - (float)p1);
+  }
+  reinterpret_cast<bf16x8*>(frag)[e] = o;
+}
+
 // 32 x 32 transpose through LDS: out[c][r] = in[r][c] for an R x C matrix
 // (in row stride C, out row stride R), converting the element type
 template <class Tin, class Tout>

@@ -12,29 +12,57 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB = os.path.join(ROOT, "firtez_dz_amd", "libfirtez_gpu.so")
 
 
+def psf_launches(d):
+    d.watch["psf_"] = lambda x: (("operands" if "operand" in x.name else "split" if "split" in x.name else "vector"),
+                                 x.arg(1, ctypes.c_void_p).value if "split" in x.name else None)
+
+    def convolve(ctx, nx, ny, _buf=[]):
+        if not _buf:
+            _buf.append((d.malloc(1 << 24), d.malloc(1 << 24)))
+        return ctx.lib.fz_psf_convolve_dev(ctx.h, nx, ny, 2, _buf[0][0], _buf[0][1], 0, None)
+    return convolve
+
+
 def case_psf_failed_operands():
-    """A failed allocation while the taps are cut for another map size leaves
-    no state that a later convolution would launch with missing operands."""
+    """A failed allocation while the taps are cut leaves no state that a
+    later convolution would launch with missing operands."""
     import numpy as np
     d = hostdouble.load()
     ctx = d.gpu.Context(0)
+    convolve = psf_launches(d)
+    ctx.set_psf(np.full((17, 17), 1.0 / 289.0))
+    assert convolve(ctx, 64, 64) == 0
     ctx.set_psf(np.full((31, 31), 1.0 / 961.0))
-    d.watch["psf_"] = lambda x: (x.name, x.arg(1, ctypes.c_void_p).value if "split" in x.name else None)
-    maps = d.malloc(4 * 2 * 128 * 128)
-    out = d.malloc(4 * 2 * 128 * 128)
-
-    def convolve(n):
-        return ctx.lib.fz_psf_convolve_dev(ctx.h, n, n, 2, maps, out, 0, None)
-
-    assert convolve(64) == 0
-    for fail in range(3):           # taps, operands, nothing
+    d.seen.clear()
+    for fail in range(2):           # the tables, nothing
         d.lib.double_fail_after(fail)
-        rc = convolve(70)
-        assert (rc != 0) == (fail < 2), (fail, rc)
-        d.lib.double_fail_after(-1)
-        for n in (64, 70, 64):
-            assert convolve(n) == 0
-    assert len(d.seen) == 11 and all("psf_split" in n and frag for n, frag in d.seen), d.seen
+        rc = convolve(ctx, 64, 64)
+        assert (rc != 0) == (fail < 1) and len(d.seen) == 2 * fail, (fail, rc)
+    d.lib.double_fail_after(-1)
+    for n in (64, 70, 64):
+        assert convolve(ctx, n, n) == 0
+    assert [k for k, _ in d.seen] == ["operands"] + 4 * ["split"] and all(f for k, f in d.seen if k == "split"), d.seen
+
+
+def case_psf_tables_of_a_psf():
+    """The tables are made once for a PSF, whatever maps it is applied to, and
+    again for another one; maps narrower than the PSF are refused."""
+    import numpy as np
+    d = hostdouble.load()
+    ctx = d.gpu.Context(0)
+    convolve = psf_launches(d)
+    for side, kind in ((31, "split"), (15, "vector"), (43, "split"), (63, "split"), (17, "split")):
+        ctx.set_psf(np.full((side, side), 1.0 / side ** 2))
+        d.seen.clear()
+        assert convolve(ctx, side, side) == 0
+        n = d.lib.double_mallocs()
+        for nx, ny in ((64, 70), (200, 63), (63, 200), (64, 70)):
+            assert convolve(ctx, nx, ny) == 0
+            assert convolve(ctx, side - 1, ny) != 0 and convolve(ctx, nx, side - 1) != 0
+        assert d.lib.double_mallocs() == n
+        assert [k for k, _ in d.seen] == (["operands"] if kind == "split" else []) + 5 * [kind], d.seen
+    ctx.set_psf(None)
+    assert convolve(ctx, 64, 64) != 0
 
 
 def case_network_buffers_only_grow():
