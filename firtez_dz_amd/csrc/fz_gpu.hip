@@ -2356,7 +2356,7 @@ static int psf_taps(fz_ctx* c, int nx, int ny) {
   for (float v : t)
     if (v != 0.f && !(std::fabs(v) > 0x1p-100f && std::fabs(v) < 0x1p100f)) split = false;
   // taps, then operands: [direction][u][x tile][step][part][lane][8]
-  const int ks = ntx > 32 ? 3 : 2, npiece = split ? 2 * nu * 2 * ks * 3 * 64 : 0;
+  const int ks = psf_steps(ntx), npiece = split ? 2 * nu * 2 * ks * 3 * 64 : 0;
   const size_t off = (sizeof(float) * t.size() + 255) / 256 * 256;
   HIPCHK(c, hipSetDevice(c->device));
   // convolutions with the tables of another PSF may be running
@@ -2380,16 +2380,26 @@ static int psf_taps(fz_ctx* c, int nx, int ny) {
   return FZ_OK;
 }
 
-template <int KS, int YT>
-static void launch_psf_split(fz_ctx* c, const PsfArgs& a, int adjoint, hipStream_t st) {
-  const int ntx = c->taps_ntx, ty = 32 * YT, nu = 2 * a.ry + 1;
+template <int NTX, int YT>
+static void launch_psf_split_y(fz_ctx* c, const PsfArgs& a, int adjoint, hipStream_t st) {
+  constexpr int KS = psf_steps(NTX);
+  const int ty = 32 * YT, nu = 2 * a.ry + 1;
   const size_t lds = std::max(sizeof(bf16) * 3 * (ty + 2 * a.ry) * (32 * KS + 8),
-                              sizeof(float) * (PSF_TX + ntx - 1) * (PSF_TY + 2 * a.ry));
-  (void)hipFuncSetAttribute((const void*)psf_split_kernel<KS, YT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              sizeof(float) * (PSF_TX + NTX - 1) * (PSF_TY + 2 * a.ry));
+  (void)hipFuncSetAttribute((const void*)psf_split_kernel<NTX, YT>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             144 * 1024);
   const dim3 grid((unsigned)((a.ny + ty - 1) / ty), (unsigned)((a.nx + PSF_TX - 1) / PSF_TX), (unsigned)a.nmaps);
-  hipLaunchKernelGGL((psf_split_kernel<KS, YT>), grid, dim3(256), lds, st, a,
-                     (const bf16*)c->d_tapfrag + (adjoint ? (size_t)nu * 2 * KS * 3 * 512 : 0), ntx);
+  hipLaunchKernelGGL((psf_split_kernel<NTX, YT>), grid, dim3(256), lds, st, a,
+                     (const bf16*)c->d_tapfrag + (adjoint ? (size_t)nu * 2 * KS * 3 * 512 : 0));
+}
+
+template <int NTX>
+static void launch_psf_split(fz_ctx* c, const PsfArgs& a, int adjoint, hipStream_t st) {
+  // 128 y a workgroup, 64 where that covers the map with fewer
+  if ((a.ny + 127) / 128 * 2 <= (a.ny + 63) / 64)
+    launch_psf_split_y<NTX, 4>(c, a, adjoint, st);
+  else
+    launch_psf_split_y<NTX, 2>(c, a, adjoint, st);
 }
 
 static void launch_psf(fz_ctx* c, int nx, int ny, int nmaps, const float* in, float* out, int adjoint, hipStream_t st) {
@@ -2405,12 +2415,14 @@ static void launch_psf(fz_ctx* c, int nx, int ny, int nmaps, const float* in, fl
   a.in = in;
   a.out = out;
   if (c->taps_split) {
-    // 128 y a workgroup, 64 where that covers the map with fewer
-    const bool wide = (ny + 127) / 128 * 2 <= (ny + 63) / 64;
-    if (ntx <= 32)
-      wide ? launch_psf_split<2, 4>(c, a, adjoint, st) : launch_psf_split<2, 2>(c, a, adjoint, st);
-    else
-      wide ? launch_psf_split<3, 4>(c, a, adjoint, st) : launch_psf_split<3, 2>(c, a, adjoint, st);
+    switch (ntx) {
+      case 24: launch_psf_split<24>(c, a, adjoint, st); break;
+      case 32: launch_psf_split<32>(c, a, adjoint, st); break;
+      case 40: launch_psf_split<40>(c, a, adjoint, st); break;
+      case 48: launch_psf_split<48>(c, a, adjoint, st); break;
+      case 56: launch_psf_split<56>(c, a, adjoint, st); break;
+      default: launch_psf_split<64>(c, a, adjoint, st); break;
+    }
     return;
   }
   const size_t lds = sizeof(float) * (PSF_TX + ntx - 1) * (PSF_TY + 2 * a.ry);

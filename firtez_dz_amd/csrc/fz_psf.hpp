@@ -38,6 +38,9 @@ constexpr int PSF_TX = 4 * PSF_OX;         // output tile along x (four waves)
 constexpr int PSF_TY = 64;                 // output tile along y (the lanes of a wave)
 constexpr int PSF_RMAX = 31;               // largest tap radius (63 x 63 PSF)
 
+// K steps of 32 that the band of 32 outputs and ntx taps takes
+constexpr int psf_steps(int ntx) { return ntx > 32 ? 3 : 2; }
+
 struct PsfArgs {
   int nx, ny, nmaps, rx, ry;
   long npix;
@@ -49,15 +52,13 @@ struct PsfArgs {
   float* out;
 };
 
+// One 32 x 64 tile from (x0, y0), by all 256 threads; tile: LDS
 template <int NTX>
-__global__ void __launch_bounds__(256) psf_conv_kernel(PsfArgs a) {
-  extern __shared__ float tile[];
+__device__ __forceinline__ void psf_vector(const PsfArgs& a, int x0, int y0, const float* __restrict__ src,
+                                           float* __restrict__ dst, float* tile) {
   constexpr int NW = PSF_OX + NTX - 1;     // register strip along x
   constexpr int ROWS = PSF_TX + NTX - 1;   // tile rows (x)
-  const int m = blockIdx.z;
-  const int x0 = blockIdx.y * PSF_TX, y0 = blockIdx.x * PSF_TY;
   const int cols = PSF_TY + 2 * a.ry;      // tile columns (y)
-  const float* src = a.in + (long)m * a.npix;
   // tile[i][j] = in(x0 - rx + i, y0 - ry + j), periodic in x and y
   for (int e = threadIdx.x; e < ROWS * cols; e += 256) {
     const int i = e / cols, j = e - i * cols;
@@ -89,53 +90,18 @@ __global__ void __launch_bounds__(256) psf_conv_kernel(PsfArgs a) {
   }
   const int y = y0 + ty;
   if (y >= a.ny) return;
-  float* dst = a.out + (long)m * a.npix + y;
 #pragma unroll
   for (int i = 0; i < PSF_OX; ++i) {
     const int x = x0 + xw + i;
-    if (x < a.nx) dst[(long)x * a.ny] = acc[i];
+    if (x < a.nx) dst[(long)x * a.ny + y] = acc[i];
   }
 }
 
-// The same tile (64 columns from y0) with the tap count at run time, by all
-// 256 threads: the sums of psf_conv_kernel in its order.
-__device__ __forceinline__ void psf_direct(const PsfArgs& a, int ntx, int x0, int y0, const float* __restrict__ src,
-                                           float* __restrict__ dst, float* tile) {
-  const int rows = PSF_TX + ntx - 1, cols = PSF_TY + 2 * a.ry;
-  __syncthreads();
-  for (int e = threadIdx.x; e < rows * cols; e += 256) {
-    const int i = e / cols, j = e - i * cols;
-    int x = (x0 - a.rx + i) % a.nx;
-    if (x < 0) x += a.nx;
-    int y = (y0 - a.ry + j) % a.ny;
-    if (y < 0) y += a.ny;
-    tile[e] = src[(long)x * a.ny + y];
-  }
-  __syncthreads();
-  const int ty = threadIdx.x & 63, xw = (threadIdx.x >> 6) * PSF_OX;
-  float acc[PSF_OX];
-#pragma unroll
-  for (int i = 0; i < PSF_OX; ++i) acc[i] = 0.f;
-  for (int u = 0; u <= 2 * a.ry; ++u) {
-    const float* colp = tile + xw * cols + ty + u;
-    float v[2 * PSF_OX - 1];
-#pragma unroll
-    for (int j = 0; j < PSF_OX - 1; ++j) v[j] = colp[j * cols];
-    for (int t0 = 0; t0 < ntx; t0 += PSF_OX) {
-#pragma unroll
-      for (int j = PSF_OX - 1; j < 2 * PSF_OX - 1; ++j) v[j] = colp[(t0 + j) * cols];
-#pragma unroll
-      for (int t = 0; t < PSF_OX; ++t)
-#pragma unroll
-        for (int i = 0; i < PSF_OX; ++i) acc[i] = fmaf(a.taps[u * ntx + t0 + t], v[i + t], acc[i]);
-#pragma unroll
-      for (int j = 0; j < PSF_OX - 1; ++j) v[j] = v[j + PSF_OX];
-    }
-  }
-  const int y = y0 + ty;
-#pragma unroll
-  for (int i = 0; i < PSF_OX; ++i)
-    if (y < a.ny && x0 + xw + i < a.nx) dst[(long)(x0 + xw + i) * a.ny + y] = acc[i];
+template <int NTX>
+__global__ void __launch_bounds__(256) psf_conv_kernel(PsfArgs a) {
+  extern __shared__ float tile[];
+  psf_vector<NTX>(a, blockIdx.y * PSF_TX, blockIdx.x * PSF_TY, a.in + (long)blockIdx.z * a.npix,
+                  a.out + (long)blockIdx.z * a.npix, tile);
 }
 
 // The convolution on the matrix cores.  Inputs and taps are split into three BF16
@@ -154,12 +120,16 @@ __device__ __forceinline__ void psf_direct(const PsfArgs& a, int ntx, int x0, in
 // result, with the vector units' sums 4.7e-7; time 0.49 ms for 0.97.
 //
 // A tile with an input that is not finite, beyond 2^120 or, not being zero,
-// below 2^-100, where the parts would leave BF16's range, takes psf_direct.
-template <int KS, int YT>
-__global__ void __launch_bounds__(256) psf_split_kernel(PsfArgs a, const bf16* __restrict__ frag, int ntx) {
+// below 2^-100, where the parts would leave BF16's range, takes psf_vector.  All
+// tiles there, ms for psf_conv_kernel's: 448 maps of 256 x 256, 31 x 31 taps 0.96 (0.96);
+// 4 maps of 64 x 64, 63 x 63 0.112 (0.108); 64 maps of 256 x 256, 63 x 63, where the
+// operands' LDS leaves one workgroup to a CU, 0.88 (0.56).  (With the tap count at run
+// time 1.14, 0.147 and 1.06; a row's inputs a row ahead 1.10, 0.118 and 1.02.)
+template <int NTX, int YT>
+__global__ void __launch_bounds__(256) psf_split_kernel(PsfArgs a, const bf16* __restrict__ frag) {
   extern __shared__ __attribute__((aligned(16))) char psf_lds[];
   __shared__ int flag[4];
-  constexpr int XP = 32 * KS + 8, TY = 32 * YT;
+  constexpr int KS = psf_steps(NTX), XP = 32 * KS + 8, TY = 32 * YT;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int lr = lane & 15, lg = lane >> 4;
   const int x0 = blockIdx.y * PSF_TX, y0 = blockIdx.x * TY;
@@ -202,8 +172,11 @@ __global__ void __launch_bounds__(256) psf_split_kernel(PsfArgs a, const bf16* _
   if (lane == 0) flag[wave] = any;
   __syncthreads();
   if (flag[0] | flag[1] | flag[2] | flag[3]) {
-    for (int h = 0; h < TY; h += PSF_TY)
-      psf_direct(a, ntx, x0, y0 + h, src, dst, reinterpret_cast<float*>(psf_lds));
+#pragma unroll 1
+    for (int h = 0; h < TY && y0 + h < a.ny; h += PSF_TY) {
+      __syncthreads();
+      psf_vector<NTX>(a, x0, y0 + h, src, dst, reinterpret_cast<float*>(psf_lds));
+    }
     return;
   }
   f32x4 acc[2][YT];
