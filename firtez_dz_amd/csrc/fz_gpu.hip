@@ -1894,6 +1894,8 @@ struct fz_ctx {
   LmArgs lm;                  // per-cycle constants; per-call pointers filled at launch
   std::vector<int> slot_of;   // [np] physical parameter (= Cartesian slot) of each free parameter
   std::vector<int> kbeg, kend;  // [np] support of each node's hat function
+  float* d_invtab = nullptr;  // one buffer for the tables that follow
+  size_t invtab_cap = 0;
   int* d_eqvnode = nullptr;   // [3][np]: kbeg, kend, Cartesian slot
   int* d_eqvtab_j = nullptr;  // [nparam][nz] node table of the pairwise contraction
   double* d_eqvtab_c = nullptr;  // [nparam][nz][2]
@@ -2056,12 +2058,7 @@ void fz_destroy(fz_ctx* c) {
   if (c->d_gain) (void)hipFree(c->d_gain);
   if (c->d_micro) (void)hipFree(c->d_micro);
   if (c->d_scratch) (void)hipFree(c->d_scratch);
-  if (c->d_coefs) (void)hipFree(c->d_coefs);
-  if (c->d_colsum) (void)hipFree(c->d_colsum);
-  if (c->d_eqvnode) (void)hipFree(c->d_eqvnode);
-  if (c->d_eqvtab_j) (void)hipFree(c->d_eqvtab_j);
-  if (c->d_eqvtab_c) (void)hipFree(c->d_eqvtab_c);
-  if (c->d_nodetab) (void)hipFree(c->d_nodetab);
+  if (c->d_invtab) (void)hipFree(c->d_invtab);
   if (c->d_lmwork) (void)hipFree(c->d_lmwork);
   if (c->d_jtile) (void)hipFree(c->d_jtile);
   if (c->d_sbuf) (void)hipFree(c->d_sbuf);
@@ -3372,12 +3369,6 @@ int fz_set_inversion(fz_ctx* c, const fz_inversion* inv, int* ifreep, int* nfreq
   c->lm_work = c->lm_big ? (lm_lds_bytes(np, nz, L.regul != 0, LM_BIG_THREADS) + 255) / 256 * 256 : 0;
   if (c->lm_lds > 160 * 1024 - 512) return set_err(c, FZ_ECONFIG, "inversion set-up exceeds the LDS of one workgroup");
   HIPCHK(c, hipSetDevice(c->device));
-  if (c->d_coefs) (void)hipFree(c->d_coefs);
-  if (c->d_colsum) (void)hipFree(c->d_colsum);
-  if (c->d_eqvnode) (void)hipFree(c->d_eqvnode);
-  c->d_coefs = nullptr;
-  c->d_colsum = nullptr;
-  c->d_eqvnode = nullptr;
   // node table of the contraction: supports, Cartesian slot
   std::vector<int> node((size_t)3 * np);
   for (int j = 0; j < np; ++j) {
@@ -3385,12 +3376,6 @@ int fz_set_inversion(fz_ctx* c, const fz_inversion* inv, int* ifreep, int* nfreq
     node[np + j] = c->kend[j];
     node[2 * np + j] = c->slot_of[j];
   }
-  HIPCHK(c, hipMalloc((void**)&c->d_coefs, sizeof(double) * coefs.size()));
-  HIPCHK(c, hipMalloc((void**)&c->d_colsum, sizeof(double) * np));
-  HIPCHK(c, hipMalloc((void**)&c->d_eqvnode, sizeof(int) * node.size()));
-  HIPCHK(c, hipMemcpy(c->d_coefs, coefs.data(), sizeof(double) * coefs.size(), hipMemcpyHostToDevice));
-  HIPCHK(c, hipMemcpy(c->d_colsum, colsum.data(), sizeof(double) * np, hipMemcpyHostToDevice));
-  HIPCHK(c, hipMemcpy(c->d_eqvnode, node.data(), sizeof(int) * node.size(), hipMemcpyHostToDevice));
   // the pairwise contraction applies when every parameter's node supports
   // overlap at most pairwise and move up with the node index (the hat basis
   // of GET_INT_COEFS); its per-height table
@@ -3402,15 +3387,12 @@ int fz_set_inversion(fz_ctx* c, const fz_inversion* inv, int* ifreep, int* nfreq
       if (j + 1 <= je && (c->kbeg[j + 1] < c->kbeg[j] || c->kend[j + 1] < c->kend[j])) c->eqv_pairs = false;
       if (j + 2 <= je && c->kbeg[j + 2] <= c->kend[j]) c->eqv_pairs = false;
     }
-  if (c->d_eqvtab_j) (void)hipFree(c->d_eqvtab_j);
-  if (c->d_eqvtab_c) (void)hipFree(c->d_eqvtab_c);
-  if (c->d_nodetab) (void)hipFree(c->d_nodetab);
-  c->d_eqvtab_j = nullptr;
-  c->d_eqvtab_c = nullptr;
-  c->d_nodetab = nullptr;
+  std::vector<int> tj;
+  std::vector<double> tc;
+  std::vector<NodeTab> nt;
   if (c->eqv_pairs) {
-    std::vector<int> tj((size_t)npar * nz, 0);
-    std::vector<double> tc((size_t)npar * nz * 2, 0.0);
+    tj.assign((size_t)npar * nz, 0);
+    tc.assign((size_t)npar * nz * 2, 0.0);
     for (int ip = 0; ip < npar; ++ip) {
       const int jb = L.j0[ip], je = jb + L.nj[ip] - 1;
       int jl = jb;
@@ -3428,12 +3410,8 @@ int fz_set_inversion(fz_ctx* c, const fz_inversion* inv, int* ifreep, int* nfreq
         tj[(size_t)ip * nz + k] = w;
       }
     }
-    HIPCHK(c, hipMalloc((void**)&c->d_eqvtab_j, sizeof(int) * tj.size()));
-    HIPCHK(c, hipMalloc((void**)&c->d_eqvtab_c, sizeof(double) * tc.size()));
-    HIPCHK(c, hipMemcpy(c->d_eqvtab_j, tj.data(), sizeof(int) * tj.size(), hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(c->d_eqvtab_c, tc.data(), sizeof(double) * tc.size(), hipMemcpyHostToDevice));
     // the same per height for the five slots T, Bx, By, Bz, v_z
-    std::vector<NodeTab> nt((size_t)nz * 5, NodeTab{0.0, 0.0, -1, 0});
+    nt.assign((size_t)nz * 5, NodeTab{0.0, 0.0, -1, 0});
     for (int ip = 0; ip < npar; ++ip) {
       const int sl = TBV_SLOT[L.par[ip]];
       if (sl < 0) continue;
@@ -3442,9 +3420,33 @@ int fz_set_inversion(fz_ctx* c, const fz_inversion* inv, int* ifreep, int* nfreq
         nt[(size_t)k * 5 + sl] = {tc[((size_t)ip * nz + k) * 2], tc[((size_t)ip * nz + k) * 2 + 1], w & 0xffff, 0};
       }
     }
-    HIPCHK(c, hipMalloc((void**)&c->d_nodetab, sizeof(NodeTab) * nt.size()));
-    HIPCHK(c, hipMemcpy(c->d_nodetab, nt.data(), sizeof(NodeTab) * nt.size(), hipMemcpyHostToDevice));
   }
+  // all tables with one copy into one buffer, which is kept (an allocation and a
+  // copy each took 96 us for five parameters of four nodes): doubles, then integers
+  std::vector<char> tab;
+  auto put = [&](const void* src, size_t bytes) {
+    const size_t at = tab.size();
+    tab.resize(at + bytes);
+    if (bytes) memcpy(tab.data() + at, src, bytes);
+    return at;
+  };
+  const size_t o_coefs = put(coefs.data(), sizeof(double) * coefs.size());
+  const size_t o_colsum = put(colsum.data(), sizeof(double) * np);
+  const size_t o_tc = put(tc.data(), sizeof(double) * tc.size());
+  const size_t o_nt = put(nt.data(), sizeof(NodeTab) * nt.size());
+  const size_t o_node = put(node.data(), sizeof(int) * node.size());
+  const size_t o_tj = put(tj.data(), sizeof(int) * tj.size());
+  HIPCHK(c, hipDeviceSynchronize());   // work with the tables of another set-up may be running
+  const int re = ensure(c, &c->d_invtab, &c->invtab_cap, tab.size());
+  if (re) return re;
+  HIPCHK(c, hipMemcpy(c->d_invtab, tab.data(), tab.size(), hipMemcpyHostToDevice));
+  char* base = reinterpret_cast<char*>(c->d_invtab);
+  c->d_coefs = reinterpret_cast<double*>(base + o_coefs);
+  c->d_colsum = reinterpret_cast<double*>(base + o_colsum);
+  c->d_eqvtab_c = reinterpret_cast<double*>(base + o_tc);
+  c->d_nodetab = reinterpret_cast<NodeTab*>(base + o_nt);
+  c->d_eqvnode = reinterpret_cast<int*>(base + o_node);
+  c->d_eqvtab_j = reinterpret_cast<int*>(base + o_tj);
   if (!c->lm_big)
     HIPCHK(c, hipFuncSetAttribute((const void*)lm_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                   (int)c->lm_lds));
