@@ -358,8 +358,13 @@ __device__ __forceinline__ void jacobi_rotation(double app, double aqq, double a
 // the rotations are formed (by the lanes of the diagonal blocks, from those
 // blocks) and one exchange through LDS hands the rotations out.  A round of 20
 // parameters took 1.3 us with the loads behind the exchange.
+//
+// Inlined into its kernels: as a function it could not know that its arrays are in
+// LDS, and its kernels took 197 registers and a stack (here 174 and 88): the step of 4096
+// pixels with 20 parameters 0.85 -> 0.65 ms (CG the same), with 64 parameters of 1024
+// 7.0 -> 6.1 ms; a single CG solve of 20 parameters 44.4 -> 42.1 us.
 template <int NT>
-__device__ void damped_solve(int solver, double svdtol, int np, double* A, double* V, const double* g,
+__device__ __forceinline__ void damped_solve(int solver, double svdtol, int np, double* A, double* V, const double* g,
                              double* dv, double* del, double* red, double* rot, double* nod) {
   const int t = threadIdx.x;
   const int ld = np + 1;
