@@ -191,7 +191,7 @@ __global__ void __launch_bounds__(256) saha_kernel(MicroTile a) {
 // Against the sequential fold of 91 terms through LDS with eight lanes per
 // column that this replaces: hydrostatic integration of 16 columns x 64
 // heights 8.9 -> 0.55 ms, of 9216 x 96 heights 26.9 -> 2.2 ms; the forward's
-// fixed point of 82944 columns x 96 heights 24.4 -> 6.5 ms.
+// fixed point of 82944 columns x 96 heights 24.4 -> 5.9 ms.
 template <int CTRL>
 __device__ __forceinline__ double dpp64(double x) {
   const int lo = __double2loint(x), hi = __double2hiint(x);
