@@ -4646,12 +4646,13 @@ void mlp_forward_rows(MlpState& M, int n, float* y, bool grad, hipStream_t st) {
   }
 }
 
-// Output layer, loss and gradient of the parameters for n rows (targets t,
-// rows gathered by idx when given): the mean squared error into loss[0].
-void mlp_backward_rows(MlpState& M, int n, const float* d_t, const int32_t* d_idx, float* loss, float* grad,
-                       hipStream_t st) {
+// Output layer, loss and gradient of the parameters for n of a batch's rows
+// (targets t, rows gathered by idx when given): their part of the mean squared
+// error into loss[0], or added to it.
+void mlp_backward_rows(MlpState& M, int n, int rows, bool add, const float* d_t, const int32_t* d_idx, float* loss,
+                       float* grad, hipStream_t st) {
   const float* tmean = M.norms + 2 * M.nin;
-  LossArgs ls = {d_t, tmean, tmean + M.nout, d_idx, M.partial};
+  LossArgs ls = {d_t, tmean, tmean + M.nout, d_idx, M.partial, rows};
   DwArgs dw;
   memset(&dw, 0, sizeof(dw));
   const bf16* dz = nullptr;
@@ -4694,8 +4695,9 @@ void mlp_backward_rows(MlpState& M, int n, const float* d_t, const int32_t* d_id
   dw.loss_blk = nb;
   dw.nloss = 4 * (pad32(n) / 32) * (pad32(M.nout) / 32);
   dw.lpart = M.partial;
-  dw.lscale = (float)((long)n * M.nout);
+  dw.lscale = (float)((long)rows * M.nout);
   dw.loss = loss;
+  dw.add = add;
   hipLaunchKernelGGL(mlp_dw_kernel, dim3((unsigned)(nb + 1)), dim3(256), 0, st, dw);
 }
 
@@ -4977,12 +4979,20 @@ int fz_mlp_gradient_dev(fz_ctx* c, int n, const float* d_x, const float* d_t, co
   MlpState& M = c->mlp;
   hipStream_t st = (hipStream_t)stream;
   HIPCHK(c, hipSetDevice(c->device));
-  int r = mlp_work(c, n, true);
+  // a million rows at a time (15 GB of work buffers for 448-512-512-512-20),
+  // their sums added up
+  const int chunk = 1 << 20;
+  int r = mlp_work(c, std::min(n, chunk), true);
   if (r) return r;
-  r = mlp_input(c, n, d_x, nullptr, d_idx, true, st);
-  if (r) return r;
-  mlp_forward_rows(M, n, nullptr, true, st);
-  mlp_backward_rows(M, n, d_t, d_idx, d_loss ? d_loss : M.loss, d_grad ? d_grad : M.g, st);
+  for (int r0 = 0; r0 < n; r0 += std::min(chunk, n - r0)) {
+    const int nr = std::min(chunk, n - r0);
+    const float *x = d_idx ? d_x : d_x + (size_t)r0 * M.nin, *t = d_idx ? d_t : d_t + (size_t)r0 * M.nout;
+    const int32_t* idx = d_idx ? d_idx + r0 : nullptr;
+    r = mlp_input(c, nr, x, nullptr, idx, true, st);
+    if (r) return r;
+    mlp_forward_rows(M, nr, nullptr, true, st);
+    mlp_backward_rows(M, nr, n, r0 > 0, t, idx, d_loss ? d_loss : M.loss, d_grad ? d_grad : M.g, st);
+  }
   HIPCHK(c, hipGetLastError());
   return FZ_OK;
 }

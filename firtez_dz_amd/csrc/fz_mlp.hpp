@@ -127,13 +127,14 @@ struct LossArgs {
   const float *T, *tmean, *tstd;
   const int32_t* idx;
   float* part;              // [4 tiles] sums of the squares
+  int rows;                 // of the whole batch, whose mean the loss is
 };
 
 enum { MLP_HIDDEN = 0, MLP_OUT = 1, MLP_LOSS = 2, MLP_DACT = 3 };
 
 // HIDDEN: Cb = ReLU(D + bias).  OUT: Cf = D + bias.  LOSS: the squared
 // differences of D + bias from the standardised targets, and their gradient
-// dY = 2 (Y - (T - tmean) / tstd) / (M N) into Cb.  DACT: Cb = D where the mask is
+// dY = 2 (Y - (T - tmean) / tstd) / (rows N) into Cb.  DACT: Cb = D where the mask is
 // positive.  CbT gets Cb's transpose, csum the column sums of the FP32 values.
 // The sums over K run in one order whatever the tile (a regrouped sum
 // rounds some activations the other way).  Each of the four waves has FR x FR
@@ -180,7 +181,7 @@ __global__ void __launch_bounds__(256) mlp_layer_kernel(GemmArgs g, LossArgs ls)
               const float tn = (ls.T[row * g.N + n + q] - ls.tmean[n + q]) / ls.tstd[n + q];
               const float df = v[q] - tn;
               e2 += df * df;
-              v[q] = 2.f * df / ((float)g.M * (float)g.N);
+              v[q] = 2.f * df / ((float)ls.rows * (float)g.N);
             }
           }
           if (!in) v[q] = 0.f;
@@ -249,6 +250,7 @@ struct DwArgs {
   const float* lpart;
   float lscale;
   float* loss;
+  int add;                           // to what the rows before this launch's gave
 };
 
 __global__ void __launch_bounds__(256) mlp_dw_kernel(DwArgs a) {
@@ -260,9 +262,13 @@ __global__ void __launch_bounds__(256) mlp_dw_kernel(DwArgs a) {
     while (l + 1 < a.n && blk >= a.g[l + 1].tile0) ++l;
     const GemmArgs& g = a.g[l];
     int m, n;
-    const f32x4 d = gemm_tile(g, blk - g.tile0, red, m, n);
+    f32x4 d = gemm_tile(g, blk - g.tile0, red, m, n);
     if (m >= g.M) return;
     float* o = g.Cf + (size_t)m * g.N + n;
+    if (a.add)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (n + q < g.N) d[q] += o[q];
     if (n + 3 < g.N && ((uintptr_t)o & 15) == 0)
       *reinterpret_cast<f32x4*>(o) = d;
     else
@@ -285,7 +291,7 @@ __global__ void __launch_bounds__(256) mlp_dw_kernel(DwArgs a) {
       if (t < h) fr[t] += fr[t + h];
       __syncthreads();
     }
-    if (t < 16 && o < no) a.bg[l][o] = fr[t];
+    if (t < 16 && o < no) a.bg[l][o] = a.add ? a.bg[l][o] + fr[t] : fr[t];
     return;
   }
   float s = 0.f;
@@ -296,7 +302,7 @@ __global__ void __launch_bounds__(256) mlp_dw_kernel(DwArgs a) {
     if (t < h) fr[t] += fr[t + h];
     __syncthreads();
   }
-  if (t == 0) a.loss[0] = fr[0] / a.lscale;
+  if (t == 0) a.loss[0] = a.add ? a.loss[0] + fr[0] / a.lscale : fr[0] / a.lscale;
 }
 
 // X(m, i) = bf16((x[row][i] - mean[i]) / std[i]), row = idx ? idx[m] : m, and

@@ -97,6 +97,37 @@ def test_training_after_larger_and_smaller_batches(gpu_ctx):
     assert torch.equal(l0, l1) and torch.equal(g0[:npar], g1[:npar])
 
 
+def test_gradient_of_large_tiles(gpu_ctx):
+    """A batch whose hidden layers take 64 x 64 tiles, forward and backward."""
+    check_gradient(gpu_ctx, 64, 513, 2, 2, 4100)
+
+
+@pytest.mark.parametrize("indexed", [False, True])
+def test_gradient_in_parts(gpu_ctx, indexed):
+    """More rows than one pass takes (2^20): loss and gradient of all of them."""
+    check_gradient(gpu_ctx, 5, 17, 1, 1, (1 << 20) + 37, indexed)
+
+
+def check_gradient(gpu_ctx, nin, nh, nl, nodes, n, indexed=True):
+    import torch
+    p, nout, rng = make(gpu_ctx, nin, nh, nl, nodes)
+    x = rng.normal(0.3, 0.15, (n + 9, nin)).astype(np.float32)
+    t = rng.normal(0, 1, (n + 9, nout)).astype(np.float32)
+    idx = rng.permutation(n + 9)[:n].astype(np.int32) if indexed else np.arange(n)
+    loss, g = gpu_ctx.mlp_gradient_torch(*(torch.from_numpy(v if indexed else v[:n]).cuda() for v in (x, t)),
+                                         torch.from_numpy(idx).cuda() if indexed else None)
+    rl, rg = omlp.loss_and_grad(p, x[idx], t[idx], nin, nh, nl, nout, emulate=True)
+    tol = (nl + 1) * 2.0 ** -8
+    assert abs(float(loss.item()) - rl) <= 2 * tol * rl
+    g = g.cpu().numpy()
+    dims = [nin] + [nh] * nl + [nout]
+    o = 0
+    for i, k in zip(dims[:-1], dims[1:]):
+        for sl in (slice(o, o + i * k), slice(o + i * k, o + i * k + k)):
+            assert np.max(np.abs(g[sl] - rg[sl])) <= tol * max(np.abs(rg[sl]).max(), 1e-30)
+        o += i * k + k
+
+
 @pytest.mark.parametrize("nin", [100, 448])
 def test_outputs_in_the_place_of_inputs(gpu_ctx, nin):
     """The forward pass with its output at the start of its input gives the

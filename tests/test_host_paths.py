@@ -211,6 +211,28 @@ def case_inversion_that_was_not_set():
         assert (forward() == 0) == same and (len(d.seen) > n) == same
 
 
+def case_network_gradient_of_many_rows():
+    """The gradient of twenty million rows fits the card beside its data, as
+    sums over parts of the batch."""
+    import numpy as np
+    from firtez_dz_amd import lines
+    d = hostdouble.load()
+    ctx = d.gpu.Context(0)
+    ctx.configure(lines.fe6301_6302(), np.arange(64) * 15.0)
+    ctx.mlp_create(448, 512, 3, 4)
+    n = 20000000
+    x, t = d.malloc(4 * 448 * n), d.malloc(4 * 20 * n)
+    d.watch["mlp_input"] = lambda a: ("x", a.arg(0, ctypes.c_int).value, a.arg(2, ctypes.c_void_p).value)
+    d.watch["mlp_dw"] = lambda a: ("dw",)
+    ctx._check(ctx.lib.fz_mlp_gradient_dev(ctx.h, n, x, t, None, None, None, None), "gradient")
+    row = 0
+    for k in d.seen:
+        if k[0] == "x":
+            assert k[2] == x + 4 * 448 * row
+            row += k[1]
+    assert row == n and sum(k[0] == "dw" for k in d.seen) == sum(k[0] == "x" for k in d.seen)
+
+
 def case_network_outputs_over_its_inputs():
     """The forward pass of all layers in one launch is not taken where its
     outputs would overwrite inputs that other workgroups have yet to read."""
