@@ -1,6 +1,6 @@
 """The LSF contraction at the edges of its tiles (16 rows, 16 outputs in
 groups of 64, four taps a step) and on both sides of the widest region it
-takes, against the circular convolution of the same profiles in 64 bits.  Taps
+takes (904 wavelengths), against the circular convolution of the same profiles in 64 bits.  Taps
 of either sign without symmetry; a region without LSF stays as it is.
 """
 import numpy as np
@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n1,n2,ncol", [(1, 2, 1), (3, 4, 3), (15, 16, 4), (17, 63, 5), (64, 65, 9), (100, 31, 17),
-                                        (130, 1, 2), (860, 5, 5), (861, 4, 5), (1000, 3, 3)])
+                                        (130, 1, 2), (860, 5, 5), (861, 4, 5), (904, 2, 5), (905, 3, 5),
+                                        (1000, 3, 3)])
 @pytest.mark.parametrize("valid", [(1, 1), (0, 1), (1, 0)])
 def test_lsf_against_convolution(gpu_ctx, n1, n2, ncol, valid):
     import torch

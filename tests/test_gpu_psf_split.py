@@ -37,7 +37,7 @@ def run(ctx, psf, maps, adjoint):
 
 @pytest.mark.parametrize("sx,sy,nx,ny", [(15, 15, 40, 70), (17, 17, 17, 17), (17, 1, 33, 65), (31, 31, 31, 64),
                                          (31, 3, 65, 128), (33, 33, 33, 129), (33, 5, 96, 40), (43, 21, 50, 200),
-                                         (63, 63, 63, 63), (63, 1, 64, 300)])
+                                         (51, 7, 60, 100), (55, 3, 55, 257), (63, 63, 63, 63), (63, 1, 64, 300)])
 @pytest.mark.parametrize("adjoint", [False, True])
 def test_convolution_at_tile_edges(gpu_ctx, sx, sy, nx, ny, adjoint):
     rng = np.random.default_rng(sx * ny)
@@ -87,6 +87,24 @@ def test_inputs_outside_the_split(gpu_ctx, value):
         assert np.all(got[1][hit] == value)
     else:
         assert np.isnan(got[1][hit]).all()
+
+
+@pytest.mark.parametrize("sx", [17, 31, 33, 41, 55, 63])
+@pytest.mark.parametrize("ny", [40, 70, 130, 200])
+def test_tiles_outside_the_split(gpu_ctx, sx, ny):
+    """Tiles of inputs below the split's range beside ordinary ones, for every tap
+    count and tile height that is launched, last tiles partly and wholly past the map."""
+    rng = np.random.default_rng(sx + ny)
+    psf = rng.uniform(0.1, 1.0, (sx, 5))
+    nx = 100
+    maps = rng.normal(size=(2, nx, ny)).astype(np.float32).astype(np.float64)
+    maps[0] *= 1e-33
+    maps[1, 20, ny - 1] = 1e-33
+    maps = maps.astype(np.float32).astype(np.float64)
+    for adjoint in (False, True):
+        got = run(gpu_ctx, psf, maps, adjoint)
+        ref, mag = reference(psf, maps, adjoint)
+        assert np.all(np.abs(got - ref) <= (sx * 5 + 8) * 2.0 ** -24 * mag + 2.0 ** -149 * sx * 5)
 
 
 def test_taps_outside_the_split(gpu_ctx):
